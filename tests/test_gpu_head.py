@@ -659,3 +659,17 @@ def test_pad_to_response_window(dev, geometry):
     assert torch.equal(dv[0].grad.cpu(), ov[0].grad) and torch.equal(dv[1].grad.cpu(), ov[1].grad)
     only, = pad_to_response_window(indices.to(dev), B, S, Lr, vals[0].to(dev))
     assert torch.equal(only.cpu(), want[0].detach())
+
+
+@pytest.mark.parametrize("n,v", [(1, 152), (5, 700), (93, 66000), (257, 33001), (1100, 5000)])
+def test_merge_of_vocabulary_splits(dev, n, v):
+    """The partial softmax states of a token, however many vocabulary splits the launch had (1, 2, 256, 128 and 19
+    here, so 1 to 64 lanes of the merge share a token), combine to the fp32 ground truth."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    from oracle import masked as OM
+    hidden, weight, labels = (t.to(dev) for t in _make(n, 128, v, seed=n + v))
+    lp, ent, pi2 = K.linear_cross_entropy_with_sum_pi_squared(hidden, weight, labels, 0.8)
+    want_lp, want_ent = OH.head_fp32_ground_truth(hidden.float(), weight.float(), labels, 0.8)
+    want_pi2 = OM.sum_pi_squared_from_logits(hidden.float() @ weight.float().t() / 0.8)
+    assert (lp - want_lp).abs().max() <= ATOL and (ent - want_ent).abs().max() <= ATOL
+    assert torch.allclose(pi2, want_pi2, rtol=2e-3, atol=1e-9)

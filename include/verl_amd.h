@@ -165,8 +165,11 @@ int vamd_lce_forward_static(const void* hidden, const void* weight, const int64_
  *   reference's torch backend, which allocates and accumulates only the gradients whose inputs require them
  *   (verl/utils/experimental/torch_functional.py:150-156, :184-187); one of the two must be asked for.
  * vocab_chunk = 0 lets the library choose how many vocabulary columns of d_logits are staged
- * at a time (the workspace holds one [n_pad, vocab_chunk] bf16 panel plus an fp32 d_hidden
- * accumulator); pass the same value to the workspace query.
+ * at a time (the workspace holds one [n_pad, vocab_chunk] bf16 panel plus fp32 d_hidden
+ * accumulators); pass the same value to the workspace query.
+ *   vamd_lce_backward_subset is the same over some of the tokens of a call with planned_tokens (>= n_tokens) tokens,
+ *   gathered by the caller because the others have no upstream gradient: d_hidden's k range is cut as for the whole
+ *   call, so with one vocabulary chunk its rows are the bits the whole call would have given them.
  */
 #define VAMD_DW_STORE 0
 #define VAMD_DW_ADD_BF16 1
@@ -181,6 +184,14 @@ int vamd_lce_backward(const void* hidden, const void* weight, const int64_t* lab
                       const float* logits_cache, void* d_hidden, void* d_weight, int d_weight_mode,
                       float* d_weight_acc32, int64_t vocab_chunk, void* workspace, size_t workspace_bytes,
                       void* stream);
+size_t vamd_lce_backward_subset_workspace_bytes(int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size,
+                                                int64_t vocab, int64_t vocab_chunk);
+int vamd_lce_backward_subset(const void* hidden, const void* weight, const int64_t* labels, int64_t n_tokens,
+                             int64_t planned_tokens, int64_t hidden_size, int64_t vocab, float rcp_temperature,
+                             const float* lse, const float* mean_z, const float* d_logprobs, const float* d_entropy,
+                             float d_entropy_scalar, const float* logits_cache, void* d_hidden, void* d_weight,
+                             int d_weight_mode, float* d_weight_acc32, int64_t vocab_chunk, void* workspace,
+                             size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Per-token log-prob / entropy from materialised logits: the unfused definitions the actor uses when the

@@ -673,3 +673,27 @@ def test_merge_of_vocabulary_splits(dev, n, v):
     want_pi2 = OM.sum_pi_squared_from_logits(hidden.float() @ weight.float().t() / 0.8)
     assert (lp - want_lp).abs().max() <= ATOL and (ent - want_ent).abs().max() <= ATOL
     assert torch.allclose(pi2, want_pi2, rtol=2e-3, atol=1e-9)
+
+
+@pytest.mark.parametrize("n,h,v,chunk", [
+    (1, 128, 40000, 0),          # one d_hidden tile cut into as many pieces as pay
+    (300, 384, 30011, 0),        # 2 x 2 tiles, ragged in both directions, last piece shorter
+    (520, 256, 20000, 8192),     # several chunks, the last one narrower than a piece count would fill
+    (2500, 640, 9000, 0),        # whole tiles and pieces side by side with d_weight tiles
+])
+@pytest.mark.parametrize("need", [(True, True), (True, False)])
+def test_backward_shares_d_hidden_out_in_pieces(dev, n, h, v, chunk, need):
+    """d_hidden whose k range is cut into pieces, and d_weight shared out around them, against the fp32 ground truth
+    with the bound for d_logits staged in bf16."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    hidden, weight, labels = _make(n, h, v, seed=n + v, dist="normal")
+    g = torch.Generator().manual_seed(n)
+    g_lp = torch.randn(n, generator=g)
+    hd, wd, ld = hidden.to(dev), weight.to(dev), labels.to(dev)
+    _, _, lse, mz = K.efficient_entropy_forward(hd, wd, ld, 0, 0.9)
+    dh, dw = K.efficient_entropy_backward(g_lp.to(dev), None, hd, wd, ld, lse, mz, 0, 0.9, vocab_chunk=chunk,
+                                          need_d_hidden=need[0], need_d_weight=need[1])
+    _, _, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)
+    _close_bf16(dh, want_dh, "d_hidden", e_dh)
+    if need[1]:
+        _close_bf16(dw, want_dw, "d_weight", e_dw)

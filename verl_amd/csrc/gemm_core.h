@@ -345,7 +345,8 @@ static_assert(kLoads == 4, "the s_waitcnt vmcnt(4 / 6) of slab_iter counts the t
 // Persistent, software-pipelined walk over a list of output tiles.
 //
 //   Sched : int count();  void tile(int i, int& r0, int& c0);
-//   Epi   : void operator()(Accum& acc, int r0, int c0);   (registers + global memory only, or LDS
+//           int slab0(int i), slabs(int i): first slab and number of slabs (> 0) of tile i's k range
+//   Epi   : void operator()(Accum& acc, int tile, int r0, int c0);   (registers + global memory only, or LDS
 //           beyond the first kLdsBytes)
 //           void prefetch(int tile, int r0, int c0);  called by every wavefront before the first slab of tile
 //           `tile` is multiplied: memory -> LDS transfers issued here have landed, and are visible to the
@@ -362,8 +363,7 @@ static_assert(kLoads == 4, "the s_waitcnt vmcnt(4 / 6) of slab_iter counts the t
 // calling wavefront has landed; the caller must pass a workgroup barrier before it reuses the
 // first kLdsBytes of LDS.
 template <bool R_KMAJOR, bool C_KMAJOR, class Sched, class Epi>
-__device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, int k_slabs, Sched& sched, Epi& epi,
-                                          char* lds) {
+__device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, Sched& sched, Epi& epi, char* lds) {
   const int ntiles = sched.count();
   if (ntiles <= 0) return;
   const LanePos pos = lane_pos();
@@ -376,16 +376,17 @@ __device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, in
   fr.init(pos.wr * kNB, kNB);
   fc.init(pos.wc * kMB, kMB);
 
-  // fetch cursor: (t2, k2) names the slab whose sources are (src_r, src_c)
-  int t2 = 0, k2 = 0, r0, c0;
+  // fetch cursor: (t2, k2) names the slab whose sources are (src_r, src_c), k2_end is the end of tile t2's k range
+  int t2 = 0, k2 = sched.slab0(0), k2_end = k2 + sched.slabs(0), r0, c0;
   sched.tile(0, r0, c0);
   u32x4 rs_r = tile_rsrc<R_KMAJOR>(R, r0), rs_c = tile_rsrc<C_KMAJOR>(C, c0);
-  SlabSrc src_r{rs_r, 0u}, src_c{rs_c, 0u};
+  SlabSrc src_r{rs_r, slab_soff<R_KMAJOR>(R, k2 * kBK)}, src_c{rs_c, slab_soff<C_KMAJOR>(C, k2 * kBK)};
   auto advance = [&]() {
-    if (t2 == ntiles - 1 && k2 == k_slabs - 1) return;
-    if (++k2 == k_slabs) {
-      k2 = 0;
+    if (t2 == ntiles - 1 && k2 == k2_end - 1) return;
+    if (++k2 == k2_end) {
       ++t2;
+      k2 = sched.slab0(t2);
+      k2_end = k2 + sched.slabs(t2);
       int tr, tc;
       sched.tile(t2, tr, tc);
       rs_r = tile_rsrc<R_KMAJOR>(R, tr);
@@ -422,14 +423,15 @@ __device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, in
     accum_zero(acc);
     sched.tile(tile, r0, c0);
     if (tile > 0) epi.prefetch(tile, r0, c0);
-    for (int kt = 0; kt < k_slabs; ++kt) {
+    const int slabs = sched.slabs(tile);
+    for (int kt = 0; kt < slabs; ++kt) {
       char* cur = lds + stage * 2 * kSlabBytes;
       const char* nxt = lds + (stage ^ 1) * 2 * kSlabBytes;
       slab_iter<R_KMAJOR, C_KMAJOR>(dr, dc, src_r, src_c, cur, nxt, fr, fc, f, acc);
       advance();
       stage ^= 1;
     }
-    epi(acc, r0, c0);
+    epi(acc, tile, r0, c0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
@@ -441,14 +443,9 @@ __device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, in
 // owns a contiguous run of the tile sequence, then the sequence walks r fastest inside bands
 // of 8 r-tiles, so the 32 workgroups resident on one XCD cover an 8 x 4 patch and share their
 // R / C slabs through that XCD's L2.
-struct GroupedSched {
-  int r_tiles, c_tiles, nwg, wg;
-  __device__ __forceinline__ int count() const {
-    const int total = r_tiles * c_tiles;
-    return (total - wg + nwg - 1) / nwg;
-  }
-  __device__ __forceinline__ void tile(int i, int& r0, int& c0) const {
-    const int q = i * nwg + wg;
+struct TileGrid {
+  int r_tiles, c_tiles;
+  __device__ __forceinline__ void at(int q, int& r0, int& c0) const {
     const int band = 8 * c_tiles;
     const int b = q / band;
     const int first_r = b * 8;
@@ -457,6 +454,56 @@ struct GroupedSched {
     r0 = (first_r + w % rows) * kTile;
     c0 = (w / rows) * kTile;
   }
+};
+
+struct GroupedSched {
+  TileGrid grid;
+  int k_slabs, nwg, wg;
+  __device__ __forceinline__ int count() const {
+    const int total = grid.r_tiles * grid.c_tiles;
+    return (total - wg + nwg - 1) / nwg;
+  }
+  __device__ __forceinline__ void tile(int i, int& r0, int& c0) const { grid.at(i * nwg + wg, r0, c0); }
+  __device__ __forceinline__ int slab0(int) const { return 0; }
+  __device__ __forceinline__ int slabs(int) const { return k_slabs; }
+};
+
+// Two products in one launch.  Every workgroup first walks units of product 1, then tiles of product 2:
+//   product 1: its output tiles, each cut into `splits` pieces of at most `split_slabs` slabs along k; unit p is piece
+//              p / tiles of tile p % tiles, so that the workgroups of an XCD work on the same k range of neighbouring
+//              tiles; workgroup w takes units w, w + nwg, ...
+//   product 2: whole tiles.  The first `extra` workgroups have one unit of product 1 more than the others and start
+//              `late` rounds of product-2 tiles later; until then a round is the other nwg - extra workgroups.
+struct SplitKSched {
+  TileGrid grid;
+  int splits, split_slabs, k_slabs, nwg, wg;
+  __device__ __forceinline__ int tiles() const { return grid.r_tiles * grid.c_tiles; }
+  __device__ __forceinline__ int count() const { return (tiles() * splits - wg + nwg - 1) / nwg; }
+  __device__ __forceinline__ int piece(int i) const { return (i * nwg + wg) / tiles(); }
+  __device__ __forceinline__ void tile(int i, int& r0, int& c0) const { grid.at((i * nwg + wg) % tiles(), r0, c0); }
+  __device__ __forceinline__ int slab0(int i) const { return piece(i) * split_slabs; }
+  __device__ __forceinline__ int slabs(int i) const {
+    const int left = k_slabs - slab0(i);
+    return left < split_slabs ? left : split_slabs;
+  }
+};
+struct LateStartSched {
+  TileGrid grid;
+  int k_slabs, nwg, wg, extra, late;
+  __device__ __forceinline__ int index(int i) const {
+    const int early = nwg - extra;  // workgroups of a round before the late ones join
+    if (wg < extra) return late * early + i * nwg + wg;
+    return i < late ? i * early + (wg - extra) : late * early + (i - late) * nwg + wg;
+  }
+  __device__ __forceinline__ int count() const {
+    const int total = grid.r_tiles * grid.c_tiles, early = nwg - extra, before = late * early;
+    if (wg >= extra && total <= before) return (total - (wg - extra) + early - 1) / early;
+    const int joint = total > before ? (total - before - wg + nwg - 1) / nwg : 0;
+    return wg < extra ? joint : late + joint;
+  }
+  __device__ __forceinline__ void tile(int i, int& r0, int& c0) const { grid.at(index(i), r0, c0); }
+  __device__ __forceinline__ int slab0(int) const { return 0; }
+  __device__ __forceinline__ int slabs(int) const { return k_slabs; }
 };
 
 // Regroup a hardware workgroup id so that XCD x owns ids [x*n/8, (x+1)*n/8).

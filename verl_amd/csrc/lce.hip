@@ -84,12 +84,14 @@ struct FwdArgs {
 };
 
 struct SplitSched {
-  int r0_, vt_begin, vt_count;
+  int r0_, vt_begin, vt_count, k_slabs;
   __device__ __forceinline__ int count() const { return vt_count; }
   __device__ __forceinline__ void tile(int i, int& r0, int& c0) const {
     r0 = r0_;
     c0 = (vt_begin + i) * kTile;
   }
+  __device__ __forceinline__ int slab0(int) const { return 0; }
+  __device__ __forceinline__ int slabs(int) const { return k_slabs; }
 };
 
 // The epilogues that write matrices hand the accumulators through a 4 KB LDS patch private to the
@@ -161,7 +163,7 @@ struct FwdEpi {
   int n_tokens;
 
   __device__ __forceinline__ void prefetch(int, int, int) {}
-  __device__ __forceinline__ void operator()(Accum& acc, int /*r0*/, int c0) {
+  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int /*r0*/, int c0) {
     const bool ragged = c0 + kTile > vocab;
     if constexpr (CACHE) {
 #pragma unroll
@@ -284,6 +286,7 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   const int sp = w / rows;
 
   SplitSched sched;
+  sched.k_slabs = a.k_slabs;
   sched.r0_ = tn * kTile;
   sched.vt_begin = (int)(((int64_t)sp * a.voc_tiles) / a.splits);
   sched.vt_count = (int)(((int64_t)(sp + 1) * a.voc_tiles) / a.splits) - sched.vt_begin;
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   epi.tok0 = sched.r0_ + epi.p.wr * (kNB * kBlk);
   epi.n_tokens = a.n_tokens;
 
-  run_tiles<false, false>(a.hidden, a.weight, a.k_slabs, sched, epi, lds);
+  run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 
   float zl[kNB];
 #pragma unroll
@@ -584,7 +587,7 @@ struct RecomputeEpi {
     }
   }
 
-  __device__ __forceinline__ void operator()(Accum& acc, int r0, int c0) {
+  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int r0, int c0) {
     const RecomputeArgs& A = *a;
     // read through LDS-typed pointers: as generic pointers some of these became flat loads, whose wait also
     // waits out every slab transfer in flight
@@ -626,13 +629,13 @@ struct RecomputeEpi {
 __global__ __launch_bounds__(kThreads) void lce_recompute_kernel(RecomputeArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   GroupedSched sched;
-  sched.r_tiles = a.tok_tiles;
-  sched.c_tiles = a.chunk_tiles;
+  sched.grid = TileGrid{a.tok_tiles, a.chunk_tiles};
+  sched.k_slabs = a.k_slabs;
   sched.nwg = gridDim.x;
   sched.wg = xcd_regroup(blockIdx.x, gridDim.x);
   RecomputeEpi epi;
   epi.init(lds + kLdsBytes, lane_pos(), &a);
-  run_tiles<false, false>(a.hidden, a.weight, a.k_slabs, sched, epi, lds);
+  run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 }
 
 // d_logits panel of one vocabulary chunk from cached logits: the same arithmetic as RecomputeEpi,
@@ -686,6 +689,8 @@ enum : int { kStoreF32 = 0, kAddF32 = 1, kFinalBf16 = 2, kFinalBf16AddPrev = 3 }
 struct GemmOutArgs {
   Operand R, C;
   int k_slabs, r_tiles, c_tiles;
+  int splits, split_slabs;  // d_hidden: pieces along k, each summed into its own fp32 accumulator when there are several
+  int extra, late;          // d_weight: LateStartSched
   int r_valid, c_valid;  // rows / cols of the output that exist
   int mode;              // d_hidden: one of the enum above; d_weight: a VAMD_DW_* value
   float* acc32;          // fp32 accumulator [r_valid][ld_out]
@@ -696,10 +701,12 @@ struct GemmOutArgs {
 struct DHiddenEpi {
   LanePos p;
   const GemmOutArgs* a;
+  SplitKSched sched;
   BlockExchange ex;
   __device__ __forceinline__ void prefetch(int, int, int) {}
-  __device__ __forceinline__ void operator()(Accum& acc, int r0, int c0) {
+  __device__ __forceinline__ void operator()(Accum& acc, int tile, int r0, int c0) {
     const GemmOutArgs& A = *a;
+    float* const acc32 = A.acc32 + (int64_t)sched.piece(tile) * A.r_valid * A.ld_out;
     const bool read_prev = A.mode == kAddF32 || A.mode == kFinalBf16AddPrev;
     const bool to_f32 = A.mode == kStoreF32 || A.mode == kAddF32;
 #pragma unroll
@@ -716,7 +723,7 @@ struct DHiddenEpi {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             prev[i] = (row0 + 8 * i < A.r_valid)
-                          ? *reinterpret_cast<const f32x4*>(A.acc32 + (int64_t)(row0 + 8 * i) * A.ld_out + col)
+                          ? *reinterpret_cast<const f32x4*>(acc32 + (int64_t)(row0 + 8 * i) * A.ld_out + col)
                           : f32x4{0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
@@ -726,7 +733,7 @@ struct DHiddenEpi {
           f32x4 x = v[i];
           if (read_prev) x = x + prev[i];
           const int64_t off = (int64_t)row * A.ld_out + col;
-          if (to_f32) *reinterpret_cast<f32x4*>(A.acc32 + off) = x;
+          if (to_f32) *reinterpret_cast<f32x4*>(acc32 + off) = x;
           else *reinterpret_cast<u32x2*>(A.out + off) = pack_bf16x4(x[0], x[1], x[2], x[3]);
         }
       }
@@ -738,7 +745,7 @@ struct DWeightEpi {
   const GemmOutArgs* a;
   BlockExchange ex;
   __device__ __forceinline__ void prefetch(int, int, int) {}
-  __device__ __forceinline__ void operator()(Accum& acc, int r0, int c0) {
+  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int r0, int c0) {
     const GemmOutArgs& A = *a;
 #pragma unroll
     for (int nb = 0; nb < kNB2; ++nb)
@@ -774,42 +781,42 @@ struct DWeightEpi {
   }
 };
 
-// Both gradient GEMMs of one vocabulary chunk in a single launch: a workgroup first walks its
-// share of the d_hidden tiles, then its share of the d_weight tiles.  The second walk starts at
-// the workgroup after the last one that received an extra tile in the first, so the combined
-// tile count, not each GEMM's, decides how full the last round is (896 + 896 tiles on 256 CUs:
-// 7 full rounds instead of 2 x 3.5).
+// Both gradient GEMMs of one vocabulary chunk in a single launch: a workgroup first walks its share of the d_hidden
+// units, then its share of the d_weight tiles, shared out by plan_gradients() so that all workgroups finish together.
 __global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, GemmOutArgs gw) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int nwg = gridDim.x;
   const int wg = xcd_regroup(blockIdx.x, nwg);
   const LanePos pos = lane_pos();
-  {
-    GroupedSched sched;
-    sched.r_tiles = gh.r_tiles;
-    sched.c_tiles = gh.c_tiles;
-    sched.nwg = nwg;
-    sched.wg = wg;
+  if (gh.r_tiles > 0) {
+    SplitKSched sched{TileGrid{gh.r_tiles, gh.c_tiles}, gh.splits, gh.split_slabs, gh.k_slabs, nwg, wg};
     DHiddenEpi epi;
     epi.p = pos;
     epi.a = &gh;
+    epi.sched = sched;
     epi.ex.init(lds + kLdsBytes, pos);
-    run_tiles<false, true>(gh.R, gh.C, gh.k_slabs, sched, epi, lds);
+    run_tiles<false, true>(gh.R, gh.C, sched, epi, lds);
   }
   __syncthreads();
   {
-    const int rem = (gh.r_tiles * gh.c_tiles) % nwg;
-    GroupedSched sched;
-    sched.r_tiles = gw.r_tiles;
-    sched.c_tiles = gw.c_tiles;
-    sched.nwg = nwg;
-    sched.wg = (wg - rem + nwg) % nwg;
+    LateStartSched sched{TileGrid{gw.r_tiles, gw.c_tiles}, gw.k_slabs, nwg, wg, gw.extra, gw.late};
     DWeightEpi epi;
     epi.p = pos;
     epi.a = &gw;
     epi.ex.init(lds + kLdsBytes, pos);
-    run_tiles<true, true>(gw.R, gw.C, gw.k_slabs, sched, epi, lds);
+    run_tiles<true, true>(gw.R, gw.C, sched, epi, lds);
   }
+}
+
+// d_hidden = sum of the pieces' fp32 accumulators, rounded once.
+__global__ __launch_bounds__(256) void lce_dhidden_sum_kernel(const float* acc32, int pieces, int64_t elements,
+                                                              uint16_t* out) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= elements) return;
+  f32x4 s = *reinterpret_cast<const f32x4*>(acc32 + i);
+#pragma unroll 4
+  for (int k = 1; k < pieces; ++k) s = s + *reinterpret_cast<const f32x4*>(acc32 + (int64_t)k * elements + i);
+  *reinterpret_cast<u32x2*>(out + i) = pack_bf16x4(s[0], s[1], s[2], s[3]);
 }
 
 // =============================================================================================
@@ -893,6 +900,60 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
   if (cv < kTile) cv = kTile;
   if (cv > v_pad) cv = v_pad;
   return cv;
+}
+
+// How the gradient GEMMs of one vocabulary chunk are shared out over the workgroups (one per CU).
+struct GradPlan {
+  int splits = 1, split_slabs = 1;  // pieces of a d_hidden tile's k range
+  int extra = 0, late = 0;          // d_weight: LateStartSched
+};
+
+// d_hidden has few tiles with a long k range (the chunk's vocabulary), d_weight many tiles with a short one (the tokens),
+// and both sum up to the same number of slabs.  Whole d_hidden tiles only balance when there are several per CU: 777
+// tokens x 896 have 16 tiles of 2374 slabs, which kept 16 CUs busy while 240 waited (2983 us; cut into 15 pieces 420 us),
+// 7339 x 3584 have 406 on 256 CUs (87 % of the launch busy).  So a tile's k range is cut into pieces of equal length,
+// each summed in fp32 into an accumulator of its own, and the d_weight tiles are shared out so that the workgroups
+// with a piece more get correspondingly fewer tiles.  The number of pieces is the one whose slowest workgroup is
+// quickest, counting in slabs (1.4 us each): a tile's epilogue about 2, and the accumulators' way to memory and back.
+constexpr int kEpilogueSlabs = 2, kMaxSplits = 64, kMinPieceSlabs = 32;
+constexpr int64_t kMaxPieceBytes = 256ll << 20;  // bound on the pieces' accumulators
+static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t cols, bool want_dh, bool want_dw,
+                               int cus, int fixed_pieces = 0) {
+  const int64_t h_tiles = ceil_div(hidden_size, kTile);
+  const int64_t th = want_dh ? ceil_div(n_tokens, kTile) * h_tiles : 0, kh = ceil_div(cols, kBK);
+  const int64_t tw = want_dw ? ceil_div(cols, kTile) * h_tiles : 0, cost_w = ceil_div(n_tokens, kBK) + kEpilogueSlabs;
+  const int64_t piece_bytes = n_tokens * hidden_size * 4;
+  GradPlan best;
+  best.split_slabs = (int)kh;
+  double best_cost = 0;
+  bool first = true;
+  for (int64_t want = fixed_pieces ? fixed_pieces : 1; want <= (fixed_pieces ? fixed_pieces : want_dh ? kMaxSplits : 1);
+       ++want) {
+    const int64_t len = ceil_div(kh, want), pieces = ceil_div(kh, len);
+    if (pieces != want && !fixed_pieces) continue;  // the same cut as for a smaller count
+    if (want > 1 && len < kMinPieceSlabs && !fixed_pieces) break;  // nothing to gain that pays for the summing launch
+    if (pieces > 1 && pieces * piece_bytes > kMaxPieceBytes && !fixed_pieces) break;
+    const int64_t units = th * pieces, cost_h = len + kEpilogueSlabs;
+    const int64_t extra = units % cus, few = units / cus * cost_h, many = few + (extra ? cost_h : 0);
+    // least time in which all d_weight tiles fit behind the d_hidden units
+    int64_t lo = many, hi = many + (ceil_div(tw, cus) + 1) * cost_w;
+    while (lo < hi) {
+      const int64_t t = (lo + hi) / 2;
+      const int64_t fit = extra * ((t - many) / cost_w) + (cus - extra) * ((t - few) / cost_w);
+      if (fit >= tw) hi = t;
+      else lo = t + 1;
+    }
+    const double cost = (double)lo + (pieces > 1 ? 4.0 + (double)(2 * pieces * piece_bytes) / 7.0e6 : 0.0);  // a launch, 5 TB/s
+    if (first || cost < best_cost) {
+      first = false;
+      best_cost = cost;
+      best.splits = (int)pieces;
+      best.split_slabs = (int)len;
+      best.extra = (int)extra;
+      best.late = (int)((lo - few) / cost_w - (lo - many) / cost_w);
+    }
+  }
+  return best;
 }
 
 }  // namespace vamd
@@ -1079,14 +1140,30 @@ extern "C" int vamd_lce_forward_static(const void* hidden, const void* weight, c
                             lse, mean_z, nullptr, sum_pi_squared, ws, stream, VAMD_LCE_STATIC_MAX_TOKENS);
 }
 
-extern "C" size_t vamd_lce_backward_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab,
-                                                    int64_t vocab_chunk) {
+namespace vamd {
+// Pieces of a d_hidden tile's k range.  Decided for a call with both gradients over `planned_tokens` tokens, whatever
+// part of that is asked for, so that d_hidden is the same bits in all of them; the first (widest) vocabulary chunk
+// decides for all chunks.
+static int d_hidden_pieces(int64_t planned_tokens, int64_t hidden_size, int64_t first_cols) {
+  return plan_gradients(planned_tokens, hidden_size, first_cols, true, true, device_cu_count()).splits;
+}
+}  // namespace vamd
+
+extern "C" size_t vamd_lce_backward_subset_workspace_bytes(int64_t n_tokens, int64_t planned_tokens,
+                                                           int64_t hidden_size, int64_t vocab, int64_t vocab_chunk) {
   if (n_tokens <= 0 || vocab <= 0 || hidden_size <= 0) return 0;
   const int64_t n_pad = ceil_div(n_tokens, kTile) * kTile;
   const int64_t cv = default_vocab_chunk(n_tokens, hidden_size, vocab, vocab_chunk);
   size_t bytes = align_up((size_t)n_pad * dz_pitch(cv) * 2, 256);
-  if (cv < ceil_div(vocab, kTile) * kTile) bytes += align_up((size_t)n_tokens * hidden_size * 4, 256);
+  const int pieces = d_hidden_pieces(planned_tokens, hidden_size, cv < vocab ? cv : vocab);
+  if (pieces > 1 || cv < ceil_div(vocab, kTile) * kTile)
+    bytes += align_up((size_t)pieces * n_tokens * hidden_size * 4, 256);
   return bytes;
+}
+
+extern "C" size_t vamd_lce_backward_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab,
+                                                    int64_t vocab_chunk) {
+  return vamd_lce_backward_subset_workspace_bytes(n_tokens, n_tokens, hidden_size, vocab, vocab_chunk);
 }
 
 extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const int64_t* labels, int64_t n_tokens,
@@ -1095,6 +1172,18 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
                                  float d_entropy_scalar, const float* logits_cache, void* d_hidden, void* d_weight,
                                  int d_weight_mode, float* d_weight_acc32, int64_t vocab_chunk, void* workspace,
                                  size_t workspace_bytes, void* stream) {
+  return vamd_lce_backward_subset(hidden, weight, labels, n_tokens, n_tokens, hidden_size, vocab, rcp_temperature, lse,
+                                  mean_z, d_logprobs, d_entropy, d_entropy_scalar, logits_cache, d_hidden, d_weight,
+                                  d_weight_mode, d_weight_acc32, vocab_chunk, workspace, workspace_bytes, stream);
+}
+
+extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, const int64_t* labels,
+                                        int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size, int64_t vocab,
+                                        float rcp_temperature, const float* lse, const float* mean_z,
+                                        const float* d_logprobs, const float* d_entropy, float d_entropy_scalar,
+                                        const float* logits_cache, void* d_hidden, void* d_weight, int d_weight_mode,
+                                        float* d_weight_acc32, int64_t vocab_chunk, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
   int st = check_head_shapes(n_tokens, hidden_size, vocab, logits_cache);
   if (st != VAMD_OK) return st;
   VAMD_REQUIRE(hidden && weight && labels && lse && mean_z, "lce_backward: null pointer");
@@ -1117,7 +1206,10 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
                  "lce_backward: hidden states (%lld x %lld) or the d_logits panel exceed 4 GiB; split the tokens into "
                  "chunks and accumulate d_weight", (long long)n_tokens, (long long)hidden_size);
   }
-  const size_t need = vamd_lce_backward_workspace_bytes(n_tokens, hidden_size, vocab, vocab_chunk);
+  VAMD_REQUIRE(planned_tokens >= n_tokens, "lce_backward: %lld tokens are no part of %lld", (long long)n_tokens,
+               (long long)planned_tokens);
+  const size_t need =
+      vamd_lce_backward_subset_workspace_bytes(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk);
   if (!workspace || workspace_bytes < need) {
     set_error("lce_backward: workspace %zu bytes, need %zu", workspace_bytes, need);
     return VAMD_EWORKSPACE;
@@ -1133,7 +1225,10 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
   Carver carve(workspace);
   const int64_t pitch = dz_pitch(cv);
   uint16_t* dz = carve.take<uint16_t>((size_t)n_pad * pitch);
-  float* acc32 = (n_chunks > 1 && d_hidden) ? carve.take<float>((size_t)n_tokens * hidden_size) : nullptr;
+  // a narrower last chunk may fill fewer pieces than the first
+  const int pieces = d_hidden ? d_hidden_pieces(planned_tokens, hidden_size, cv < vocab ? cv : vocab) : 1;
+  float* acc32 = (d_hidden && (n_chunks > 1 || pieces > 1)) ? carve.take<float>((size_t)pieces * n_tokens * hidden_size)
+                                                            : nullptr;
   const uint16_t* hid = static_cast<const uint16_t*>(hidden);
   const uint16_t* wgt = static_cast<const uint16_t*>(weight);
   const int h_tiles = (int)ceil_div(hidden_size, kTile);
@@ -1206,9 +1301,13 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
     gh.c_tiles = h_tiles;
     gh.r_valid = (int)n_tokens;
     gh.c_valid = (int)hidden_size;
-    if (n_chunks == 1) gh.mode = kFinalBf16;
+    const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, d_hidden != nullptr, want_dw, cus, pieces);
+    gh.splits = plan.splits;
+    gh.split_slabs = plan.split_slabs;
+    gh.extra = gh.late = 0;
+    if (n_chunks == 1 && pieces == 1) gh.mode = kFinalBf16;
     else if (ci == 0) gh.mode = kStoreF32;
-    else if (ci == n_chunks - 1) gh.mode = kFinalBf16AddPrev;
+    else if (ci == n_chunks - 1 && pieces == 1) gh.mode = kFinalBf16AddPrev;
     else gh.mode = kAddF32;
     gh.acc32 = acc32;
     gh.out = static_cast<uint16_t*>(d_hidden);
@@ -1219,6 +1318,10 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
     gw.C = Operand{hid, hidden_size, (int)hidden_size, (int)n_tokens};
     gw.k_slabs = (int)ceil_div(n_tokens, kBK);
     gw.r_tiles = want_dw ? chunk_tiles : 0;
+    gw.splits = 1;
+    gw.split_slabs = gw.k_slabs;
+    gw.extra = plan.extra;
+    gw.late = plan.late;
     gw.c_tiles = h_tiles;
     gw.r_valid = (int)cols;
     gw.c_valid = (int)hidden_size;
@@ -1227,11 +1330,15 @@ extern "C" int vamd_lce_backward(const void* hidden, const void* weight, const i
     gw.out = d_weight ? static_cast<uint16_t*>(d_weight) + c0 * hidden_size : nullptr;
     gw.ld_out = hidden_size;
     {
-      const int tiles = gh.r_tiles * gh.c_tiles + gw.r_tiles * gw.c_tiles;
-      const int grid = tiles < cus ? tiles : cus;
       ScopedTiming tm(kTagDGrad, s);
-      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(grid), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw);
+      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(cus), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw);
     }
+    VAMD_LAUNCH_CHECK();
+  }
+  if (pieces > 1) {
+    const int64_t elements = n_tokens * hidden_size;
+    hipLaunchKernelGGL(lce_dhidden_sum_kernel, dim3((unsigned)ceil_div(elements, 1024)), dim3(256), 0, s, acc32, pieces,
+                       elements, static_cast<uint16_t*>(d_hidden));
     VAMD_LAUNCH_CHECK();
   }
   return VAMD_OK;

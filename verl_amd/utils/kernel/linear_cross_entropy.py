@@ -105,7 +105,7 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
                                d_weight_out: torch.Tensor | None = None, vocab_chunk: int = 0,
                                logits_cache: torch.Tensor | None = None,
                                d_weight_acc32: torch.Tensor | None = None, acc32_step: str | None = None,
-                               need_d_hidden: bool = True, need_d_weight: bool = True):
+                               need_d_hidden: bool = True, need_d_weight: bool = True, planned_tokens: int | None = None):
     """Host side of the backward kernels (reference kernels.py:1512-1723).
 
     ``dlogprobs`` / ``dentropy`` may be ``None`` (no contribution).  ``d_entropy_scalar`` adds a
@@ -120,6 +120,7 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
     detached hidden states): its gradient GEMM is not run and ``None`` is returned in its place, as the reference's
     torch backend allocates and accumulates only the gradients its inputs require
     (verl/utils/experimental/torch_functional.py:150-156, :184-187).
+    ``planned_tokens``: set when the arguments are some of the tokens of a larger call, to that call's token count.
     Returns ``(d_hidden, d_weight)`` in ``hidden.dtype``; ``d_weight`` is ``None`` for the "first" and
     "middle" steps of an fp32 accumulation.
     """
@@ -168,13 +169,14 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
         d_weight = d_weight_out if d_weight_out is not None else torch.empty_like(weight)
     if d_weight is not None:
         assert d_weight.shape == weight.shape and d_weight.dtype == weight.dtype and d_weight.is_contiguous()
-    ws = _cabi.workspace(L.vamd_lce_backward_workspace_bytes(n, h, v, vocab_chunk), dev)
+    planned = n if planned_tokens is None else planned_tokens
+    ws = _cabi.workspace(L.vamd_lce_backward_subset_workspace_bytes(n, planned, h, v, vocab_chunk), dev)
     with _cabi.device_guard(dev):
-        _cabi.check(L.vamd_lce_backward(hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(), n, h, v,
-                                        1.0 / temperature, lse.data_ptr(), mean_z.data_ptr(), _cabi.ptr(dlogprobs),
-                                        _cabi.ptr(dentropy), float(d_entropy_scalar), _cabi.ptr(logits_cache),
-                                        _cabi.ptr(d_hidden), _cabi.ptr(d_weight), mode, _cabi.ptr(d_weight_acc32),
-                                        int(vocab_chunk), ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
+        _cabi.check(L.vamd_lce_backward_subset(
+            hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(), n, planned, h, v, 1.0 / temperature,
+            lse.data_ptr(), mean_z.data_ptr(), _cabi.ptr(dlogprobs), _cabi.ptr(dentropy), float(d_entropy_scalar),
+            _cabi.ptr(logits_cache), _cabi.ptr(d_hidden), _cabi.ptr(d_weight), mode, _cabi.ptr(d_weight_acc32),
+            int(vocab_chunk), ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
     return d_hidden, d_weight
 
 
@@ -227,7 +229,8 @@ def backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels
     take = lambda t: None if t is None else t.index_select(0, idx)
     dh, d_weight = efficient_entropy_backward(take(dlogprobs), take(dentropy), take(hidden), weight, take(labels),
                                               take(lse), take(mean_z), 0, temperature,
-                                              need_d_hidden=need_d_hidden, need_d_weight=need_d_weight)
+                                              need_d_hidden=need_d_hidden, need_d_weight=need_d_weight,
+                                              planned_tokens=hidden.shape[0])
     if need_d_hidden:
         d_hidden.index_copy_(0, idx, dh)
     return d_hidden, d_weight

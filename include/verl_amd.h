@@ -130,7 +130,7 @@ int vamd_lce_forward(const void* hidden, const void* weight, const int64_t* labe
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference.  Same arguments, arithmetic and results as vamd_lce_forward without a logits cache; the
  * softmax partials of the (token tile, vocabulary split) workgroups go to a buffer built into the library
- * (VAMD_LCE_STATIC_MAX_TOKENS * 20 + 512 bytes of device memory, held by every GPU the library is
+ * (VAMD_LCE_STATIC_MAX_TOKENS * 105 + 512 bytes of device memory, held by every GPU the library is
  * used on until the process ends).  n_tokens above VAMD_LCE_STATIC_MAX_TOKENS is refused with VAMD_EINVAL.
  * The call allocates nothing and records no memset.  All calls on one GPU share the one buffer: calls on
  * different streams of the same GPU that may overlap race on it; calls ordered on one stream do not.

@@ -697,3 +697,25 @@ def test_backward_shares_d_hidden_out_in_pieces(dev, n, h, v, chunk, need):
     _close_bf16(dh, want_dh, "d_hidden", e_dh)
     if need[1]:
         _close_bf16(dw, want_dw, "d_weight", e_dw)
+
+
+@pytest.mark.parametrize("n,v", [
+    (10999, 33001),   # 43 token tiles: bands of 8, 2 and 1, shares that cross from band to band
+    (32900, 1000),    # 129 token tiles, 4 vocabulary tiles: several bands per share, fewer columns than workgroups
+    (2100, 151936),   # 9 token tiles: one full band and a single tile
+])
+def test_forward_in_bands_of_token_tiles(dev, n, v):
+    """Token counts whose tiles do not divide the chip go through the band schedule of the forward pass, where a
+    workgroup may hand over its softmax state in the middle of its tiles."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    from oracle import masked as OM
+    hidden, weight, labels = (t.to(dev) for t in _make(n, 128, v, seed=n + v))
+    lp, ent, pi2 = K.linear_cross_entropy_with_sum_pi_squared(hidden, weight, labels, 0.8)
+    lp0, ent0, _, _ = K.efficient_entropy_forward(hidden, weight, labels, 0, 0.8)
+    assert torch.equal(lp, lp0) and torch.equal(ent, ent0)
+    for lo in range(0, n, 4096):
+        h, y = hidden[lo:lo + 4096].float(), labels[lo:lo + 4096]
+        want_lp, want_ent = OH.head_fp32_ground_truth(h, weight.float(), y, 0.8)
+        assert (lp[lo:lo + 4096] - want_lp).abs().max() <= ATOL and (ent[lo:lo + 4096] - want_ent).abs().max() <= ATOL
+        want_pi2 = OM.sum_pi_squared_from_logits(h @ weight.float().t() / 0.8)
+        assert torch.allclose(pi2[lo:lo + 4096], want_pi2, rtol=2e-3, atol=1e-9)

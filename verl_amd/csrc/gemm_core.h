@@ -419,10 +419,10 @@ __device__ __forceinline__ void run_tiles(const Operand& R, const Operand& C, Sc
 
   int stage = 0;
   for (int tile = 0; tile < ntiles; ++tile) {
-    Accum acc;
-    accum_zero(acc);
     sched.tile(tile, r0, c0);
     if (tile > 0) epi.prefetch(tile, r0, c0);
+    Accum acc;
+    accum_zero(acc);
     const int slabs = sched.slabs(tile);
     for (int kt = 0; kt < slabs; ++kt) {
       char* cur = lds + stage * 2 * kSlabBytes;

@@ -70,25 +70,159 @@ struct ScopedTiming {
 // =============================================================================================
 // Forward
 // =============================================================================================
+// How the logits tiles (token tile x vocabulary tile) of a forward launch are shared out over the workgroups.
+//
+// splits: one round of workgroups, each with one token tile and one of `splits` equal ranges of the vocabulary.  Right when
+//   token tiles x splits comes close to the CU count; 45 token tiles (5 splits) leave 31 of 256 CUs idle, 86 tiles
+//   (2 splits) leave 84, and 129 tiles run at half rate.
+// bands: the token tiles are cut into bands of 8 (then 4, 2, 1 for what is left), and a band of R tiles is walked by the
+//   P workgroups of an XCD together: R token tiles x P / R vocabulary tiles per round, so that they share operand slabs
+//   through that XCD's L2 as they do with splits.  Bands go to the XCDs eight at a time while there are eight (a wave);
+//   the rounds of what is left form one sequence, of which each XCD takes an equal share.  A workgroup whose share crosses
+//   into another band writes out its softmax state and starts afresh.  Within a share the part of the later band, which
+//   begins at the start of the vocabulary, comes first: then all XCDs walk the vocabulary together, in two groups that are
+//   a fixed distance apart, and the weight comes out of HBM about twice per wave instead of once per band (in order of
+//   the sequence 21503 x 3584 x 152064 took 16.95 instead of 16.41 ms: on a board at its power limit traffic is time).
+constexpr int kXcds = 8;
+struct FwdPlan {
+  int tok_tiles, voc_tiles;
+  int splits;     // 0: bands
+  int group;      // bands: P, workgroups per XCD (a multiple of 8)
+  int waves;      // bands: eight full bands each, one per XCD
+  int count[4];   // bands: rounds of a band of 1, 2, 4, 8 token tiles
+  int rounds;     // bands: rounds of all bands after the waves together, below 2^27
+
+  // Everything a workgroup asks of the plan is additions, shifts and comparisons of uniform 32-bit values: it is asked
+  // with a tile's accumulators in registers, where a division would spill them.
+  struct Band {
+    // place among the bands after the waves, first token tile, log2 of its token tiles, rounds, first round
+    int index, first, log2_rows, count, start;
+    __host__ __device__ __forceinline__ int rows() const { return 1 << log2_rows; }
+  };
+  __host__ __device__ __forceinline__ int bands() const {  // after the waves
+    const int left = tok_tiles - 64 * waves;
+    return (left >> 3) + ((left >> 2) & 1) + ((left >> 1) & 1) + (left & 1);
+  }
+  __host__ __device__ __forceinline__ Band first_band() const {
+    Band b{0, 64 * waves, 3, count[3], 0};
+    shrink(b);
+    return b;
+  }
+  // the band after b; past the last one its count is 0 and its start is `rounds`
+  __host__ __device__ __forceinline__ void next(Band& b) const {
+    b.first += b.rows();
+    b.start += b.count;
+    ++b.index;
+    shrink(b);
+  }
+  __host__ __device__ __forceinline__ void shrink(Band& b) const {
+    const int left = tok_tiles - b.first;
+    if (left >= 8) return;
+    b.log2_rows = left >= 4 ? 2 : left >= 2 ? 1 : 0;
+    b.count = left <= 0 ? 0 : left >= 4 ? count[2] : left >= 2 ? count[1] : count[0];
+  }
+  // the first band that ends after round q
+  __device__ __forceinline__ Band band_of_round(int q) const {
+    Band b = first_band();
+    while (b.count > 0 && q >= b.start + b.count) next(b);
+    return b;
+  }
+  __device__ __forceinline__ int share_begin(int xcd) const { return (rounds * xcd) >> 3; }
+  // Where the state of (band, XCD, workgroup of the XCD) goes, in rows of 256 tokens: first the bands of the waves, then
+  // the others.  Those and the XCDs are walked in order, so index + xcd is different for every pair that meets.
+  __device__ __forceinline__ int64_t wave_slot(int wave, int xcd, int member) const {
+    return (int64_t)(kXcds * wave + xcd) * group + member;
+  }
+  __device__ __forceinline__ int64_t slot(int band_index, int xcd, int member) const {
+    return (int64_t)(kXcds * waves + band_index + xcd) * group + member;
+  }
+  __host__ __device__ __forceinline__ int64_t slots() const {
+    return splits ? (int64_t)splits * tok_tiles : (int64_t)(kXcds * waves + bands() + kXcds) * group;
+  }
+};
+static_assert(kXcds == 8, "share_begin() divides by shifting, a wave is 64 token tiles");
+
 struct FwdArgs {
   Operand hidden;  // R operand: [n_tokens][H]
   Operand weight;  // C operand: [vocab][H]
   const int64_t* labels;
   int n_tokens, vocab, k_slabs;
-  int tok_tiles, voc_tiles, splits;
+  FwdPlan plan;
   float scale2;      // log2(e) / temperature
   float rcp_t;       // 1 / temperature
-  float4* partials;  // [splits][tok_tiles * 256] : (max in the log2 domain, sum e, sum e x with x = hidden . weight, label logit)
-  float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward
-  float* pi2_partials;  // optional [splits][tok_tiles * 256] : sum of e^2 relative to the same max
+  float4* partials;  // [plan.slots()][256] : (max in the log2 domain, sum e, sum e x with x = hidden . weight, label logit)
+  float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward (splits only)
+  float* pi2_partials;  // optional [plan.slots()][256] : sum of e^2 relative to the same max
 };
 
-struct SplitSched {
-  int r0_, vt_begin, vt_count, k_slabs;
-  __device__ __forceinline__ int count() const { return vt_count; }
+// The tiles of one workgroup: its range of the vocabulary for one token tile (splits), or its column of every band its
+// XCD's share of the rounds touches (bands).
+struct FwdSched {
+  const FwdPlan* plan;
+  int k_slabs;
+  int tn_, vt_begin, ntiles, slot_;  // splits (ntiles: both)
+  int xcd, member, wave_count;       // bands: this XCD, workgroup within it, its tiles of a wave
+  FwdPlan::Band band0;               // bands: the band its share starts in
+
+  struct Place {
+    int tn, vt;    // token tile, vocabulary tile
+    int64_t slot;  // where the state goes
+  };
+  struct Column {
+    int first, count;  // first vocabulary tile, and how many; they are group >> log2_rows apart
+  };
+  __device__ __forceinline__ Column column(const FwdPlan::Band& b) const {
+    const int q0 = plan->share_begin(xcd) - b.start, q1 = plan->share_begin(xcd + 1) - b.start;
+    const int lo = q0 > 0 ? q0 : 0, hi = q1 < b.count ? q1 : b.count, cols = plan->group >> b.log2_rows;
+    const int first = (member >> b.log2_rows) + cols * lo;
+    int n = hi > lo ? hi - lo : 0;  // the last round of a band may have fewer columns than workgroups
+    if (n > 0 && first + cols * (n - 1) >= plan->voc_tiles) --n;
+    return Column{first, n};
+  }
+  __device__ __forceinline__ void init(const FwdPlan& p, int wg) {
+    plan = &p;
+    if (p.splits) {
+      // bands of 8 token tiles x all splits per XCD
+      const int band = 8 * p.splits, b = wg / band, first = b * 8, w = wg - b * band;
+      const int rows = (p.tok_tiles - first) < 8 ? (p.tok_tiles - first) : 8;
+      const int sp = w / rows;
+      tn_ = first + w % rows;
+      vt_begin = (int)(((int64_t)sp * p.voc_tiles) / p.splits);
+      ntiles = (int)(((int64_t)(sp + 1) * p.voc_tiles) / p.splits) - vt_begin;
+      slot_ = sp * p.tok_tiles + tn_;
+    } else {
+      xcd = wg / p.group;
+      member = wg % p.group;
+      band0 = p.band_of_round(p.share_begin(xcd));
+      const int cols = p.group >> 3;
+      wave_count = p.voc_tiles > (member >> 3) ? (p.voc_tiles - (member >> 3) + cols - 1) / cols : 0;
+      ntiles = p.waves * wave_count;
+      for (FwdPlan::Band b = band0; b.start < p.share_begin(xcd + 1); p.next(b)) ntiles += column(b).count;
+    }
+  }
+  __device__ __forceinline__ int count() const { return ntiles; }
+  __device__ __forceinline__ Place at(int i) const {
+    if (plan->splits) return Place{tn_, vt_begin + i, slot_};
+    int left = ntiles;
+    for (int w = 0; w < plan->waves; ++w, i -= wave_count, left -= wave_count)
+      if (i < wave_count)
+        return Place{8 * (kXcds * w + xcd) + (member & 7), (member >> 3) + (plan->group >> 3) * i,
+                     plan->wave_slot(w, xcd, member)};
+    // the bands of the share from the last to the first
+    FwdPlan::Band b = band0;
+    Column c = column(b);
+    while (i < left - c.count) {
+      left -= c.count;
+      plan->next(b);
+      c = column(b);
+    }
+    return Place{b.first + (member & (b.rows() - 1)), c.first + (plan->group >> b.log2_rows) * (i - (left - c.count)),
+                 plan->slot(b.index, xcd, member)};
+  }
   __device__ __forceinline__ void tile(int i, int& r0, int& c0) const {
-    r0 = r0_;
-    c0 = (vt_begin + i) * kTile;
+    const Place p = at(i);
+    r0 = p.tn * kTile;
+    c0 = p.vt * kTile;
   }
   __device__ __forceinline__ int slab0(int) const { return 0; }
   __device__ __forceinline__ int slabs(int) const { return k_slabs; }
@@ -137,7 +271,26 @@ struct BlockExchange {
 };
 
 constexpr int kCacheStageBytes = (kThreads / 64) * 4096;  // one 32 x 32 fp32 patch per wavefront
-constexpr int kFwdTokenLds = kTile * 4 + kThreads * kNB * 4;  // forward without a cache: labels + label-logit sums
+// forward without a cache: two sets of labels, label-logit sums, states of one half of the wavefronts (and squared sums)
+constexpr int kFwdTokenLds = 2 * kTile * 4 + kThreads * kNB * 4 + kTile * (16 + 4);
+
+__device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float m2, float s2, float sy2) {
+  const float mm = fmaxf(m, m2);
+  const float a = fast_exp2(m - mm), b = fast_exp2(m2 - mm);
+  s = s * a + s2 * b;
+  sy = sy * a + sy2 * b;
+  m = mm;
+}
+// the same with the squared sums q
+__device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float& q, float m2, float s2, float sy2,
+                                            float q2) {
+  const float mm = fmaxf(m, m2);
+  const float a = fast_exp2(m - mm), b = fast_exp2(m2 - mm);
+  s = s * a + s2 * b;
+  sy = sy * a + sy2 * b;
+  q = q * a * a + q2 * b * b;
+  m = mm;
+}
 
 // Per-lane online-softmax state for the kNB token slots (nb) the lane owns.  With CACHE the
 // scaled logits of every valid (token, vocabulary column) are also written out in fp32, so the
@@ -149,22 +302,125 @@ struct FwdEpi {
   LanePos p;
   float scale2;
   int vocab;
-  float m[kNB], s[kNB], sy[kNB], s2[kNB];
+  // vectors and not arrays: an array here ends up in scratch memory
+  f32x4 m, s, sy, s2;
   // The labels of the lane's token rows and the label-logit sums live in LDS behind the pipeline's stages when the
   // kernel has LDS to spare (no logits cache), in registers otherwise: with them in registers the kernel spilled,
   // and every reload of a spilled value waits out the slab transfers in flight (one counter counts both).
-  float zl[CACHE ? kNB : 1];
-  int lab[CACHE ? kNB : 1];
-  unsigned lab_lds, zl_lds;  // LDS byte addresses: labels [256] by tile row; sums [kThreads][kNB]
+  f32x4 zl;  // CACHE
+  int lab[kNB];  // CACHE
+  unsigned lab_lds, zl_lds, red_lds;  // LDS byte addresses: labels [2][256] by tile parity and row; sums [kThreads][kNB];
+                                      // states [256] float4, then squared sums [256]
+  const FwdArgs* args;
+  FwdSched sched;
+  int64_t slot;  // where the state of the token tile at hand goes
   float rcp_t;
   float* z_cache;  // CACHE: [n_tokens][vocab]
   BlockExchange ex;  // CACHE
   int tok0;        // CACHE: first token row of the wavefront
   int n_tokens;
 
-  __device__ __forceinline__ void prefetch(int, int, int) {}
-  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int /*r0*/, int c0) {
+  // the low dwords of the tile's 256 labels, 64 per wavefront of the first four, straight into LDS; a token past the end
+  // reads as label 0, whose sums nobody looks at
+  __device__ __forceinline__ void prefetch(int tile, int r0, int) {
+    if constexpr (!CACHE) {
+      const FwdSched::Place here = sched.at(tile);
+      if (here.slot != slot) {  // the token tile is another one (here no accumulators are alive)
+        if (tile > 0) write_state();
+        slot = here.slot;
+      }
+      const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+      if (w < 4) {
+        const u32x4 rs = span_rsrc(args->labels, (int64_t)args->n_tokens * 8);
+        load_to_lds_4(rs, ((unsigned)r0 + 64u * w + (threadIdx.x & 63u)) * 8u, label_set(tile) + 64u * w * 4u);
+      }
+    }
+  }
+  __device__ __forceinline__ unsigned label_set(int tile) const { return lab_lds + (unsigned)(tile & 1) * (kTile * 4); }
+
+  __device__ __forceinline__ void reset() {
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      m[nb] = kNegBig;
+      s[nb] = 0.f;
+      sy[nb] = 0.f;
+      s2[nb] = 0.f;
+    }
+  }
+
+  // merge the four lane quarters (they hold disjoint vocabulary columns of the same token)
+  __device__ __forceinline__ void merge_lanes(f32x4& z, int thread) {
+    merge_with_peer(z, ((thread & 63) ^ 16) << 2);
+    merge_with_peer(z, ((thread & 63) ^ 32) << 2);
+  }
+  static __device__ __forceinline__ float from_peer(int peer, float x) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(peer, __float_as_int(x)));
+  }
+  __device__ __forceinline__ void merge_with_peer(f32x4& z, int peer) {
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      merge_into(nb, from_peer(peer, m[nb]), from_peer(peer, s[nb]), from_peer(peer, sy[nb]),
+                 PI2 ? from_peer(peer, s2[nb]) : 0.f);
+      z[nb] += from_peer(peer, z[nb]);
+    }
+  }
+  __device__ __forceinline__ void merge_into(int nb, float m2, float sm2, float sy2, float q2) {
+    float a = m[nb], b = s[nb], c = sy[nb], q = s2[nb];
+    if (PI2) merge_state(a, b, c, q, m2, sm2, sy2, q2);
+    else merge_state(a, b, c, m2, sm2, sy2);
+    m[nb] = a;
+    s[nb] = b;
+    sy[nb] = c;
+    s2[nb] = q;
+  }
+
+  // The token tile is done for this workgroup: combine the lanes, then the two wavefronts that share a token quarter
+  // (wc = 0 / 1, through LDS), write the state out and start afresh.
+  __device__ __forceinline__ void write_state() {
+    typedef float __attribute__((address_space(3))) * lds_f32_t;
+    typedef f32x4 __attribute__((address_space(3))) * lds_f32x4_t;
+    // The thread's number as a value made here: everything addressed with it is then computed here too.  From threadIdx.x
+    // the compiler computes the lot ahead of the tile loop and, with the accumulators in the way, spills 110 registers.
+    int thread = threadIdx.x;
+    asm volatile("" : "+v"(thread));
+    const int row0 = ((thread >> 6) % kWavesR) * (kNB * kBlk) + (thread & 15);  // acc_row(p, 0)
+    f32x4 z;
+    const lds_f32_t sums = (lds_f32_t)(uintptr_t)(zl_lds + 4u * (unsigned)(thread * kNB));
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      z[nb] = sums[nb];
+      sums[nb] = 0.f;
+    }
+    merge_lanes(z, thread);
+    const lds_f32x4_t red = (lds_f32x4_t)(uintptr_t)red_lds;
+    const lds_f32_t redq = (lds_f32_t)(uintptr_t)(red_lds + kTile * 16);
+    const bool lq0 = (thread & 48) == 0;
+    if (thread >= 64 * kWavesR && lq0) {  // wc = 1
+#pragma unroll
+      for (int nb = 0; nb < kNB; ++nb) {
+        red[row0 + kBlk * nb] = f32x4{m[nb], s[nb], sy[nb], z[nb]};
+        if (PI2) redq[row0 + kBlk * nb] = s2[nb];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (thread < 64 * kWavesR && lq0) {
+#pragma unroll
+      for (int nb = 0; nb < kNB; ++nb) {
+        const int row = row0 + kBlk * nb;
+        const f32x4 o = red[row];
+        merge_into(nb, o[0], o[1], o[2], PI2 ? redq[row] : 0.f);
+        if (PI2) args->pi2_partials[slot * kTile + row] = s2[nb];
+        args->partials[slot * kTile + row] = make_float4(m[nb], s[nb], sy[nb], z[nb] + o[3]);
+      }
+    }
+    reset();
+  }
+
+  __device__ __forceinline__ void operator()(Accum& acc, int tile, int /*r0*/, int c0) {
     const bool ragged = c0 + kTile > vocab;
+    // element (mb, v) of the lane is column 16 mb + v of this: comparing immediates with one register, where a column
+    // number per element would be computed ahead of the tile loop and held (or spilled) through it
+    const int cols_left = vocab - c0 - p.wc * 128 - 4 * p.lq;
     if constexpr (CACHE) {
 #pragma unroll
       for (int nb2 = 0; nb2 < kNB2; ++nb2)
@@ -197,7 +453,7 @@ struct FwdEpi {
         for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const float x = (c0 + acc_col(p, mb, v) < vocab) ? acc.a[mb][nb][v] : kNoColumn;
+            const float x = mb * kBlk + v < cols_left ? acc.a[mb][nb][v] : kNoColumn;
             acc.a[mb][nb][v] = x;
             xmax = fmaxf(xmax, x);
           }
@@ -212,16 +468,16 @@ struct FwdEpi {
       typedef float __attribute__((address_space(3))) * lds_f32_t;
       int label;
       if constexpr (CACHE) label = lab[nb];
-      else label = *(lds_i32_t)(uintptr_t)(lab_lds + 4u * (unsigned)acc_row(p, nb));
+      else label = *(lds_i32_t)(uintptr_t)(label_set(tile) + 4u * (unsigned)acc_row(p, nb));
       const int rel = label - c0 - p.wc * 128;
       if (__any(rel >= 0 && rel < 128)) {
         float add = 0.f;
+        const int mine = rel - 4 * p.lq;
 #pragma unroll
         for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int col = mb * kBlk + 4 * p.lq + v;
-            add += (col == rel) ? acc.a[mb][nb][v] * rcp_t : 0.f;
+            add += mb * kBlk + v == mine ? acc.a[mb][nb][v] * rcp_t : 0.f;
           }
         if constexpr (CACHE) {
           zl[nb] += add;
@@ -253,140 +509,82 @@ struct FwdEpi {
   }
 };
 
-__device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float m2, float s2, float sy2) {
-  const float mm = fmaxf(m, m2);
-  const float a = fast_exp2(m - mm), b = fast_exp2(m2 - mm);
-  s = s * a + s2 * b;
-  sy = sy * a + sy2 * b;
-  m = mm;
-}
-// the same with the squared sums q
-__device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float& q, float m2, float s2, float sy2,
-                                            float q2) {
-  const float mm = fmaxf(m, m2);
-  const float a = fast_exp2(m - mm), b = fast_exp2(m2 - mm);
-  s = s * a + s2 * b;
-  sy = sy * a + sy2 * b;
-  q = q * a * a + q2 * b * b;
-  m = mm;
-}
-
 template <bool CACHE, bool PI2>
 __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  // workgroup -> (token tile, vocabulary split); bands of 8 token tiles x all splits per XCD
-  const int nwg = a.tok_tiles * a.splits;
-  const int q = xcd_regroup(blockIdx.x, nwg);
-  const int band = 8 * a.splits;
-  const int bidx = q / band;
-  const int first = bidx * 8;
-  const int rows = (a.tok_tiles - first) < 8 ? (a.tok_tiles - first) : 8;
-  const int w = q - bidx * band;
-  const int tn = first + w % rows;
-  const int sp = w / rows;
-
-  SplitSched sched;
+  FwdSched sched;
+  sched.init(a.plan, xcd_regroup(blockIdx.x, gridDim.x));
   sched.k_slabs = a.k_slabs;
-  sched.r0_ = tn * kTile;
-  sched.vt_begin = (int)(((int64_t)sp * a.voc_tiles) / a.splits);
-  sched.vt_count = (int)(((int64_t)(sp + 1) * a.voc_tiles) / a.splits) - sched.vt_begin;
 
   FwdEpi<CACHE, PI2> epi;
   epi.p = lane_pos();
   epi.scale2 = a.scale2;
   epi.vocab = a.vocab;
   epi.rcp_t = a.rcp_t;
+  epi.args = &a;
+  epi.sched = sched;
+  epi.slot = -1;
+  epi.reset();
+  if constexpr (CACHE) {
 #pragma unroll
-  for (int nb = 0; nb < kNB; ++nb) {
-    epi.m[nb] = kNegBig;
-    epi.s[nb] = 0.f;
-    epi.sy[nb] = 0.f;
-    epi.s2[nb] = 0.f;
-    if constexpr (CACHE) {
+    for (int nb = 0; nb < kNB; ++nb) {
       epi.zl[nb] = 0.f;
-      const int tok = sched.r0_ + acc_row(epi.p, nb);
+      const int tok = sched.tn_ * kTile + acc_row(epi.p, nb);
       epi.lab[nb] = tok < a.n_tokens ? (int)a.labels[tok] : -1;
     }
-  }
-  if constexpr (!CACHE) {
+    epi.z_cache = a.z_cache;
+    epi.ex.init(lds + kLdsBytes, epi.p);
+    epi.tok0 = sched.tn_ * kTile + epi.p.wr * (kNB * kBlk);
+    epi.n_tokens = a.n_tokens;
+  } else {
     typedef float __attribute__((address_space(3))) * lds_f32_t;
     epi.lab_lds = lds_address(lds + kLdsBytes);
-    epi.zl_lds = epi.lab_lds + kTile * 4;
+    epi.zl_lds = epi.lab_lds + 2 * kTile * 4;
+    epi.red_lds = epi.zl_lds + kThreads * kNB * 4;
 #pragma unroll
     for (int nb = 0; nb < kNB; ++nb) *(lds_f32_t)(uintptr_t)(epi.zl_lds + 4u * (threadIdx.x * kNB + nb)) = 0.f;
-    // the low dwords of the tile's 256 labels, 64 per wavefront of the first four, straight into LDS; a token past
-    // the end reads as label 0, whose sums nobody looks at.  The transfers are older than every slab transfer, so
-    // the pipeline's first wait and barrier cover them.
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (w < 4) {
-      const u32x4 rs = span_rsrc(a.labels, (int64_t)a.n_tokens * 8);
-      load_to_lds_4(rs, ((unsigned)sched.r0_ + 64u * w + (threadIdx.x & 63u)) * 8u, epi.lab_lds + 64u * w * 4u);
-    }
   }
-  epi.z_cache = a.z_cache;
-  epi.ex.init(lds + kLdsBytes, epi.p);
-  epi.tok0 = sched.r0_ + epi.p.wr * (kNB * kBlk);
-  epi.n_tokens = a.n_tokens;
 
   run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 
-  float zl[kNB];
+  if constexpr (!CACHE) {
+    if (sched.count() > 0) epi.write_state();
+  } else {  // one token tile per workgroup (splits): its state is written once, at the end
+    epi.merge_lanes(epi.zl, threadIdx.x);
+    // the two wavefronts that share a token quarter, through LDS (once every wavefront's last slab transfers have landed)
+    __syncthreads();
+    float4* red = reinterpret_cast<float4*>(lds);                     // [2][256]
+    float* redq = reinterpret_cast<float*>(lds + 2 * kTile * 16);    // [2][256] squared sums
+    if (epi.p.lq == 0) {
 #pragma unroll
-  for (int nb = 0; nb < kNB; ++nb) {
-    typedef float __attribute__((address_space(3))) * lds_f32_t;
-    if constexpr (CACHE) zl[nb] = epi.zl[nb];
-    else zl[nb] = *(lds_f32_t)(uintptr_t)(epi.zl_lds + 4u * (threadIdx.x * kNB + nb));
-  }
-  // merge the four lane quarters (they hold disjoint vocabulary columns of the same token) ...
-#pragma unroll
-  for (int step = 16; step <= 32; step *= 2)
-#pragma unroll
-    for (int nb = 0; nb < kNB; ++nb) {
-      const float m2 = __shfl_xor(epi.m[nb], step, 64);
-      const float s2 = __shfl_xor(epi.s[nb], step, 64);
-      const float sy2 = __shfl_xor(epi.sy[nb], step, 64);
-      const float z2 = __shfl_xor(zl[nb], step, 64);
-      if (PI2) {
-        const float q2 = __shfl_xor(epi.s2[nb], step, 64);
-        merge_state(epi.m[nb], epi.s[nb], epi.sy[nb], epi.s2[nb], m2, s2, sy2, q2);
-      } else {
-        merge_state(epi.m[nb], epi.s[nb], epi.sy[nb], m2, s2, sy2);
+      for (int nb = 0; nb < kNB; ++nb) {
+        red[epi.p.wc * kTile + acc_row(epi.p, nb)] = make_float4(epi.m[nb], epi.s[nb], epi.sy[nb], epi.zl[nb]);
+        if (PI2) redq[epi.p.wc * kTile + acc_row(epi.p, nb)] = epi.s2[nb];
       }
-      zl[nb] += z2;
     }
-  // ... then the two wavefronts that share a token quarter (wc = 0/1), through LDS (once every
-  // wavefront's last slab transfers have landed).
-  __syncthreads();
-  float4* red = reinterpret_cast<float4*>(lds);                     // [2][256]
-  float* redq = reinterpret_cast<float*>(lds + 2 * kTile * 16);    // [2][256] squared sums
-  if (epi.p.lq == 0) {
-#pragma unroll
-    for (int nb = 0; nb < kNB; ++nb) {
-      red[epi.p.wc * kTile + acc_row(epi.p, nb)] = make_float4(epi.m[nb], epi.s[nb], epi.sy[nb], zl[nb]);
-      if (PI2) redq[epi.p.wc * kTile + acc_row(epi.p, nb)] = epi.s2[nb];
+    __syncthreads();
+    if (threadIdx.x < kTile) {
+      const int t = threadIdx.x;
+      float4 x = red[t], y = red[kTile + t];
+      const int64_t slot = (int64_t)sched.slot_ * kTile + t;
+      if (PI2) {
+        float q = redq[t];
+        merge_state(x.x, x.y, x.z, q, y.x, y.y, y.z, redq[kTile + t]);
+        a.pi2_partials[slot] = q;
+      } else {
+        merge_state(x.x, x.y, x.z, y.x, y.y, y.z);
+      }
+      x.w += y.w;
+      a.partials[slot] = x;
     }
-  }
-  __syncthreads();
-  if (threadIdx.x < kTile) {
-    const int t = threadIdx.x;
-    float4 x = red[t], y = red[kTile + t];
-    const int64_t slot = (int64_t)sp * a.tok_tiles * kTile + tn * kTile + t;
-    if (PI2) {
-      float q = redq[t];
-      merge_state(x.x, x.y, x.z, q, y.x, y.y, y.z, redq[kTile + t]);
-      a.pi2_partials[slot] = q;
-    } else {
-      merge_state(x.x, x.y, x.z, y.x, y.y, y.z);
-    }
-    x.w += y.w;
-    a.partials[slot] = x;
   }
 }
 
 struct MergeArgs {
   const float4* partials;
   const float* pi2_partials;  // null unless sum_pi_squared is wanted
-  int splits, stride, n_tokens;
+  FwdPlan plan;
+  int n_tokens;
   int lanes_log2;  // lanes that share a token, as a power of two
   float rcp_t;  // the partial sums of e * (hidden . weight) carry no 1 / temperature yet
   float* logprobs;
@@ -406,11 +604,33 @@ __global__ __launch_bounds__(256) void lce_merge_kernel(MergeArgs a) {
   const bool exists = tok < a.n_tokens;
   float m = kNegBig, s = 0.f, sy = 0.f, zl = 0.f, q = 0.f;
   if (exists) {
-    for (int sp = threadIdx.x & (lanes - 1); sp < a.splits; sp += lanes) {
-      const float4 x = a.partials[(int64_t)sp * a.stride + tok];
-      if (a.pi2_partials) merge_state(m, s, sy, q, x.x, x.y, x.z, a.pi2_partials[(int64_t)sp * a.stride + tok]);
+    const int tn = (int)(tok / kTile), row = (int)(tok % kTile), mine = threadIdx.x & (lanes - 1);
+    auto add = [&](int64_t slot) {
+      const float4 x = a.partials[slot * kTile + row];
+      if (a.pi2_partials) merge_state(m, s, sy, q, x.x, x.y, x.z, a.pi2_partials[slot * kTile + row]);
       else merge_state(m, s, sy, x.x, x.y, x.z);
       zl += x.w;
+    };
+    if (a.plan.splits) {
+      for (int sp = mine; sp < a.plan.splits; sp += lanes) add((int64_t)sp * a.plan.tok_tiles + tn);
+    } else {  // every workgroup column of every XCD whose share of the rounds touches the token tile's band
+      const bool in_wave = tn < 64 * a.plan.waves;
+      FwdPlan::Band b = a.plan.first_band();
+      while (!in_wave && tn >= b.first + b.rows()) a.plan.next(b);
+      const int cols = a.plan.group >> (in_wave ? 3 : b.log2_rows);
+      if (in_wave)
+        for (int col = mine; col < cols && col < a.plan.voc_tiles; col += lanes)
+          add(a.plan.wave_slot(tn / 64, tn / 8 % kXcds, col * 8 + tn % 8));
+      int x0 = 0, x1;  // the XCDs whose shares touch the band
+      while (!in_wave && a.plan.share_begin(x0 + 1) <= b.start) ++x0;
+      for (x1 = x0; x1 + 1 < kXcds && a.plan.share_begin(x1 + 1) < b.start + b.count;) ++x1;
+      for (int j = mine; !in_wave && j < (x1 - x0 + 1) * cols; j += lanes) {
+        const int xcd = x0 + j / cols, col = j % cols;
+        const int q0 = a.plan.share_begin(xcd), q1 = a.plan.share_begin(xcd + 1);
+        const int lo = q0 > b.start ? q0 - b.start : 0;
+        if (q1 > b.start + lo && col + cols * lo < a.plan.voc_tiles)  // it had a tile to do
+          add(a.plan.slot(b.index, xcd, col * b.rows() + (tn - b.first)));
+      }
     }
   }
   for (int step = 1; step < lanes; step <<= 1) {
@@ -857,15 +1077,33 @@ static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // channels instead of landing on a power-of-two stride.
 static inline int64_t dz_pitch(int64_t cv) { return cv + 128; }
 
-// max_rows: most partial-state rows (splits x padded tokens) the caller's buffer holds; the built-in buffer of the
-// entry point that allocates nothing is sized for 256 CUs and must serve a part with more of them too.
-static int fwd_splits(int64_t tok_tiles, int64_t voc_tiles, int64_t max_rows = INT64_MAX) {
-  const int cus = device_cu_count();
+// max_slots: most partial states (of 256 tokens each) the caller's buffer holds; the built-in buffer of the entry point that
+// allocates nothing is sized for 256 CUs and must serve a part with more of them too.
+static FwdPlan plan_forward(int64_t tok_tiles, int64_t voc_tiles, bool one_tile_only, int64_t max_slots = INT64_MAX) {
+  const int64_t cus = device_cu_count();
+  FwdPlan p{};
+  p.tok_tiles = (int)tok_tiles;
+  p.voc_tiles = (int)voc_tiles;
   int64_t sp = cus / tok_tiles;  // as many workgroups as fit in one round over the CUs
-  if (sp > max_rows / (tok_tiles * kTile)) sp = max_rows / (tok_tiles * kTile);
+  if (sp > max_slots / tok_tiles) sp = max_slots / tok_tiles;
   if (sp < 1) sp = 1;
   if (sp > voc_tiles) sp = voc_tiles;
-  return (int)sp;
+  p.splits = (int)sp;
+  if (one_tile_only || cus % (8 * kXcds) != 0) return p;
+  const int64_t split_rounds = ceil_div(tok_tiles * sp, cus) * ceil_div(voc_tiles, sp);
+  FwdPlan b = p;
+  b.splits = 0;
+  b.group = (int)(cus / kXcds);
+  for (int k = 0; k < 4; ++k) b.count[k] = (int)ceil_div(voc_tiles, b.group >> k);
+  b.waves = (int)(tok_tiles / 64);
+  int64_t rounds = tok_tiles % 64 / 8 * b.count[3];
+  for (int k = 0; k < 3; ++k) rounds += (tok_tiles >> k & 1) * b.count[k];
+  b.rounds = (int)rounds;
+  const int64_t band_rounds = (int64_t)b.waves * b.count[3] + ceil_div(rounds, kXcds);
+  // Bands cost what 1 - 2 % more rounds would (more of the weight's traffic, states written more than once): 9000 tokens x
+  // 3584 x 152064, 84 rounds in bands and 85 in splits, 7.07 and 6.97 ms; 3300 x 896 x 151936, 31 and 32, 0.710 and
+  // 0.736; 11290 x 3584 x 152064, 105 and 119, 8.81 and 9.24; 22000 tokens, 200 and 297, 16.9 and 19.9.
+  return rounds < (1 << 27) && 34 * band_rounds <= 33 * split_rounds && b.slots() <= max_slots ? b : p;
 }
 
 // Any vocabulary size is served; only the fp32 logits cache, whose rows are read and written 32 bytes at a time,
@@ -993,9 +1231,12 @@ extern "C" size_t vamd_lce_forward_workspace_bytes(int64_t n_tokens, int64_t hid
   (void)hidden_size;
   if (n_tokens <= 0 || vocab <= 0) return 0;
   const int64_t tok_tiles = ceil_div(n_tokens, kTile), voc_tiles = ceil_div(vocab, kTile);
-  const int sp = fwd_splits(tok_tiles, voc_tiles);
-  return align_up((size_t)sp * tok_tiles * kTile * sizeof(float4), 256) +
-         align_up((size_t)sp * tok_tiles * kTile * sizeof(float), 256);  // state + squared sums
+  int64_t slots = 0;  // with a logits cache the launch has one token tile per workgroup
+  for (bool one_tile_only : {false, true}) {
+    const int64_t n = plan_forward(tok_tiles, voc_tiles, one_tile_only).slots();
+    if (n > slots) slots = n;
+  }
+  return (size_t)slots * kTile * (sizeof(float4) + sizeof(float));  // state + squared sums
 }
 
 // Forward launches shared by the two entry points; `workspace` holds at least
@@ -1003,7 +1244,7 @@ extern "C" size_t vamd_lce_forward_workspace_bytes(int64_t n_tokens, int64_t hid
 static int lce_forward_launch(const void* hidden, const void* weight, const int64_t* labels, int64_t n_tokens,
                               int64_t hidden_size, int64_t vocab, float rcp_temperature, float* logprobs,
                               float* entropy, float* lse, float* mean_z, float* logits_cache, float* sum_pi_squared,
-                              void* workspace, void* stream, int64_t max_rows = INT64_MAX) {
+                              void* workspace, void* stream, int64_t max_slots = INT64_MAX) {
 
   FwdArgs a;
   a.hidden = Operand{static_cast<const uint16_t*>(hidden), hidden_size, (int)n_tokens, (int)hidden_size};
@@ -1012,21 +1253,19 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   a.n_tokens = (int)n_tokens;
   a.vocab = (int)vocab;
   a.k_slabs = (int)(hidden_size / kBK);
-  a.tok_tiles = (int)ceil_div(n_tokens, kTile);
-  a.voc_tiles = (int)ceil_div(vocab, kTile);
-  a.splits = fwd_splits(a.tok_tiles, a.voc_tiles, max_rows);
+  a.plan = plan_forward(ceil_div(n_tokens, kTile), ceil_div(vocab, kTile), logits_cache != nullptr, max_slots);
   a.scale2 = rcp_temperature * kLog2e;
   a.rcp_t = rcp_temperature;
   a.partials = static_cast<float4*>(workspace);
   a.pi2_partials = sum_pi_squared
                        ? reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                                  align_up((size_t)a.splits * a.tok_tiles * kTile * sizeof(float4), 256))
+                                                  (size_t)a.plan.slots() * kTile * sizeof(float4))
                        : nullptr;
   a.z_cache = logits_cache;
   hipStream_t s = static_cast<hipStream_t>(stream);
   {
     ScopedTiming tm(kTagForward, s);
-    const dim3 grid(a.tok_tiles * a.splits), block(kThreads);
+    const dim3 grid(a.plan.splits ? a.plan.tok_tiles * a.plan.splits : a.plan.group * kXcds), block(kThreads);
     if (logits_cache) {
       if (sum_pi_squared)
         hipLaunchKernelGGL((lce_forward_kernel<true, true>), grid, block, kLdsBytes + kCacheStageBytes, s, a);
@@ -1045,11 +1284,11 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   m.partials = a.partials;
   m.pi2_partials = a.pi2_partials;
   m.sum_pi_squared = sum_pi_squared;
-  m.splits = a.splits;
-  m.stride = a.tok_tiles * kTile;
-  // a lane per split up to a wavefront per token: fewer splits than lanes would leave lanes idle
+  m.plan = a.plan;
+  // a lane per state up to a wavefront per token: fewer states than lanes would leave lanes idle
+  const int states = a.plan.splits ? a.plan.splits : (int)(a.plan.slots() / a.plan.tok_tiles);
   m.lanes_log2 = 0;
-  while (m.lanes_log2 < 6 && (2 << m.lanes_log2) <= a.splits) ++m.lanes_log2;
+  while (m.lanes_log2 < 6 && (2 << m.lanes_log2) <= states) ++m.lanes_log2;
   m.n_tokens = (int)n_tokens;
   m.rcp_t = rcp_temperature;
   m.logprobs = logprobs;
@@ -1098,7 +1337,9 @@ extern "C" int vamd_lce_forward(const void* hidden, const void* weight, const in
 // The array's name is only a host-side handle for that lookup: launches and copies use the
 // looked-up pointer.
 namespace vamd {
-constexpr size_t kStaticScratchBytes = (size_t)VAMD_LCE_STATIC_MAX_TOKENS * (sizeof(float4) + sizeof(float)) + 512;
+// up to 65536 tokens in bands: (34 bands + 8 XCDs) x 32 workgroups x 256 tokens
+constexpr int64_t kStaticSlots = (VAMD_LCE_STATIC_MAX_TOKENS / (8 * kTile) + 2 + kXcds) * 32;
+constexpr size_t kStaticScratchBytes = (size_t)kStaticSlots * kTile * (sizeof(float4) + sizeof(float)) + 512;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 static int static_scratch_pointer(void** out) {
@@ -1135,9 +1376,9 @@ extern "C" int vamd_lce_forward_static(const void* hidden, const void* weight, c
   if ((st = static_scratch_pointer(&ws)) != VAMD_OK) return st;
   // Every partial the merge kernel reads is written by the forward kernel of the same call, so
   // nothing in the buffer has to start at zero and a previous call's contents do not matter.
-  // the vocabulary splits are capped so that splits x padded tokens fits the buffer whatever the CU count
+  // the plan is made so that its states fit the buffer whatever the CU count
   return lce_forward_launch(hidden, weight, labels, n_tokens, hidden_size, vocab, rcp_temperature, logprobs, entropy,
-                            lse, mean_z, nullptr, sum_pi_squared, ws, stream, VAMD_LCE_STATIC_MAX_TOKENS);
+                            lse, mean_z, nullptr, sum_pi_squared, ws, stream, kStaticSlots);
 }
 
 namespace vamd {

@@ -2001,3 +2001,53 @@ def test_c_abi_chain_replays_from_a_hip_graph(dev):
             assert torch.equal(captured[name], eager[name]), name
         assert _counter_area_is_clear(ws)        # the arrival counters are back at zero
 
+
+
+# ---- rows that are aligned to their elements only --------------------------------------------------
+def _at_offset(t, k):
+    """The same values, contiguous, k elements into a fresh buffer."""
+    flat = torch.empty(t.numel() + k, dtype=t.dtype, device=t.device)
+    flat[k:] = t.flatten()
+    return flat[k:].view(t.shape)
+
+
+@pytest.mark.parametrize("cols", [4, 1028, 4096, 4100])
+@pytest.mark.parametrize("mdtype", [torch.float32, torch.int64, torch.bool, torch.int32])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_misaligned_tensors_give_the_bits_of_aligned_ones(dev, cols, mdtype, offset):
+    """The same threads hold the same elements whatever the alignment, so every result is the same bits."""
+    from verl_amd.trainer.ppo import core_algos as CA, rollout_corr_helper as RC
+    g = torch.Generator().manual_seed(cols + offset)
+    B = 5
+    mask = _prefix_mask(B, cols, g)[0].to(dev).to(mdtype)
+    old, new, adv = (torch.randn(B, cols, generator=g).to(dev) for _ in range(3))
+
+    def results(place):
+        lp = place(new).requires_grad_()
+        m = place(mask)
+        loss, metrics = CA.compute_policy_loss_vanilla(place(old), lp, place(adv), m, "token-mean", _cfg())
+        kl = CA.compute_kl_loss(lp, place(old), m, "low_var_kl", "seq-mean-token-mean")
+        (grad,) = torch.autograd.grad(loss + kl, (lp,))
+        kept, rs = RC.compute_rollout_rejection_mask(place(0.1 * old), m, "token_k1", "0.9_1.1")
+        return (loss.detach(), kl.detach(), grad, kept), metrics, rs
+
+    (a, am, ars), (b, bm, brs) = results(lambda t: t.clone()), results(lambda t: _at_offset(t, offset))
+    for x, y in zip(a, b):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+    assert am == bm and ars == brs
+
+
+@pytest.mark.parametrize("cols", [1, 2, 3, 5, 1023, 4097, 8190])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_odd_rows_are_written_to_their_last_column_and_no_further(dev, cols, offset):
+    from verl_amd import _cabi
+    B, guard = 4, 8
+    x = _at_offset(torch.arange(B * cols, dtype=torch.float32, device=dev).view(B, cols), offset)
+    buf = torch.full((guard + offset + B * cols + guard,), -7.0, device=dev)
+    out = buf[guard + offset:guard + offset + B * cols]
+    coef = torch.tensor([1.0, 2.0, 4.0, 8.0], device=dev)
+    one = torch.ones(1, device=dev)
+    _cabi.check(_cabi.lib().vamd_scale_rows(x.data_ptr(), coef.data_ptr(), one.data_ptr(), 0.5, B, cols, out.data_ptr(),
+                                            _cabi.stream_ptr(dev)))
+    assert torch.equal(out.view(B, cols), x * (0.5 * coef[:, None]))
+    assert bool((buf[:guard + offset] == -7.0).all()) and bool((buf[guard + offset + B * cols:] == -7.0).all())

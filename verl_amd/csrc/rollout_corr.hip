@@ -513,8 +513,8 @@ __global__ __launch_bounds__(kRcThreads) void rs_apply_kernel(const float* __res
       out[e] = keep ? static_cast<M>(m[g][e]) : static_cast<M>(0);
     }
     if (pos.valid[g] > 0) {
-      if constexpr (VEC) {
-        struct alignas(sizeof(M) * 4) Pack { M v[4]; };
+      if (VEC || pos.valid[g] == 4) {
+        struct alignas(VEC ? sizeof(M) * 4 : alignof(M)) Pack { M v[4]; };
         Pack p;
 #pragma unroll
         for (int e = 0; e < 4; ++e) p.v[e] = out[e];

@@ -12,6 +12,8 @@
 // Workspace contract of these kernels: the first 256 bytes hold the ticket counter; they must be
 // zero on entry and are zero again when the kernel has finished.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace vamd {
@@ -47,6 +49,17 @@ __device__ __forceinline__ bool streams_past_caches(int64_t elements) {
 typedef float nt_f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned nt_u32x4 __attribute__((ext_vector_type(4)));
 
+// VEC = false: the rows of the matrix (or its base) are only aligned to their elements, as every second row is when the
+// column count is odd.  The memory pipeline takes a 16-byte access at any 4-byte boundary (8-byte for int64 masks, any
+// byte for bool masks), so a whole group still moves as one instruction per 16 bytes, through these types that promise
+// the element's alignment only; the group that a row ends in goes element by element, so nothing is touched past it.
+// One instruction per element, as it was, moves a quarter of the bytes per instruction.  At 1000 x 11999 with an int64
+// mask: policy loss with gradient 81.6 -> 64.7 us, KL loss with gradient 62.6 -> 47.2 us, GRPO 61.5 -> 44.9 us,
+// scale_rows 28.6 -> 18.0 us, agg_loss forward / backward 34.5 / 32.5 -> 28.0 / 23.0 us.
+typedef float un_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned un_u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned un_u32 __attribute__((aligned(1)));
+
 template <bool VEC>
 __device__ __forceinline__ void ld4(const float* __restrict__ p, int64_t i, int valid, float (&x)[4],
                                     bool streaming = launch_streams_past_caches()) {
@@ -58,6 +71,15 @@ __device__ __forceinline__ void ld4(const float* __restrict__ p, int64_t i, int 
     } else {
       const float4 v = *reinterpret_cast<const float4*>(p + i);
       x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    }
+  } else if (valid == 4) {
+    if (streaming) {
+      const un_f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const un_f32x4*>(p + i));
+      x[0] = v[0]; x[1] = v[1]; x[2] = v[2]; x[3] = v[3];
+    } else {
+      const un_u32x4 v = *reinterpret_cast<const un_u32x4*>(p + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(v[e]);
     }
   } else {
 #pragma unroll
@@ -75,6 +97,13 @@ __device__ __forceinline__ void st4(float* __restrict__ p, int64_t i, int valid,
     } else {
       *reinterpret_cast<float4*>(p + i) = make_float4(x[0], x[1], x[2], x[3]);
     }
+  } else if (valid == 4) {
+    if (streaming) {
+      const un_u32x4 v = {__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]), __float_as_uint(x[3])};
+      __builtin_nontemporal_store(v, reinterpret_cast<un_u32x4*>(p + i));
+    } else {
+      *reinterpret_cast<un_f32x4*>(p + i) = un_f32x4{x[0], x[1], x[2], x[3]};
+    }
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -85,24 +114,28 @@ __device__ __forceinline__ void st4(float* __restrict__ p, int64_t i, int valid,
 template <bool VEC, class M>
 __device__ __forceinline__ void ldmask4(const M* __restrict__ p, int64_t i, int valid, float (&w)[4],
                                         bool streaming = launch_streams_past_caches()) {
-  if constexpr (VEC) {
-    struct alignas(sizeof(M) * 4) Pack { M v[4]; };
+  // the same instructions at either alignment; VEC only says what the compiler may assume
+  typedef std::conditional_t<VEC, nt_f32x4, un_f32x4> F4;
+  typedef std::conditional_t<VEC, nt_u32x4, un_u32x4> U4;
+  typedef std::conditional_t<VEC, unsigned, un_u32> U1;
+  if (VEC || valid == 4) {
+    struct alignas(VEC ? sizeof(M) * 4 : alignof(M)) Pack { M v[4]; };
     Pack k;
     if (streaming) {
       if constexpr (sizeof(M) == 4 && static_cast<M>(0.5f) != static_cast<M>(0)) {  // fp32 mask: load as integers
-        const nt_u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const nt_u32x4*>(p + i));
+        const U4 raw = __builtin_nontemporal_load(reinterpret_cast<const U4*>(p + i));
         k = __builtin_bit_cast(Pack, raw);
       } else if constexpr (sizeof(M) == 4) {  // int32 mask: load as floats (a type the default path does not use)
-        const nt_f32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const nt_f32x4*>(p + i));
+        const F4 raw = __builtin_nontemporal_load(reinterpret_cast<const F4*>(p + i));
         k = __builtin_bit_cast(Pack, raw);
       } else if constexpr (sizeof(M) == 8) {
-        struct Two { nt_u32x4 lo, hi; };
+        struct Two { U4 lo, hi; };
         Two raw;
-        raw.lo = __builtin_nontemporal_load(reinterpret_cast<const nt_u32x4*>(p + i));
-        raw.hi = __builtin_nontemporal_load(reinterpret_cast<const nt_u32x4*>(p + i) + 1);
+        raw.lo = __builtin_nontemporal_load(reinterpret_cast<const U4*>(p + i));
+        raw.hi = __builtin_nontemporal_load(reinterpret_cast<const U4*>(p + i) + 1);
         k = __builtin_bit_cast(Pack, raw);
       } else {
-        const unsigned raw = __builtin_nontemporal_load(reinterpret_cast<const unsigned*>(p + i));
+        const unsigned raw = __builtin_nontemporal_load(reinterpret_cast<const U1*>(p + i));
         k = __builtin_bit_cast(Pack, raw);
       }
     } else {

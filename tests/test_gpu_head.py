@@ -663,8 +663,8 @@ def test_pad_to_response_window(dev, geometry):
 
 @pytest.mark.parametrize("n,v", [(1, 152), (5, 700), (93, 66000), (257, 33001), (1100, 5000)])
 def test_merge_of_vocabulary_splits(dev, n, v):
-    """The partial softmax states of a token, however many vocabulary splits the launch had (1, 2, 256, 128 and 19
-    here, so 1 to 64 lanes of the merge share a token), combine to the fp32 ground truth."""
+    """The partial softmax states of a token, however many vocabulary splits the launch had (3, 11, 256, 128 and 19
+    here, so 2 to 64 lanes of the merge share a token), combine to the fp32 ground truth."""
     from verl_amd.utils.kernel import linear_cross_entropy as K
     from oracle import masked as OM
     hidden, weight, labels = (t.to(dev) for t in _make(n, 128, v, seed=n + v))
@@ -719,3 +719,30 @@ def test_forward_in_bands_of_token_tiles(dev, n, v):
         assert (lp[lo:lo + 4096] - want_lp).abs().max() <= ATOL and (ent[lo:lo + 4096] - want_ent).abs().max() <= ATOL
         want_pi2 = OM.sum_pi_squared_from_logits(h @ weight.float().t() / 0.8)
         assert torch.allclose(pi2[lo:lo + 4096], want_pi2, rtol=2e-3, atol=1e-9)
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (1, 128, 16),          # one workgroup, one block of columns
+    (128, 128, 64),        # one full range
+    (127, 256, 257),       # five ranges, the last of one column
+    (128, 896, 16641),     # ranges of 80 columns, the last of one
+    (77, 128, 66001),      # ranges of 272 columns: two tiles of 144 and 128, the last range ragged
+    (128, 256, 140000),    # ranges of 560 columns: three tiles
+])
+@pytest.mark.parametrize("T", [1.0, 0.3])
+def test_forward_over_few_tokens(dev, n, h, v, T):
+    """Up to 128 tokens every workgroup streams an equal range of the vocabulary; labels sit on the first and last column
+    of the vocabulary and around the edges of ranges and tiles."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    from oracle import masked as OM
+    hidden, weight, labels = (t.to(dev) for t in _make(n, h, v, seed=n + v))
+    edges = [0, v - 1, 63, 64, 79, 80, 143, 144, 191, 192, 255, 256, 271, 272, 559, 560]
+    for i, e in enumerate(edges[:n]):
+        labels[i] = min(e, v - 1)
+    lp, ent, pi2 = K.linear_cross_entropy_with_sum_pi_squared(hidden, weight, labels, T)
+    lp0, ent0, _, _ = K.efficient_entropy_forward(hidden, weight, labels, 0, T)
+    assert torch.equal(lp, lp0) and torch.equal(ent, ent0)
+    want_lp, want_ent = OH.head_fp32_ground_truth(hidden.float(), weight.float(), labels, T)
+    assert (lp - want_lp).abs().max() <= ATOL and (ent - want_ent).abs().max() <= ATOL
+    want_pi2 = OM.sum_pi_squared_from_logits(hidden.float() @ weight.float().t() / T)
+    assert torch.allclose(pi2, want_pi2, rtol=2e-3, atol=1e-9)

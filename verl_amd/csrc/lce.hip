@@ -91,6 +91,7 @@ struct FwdPlan {
   int waves;      // bands: eight full bands each, one per XCD
   int count[4];   // bands: rounds of a band of 1, 2, 4, 8 token tiles
   int rounds;     // bands: rounds of all bands after the waves together, below 2^27
+  int few_cols;   // not 0: lce_forward_few_kernel, `splits` workgroups of this many columns each
 
   // Everything a workgroup asks of the plan is additions, shifts and comparisons of uniform 32-bit values: it is asked
   // with a tile's accumulators in registers, where a division would spill them.
@@ -580,6 +581,189 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   }
 }
 
+// The forward pass over at most kFewTokens tokens.  It is bound by reading the weight: with a 256-token tile the matrix cores
+// spend most of their time on padding (93 tokens x 896 x 151936: 68 us, 4 TB/s), with 128 tokens the MFMAs of a 256-row slab
+// of the weight take about half as long as the slab takes out of HBM.  Every workgroup streams an equal range of weight rows,
+// cut into tiles of equal height up to 256 whose rows only are fetched, through three LDS stages, so that two slabs (up to
+// 16 MB over the chip) are in flight while one is multiplied; one barrier per slab: 53.6 us, 5.1 TB/s; whole pass 76 -> 60 us;
+// 93 x 3584 x 152064 5.4 TB/s, 93 x 4096 x 128256 5.7 TB/s.  From 129 tokens on the 256-token tile's padding is less than half.  A wavefront owns 64 tokens
+// x 64 columns (2 x 4 wavefronts) and keeps the softmax state of its tokens in registers to the end.
+constexpr int kFewTokens = 128;
+constexpr int kFewStageBytes = (kFewTokens + kTile) * kBK * 2;
+constexpr int kFewStages = 3;
+constexpr int kFewLds = kFewStages * kFewStageBytes;
+constexpr int kFewWavesR = 2, kFewWavesC = 4, kFewMB = kTile / kBlk / kFewWavesC;
+constexpr int kFewLoadsR = kFewTokens * 8 / kThreads;  // transfers per lane of one slab of hidden (2)
+static_assert(kFewLoadsR + kLoads == 6, "the s_waitcnt vmcnt(6) of lce_forward_few_kernel counts the transfers of one slab");
+static_assert(kFewTokens == kFewWavesR * kNB * kBlk, "a wavefront owns kNB blocks of tokens");
+
+template <bool PI2>
+__global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int split = xcd_regroup(blockIdx.x, gridDim.x);
+  const int c_begin = split * a.plan.few_cols;
+  const int c_end = c_begin + a.plan.few_cols < a.vocab ? c_begin + a.plan.few_cols : a.vocab;  // > c_begin
+  const int w = threadIdx.x >> 6, lx = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
+  const int wr = w % kFewWavesR, wc = w / kFewWavesR;
+
+  // tiles of equal height, rows past a tile's read as zero without being fetched
+  const int tiles = (c_end - c_begin + kTile - 1) / kTile, slabs = tiles * a.k_slabs;
+  const int tile_cols = ((c_end - c_begin + tiles - 1) / tiles + kBlk - 1) / kBlk * kBlk;
+  auto tile_end = [&](int t) {
+    const int end = c_begin + (t + 1) * tile_cols;
+    return end < c_end ? end : c_end;
+  };
+  auto weight_rsrc = [&](int t) {
+    Operand weight = a.weight;
+    weight.x_extent = tile_end(t);
+    return tile_rsrc<false>(weight, c_begin + t * tile_cols);
+  };
+  SlabDma<false> dma;       // the same for both operands: their rows are the same distance apart
+  dma.init(a.hidden);
+  FragAddr<false> fr, fc;
+  fr.init(wr * kNB, kNB);
+  fc.init(wc * kFewMB, kFewMB);
+
+  int label[kNB];
+  float m[kNB], s[kNB], sy[kNB], s2[kNB], zl[kNB];
+#pragma unroll
+  for (int nb = 0; nb < kNB; ++nb) {
+    const int tok = wr * (kNB * kBlk) + nb * kBlk + lx;
+    label[nb] = tok < a.n_tokens ? (int)a.labels[tok] : -1;
+    m[nb] = kNegBig;
+    s[nb] = sy[nb] = s2[nb] = zl[nb] = 0.f;
+  }
+
+  // fetch cursor; past the end it stays on the last slab
+  const u32x4 rs_r = tile_rsrc<false>(a.hidden, 0);
+  u32x4 rs_c = weight_rsrc(0);
+  int t2 = 0, k2 = 0, fill = 0;
+  auto fetch = [&]() {
+    const SlabSrc r{rs_r, slab_soff<false>(a.hidden, k2 * kBK)}, c{rs_c, slab_soff<false>(a.weight, k2 * kBK)};
+    const unsigned base = lds_address(lds) + (unsigned)fill * kFewStageBytes;
+#pragma unroll
+    for (int i = 0; i < kFewLoadsR; ++i) dma.issue_one(i, r, base);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) dma.issue_one(i, c, base + kFewTokens * kBK * 2);
+    fill = fill == kFewStages - 1 ? 0 : fill + 1;
+    if (t2 == tiles - 1 && k2 == a.k_slabs - 1) return;
+    if (++k2 == a.k_slabs) {
+      k2 = 0;
+      ++t2;
+      rs_c = weight_rsrc(t2);
+    }
+  };
+  fetch();
+  fetch();
+
+  f32x4 acc[kFewMB][kNB];
+  int kt = 0, tile = 0, stage = 0;
+  for (int it = 0; it < slabs; ++it) {
+    if (kt == 0) {
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < kNB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // slab `it` has landed (all but the six transfers of the next one), and nobody reads the stage before it any more:
+    // that one takes slab it + 2
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    fetch();
+    const char* cur = lds + stage * kFewStageBytes;
+    stage = stage == kFewStages - 1 ? 0 : stage + 1;
+    bf16x8 r[kSteps][kNB], c[kSteps][kFewMB];
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) {
+#pragma unroll
+      for (int nb = 0; nb < kNB; ++nb) r[ks][nb] = fr.read(cur, ks, nb);
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb) c[ks][mb] = fc.read(cur + kFewTokens * kBK * 2, ks, mb);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < kNB; ++nb)
+          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[ks][mb], r[ks][nb], acc[mb][nb], 0, 0, 0);
+    if (++kt < a.k_slabs) continue;
+    kt = 0;
+    // the tile is done: online softmax over its columns, as in FwdEpi
+    const int col0 = c_begin + tile * tile_cols + wc * (kFewMB * kBlk) + 4 * lq;  // column of element (0, 0) of the lane
+    const int cols_left = tile_end(tile) - col0;
+    ++tile;
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      float xmax = kNegBig, add = 0.f;
+      const int mine = label[nb] - col0;
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float x = mb * kBlk + v < cols_left ? acc[mb][nb][v] : kNoColumn;
+          acc[mb][nb][v] = x;
+          xmax = fmaxf(xmax, x);
+          add += mb * kBlk + v == mine && mine < cols_left ? x * a.rcp_t : 0.f;
+        }
+      zl[nb] += add;
+      const float m_new = fmaxf(m[nb], xmax * a.scale2);
+      const float resc = fast_exp2(m[nb] - m_new);
+      float s_ = s[nb] * resc, sy_ = sy[nb] * resc, s2_ = PI2 ? s2[nb] * resc * resc : 0.f;
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float x = acc[mb][nb][v];
+          const float e = fast_exp2(fmaf(x, a.scale2, -m_new));
+          s_ += e;
+          sy_ = fmaf(e, x, sy_);
+          if (PI2) s2_ = fmaf(e, e, s2_);
+        }
+      m[nb] = m_new;
+      s[nb] = s_;
+      sy[nb] = sy_;
+      if (PI2) s2[nb] = s2_;
+    }
+  }
+
+  // the four lane quarters, then the four wavefronts that share 64 tokens, hold disjoint columns
+#pragma unroll
+  for (int step = 16; step <= 32; step <<= 1)
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      zl[nb] += __shfl_xor(zl[nb], step, 64);
+      const float m2 = __shfl_xor(m[nb], step, 64), b2 = __shfl_xor(s[nb], step, 64), y2 = __shfl_xor(sy[nb], step, 64);
+      if (PI2) merge_state(m[nb], s[nb], sy[nb], s2[nb], m2, b2, y2, __shfl_xor(s2[nb], step, 64));
+      else merge_state(m[nb], s[nb], sy[nb], m2, b2, y2);
+    }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the stages are free
+  float4* red = reinterpret_cast<float4*>(lds);                                          // [4][128]
+  float* redq = reinterpret_cast<float*>(lds + kFewWavesC * kFewTokens * sizeof(float4));  // [4][128] squared sums
+  if (lq == 0) {
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) {
+      const int row = wr * (kNB * kBlk) + nb * kBlk + lx;
+      red[wc * kFewTokens + row] = make_float4(m[nb], s[nb], sy[nb], zl[nb]);
+      if (PI2) redq[wc * kFewTokens + row] = s2[nb];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < kFewTokens) {
+    const int row = threadIdx.x;
+    float4 x = red[row];
+    float q = PI2 ? redq[row] : 0.f;
+#pragma unroll
+    for (int j = 1; j < kFewWavesC; ++j) {
+      const float4 y = red[j * kFewTokens + row];
+      if (PI2) merge_state(x.x, x.y, x.z, q, y.x, y.y, y.z, redq[j * kFewTokens + row]);
+      else merge_state(x.x, x.y, x.z, y.x, y.y, y.z);
+      x.w += y.w;
+    }
+    a.partials[(int64_t)split * kTile + row] = x;
+    if (PI2) a.pi2_partials[(int64_t)split * kTile + row] = q;
+  }
+}
+
 struct MergeArgs {
   const float4* partials;
   const float* pi2_partials;  // null unless sum_pi_squared is wanted
@@ -1064,6 +1248,8 @@ static int ensure_lds_attributes() {
   if ((s = allow_big_lds(lce_forward_kernel<false, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_kernel<true, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_kernel<true, true>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<false>, kFewLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<true>, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_dgrad_kernel, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
   done[dev] = true;
@@ -1079,8 +1265,8 @@ static inline int64_t dz_pitch(int64_t cv) { return cv + 128; }
 
 // max_slots: most partial states (of 256 tokens each) the caller's buffer holds; the built-in buffer of the entry point that
 // allocates nothing is sized for 256 CUs and must serve a part with more of them too.
-static FwdPlan plan_forward(int64_t tok_tiles, int64_t voc_tiles, bool one_tile_only, int64_t max_slots = INT64_MAX) {
-  const int64_t cus = device_cu_count();
+static FwdPlan plan_forward(int64_t n_tokens, int64_t vocab, bool one_tile_only, int64_t max_slots = INT64_MAX) {
+  const int64_t cus = device_cu_count(), tok_tiles = ceil_div(n_tokens, kTile), voc_tiles = ceil_div(vocab, kTile);
   FwdPlan p{};
   p.tok_tiles = (int)tok_tiles;
   p.voc_tiles = (int)voc_tiles;
@@ -1089,6 +1275,13 @@ static FwdPlan plan_forward(int64_t tok_tiles, int64_t voc_tiles, bool one_tile_
   if (sp < 1) sp = 1;
   if (sp > voc_tiles) sp = voc_tiles;
   p.splits = (int)sp;
+  if (n_tokens <= kFewTokens && !one_tile_only) {
+    // equal ranges of weight rows; 64 rows are the least that is worth a workgroup
+    const int64_t even = ceil_div(ceil_div(vocab, cus < max_slots ? cus : max_slots), kBlk) * kBlk;
+    p.few_cols = (int)(even < 64 ? 64 : even);
+    p.splits = (int)ceil_div(vocab, p.few_cols);
+    return p;
+  }
   if (one_tile_only || cus % (8 * kXcds) != 0) return p;
   const int64_t split_rounds = ceil_div(tok_tiles * sp, cus) * ceil_div(voc_tiles, sp);
   FwdPlan b = p;
@@ -1230,10 +1423,9 @@ extern "C" int vamd_lce_timing_collect(double* ms_by_kernel, int64_t* launches_b
 extern "C" size_t vamd_lce_forward_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab) {
   (void)hidden_size;
   if (n_tokens <= 0 || vocab <= 0) return 0;
-  const int64_t tok_tiles = ceil_div(n_tokens, kTile), voc_tiles = ceil_div(vocab, kTile);
   int64_t slots = 0;  // with a logits cache the launch has one token tile per workgroup
   for (bool one_tile_only : {false, true}) {
-    const int64_t n = plan_forward(tok_tiles, voc_tiles, one_tile_only).slots();
+    const int64_t n = plan_forward(n_tokens, vocab, one_tile_only).slots();
     if (n > slots) slots = n;
   }
   return (size_t)slots * kTile * (sizeof(float4) + sizeof(float));  // state + squared sums
@@ -1253,7 +1445,7 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   a.n_tokens = (int)n_tokens;
   a.vocab = (int)vocab;
   a.k_slabs = (int)(hidden_size / kBK);
-  a.plan = plan_forward(ceil_div(n_tokens, kTile), ceil_div(vocab, kTile), logits_cache != nullptr, max_slots);
+  a.plan = plan_forward(n_tokens, vocab, logits_cache != nullptr, max_slots);
   a.scale2 = rcp_temperature * kLog2e;
   a.rcp_t = rcp_temperature;
   a.partials = static_cast<float4*>(workspace);
@@ -1271,6 +1463,11 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
         hipLaunchKernelGGL((lce_forward_kernel<true, true>), grid, block, kLdsBytes + kCacheStageBytes, s, a);
       else
         hipLaunchKernelGGL((lce_forward_kernel<true, false>), grid, block, kLdsBytes + kCacheStageBytes, s, a);
+    } else if (a.plan.few_cols) {
+      if (sum_pi_squared)
+        hipLaunchKernelGGL((lce_forward_few_kernel<true>), grid, block, kFewLds, s, a);
+      else
+        hipLaunchKernelGGL((lce_forward_few_kernel<false>), grid, block, kFewLds, s, a);
     } else {
       if (sum_pi_squared)
         hipLaunchKernelGGL((lce_forward_kernel<false, true>), grid, block, kLdsBytes + kFwdTokenLds, s, a);

@@ -57,6 +57,26 @@ def test_logprobs_and_entropy_from_logits_forward(dev, dtype, n, v):
     assert (ent32 >= -1e-4).all() and (ent32 <= math.log(v) + 1e-4).all()
 
 
+@pytest.mark.parametrize("dtype,v", [(torch.float32, 16383), (torch.float32, 16384), (torch.float32, 33001),
+                                     (torch.bfloat16, 32767), (torch.bfloat16, 32768), (torch.bfloat16, 66007),
+                                     (torch.float16, 32776), (torch.float16, 98304)])
+@pytest.mark.parametrize("extra_rows", [None, 0, 1])
+def test_few_long_rows_and_one_row_more_than_compute_units(dev, dtype, v, extra_rows):
+    """Rows of 64 KB and more take a wider workgroup while there are no more of them than compute units; both sides of
+    both lines, labels on the first and last column."""
+    import verl_amd.utils.torch_functional as F
+    n = 3 if extra_rows is None else torch.cuda.get_device_properties(dev).multi_processor_count + extra_rows
+    z, labels = _logits(n, v, dtype, seed=n + v)
+    labels[0], labels[1] = 0, v - 1
+    z64 = z.double()
+    lse = torch.logsumexp(z64, -1)
+    want_lp = z64.gather(1, labels[:, None])[:, 0] - lse
+    want_ent = lse - (torch.exp(z64 - lse[:, None]) * z64).sum(-1)
+    zd = z.to(dev)
+    _assert_close(F.logprobs_from_logits(zd, labels.to(dev)), want_lp, dtype, "logprobs")
+    _assert_close(F.entropy_from_logits_with_chunking(zd), want_ent, torch.float32, "entropy", atol=2e-5)
+
+
 def test_logits_with_batch_dimensions_row_pitch_and_infinities(dev):
     import verl_amd.utils.torch_functional as F
     b, s, v = 3, 50, 777

@@ -3,8 +3,8 @@
 // :224-263 entropy_from_logits / _with_chunking, :203-221 clip_by_value).
 //
 // Forward: one pass over a row of logits with an online softmax (running max, sum e, sum e*z per thread, merged over
-// the workgroup), one workgroup per row, 16-byte loads, four of them in flight per thread.  Algorithmic traffic: the
-// logits once.  Backward: elementwise over [rows, vocab], d_logits = g_lp (onehot - p) - g_ent p (z - mean_z) with
+// the workgroup), one workgroup per row, 16-byte loads, four of them in flight per thread; bound by HBM, over few rows by
+// the latency of a row's trips.  Algorithmic traffic: the logits once.  Backward: elementwise over [rows, vocab], d_logits = g_lp (onehot - p) - g_ent p (z - mean_z) with
 // p = exp(z - lse): logits in, gradient out (in place if the caller passes the same buffer).
 #include "common.h"
 
@@ -12,6 +12,8 @@ namespace vamd {
 namespace {
 
 constexpr int kRowThreads = 256;
+constexpr int kWideRowThreads = 1024;           // forward, few long rows: launch_stats()
+constexpr int64_t kWideRowBytes = 64 * 1024;
 constexpr int kInFlight = 4;  // 16-byte loads a thread issues before it consumes them
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -89,15 +91,15 @@ struct StatsArgs {
   float* mean_z;
 };
 
-template <class D, bool VEC>
-__global__ __launch_bounds__(kRowThreads) void row_softmax_stats_kernel(StatsArgs a) {
+template <class D, bool VEC, int NT>
+__global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
   using T = typename D::type;
   constexpr int G = D::kVec;
   const int64_t r = blockIdx.x;
   const T* __restrict__ row = static_cast<const T*>(a.logits) + r * a.ld;
   // running state in the log2 domain: m = max of z log2(e), s = sum 2^(y - m), sz = sum 2^(y - m) z
   float m = kNegBig, s = 0.f, sz = 0.f;
-  const int64_t stride = (int64_t)kRowThreads * G;
+  const int64_t stride = (int64_t)NT * G;
   for (int64_t c0 = (int64_t)threadIdx.x * G; c0 < a.cols; c0 += stride * kInFlight) {
     // whole 16-byte groups are all requested first; a ragged last group is fetched element by element afterwards
     u32x4_t raw[kInFlight];
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_stats_kernel(StatsArg
     const float m2 = __shfl_xor(m, off, 64), s2 = __shfl_xor(s, off, 64), sz2 = __shfl_xor(sz, off, 64);
     merge(m, s, sz, m2, s2, sz2);
   }
-  __shared__ float red[3][kRowThreads / 64];
+  __shared__ float red[3][NT / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) {
     red[0][w] = m;
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_stats_kernel(StatsArg
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int j = 1; j < kRowThreads / 64; ++j) merge(m, s, sz, red[0][j], red[1][j], red[2][j]);
+    for (int j = 1; j < NT / 64; ++j) merge(m, s, sz, red[0][j], red[1][j], red[2][j]);
     const float lse = (m + log2f(s)) * kLn2;
     const float mz = sz / s;
     if (a.lse) a.lse[r] = lse;
@@ -293,6 +295,21 @@ int check_rows(const char* what, const void* logits, int dtype, int64_t n_rows, 
   return VAMD_OK;
 }
 
+// Threads per row.  Up to one row per CU a workgroup has the CU to itself, and a row is a chain of dependent trips to HBM, each
+// as long as NT * kInFlight * 16 bytes: 1024 threads make it a quarter of the length (64 rows x 152064 bf16 24.4 -> 13.3 us,
+// 200 rows 25.5 -> 15.2; 64 rows x 128256 fp32 32.8 -> 14.0, 200 rows 35.1 -> 18.6).  From more rows than CUs on, 256-thread
+// workgroups (eight to a CU) fill the chip more evenly: 520 x 152064 bf16 32.8 us against 38.4, 3001 rows 142 against 153,
+// 4096 rows 188 against 199.  A row below 64 KB (a trip of the wide workgroup) is not worth the wider reduction: 64 rows x
+// 16384 bf16 4.8 us against 5.2; at 64 KB 7.1 against 5.4.  512 threads or eight loads in flight lie between the two.
+template <class D, bool VEC>
+void launch_stats(const StatsArgs& a, int64_t n_rows, hipStream_t s) {
+  const dim3 grid((unsigned)n_rows);
+  if (n_rows <= device_cu_count() && a.cols * (int64_t)sizeof(typename D::type) >= kWideRowBytes)
+    hipLaunchKernelGGL((row_softmax_stats_kernel<D, VEC, kWideRowThreads>), grid, dim3(kWideRowThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((row_softmax_stats_kernel<D, VEC, kRowThreads>), grid, dim3(kRowThreads), 0, s, a);
+}
+
 }  // namespace
 }  // namespace vamd
 
@@ -315,10 +332,8 @@ extern "C" int vamd_row_softmax_stats(const void* logits, int dtype, int64_t n_r
   StatsArgs a{logits, ld, labels, vocab, logprobs, entropy, lse, mean_z};
   hipStream_t s = static_cast<hipStream_t>(stream);
   VAMD_DTYPE_DISPATCH(dtype, D, {
-    if (rows_vectorizable<D>(logits, ld))
-      hipLaunchKernelGGL((row_softmax_stats_kernel<D, true>), dim3((unsigned)n_rows), dim3(kRowThreads), 0, s, a);
-    else
-      hipLaunchKernelGGL((row_softmax_stats_kernel<D, false>), dim3((unsigned)n_rows), dim3(kRowThreads), 0, s, a);
+    if (rows_vectorizable<D>(logits, ld)) launch_stats<D, true>(a, n_rows, s);
+    else launch_stats<D, false>(a, n_rows, s);
   });
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;

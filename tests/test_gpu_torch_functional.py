@@ -77,6 +77,34 @@ def test_few_long_rows_and_one_row_more_than_compute_units(dev, dtype, v, extra_
     _assert_close(F.entropy_from_logits_with_chunking(zd), want_ent, torch.float32, "entropy", atol=2e-5)
 
 
+@pytest.mark.parametrize("dtype,v", [(torch.float32, 3), (torch.float32, 1001), (torch.bfloat16, 7), (torch.bfloat16, 1003),
+                                     (torch.bfloat16, 33001), (torch.float16, 9), (torch.float16, 2049)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rows_aligned_to_their_elements_only(dev, dtype, v, offset):
+    """Rows of an odd pitch, and rows that begin one element into their storage: values and gradients, and nothing outside
+    the rows is touched by the in-place gradient."""
+    from verl_amd import _cabi
+    import verl_amd.utils.torch_functional as F
+    n, guard = 5, 16
+    z, labels = _logits(n, v, dtype, seed=v + offset)
+    z64 = z.double().requires_grad_()
+    lse = torch.logsumexp(z64, -1)
+    want = z64.gather(1, labels[:, None])[:, 0] - lse
+    g = torch.randn(n, generator=torch.Generator().manual_seed(v))
+    (want_d,) = torch.autograd.grad(want, z64, g.double())
+    buf = torch.full((guard + offset + n * v + guard,), 77.0, dtype=dtype, device=dev)
+    rows = buf[guard + offset:guard + offset + n * v].view(n, v)
+    rows.copy_(z)
+    lab = labels.to(dev)
+    logprobs, entropy, lse_d, mean_z = F._row_stats(rows, v, lab, True, True, True)
+    _assert_close(logprobs, want.detach(), torch.float32, "logprobs")
+    p64 = torch.exp(z64 - lse[:, None]).detach()
+    _assert_close(entropy, (lse - (p64 * z64).sum(-1)).detach(), torch.float32, "entropy", atol=2e-5)
+    F._row_backward(rows, v, lab, lse_d, None, g.to(dev), None, True)
+    _assert_close(rows, want_d, dtype, "d_logits")
+    assert bool((buf[:guard + offset] == 77.0).all()) and bool((buf[guard + offset + n * v:] == 77.0).all())
+
+
 def test_logits_with_batch_dimensions_row_pitch_and_infinities(dev):
     import verl_amd.utils.torch_functional as F
     b, s, v = 3, 50, 777

@@ -6,6 +6,8 @@
 // the workgroup), one workgroup per row, 16-byte loads, four of them in flight per thread; bound by HBM, over few rows by
 // the latency of a row's trips.  Algorithmic traffic: the logits once.  Backward: elementwise over [rows, vocab], d_logits = g_lp (onehot - p) - g_ent p (z - mean_z) with
 // p = exp(z - lse): logits in, gradient out (in place if the caller passes the same buffer).
+#include <type_traits>
+
 #include "common.h"
 
 namespace vamd {
@@ -41,30 +43,39 @@ struct alignas(16) Pack {
   typename D::type v[D::kVec];
 };
 
-// Load the D::kVec elements starting at column c of a row (those at or beyond `cols` read as `fill`).
+// Rows on 16-byte boundaries (VEC) promise that to the compiler; others (an odd vocabulary, a column slice) only the alignment
+// of their elements.  The memory pipeline takes a 16-byte access at either, so a whole group is one instruction in both.  Element
+// by element, as it was, an instruction moved an eighth (fp32: a quarter) of the bytes: 3001 x 152063 bf16 forward 555 -> 187 us,
+// backward 956 -> 296 (152064 columns: 141 and 283); 1500 x 152063 fp32 forward 217 -> 152, backward 566 -> 318 (140 and 298).
+typedef unsigned u32x4_at4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned u32x4_at2_t __attribute__((ext_vector_type(4), aligned(2)));
 template <class D, bool VEC>
-__device__ __forceinline__ void load_group(const typename D::type* __restrict__ row, int64_t c, int64_t cols,
-                                           float fill, float (&x)[D::kVec]) {
-  if (VEC && c + D::kVec <= cols) {
-    // logits are read once and never again by this launch: non-temporal, which is worth 7 % of HBM bandwidth here
-    const u32x4_t raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row + c));
-    const Pack<D> p = __builtin_bit_cast(Pack<D>, raw);
+struct Group {
+  using type = std::conditional_t<VEC, u32x4_t, std::conditional_t<sizeof(typename D::type) == 4, u32x4_at4_t, u32x4_at2_t>>;
+};
+
+// logits are read once and never again by a launch: non-temporal, which is worth 7 % of HBM bandwidth here
+template <class D, bool VEC>
+__device__ __forceinline__ u32x4_t load_whole(const typename D::type* __restrict__ p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const typename Group<D, VEC>::type*>(p));
+}
+
+// The ragged group a row ends in: elements at or beyond `cols` read as `fill`.
+template <class D>
+__device__ __forceinline__ void load_ragged(const typename D::type* __restrict__ row, int64_t c, int64_t cols,
+                                            float fill, float (&x)[D::kVec]) {
 #pragma unroll
-    for (int e = 0; e < D::kVec; ++e) x[e] = to_float(p.v[e], D());
-  } else {
-#pragma unroll
-    for (int e = 0; e < D::kVec; ++e) x[e] = (c + e < cols) ? to_float(row[c + e], D()) : fill;
-  }
+  for (int e = 0; e < D::kVec; ++e) x[e] = (c + e < cols) ? to_float(row[c + e], D()) : fill;
 }
 
 template <class D, bool VEC>
 __device__ __forceinline__ void store_group(typename D::type* __restrict__ row, int64_t c, int64_t cols,
                                             const float (&x)[D::kVec]) {
-  if (VEC && c + D::kVec <= cols) {
+  if (c + D::kVec <= cols) {
     Pack<D> p;
 #pragma unroll
     for (int e = 0; e < D::kVec; ++e) p.v[e] = from_float(x[e], D());
-    __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, p), reinterpret_cast<u32x4_t*>(row + c));
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, p), reinterpret_cast<typename Group<D, VEC>::type*>(row + c));
   } else {
 #pragma unroll
     for (int e = 0; e < D::kVec; ++e)
@@ -106,18 +117,18 @@ __global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
       const int64_t c = c0 + u * stride;
-      if (VEC && c + G <= a.cols) raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row + c));
+      if (c + G <= a.cols) raw[u] = load_whole<D, VEC>(row + c);
     }
     float x[kInFlight][G];
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
       const int64_t c = c0 + u * stride;
-      if (VEC && c + G <= a.cols) {
+      if (c + G <= a.cols) {
         const Pack<D> p = __builtin_bit_cast(Pack<D>, raw[u]);
 #pragma unroll
         for (int e = 0; e < G; ++e) x[u][e] = to_float(p.v[e], D());
       } else if (c < a.cols) {
-        load_group<D, false>(row, c, a.cols, kNegBig, x[u]);
+        load_ragged<D>(row, c, a.cols, kNegBig, x[u]);
       } else {
 #pragma unroll
         for (int e = 0; e < G; ++e) x[u][e] = kNegBig;
@@ -217,19 +228,19 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(Backw
 #pragma unroll
   for (int u = 0; u < F; ++u) {
     const int64_t c = c0 + u * stride;
-    if (VEC && c + G <= a.cols) raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row + c));
+    if (c + G <= a.cols) raw[u] = load_whole<D, VEC>(row + c);
   }
   float x[F][G];
 #pragma unroll
   for (int u = 0; u < F; ++u) {
     const int64_t c = c0 + u * stride;
     if (c >= a.cols) continue;
-    if (VEC && c + G <= a.cols) {
+    if (c + G <= a.cols) {
       const Pack<D> p = __builtin_bit_cast(Pack<D>, raw[u]);
 #pragma unroll
       for (int e = 0; e < G; ++e) x[u][e] = to_float(p.v[e], D());
     } else {
-      load_group<D, false>(row, c, a.cols, 0.f, x[u]);
+      load_ragged<D>(row, c, a.cols, 0.f, x[u]);
     }
     // the label's place in this group as a 32-bit index (-1: not here): one 32-bit compare per element below
     const int64_t hit64 = label - c;

@@ -703,6 +703,8 @@ def test_backward_shares_d_hidden_out_in_pieces(dev, n, h, v, chunk, need):
     (10999, 33001),   # 43 token tiles: bands of 8, 2 and 1, shares that cross from band to band
     (32900, 1000),    # 129 token tiles, 4 vocabulary tiles: several bands per share, fewer columns than workgroups
     (2100, 151936),   # 9 token tiles: one full band and a single tile
+    (22000, 33001),   # 86 token tiles: a wave of 33 rounds, then bands of 8, 8, 4 and 2 in shares of 11 or 12 rounds that
+                      # cross from band to band: a workgroup changes its labels and its state up to twice
 ])
 def test_forward_in_bands_of_token_tiles(dev, n, v):
     """Token counts whose tiles do not divide the chip go through the band schedule of the forward pass, where a

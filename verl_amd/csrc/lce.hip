@@ -16,6 +16,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -156,14 +157,45 @@ struct FwdArgs {
   float* pi2_partials;  // optional [plan.slots()][256] : sum of e^2 relative to the same max
 };
 
-// The tiles of one workgroup: its range of the vocabulary for one token tile (splits), or its column of every band its
-// XCD's share of the rounds touches (bands).
-struct FwdSched {
+// The tiles of one workgroup.  The two ways of sharing out are kernels of their own: with both in one kernel the split
+// walk, whose token tile never changes, carried the bands' lookups and the state's write-out through its tile loop, with 41
+// scalar registers spilled (16384 x 3584 x 152064 12.50 ms, apart 12.47; 3300 x 896 x 151936, in bands, 706 and 699 us).
+template <bool BANDS>
+struct FwdSched;
+
+// splits: one range of the vocabulary for one token tile
+template <>
+struct FwdSched<false> {
+  int k_slabs, tn, vt_begin, ntiles;
+  int64_t slot;  // where the state goes
+
+  __device__ __forceinline__ void init(const FwdPlan& p, int slabs, int wg) {
+    k_slabs = slabs;
+    // bands of 8 token tiles x all splits per XCD
+    const int band = 8 * p.splits, b = wg / band, first = b * 8, w = wg - b * band;
+    const int rows = (p.tok_tiles - first) < 8 ? (p.tok_tiles - first) : 8;
+    const int sp = w / rows;
+    tn = first + w % rows;
+    vt_begin = (int)(((int64_t)sp * p.voc_tiles) / p.splits);
+    ntiles = (int)(((int64_t)(sp + 1) * p.voc_tiles) / p.splits) - vt_begin;
+    slot = (int64_t)sp * p.tok_tiles + tn;
+  }
+  __device__ __forceinline__ int count() const { return ntiles; }
+  __device__ __forceinline__ void tile(int i, int& r0, int& c0) const {
+    r0 = tn * kTile;
+    c0 = (vt_begin + i) * kTile;
+  }
+  __device__ __forceinline__ int slab0(int) const { return 0; }
+  __device__ __forceinline__ int slabs(int) const { return k_slabs; }
+};
+
+// bands: the workgroup's column of every band its XCD's share of the rounds touches
+template <>
+struct FwdSched<true> {
   const FwdPlan* plan;
-  int k_slabs;
-  int tn_, vt_begin, ntiles, slot_;  // splits (ntiles: both)
-  int xcd, member, wave_count;       // bands: this XCD, workgroup within it, its tiles of a wave
-  FwdPlan::Band band0;               // bands: the band its share starts in
+  int k_slabs, ntiles;
+  int xcd, member, wave_count;  // this XCD, workgroup within it, its tiles of a wave
+  FwdPlan::Band band0;          // the band its share starts in
 
   struct Place {
     int tn, vt;    // token tile, vocabulary tile
@@ -180,30 +212,19 @@ struct FwdSched {
     if (n > 0 && first + cols * (n - 1) >= plan->voc_tiles) --n;
     return Column{first, n};
   }
-  __device__ __forceinline__ void init(const FwdPlan& p, int wg) {
+  __device__ __forceinline__ void init(const FwdPlan& p, int slabs, int wg) {
     plan = &p;
-    if (p.splits) {
-      // bands of 8 token tiles x all splits per XCD
-      const int band = 8 * p.splits, b = wg / band, first = b * 8, w = wg - b * band;
-      const int rows = (p.tok_tiles - first) < 8 ? (p.tok_tiles - first) : 8;
-      const int sp = w / rows;
-      tn_ = first + w % rows;
-      vt_begin = (int)(((int64_t)sp * p.voc_tiles) / p.splits);
-      ntiles = (int)(((int64_t)(sp + 1) * p.voc_tiles) / p.splits) - vt_begin;
-      slot_ = sp * p.tok_tiles + tn_;
-    } else {
-      xcd = wg / p.group;
-      member = wg % p.group;
-      band0 = p.band_of_round(p.share_begin(xcd));
-      const int cols = p.group >> 3;
-      wave_count = p.voc_tiles > (member >> 3) ? (p.voc_tiles - (member >> 3) + cols - 1) / cols : 0;
-      ntiles = p.waves * wave_count;
-      for (FwdPlan::Band b = band0; b.start < p.share_begin(xcd + 1); p.next(b)) ntiles += column(b).count;
-    }
+    k_slabs = slabs;
+    xcd = wg / p.group;
+    member = wg % p.group;
+    band0 = p.band_of_round(p.share_begin(xcd));
+    const int cols = p.group >> 3;
+    wave_count = p.voc_tiles > (member >> 3) ? (p.voc_tiles - (member >> 3) + cols - 1) / cols : 0;
+    ntiles = p.waves * wave_count;
+    for (FwdPlan::Band b = band0; b.start < p.share_begin(xcd + 1); p.next(b)) ntiles += column(b).count;
   }
   __device__ __forceinline__ int count() const { return ntiles; }
   __device__ __forceinline__ Place at(int i) const {
-    if (plan->splits) return Place{tn_, vt_begin + i, slot_};
     int left = ntiles;
     for (int w = 0; w < plan->waves; ++w, i -= wave_count, left -= wave_count)
       if (i < wave_count)
@@ -273,6 +294,7 @@ struct BlockExchange {
 
 constexpr int kCacheStageBytes = (kThreads / 64) * 4096;  // one 32 x 32 fp32 patch per wavefront
 // forward without a cache: two sets of labels, label-logit sums, states of one half of the wavefronts (and squared sums)
+static_assert(kLdsBytes % (2 * kTile * 4) == 0, "the sets of labels are told apart by one address bit");
 constexpr int kFwdTokenLds = 2 * kTile * 4 + kThreads * kNB * 4 + kTile * (16 + 4);
 
 __device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float m2, float s2, float sy2) {
@@ -298,22 +320,25 @@ __device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float
 // backward pass can form d_logits without repeating the GEMM.
 // With PI2 a fifth running sum, sum_j e_j^2, is carried, from which sum_j softmax(z)_j^2 follows
 // (calculate_sum_pi_squared_from_logits, verl/utils/torch_functional.py:680-694).
-template <bool CACHE, bool PI2>
+template <bool CACHE, bool PI2, bool BANDS>
 struct FwdEpi {
+  static_assert(!(CACHE && BANDS), "with a logits cache every workgroup has one token tile");
   LanePos p;
   float scale2;
   int vocab;
-  // vectors and not arrays: an array here ends up in scratch memory
-  f32x4 m, s, sy, s2;
+  // vectors where the state is written out in the middle of the tile loop: an array ends up in scratch memory there.
+  // Where it lives to the end an array takes 0.1 - 0.2 % off the pass (21503 x 4096 x 128256 15148 -> 15120 us).
+  using State = std::conditional_t<CACHE || BANDS, f32x4, float[kNB]>;
+  State m, s, sy, s2;
   // The labels of the lane's token rows and the label-logit sums live in LDS behind the pipeline's stages when the
   // kernel has LDS to spare (no logits cache), in registers otherwise: with them in registers the kernel spilled,
   // and every reload of a spilled value waits out the slab transfers in flight (one counter counts both).
   f32x4 zl;  // CACHE
   int lab[kNB];  // CACHE
-  unsigned lab_lds, zl_lds, red_lds;  // LDS byte addresses: labels [2][256] by tile parity and row; sums [kThreads][kNB];
-                                      // states [256] float4, then squared sums [256]
+  unsigned lab_lds, zl_lds, red_lds;  // LDS byte addresses: labels [256] by row, in the set in use of two; sums
+                                      // [kThreads][kNB]; states [256] float4, then squared sums [256]
   const FwdArgs* args;
-  FwdSched sched;
+  FwdSched<BANDS> sched;
   int64_t slot;  // where the state of the token tile at hand goes
   float rcp_t;
   float* z_cache;  // CACHE: [n_tokens][vocab]
@@ -321,23 +346,27 @@ struct FwdEpi {
   int tok0;        // CACHE: first token row of the wavefront
   int n_tokens;
 
-  // the low dwords of the tile's 256 labels, 64 per wavefront of the first four, straight into LDS; a token past the end
-  // reads as label 0, whose sums nobody looks at
+  // When the token tile changes: the low dwords of its 256 labels, 64 per wavefront of the first four, straight into LDS;
+  // a token past the end reads as label 0, whose sums nobody looks at.  They go into the set that is not in use: other
+  // wavefronts may still be in the epilogue that reads this one.
   __device__ __forceinline__ void prefetch(int tile, int r0, int) {
     if constexpr (!CACHE) {
-      const FwdSched::Place here = sched.at(tile);
-      if (here.slot != slot) {  // the token tile is another one (here no accumulators are alive)
-        if (tile > 0) write_state();
+      if constexpr (BANDS) {
+        const auto here = sched.at(tile);
+        if (here.slot == slot) return;
+        if (tile > 0) write_state();  // (here no accumulators are alive)
         slot = here.slot;
+        lab_lds ^= kTile * 4;
+      } else if (tile > 0) {
+        return;
       }
       const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
       if (w < 4) {
         const u32x4 rs = span_rsrc(args->labels, (int64_t)args->n_tokens * 8);
-        load_to_lds_4(rs, ((unsigned)r0 + 64u * w + (threadIdx.x & 63u)) * 8u, label_set(tile) + 64u * w * 4u);
+        load_to_lds_4(rs, ((unsigned)r0 + 64u * w + (threadIdx.x & 63u)) * 8u, lab_lds + 64u * w * 4u);
       }
     }
   }
-  __device__ __forceinline__ unsigned label_set(int tile) const { return lab_lds + (unsigned)(tile & 1) * (kTile * 4); }
 
   __device__ __forceinline__ void reset() {
 #pragma unroll
@@ -417,7 +446,7 @@ struct FwdEpi {
     reset();
   }
 
-  __device__ __forceinline__ void operator()(Accum& acc, int tile, int /*r0*/, int c0) {
+  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int /*r0*/, int c0) {
     const bool ragged = c0 + kTile > vocab;
     // element (mb, v) of the lane is column 16 mb + v of this: comparing immediates with one register, where a column
     // number per element would be computed ahead of the tile loop and held (or spilled) through it
@@ -469,7 +498,7 @@ struct FwdEpi {
       typedef float __attribute__((address_space(3))) * lds_f32_t;
       int label;
       if constexpr (CACHE) label = lab[nb];
-      else label = *(lds_i32_t)(uintptr_t)(label_set(tile) + 4u * (unsigned)acc_row(p, nb));
+      else label = *(lds_i32_t)(uintptr_t)(lab_lds + 4u * (unsigned)acc_row(p, nb));
       const int rel = label - c0 - p.wc * 128;
       if (__any(rel >= 0 && rel < 128)) {
         float add = 0.f;
@@ -510,32 +539,32 @@ struct FwdEpi {
   }
 };
 
-template <bool CACHE, bool PI2>
+template <bool CACHE, bool PI2, bool BANDS>
 __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  FwdSched sched;
-  sched.init(a.plan, xcd_regroup(blockIdx.x, gridDim.x));
-  sched.k_slabs = a.k_slabs;
+  FwdSched<BANDS> sched;
+  sched.init(a.plan, a.k_slabs, xcd_regroup(blockIdx.x, gridDim.x));
 
-  FwdEpi<CACHE, PI2> epi;
+  FwdEpi<CACHE, PI2, BANDS> epi;
   epi.p = lane_pos();
   epi.scale2 = a.scale2;
   epi.vocab = a.vocab;
   epi.rcp_t = a.rcp_t;
   epi.args = &a;
   epi.sched = sched;
-  epi.slot = -1;
+  if constexpr (BANDS) epi.slot = -1;
+  else epi.slot = sched.slot;
   epi.reset();
   if constexpr (CACHE) {
 #pragma unroll
     for (int nb = 0; nb < kNB; ++nb) {
       epi.zl[nb] = 0.f;
-      const int tok = sched.tn_ * kTile + acc_row(epi.p, nb);
+      const int tok = sched.tn * kTile + acc_row(epi.p, nb);
       epi.lab[nb] = tok < a.n_tokens ? (int)a.labels[tok] : -1;
     }
     epi.z_cache = a.z_cache;
     epi.ex.init(lds + kLdsBytes, epi.p);
-    epi.tok0 = sched.tn_ * kTile + epi.p.wr * (kNB * kBlk);
+    epi.tok0 = sched.tn * kTile + epi.p.wr * (kNB * kBlk);
     epi.n_tokens = a.n_tokens;
   } else {
     typedef float __attribute__((address_space(3))) * lds_f32_t;
@@ -567,7 +596,7 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
     if (threadIdx.x < kTile) {
       const int t = threadIdx.x;
       float4 x = red[t], y = red[kTile + t];
-      const int64_t slot = (int64_t)sched.slot_ * kTile + t;
+      const int64_t slot = sched.slot * kTile + t;
       if (PI2) {
         float q = redq[t];
         merge_state(x.x, x.y, x.z, q, y.x, y.y, y.z, redq[kTile + t]);
@@ -1244,10 +1273,12 @@ static int ensure_lds_attributes() {
   std::lock_guard<std::mutex> lock(mu);
   if (done[dev]) return VAMD_OK;
   int s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, true>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<false, false, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<false, true, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<false, false, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<false, true, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, false, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, true, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_few_kernel<false>, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_few_kernel<true>, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
@@ -1458,22 +1489,19 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   {
     ScopedTiming tm(kTagForward, s);
     const dim3 grid(a.plan.splits ? a.plan.tok_tiles * a.plan.splits : a.plan.group * kXcds), block(kThreads);
-    if (logits_cache) {
-      if (sum_pi_squared)
-        hipLaunchKernelGGL((lce_forward_kernel<true, true>), grid, block, kLdsBytes + kCacheStageBytes, s, a);
-      else
-        hipLaunchKernelGGL((lce_forward_kernel<true, false>), grid, block, kLdsBytes + kCacheStageBytes, s, a);
-    } else if (a.plan.few_cols) {
-      if (sum_pi_squared)
-        hipLaunchKernelGGL((lce_forward_few_kernel<true>), grid, block, kFewLds, s, a);
-      else
-        hipLaunchKernelGGL((lce_forward_few_kernel<false>), grid, block, kFewLds, s, a);
-    } else {
-      if (sum_pi_squared)
-        hipLaunchKernelGGL((lce_forward_kernel<false, true>), grid, block, kLdsBytes + kFwdTokenLds, s, a);
-      else
-        hipLaunchKernelGGL((lce_forward_kernel<false, false>), grid, block, kLdsBytes + kFwdTokenLds, s, a);
-    }
+    auto launch = [&](auto* kernel, size_t lds_bytes) { hipLaunchKernelGGL(kernel, grid, block, lds_bytes, s, a); };
+    const bool pi2 = sum_pi_squared != nullptr;
+    if (logits_cache)
+      launch(pi2 ? lce_forward_kernel<true, true, false> : lce_forward_kernel<true, false, false>,
+             kLdsBytes + kCacheStageBytes);
+    else if (a.plan.few_cols)
+      launch(pi2 ? lce_forward_few_kernel<true> : lce_forward_few_kernel<false>, kFewLds);
+    else if (a.plan.splits)
+      launch(pi2 ? lce_forward_kernel<false, true, false> : lce_forward_kernel<false, false, false>,
+             kLdsBytes + kFwdTokenLds);
+    else
+      launch(pi2 ? lce_forward_kernel<false, true, true> : lce_forward_kernel<false, false, true>,
+             kLdsBytes + kFwdTokenLds);
   }
   VAMD_LAUNCH_CHECK();
 

@@ -168,8 +168,9 @@ int vamd_lce_forward_static(const void* hidden, const void* weight, const int64_
  * at a time (the workspace holds one [n_pad, vocab_chunk] bf16 panel plus fp32 d_hidden
  * accumulators); pass the same value to the workspace query.
  *   vamd_lce_backward_subset is the same over some of the tokens of a call with planned_tokens (>= n_tokens) tokens,
- *   gathered by the caller because the others have no upstream gradient: d_hidden's k range is cut as for the whole
- *   call, so with one vocabulary chunk its rows are the bits the whole call would have given them.
+ *   gathered by the caller because the others have no upstream gradient.  Where the whole call has one vocabulary chunk,
+ *   d_hidden's k range is cut as there and its rows are the bits the whole call would have given them; with several
+ *   chunks, whose width depends on the token count, the two sum over different ranges and n_tokens alone decides.
  */
 #define VAMD_DW_STORE 0
 #define VAMD_DW_ADD_BF16 1

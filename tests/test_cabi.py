@@ -55,6 +55,22 @@ def test_workspace_queries(lib):
     assert lib.vamd_gae_workspace_bytes(512, 4096) >= ticket + 512 * 4 * 8
 
 
+def test_pieces_of_a_call_over_some_of_the_tokens(lib):
+    """As the workspace query shows them: cut like the whole call where that has one vocabulary chunk, on their own where
+    it has several; a planned count below the token count (which the call refuses) is answered too."""
+    subset, whole = lib.vamd_lce_backward_subset_workspace_bytes, lib.vamd_lce_backward_workspace_bytes
+
+    def pieces(n, planned, h, v=152064):
+        panel = -(-n // 256) * 256 * (v + 128) * 2
+        return (subset(n, planned, h, v, 0) - panel) // (n * h * 4)
+
+    assert pieces(200, 1500, 3584) == pieces(1500, 1500, 3584) != pieces(200, 200, 3584)
+    for n, planned, h in ((1000, 11290, 3584), (1300, 8000, 896), (200, 2000, 3584)):
+        assert subset(n, planned, h, 152064, 0) == whole(n, h, 152064, 0) and pieces(n, planned, h) > 1
+    for planned in (0, -5, 1, 99):
+        assert subset(100, planned, 3584, 152064, 0) == whole(100, 3584, 152064, 0)
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(lib):
     rc = lib.vamd_lce_forward(None, None, None, 16, 100, 128, 1.0, None, None, None, None, None, None, None, 0, None)
     assert rc == -1 and b"multiple of 128" in lib.vamd_last_error()

@@ -202,6 +202,27 @@ def test_backward_leaves_out_tokens_without_upstream_gradient(dev, monkeypatch, 
         _close_bf16(dw, grads["0"][1].float().cpu(), "d_weight: active tokens against all tokens")
 
 
+@pytest.mark.parametrize("n,h,v,active", [(1400, 256, 20000, 150), (3000, 384, 9000, 700), (600, 128, 5000, 1)])
+def test_few_active_tokens_of_a_call_with_several_vocabulary_chunks(dev, monkeypatch, n, h, v, active):
+    """The d_logits panel of all tokens takes several vocabulary chunks, that of the active ones fewer: their d_hidden tiles
+    are cut as for a call over them alone, and both gradients are those of the whole call."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    monkeypatch.setenv("VAMD_LCE_DZ_BUDGET_MB", "4")
+    hidden, weight, labels = _make(n, h, v, seed=n + v)
+    g = torch.Generator().manual_seed(n)
+    g_lp = torch.zeros(n)
+    idx = torch.randperm(n, generator=g)[:active].sort().values
+    g_lp[idx] = torch.randn(active, generator=g)
+    hd, wd, ld, gd, at = (t.to(dev) for t in (hidden, weight, labels, g_lp, idx))
+    _, _, lse, mz = K.efficient_entropy_forward(hd, wd, ld, 0, 0.9)
+    dh, dw = K.backward_over_active_tokens(at, gd, None, hd, wd, ld, lse, mz, 0.9, True, True)
+    alone, _ = K.efficient_entropy_backward(gd[at], None, hd[at], wd, ld[at], lse[at], mz[at], 0, 0.9)
+    assert torch.equal(dh[at], alone) and int((dh != 0).any(dim=1).sum()) <= active
+    _, _, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)
+    _close_bf16(dh, want_dh, "d_hidden", e_dh)
+    _close_bf16(dw, want_dw, "d_weight", e_dw)
+
+
 def test_backward_c_abi_refuses_a_call_that_asks_for_nothing(dev):
     from verl_amd import _cabi
     from verl_amd.utils.kernel.linear_cross_entropy import efficient_entropy_backward, efficient_entropy_forward

@@ -1607,11 +1607,17 @@ extern "C" int vamd_lce_forward_static(const void* hidden, const void* weight, c
 }
 
 namespace vamd {
-// Pieces of a d_hidden tile's k range.  Decided for a call with both gradients over `planned_tokens` tokens, whatever
-// part of that is asked for, so that d_hidden is the same bits in all of them; the first (widest) vocabulary chunk
-// decides for all chunks.
-static int d_hidden_pieces(int64_t planned_tokens, int64_t hidden_size, int64_t first_cols) {
-  return plan_gradients(planned_tokens, hidden_size, first_cols, true, true, device_cu_count()).splits;
+// Pieces of a d_hidden tile's k range.  Decided as if both gradients were asked for, whichever are, so that d_hidden is the
+// same bits either way; the first (widest) vocabulary chunk decides for all chunks.  For some of the tokens of a larger call
+// they are that call's pieces, so that its bits come out, where it has one vocabulary chunk.  With several chunks it sums
+// over other ranges anyway: there the tokens at hand decide (1000 of 11290 x 3584 x 152064 would run as 56 whole tiles).
+static int d_hidden_pieces(int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size, int64_t vocab,
+                           int64_t vocab_chunk) {
+  const int64_t cv = default_vocab_chunk(n_tokens, hidden_size, vocab, vocab_chunk);
+  const bool same_ranges =
+      planned_tokens > n_tokens && default_vocab_chunk(planned_tokens, hidden_size, vocab, vocab_chunk) >= vocab;
+  return plan_gradients(same_ranges ? planned_tokens : n_tokens, hidden_size, cv < vocab ? cv : vocab, true, true,
+                        device_cu_count()).splits;
 }
 }  // namespace vamd
 
@@ -1621,7 +1627,7 @@ extern "C" size_t vamd_lce_backward_subset_workspace_bytes(int64_t n_tokens, int
   const int64_t n_pad = ceil_div(n_tokens, kTile) * kTile;
   const int64_t cv = default_vocab_chunk(n_tokens, hidden_size, vocab, vocab_chunk);
   size_t bytes = align_up((size_t)n_pad * dz_pitch(cv) * 2, 256);
-  const int pieces = d_hidden_pieces(planned_tokens, hidden_size, cv < vocab ? cv : vocab);
+  const int pieces = d_hidden_pieces(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk);
   if (pieces > 1 || cv < ceil_div(vocab, kTile) * kTile)
     bytes += align_up((size_t)pieces * n_tokens * hidden_size * 4, 256);
   return bytes;
@@ -1692,7 +1698,7 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
   const int64_t pitch = dz_pitch(cv);
   uint16_t* dz = carve.take<uint16_t>((size_t)n_pad * pitch);
   // a narrower last chunk may fill fewer pieces than the first
-  const int pieces = d_hidden ? d_hidden_pieces(planned_tokens, hidden_size, cv < vocab ? cv : vocab) : 1;
+  const int pieces = d_hidden ? d_hidden_pieces(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk) : 1;
   float* acc32 = (d_hidden && (n_chunks > 1 || pieces > 1)) ? carve.take<float>((size_t)pieces * n_tokens * hidden_size)
                                                             : nullptr;
   const uint16_t* hid = static_cast<const uint16_t*>(hidden);

@@ -221,8 +221,10 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int):
 def backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels, lse, mean_z, temperature,
                                 need_d_hidden: bool, need_d_weight: bool):
     """``efficient_entropy_backward`` over the rows ``idx`` of its per-token arguments; ``d_hidden`` comes back with
-    zero rows for the tokens left out.  ``d_hidden`` rows are the same bits as over all tokens (a row depends on its
-    own token only); ``d_weight`` sums the same non-zero terms in a different grouping."""
+    zero rows for the tokens left out.  ``d_hidden`` rows are the same bits as over all tokens where the backward pass over
+    all of them stages ``d_logits`` in one vocabulary chunk (a row depends on its own token only); with several chunks,
+    whose width depends on the token count, a row is the same sum over other ranges of the vocabulary.  ``d_weight`` sums
+    the same non-zero terms in a different grouping."""
     d_hidden = torch.zeros_like(hidden) if need_d_hidden else None
     if idx.numel() == 0:
         return d_hidden, (torch.zeros_like(weight) if need_d_weight else None)

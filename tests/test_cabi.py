@@ -71,6 +71,38 @@ def test_pieces_of_a_call_over_some_of_the_tokens(lib):
         assert subset(100, planned, 3584, 152064, 0) == whole(100, 3584, 152064, 0)
 
 
+def test_head_size_queries_are_asked_on_the_tensors_device(monkeypatch):
+    """The head's workspaces depend on the compute units of the current device, so the query belongs inside the guard that
+    makes the tensors' device current for the call itself (devices need not be alike)."""
+    import contextlib
+
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    current, asked = ["another"], []
+
+    @contextlib.contextmanager
+    def guard(device):
+        current.append(device)
+        yield
+        current.pop()
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                asked.append((name, current[-1]))
+                return 4096 if name.endswith("_workspace_bytes") else 0
+            return call
+
+    monkeypatch.setattr(_cabi, "lib", Library)
+    monkeypatch.setattr(_cabi, "device_guard", guard)
+    monkeypatch.setattr(_cabi, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(K, "_check_inputs", lambda *tensors: None)
+    hidden, weight = torch.zeros(5, 128, dtype=torch.bfloat16), torch.zeros(16, 128, dtype=torch.bfloat16)
+    labels = torch.zeros(5, dtype=torch.int64)
+    _, _, lse, mean_z = K.efficient_entropy_forward(hidden, weight, labels)
+    K.efficient_entropy_backward(None, None, hidden, weight, labels, lse, mean_z)
+    assert len(asked) == 4 and all(device == hidden.device for _, device in asked), asked
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(lib):
     rc = lib.vamd_lce_forward(None, None, None, 16, 100, 128, 1.0, None, None, None, None, None, None, None, 0, None)
     assert rc == -1 and b"multiple of 128" in lib.vamd_last_error()

@@ -103,6 +103,27 @@ def test_head_size_queries_are_asked_on_the_tensors_device(monkeypatch):
     assert len(asked) == 4 and all(device == hidden.device for _, device in asked), asked
 
 
+def test_a_long_backward_pass_looks_at_its_own_gradients_whatever_ran_before(monkeypatch):
+    """Only short calls are spared the look after one that found every token active, and only with the same head."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.delenv("VAMD_LCE_SKIP_ZERO_GRAD_TOKENS", raising=False)
+    monkeypatch.setattr(K, "_ACTIVE_PROBE", {"rest": 0, "head": None})
+    small, other, large = (1024, 128), (1024, 256), (152064, 3584)
+    dense, masked = torch.ones(2000), torch.cat((torch.zeros(1600), torch.ones(400)))
+    look = lambda g, head: K.active_token_index(g, None, 2000, head)
+    for _ in range(2):                                       # the second time round starts with the first one's state
+        assert look(dense, small) is None
+        for _ in range(3):
+            assert look(masked, large).tolist() == list(range(1600, 2000))
+            assert look(masked, other).numel() == 400
+        assert look(dense, large) is None
+        assert look(masked, other).numel() == 400
+        for _ in range(K._ACTIVE_PROBE_REST):
+            assert look(masked, small) is None
+        assert look(masked, small).numel() == 400
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(lib):
     rc = lib.vamd_lce_forward(None, None, None, 16, 100, 128, 1.0, None, None, None, None, None, None, None, 0, None)
     assert rc == -1 and b"multiple of 128" in lib.vamd_last_error()

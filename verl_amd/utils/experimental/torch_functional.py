@@ -60,7 +60,9 @@ class FusedLinearForPPOFunction(torch.autograd.Function):
         # only the gradient GEMMs whose inputs require a gradient are run (reference :150-156, :184-187), and only over
         # the tokens whose upstream gradients are not both zero (prompt tokens, which the loss masks out)
         need_dh, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        idx = active_token_index(dlog_probs, dentropy, hidden_states.shape[0]) if (need_dh or need_dw) else None
+        idx = None
+        if need_dh or need_dw:
+            idx = active_token_index(dlog_probs, dentropy, hidden_states.shape[0], vocab_weights.shape)
         if idx is not None:
             dhidden_states, dvocab_weights = backward_over_active_tokens(
                 idx, dlog_probs, dentropy, hidden_states, vocab_weights, input_ids, lse, mean_z, ctx.temperature,

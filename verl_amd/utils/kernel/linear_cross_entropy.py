@@ -180,11 +180,17 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
     return d_hidden, d_weight
 
 
+# A backward pass of this many multiply-adds per product (tokens x vocabulary x hidden size) takes about 5 ms, a hundred
+# times what a look at the upstream gradients costs (35 to 60 us): from there on every call looks.  At 2 * 10**11 dense
+# passes of 3.4 ms were 1 % slower for it.
+_ACTIVE_PROBE_ALWAYS = 10**12
+# Shorter calls: how many of them do not look after one that found nearly every token active, how many of those are left,
+# and the (vocabulary, hidden size) they are left for.
 _ACTIVE_PROBE_REST = 15
-_ACTIVE_PROBE = {"rest": 0}   # calls left during which active_token_index() does not look at the gradients
+_ACTIVE_PROBE = {"rest": 0, "head": None}
 
 
-def active_token_index(dlogprobs, dentropy, n_tokens: int):
+def active_token_index(dlogprobs, dentropy, n_tokens: int, weight_shape):
     """Indices of the tokens whose upstream gradients are not both zero, or ``None`` when the backward pass should
     run over every token.
 
@@ -193,13 +199,16 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int):
     Running the backward kernels over the other tokens only gives the same gradients for a fraction of the work (the
     reference's kernels run over all of them).  The count is read on the host, so this is skipped under stream
     capture; ``VAMD_LCE_SKIP_ZERO_GRAD_TOKENS=0`` switches it off; nothing is gained, and nothing done, when more
-    than nine tokens in ten are active.  Reading the count stalls the launch queue for about 0.1 ms, so after a call
-    that found nearly every token active the next fifteen calls do not look."""
+    than nine tokens in ten are active.  Reading the count stalls the launch queue for 35 to 60 us.  A long backward pass
+    always looks, so what it does depends on its own gradients only; where the stall could be more than a hundredth of the
+    pass, fifteen calls with the same head do not look after one that found nearly every token active."""
     if os.environ.get("VAMD_LCE_SKIP_ZERO_GRAD_TOKENS", "1") == "0":
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
-    if _ACTIVE_PROBE["rest"] > 0:
+    head = tuple(weight_shape)
+    short = n_tokens * head[0] * head[1] < _ACTIVE_PROBE_ALWAYS
+    if short and _ACTIVE_PROBE["rest"] > 0 and _ACTIVE_PROBE["head"] == head:
         _ACTIVE_PROBE["rest"] -= 1
         return None
     active = None
@@ -213,7 +222,8 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int):
         return None
     n_active = int(active.sum())  # the one host synchronisation of this path
     if 10 * n_active > 9 * n_tokens:
-        _ACTIVE_PROBE["rest"] = _ACTIVE_PROBE_REST
+        if short:
+            _ACTIVE_PROBE.update(rest=_ACTIVE_PROBE_REST, head=head)
         return None
     return active.nonzero().squeeze(1)
 
@@ -313,7 +323,7 @@ class LinearCrossEntropy(torch.autograd.Function):
         need_dh, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         idx = None
         if cache is None and ctx.REDUCTION == 0 and (need_dh or need_dw):
-            idx = active_token_index(dlogprobs, dentropy, hidden.shape[0])
+            idx = active_token_index(dlogprobs, dentropy, hidden.shape[0], weight.shape)
         if idx is not None:   # tokens the loss masked out are left out of the backward kernels
             d_hidden, d_weight = backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels, lse,
                                                              mean_z, ctx.temperature, need_dh, need_dw)

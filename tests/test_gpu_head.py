@@ -223,6 +223,24 @@ def test_few_active_tokens_of_a_call_with_several_vocabulary_chunks(dev, monkeyp
     _close_bf16(dw, want_dw, "d_weight", e_dw)
 
 
+@pytest.mark.parametrize("n,v,launches", [(64, 256, 1), (300, 30000, 2)])   # whole d_hidden tiles; cut into pieces
+def test_timing_brackets_every_launch_of_the_gradients(dev, n, v, launches):
+    import ctypes
+    from verl_amd import _cabi
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    hidden, weight, labels = (t.to(dev) for t in _make(n, 128, v, seed=n))
+    _, _, lse, mz = K.efficient_entropy_forward(hidden, weight, labels)
+    L = _cabi.lib()
+    ms, count = (ctypes.c_double * _cabi.LCE_TIMING_KERNELS)(), (ctypes.c_int64 * _cabi.LCE_TIMING_KERNELS)()
+    try:
+        L.vamd_lce_timing_enable(1)
+        K.efficient_entropy_backward(torch.ones(n, device=dev), None, hidden, weight, labels, lse, mz)
+        _cabi.check(L.vamd_lce_timing_collect(ms, count))
+    finally:
+        L.vamd_lce_timing_enable(0)
+    assert list(count) == [0, 0, 1, launches, 0] and ms[3] > 0
+
+
 def test_backward_c_abi_refuses_a_call_that_asks_for_nothing(dev):
     from verl_amd import _cabi
     from verl_amd.utils.kernel.linear_cross_entropy import efficient_entropy_backward, efficient_entropy_forward

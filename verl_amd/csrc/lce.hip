@@ -1809,8 +1809,11 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
   }
   if (pieces > 1) {
     const int64_t elements = n_tokens * hidden_size;
-    hipLaunchKernelGGL(lce_dhidden_sum_kernel, dim3((unsigned)ceil_div(elements, 1024)), dim3(256), 0, s, acc32, pieces,
-                       elements, static_cast<uint16_t*>(d_hidden));
+    {
+      ScopedTiming tm(kTagDGrad, s);
+      hipLaunchKernelGGL(lce_dhidden_sum_kernel, dim3((unsigned)ceil_div(elements, 1024)), dim3(256), 0, s, acc32, pieces,
+                         elements, static_cast<uint16_t*>(d_hidden));
+    }
     VAMD_LAUNCH_CHECK();
   }
   return VAMD_OK;

@@ -71,6 +71,14 @@ def test_pieces_of_a_call_over_some_of_the_tokens(lib):
         assert subset(100, planned, 3584, 152064, 0) == whole(100, 3584, 152064, 0)
 
 
+def test_a_call_over_more_tokens_than_planned_is_refused(lib):
+    at = 4096                                                # never read: the call is refused on the host
+    for planned in (99, 0, -1):
+        rc = lib.vamd_lce_backward_subset(at, at, at, 100, planned, 128, 256, 1.0, at, at, None, None, 0.0, None, at, at,
+                                          _cabi.DW_STORE, None, 0, None, 0, None)
+        assert rc == -1 and b"tokens are no part of" in lib.vamd_last_error()
+
+
 def test_head_size_queries_are_asked_on_the_tensors_device(monkeypatch):
     """The head's workspaces depend on the compute units of the current device, so the query belongs inside the guard that
     makes the tensors' device current for the call itself (devices need not be alike)."""

@@ -1773,7 +1773,11 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     gh.c_tiles = h_tiles;
     gh.r_valid = (int)n_tokens;
     gh.c_valid = (int)hidden_size;
-    const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, d_hidden != nullptr, want_dw, cus, pieces);
+    // No more workgroups than pieces and tiles: with one on every CU, idle or not, and the tiles planned for all of them,
+    // the backward of small heads took 85 instead of 73 us (2239 x 896 x 2000: 68 tiles), 44.5 instead of 42.1 (1209 x 128 x 1000).
+    const int64_t units = (int64_t)h_tiles * ((d_hidden ? (int64_t)tok_tiles * pieces : 0) + (want_dw ? chunk_tiles : 0));
+    const int workgroups = (int)(units < cus ? units : cus);
+    const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, d_hidden != nullptr, want_dw, workgroups, pieces);
     gh.splits = plan.splits;
     gh.split_slabs = plan.split_slabs;
     gh.extra = gh.late = 0;
@@ -1803,7 +1807,7 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     gw.ld_out = hidden_size;
     {
       ScopedTiming tm(kTagDGrad, s);
-      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(cus), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw);
+      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw);
     }
     VAMD_LAUNCH_CHECK();
   }

@@ -702,7 +702,7 @@ def test_pad_to_response_window(dev, geometry):
 
 @pytest.mark.parametrize("n,v", [(1, 152), (5, 700), (93, 66000), (257, 33001), (1100, 5000)])
 def test_merge_of_vocabulary_splits(dev, n, v):
-    """The partial softmax states of a token, however many vocabulary splits the launch had (3, 11, 256, 128 and 19
+    """The partial softmax states of a token, however many vocabulary splits the launch had (3, 11, 243, 128 and 20
     here, so 2 to 64 lanes of the merge share a token), combine to the fp32 ground truth."""
     from verl_amd.utils.kernel import linear_cross_entropy as K
     from oracle import masked as OM
@@ -717,7 +717,8 @@ def test_merge_of_vocabulary_splits(dev, n, v):
 @pytest.mark.parametrize("n,h,v,chunk", [
     (1, 128, 40000, 0),          # one d_hidden tile cut into as many pieces as pay
     (300, 384, 30011, 0),        # 2 x 2 tiles, ragged in both directions, last piece shorter
-    (520, 256, 20000, 8192),     # several chunks, the last one narrower than a piece count would fill
+    (520, 256, 20000, 8192),     # several chunks, all cut into four pieces
+    (520, 256, 16704, 8192),     # several chunks, the last one so narrow (5 slabs) that it fills three of the four pieces
     (2500, 640, 9000, 0),        # whole tiles and pieces side by side with d_weight tiles
 ])
 @pytest.mark.parametrize("need", [(True, True), (True, False)])
@@ -740,7 +741,8 @@ def test_backward_shares_d_hidden_out_in_pieces(dev, n, h, v, chunk, need):
 
 @pytest.mark.parametrize("n,v", [
     (10999, 33001),   # 43 token tiles: bands of 8, 2 and 1, shares that cross from band to band
-    (32900, 1000),    # 129 token tiles, 4 vocabulary tiles: several bands per share, fewer columns than workgroups
+    (32900, 1000),    # 129 token tiles, 4 vocabulary tiles: two waves and a band of one round each, fewer columns than
+                      # workgroups, shares with nothing to do
     (2100, 151936),   # 9 token tiles: one full band and a single tile
     (22000, 33001),   # 86 token tiles: a wave of 33 rounds, then bands of 8, 8, 4 and 2 in shares of 11 or 12 rounds that
                       # cross from band to band: a workgroup changes its labels and its state up to twice

@@ -103,10 +103,6 @@ __device__ __forceinline__ LanePos lane_pos() {
   return p;
 }
 
-// Column offset inside the 256-wide tile of accumulator element (mb, v) for this lane.
-__device__ __forceinline__ int acc_col(const LanePos& p, int mb, int v) {
-  return p.wc * (kMB * kBlk) + mb * kBlk + 4 * p.lq + v;
-}
 // Row offset inside the 256-tall tile of accumulator block nb for this lane.
 __device__ __forceinline__ int acc_row(const LanePos& p, int nb) { return p.wr * (kNB * kBlk) + nb * kBlk + p.lx; }
 

@@ -1119,14 +1119,18 @@ __global__ __launch_bounds__(256) void lce_dlogits_kernel(DLogitsArgs a) {
 // d_weight[chunk] (+)= dz_panel^T . hidden    R = dz (kmajor, k = token), C = hidden (kmajor)
 enum : int { kStoreF32 = 0, kAddF32 = 1, kFinalBf16 = 2, kFinalBf16AddPrev = 3 };
 
+// How the gradient GEMMs of one vocabulary chunk are shared out over the workgroups: plan_gradients().
+struct GradPlan {
+  int splits = 1, split_slabs = 1;  // d_hidden: SplitKSched; each piece is summed into its own fp32 accumulator
+  int extra = 0, late = 0;          // d_weight: LateStartSched
+};
+
 struct GemmOutArgs {
   Operand R, C;
   int k_slabs, r_tiles, c_tiles;
-  int splits, split_slabs;  // d_hidden: pieces along k, each summed into its own fp32 accumulator when there are several
-  int extra, late;          // d_weight: LateStartSched
   int r_valid, c_valid;  // rows / cols of the output that exist
   int mode;              // d_hidden: one of the enum above; d_weight: a VAMD_DW_* value
-  float* acc32;          // fp32 accumulator [r_valid][ld_out]
+  float* acc32;          // fp32 accumulator [r_valid][ld_out], of d_hidden one per piece
   uint16_t* out;         // bf16 output
   int64_t ld_out;
 };
@@ -1216,13 +1220,13 @@ struct DWeightEpi {
 
 // Both gradient GEMMs of one vocabulary chunk in a single launch: a workgroup first walks its share of the d_hidden
 // units, then its share of the d_weight tiles, shared out by plan_gradients() so that all workgroups finish together.
-__global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, GemmOutArgs gw) {
+__global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, GemmOutArgs gw, GradPlan plan) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int nwg = gridDim.x;
   const int wg = xcd_regroup(blockIdx.x, nwg);
   const LanePos pos = lane_pos();
   if (gh.r_tiles > 0) {
-    SplitKSched sched{TileGrid{gh.r_tiles, gh.c_tiles}, gh.splits, gh.split_slabs, gh.k_slabs, nwg, wg};
+    SplitKSched sched{TileGrid{gh.r_tiles, gh.c_tiles}, plan.splits, plan.split_slabs, gh.k_slabs, nwg, wg};
     DHiddenEpi epi;
     epi.p = pos;
     epi.a = &gh;
@@ -1232,7 +1236,7 @@ __global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, Gem
   }
   __syncthreads();
   {
-    LateStartSched sched{TileGrid{gw.r_tiles, gw.c_tiles}, gw.k_slabs, nwg, wg, gw.extra, gw.late};
+    LateStartSched sched{TileGrid{gw.r_tiles, gw.c_tiles}, gw.k_slabs, nwg, wg, plan.extra, plan.late};
     DWeightEpi epi;
     epi.p = pos;
     epi.a = &gw;
@@ -1363,12 +1367,6 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
   if (cv > v_pad) cv = v_pad;
   return cv;
 }
-
-// How the gradient GEMMs of one vocabulary chunk are shared out over the workgroups (one per CU).
-struct GradPlan {
-  int splits = 1, split_slabs = 1;  // pieces of a d_hidden tile's k range
-  int extra = 0, late = 0;          // d_weight: LateStartSched
-};
 
 // d_hidden has few tiles with a long k range (the chunk's vocabulary), d_weight many tiles with a short one (the tokens),
 // and both sum up to the same number of slabs.  Whole d_hidden tiles only balance when there are several per CU: 777
@@ -1778,9 +1776,6 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     const int64_t units = (int64_t)h_tiles * ((d_hidden ? (int64_t)tok_tiles * pieces : 0) + (want_dw ? chunk_tiles : 0));
     const int workgroups = (int)(units < cus ? units : cus);
     const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, d_hidden != nullptr, want_dw, workgroups, pieces);
-    gh.splits = plan.splits;
-    gh.split_slabs = plan.split_slabs;
-    gh.extra = gh.late = 0;
     if (n_chunks == 1 && pieces == 1) gh.mode = kFinalBf16;
     else if (ci == 0) gh.mode = kStoreF32;
     else if (ci == n_chunks - 1 && pieces == 1) gh.mode = kFinalBf16AddPrev;
@@ -1794,10 +1789,6 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     gw.C = Operand{hid, hidden_size, (int)hidden_size, (int)n_tokens};
     gw.k_slabs = (int)ceil_div(n_tokens, kBK);
     gw.r_tiles = want_dw ? chunk_tiles : 0;
-    gw.splits = 1;
-    gw.split_slabs = gw.k_slabs;
-    gw.extra = plan.extra;
-    gw.late = plan.late;
     gw.c_tiles = h_tiles;
     gw.r_valid = (int)cols;
     gw.c_valid = (int)hidden_size;
@@ -1807,7 +1798,8 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     gw.ld_out = hidden_size;
     {
       ScopedTiming tm(kTagDGrad, s);
-      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw);
+      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw,
+                         plan);
     }
     VAMD_LAUNCH_CHECK();
   }

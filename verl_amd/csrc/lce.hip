@@ -16,7 +16,6 @@
 
 #include <atomic>
 #include <mutex>
-#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -326,10 +325,9 @@ struct FwdEpi {
   LanePos p;
   float scale2;
   int vocab;
-  // vectors where the state is written out in the middle of the tile loop: an array ends up in scratch memory there.
-  // Where it lives to the end an array takes 0.1 - 0.2 % off the pass (21503 x 4096 x 128256 15148 -> 15120 us).
-  using State = std::conditional_t<CACHE || BANDS, f32x4, float[kNB]>;
-  State m, s, sy, s2;
+  // vectors and not arrays: an array here ends up in scratch memory, whose set-up alone is 1 to 2 us of a launch (129 x 896 x
+  // 151936 68.4 -> 70.9 us, 400 x 1024 x 32000 32.1 -> 33.2)
+  f32x4 m, s, sy, s2;
   // The labels of the lane's token rows and the label-logit sums live in LDS behind the pipeline's stages when the
   // kernel has LDS to spare (no logits cache), in registers otherwise: with them in registers the kernel spilled,
   // and every reload of a spilled value waits out the slab transfers in flight (one counter counts both).

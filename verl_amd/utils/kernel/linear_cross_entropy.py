@@ -211,21 +211,16 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int, weight_shape):
     if short and _ACTIVE_PROBE["rest"] > 0 and _ACTIVE_PROBE["head"] == head:
         _ACTIVE_PROBE["rest"] -= 1
         return None
-    active = None
-    for g in (dlogprobs, dentropy):
-        if g is not None and g.dim() == 1 and g.shape[0] == n_tokens:
-            nz = g != 0           # NaN counts as active
-            active = nz if active is None else active.logical_or_(nz)
-        elif g is not None:
-            return None           # a scalar upstream gradient reaches every token
-    if active is None:
-        return None
-    n_active = int(active.sum())  # the one host synchronisation of this path
-    if 10 * n_active > 9 * n_tokens:
+    given = [g for g in (dlogprobs, dentropy) if g is not None]
+    if not given or any(g.dim() != 1 or g.shape[0] != n_tokens for g in given):
+        return None               # a scalar upstream gradient reaches every token
+    active = given[0] if len(given) == 1 else torch.logical_or(*given)   # NaN counts as active
+    idx = active.nonzero().squeeze(1)   # the one host synchronisation of this path
+    if 10 * idx.numel() > 9 * n_tokens:
         if short:
             _ACTIVE_PROBE.update(rest=_ACTIVE_PROBE_REST, head=head)
         return None
-    return active.nonzero().squeeze(1)
+    return idx
 
 
 def backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels, lse, mean_z, temperature,

@@ -241,6 +241,29 @@ def test_timing_brackets_every_launch_of_the_gradients(dev, n, v, launches):
     assert list(count) == [0, 0, 1, launches, 0] and ms[3] > 0
 
 
+@pytest.mark.parametrize("n", [5, 300, 32900])   # few tokens, vocabulary splits, bands of token tiles
+@pytest.mark.parametrize("cached", [False, True])
+def test_labels_outside_the_vocabulary_match_no_column(dev, n, cached):
+    """Below zero or past the vocabulary, inside its ragged last tile or not: the log-prob is -lse, and the gradient has no
+    one-hot term."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    v, T = 1000, 0.8
+    hidden, weight, labels = (t.to(dev) for t in _make(n, 128, v, seed=n))
+    outside = torch.tensor([-100, v, v + 23, 5 * v], device=dev)
+    labels[:4] = outside
+    cache = torch.empty((n, v), device=dev) if cached else None
+    lp, _, lse, mz = K.efficient_entropy_forward(hidden, weight, labels, 0, T, logits_cache=cache)
+    z = hidden.float() @ weight.float().t() / T
+    assert (lp[:4] + torch.logsumexp(z[:4], -1)).abs().max() <= ATOL
+    assert (lp[4:] - torch.log_softmax(z[4:], -1).gather(1, labels[4:, None])[:, 0]).abs().max() <= ATOL
+    g = torch.zeros(n, device=dev)
+    g[:4] = 1.0
+    dh, _ = K.efficient_entropy_backward(g, None, hidden, weight, labels, lse, mz, 0, T, logits_cache=cache)
+    d = -torch.softmax(z[:4], -1) / T
+    assert bool(((dh[:4].float() - d @ weight.float()).abs()            # d_logits and the result are rounded to bf16
+                 <= 2.0 ** -8 * (d.abs() @ weight.float().abs()) + 2.0 ** -8 * (d @ weight.float()).abs() + 1e-6).all())
+
+
 def test_backward_c_abi_refuses_a_call_that_asks_for_nothing(dev):
     from verl_amd import _cabi
     from verl_amd.utils.kernel.linear_cross_entropy import efficient_entropy_backward, efficient_entropy_forward

@@ -500,7 +500,8 @@ struct FwdEpi {
       const int rel = label - c0 - p.wc * 128;
       if (__any(rel >= 0 && rel < 128)) {
         float add = 0.f;
-        const int mine = rel - 4 * p.lq;
+        // a label past the vocabulary but inside its ragged last tile matches nothing: those columns hold kNoColumn
+        const int mine = rel - 4 * p.lq < cols_left ? rel - 4 * p.lq : -1;
 #pragma unroll
         for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll

@@ -165,8 +165,10 @@ int vamd_lce_forward_static(const void* hidden, const void* weight, const int64_
  *   reference's torch backend, which allocates and accumulates only the gradients whose inputs require them
  *   (verl/utils/experimental/torch_functional.py:150-156, :184-187); one of the two must be asked for.
  * vocab_chunk = 0 lets the library choose how many vocabulary columns of d_logits are staged
- * at a time (the workspace holds one [n_pad, vocab_chunk] bf16 panel plus fp32 d_hidden
- * accumulators); pass the same value to the workspace query.
+ * at a time (the workspace holds one [n_pad, vocab_chunk] bf16 panel plus, with several chunks, an fp32 d_hidden
+ * accumulator, or several of together up to 256 MB where d_hidden's k range is cut into pieces; the query counts them
+ * whether or not the call will ask for d_hidden);
+ * pass the same value to the workspace query.  The queries count the compute units of the current device.
  *   vamd_lce_backward_subset is the same over some of the tokens of a call with planned_tokens (>= n_tokens) tokens,
  *   gathered by the caller because the others have no upstream gradient.  Where the whole call has one vocabulary chunk,
  *   d_hidden's k range is cut as there and its rows are the bits the whole call would have given them; with several

@@ -1369,7 +1369,7 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
 
 // d_hidden has few tiles with a long k range (the chunk's vocabulary), d_weight many tiles with a short one (the tokens),
 // and both sum up to the same number of slabs.  Whole d_hidden tiles only balance when there are several per CU: 777
-// tokens x 896 have 16 tiles of 2374 slabs, which kept 16 CUs busy while 240 waited (2983 us; cut into 15 pieces 420 us),
+// tokens x 896 have 16 tiles of 2374 slabs, which kept 16 CUs busy while 240 waited (2983 us; cut into 11 pieces 463 us),
 // 7339 x 3584 have 406 on 256 CUs (87 % of the launch busy).  So a tile's k range is cut into pieces of equal length,
 // each summed in fp32 into an accumulator of its own, and the d_weight tiles are shared out so that the workgroups
 // with a piece more get correspondingly fewer tiles.  The number of pieces is the one whose slowest workgroup is

@@ -181,7 +181,7 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
 
 
 # A backward pass of this many multiply-adds per product (tokens x vocabulary x hidden size) takes about 5 ms, a hundred
-# times what a look at the upstream gradients costs (35 to 60 us): from there on every call looks.  At 2 * 10**11 dense
+# times what a look at the upstream gradients costs (35 to 60 us there): from there on every call looks.  At 2 * 10**11 dense
 # passes of 3.4 ms were 1 % slower for it.
 _ACTIVE_PROBE_ALWAYS = 10**12
 # Shorter calls: how many of them do not look after one that found nearly every token active, how many of those are left,
@@ -199,7 +199,7 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int, weight_shape):
     Running the backward kernels over the other tokens only gives the same gradients for a fraction of the work (the
     reference's kernels run over all of them).  The count is read on the host, so this is skipped under stream
     capture; ``VAMD_LCE_SKIP_ZERO_GRAD_TOKENS=0`` switches it off; nothing is gained, and nothing done, when more
-    than nine tokens in ten are active.  Reading the count stalls the launch queue for 35 to 60 us.  A long backward pass
+    than nine tokens in ten are active.  Reading the count stalls the launch queue for 35 to 110 us.  A long backward pass
     always looks, so what it does depends on its own gradients only; where the stall could be more than a hundredth of the
     pass, fifteen calls with the same head do not look after one that found nearly every token active."""
     if os.environ.get("VAMD_LCE_SKIP_ZERO_GRAD_TOKENS", "1") == "0":

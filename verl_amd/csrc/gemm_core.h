@@ -272,7 +272,10 @@ struct Frags {
 // One slab (64 k = two 32-k steps of 32 MFMAs per wavefront) of the software pipeline.
 //
 // The body is 64 slots "one MFMA + at most two memory instruction groups", each closed by a scheduling barrier so
-// the compiler keeps the order.  Slot j = 4 G + nb multiplies block (mb = G % 8, nb) of k-step G / 8.
+// the compiler keeps the order.  Slot j = 4 G + n multiplies block (mb = G % 8, nb) of k-step G / 8, with nb = n in even
+// groups and 3 - n in odd ones: from one MFMA to the next exactly one of the two operands changes, which on a board at its
+// power limit is speed (register-only loop on normal data 2020 -> 2049 TFLOP/s, with both changing every time 1960;
+// 16384 x 3584 x 152064 forward and backward 50.61 -> 50.36 ms, 21503 x 4096 x 128256 forward 15.47 -> 15.43).
 //
 //   slots  0..51 : the C fragment of group G + 3 is read from `cur` in the first slot of group G (its ring slot was
 //                  last used by group G - 1); the R fragments of k-step 1 are read in groups 1..4
@@ -297,14 +300,14 @@ __device__ __forceinline__ void slab_iter(const SlabDma<RK>& dr, const SlabDma<C
                                           const FragAddr<CK>& fc, Frags& f, Accum& acc) {
 #pragma unroll
   for (int j = 0; j < 64; ++j) {
-    const int G = j >> 2, nb = j & 3, ks = G >> 3, mb = G & 7;
+    const int G = j >> 2, n = j & 3, ks = G >> 3, mb = G & 7, nb = G & 1 ? 3 - n : n;
     acc.a[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.c[G & 3], f.r[ks][nb], acc.a[mb][nb], 0, 0, 0);
     if (j < 52) {
-      if (nb == 0) {
+      if (n == 0) {
         const int g3 = G + 3;  // <= 15: still this slab
         f.c[g3 & 3] = fc.read(cur + kSlabBytes, g3 >> 3, g3 & 7);
       }
-      if (nb == 1 && G >= 1 && G <= kNB) f.r[1][G - 1] = fr.read(cur, 1, G - 1);
+      if (n == 1 && G >= 1 && G <= kNB) f.r[1][G - 1] = fr.read(cur, 1, G - 1);
       // LDS reads return in order: with at most one read outstanding (it belongs to the C fragment of slot 20) the
       // last R fragment, read in slot 17, has arrived
       if (j == 21) asm volatile("s_waitcnt lgkmcnt(1)\n\ts_barrier" ::: "memory");

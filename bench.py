@@ -822,7 +822,7 @@ def main() -> None:
     import torch
 
     from verl_amd import _cabi
-    from verl_amd.utils.kernel.linear_cross_entropy import linear_cross_entropy, logits_cache_budget_bytes
+    from verl_amd.utils.kernel.linear_cross_entropy import keeps_logits, linear_cross_entropy
 
     assert torch.cuda.is_available(), "bench.py needs a GPU"
     dev = torch.device("cuda:0")
@@ -866,8 +866,9 @@ def main() -> None:
     del src, dst
 
     # The headline is the mode the library ships as its default (whatever VAMD_LCE_LOGITS_CACHE_GB says in this
-    # process's environment; unset = no cache, the backward pass recomputes the logits).
-    default_cached = 4 * n * v <= logits_cache_budget_bytes()
+    # process's environment; unset = the logits are kept for the backward pass where they are a small part of the free
+    # memory).
+    default_cached = keeps_logits(n, v, dev)
     head = time_head_mode(step, args.steps, args.warmup, n, dev)
     ms_per_step, tokens_per_s = head["ms_per_step"], head["tokens_per_s"]
     prof_steps = max(1, min(args.steps, 5))

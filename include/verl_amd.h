@@ -173,6 +173,9 @@ int vamd_lce_forward_static(const void* hidden, const void* weight, const int64_
  *   gathered by the caller because the others have no upstream gradient.  Where the whole call has one vocabulary chunk,
  *   d_hidden's k range is cut as there and its rows are the bits the whole call would have given them; with several
  *   chunks, whose width depends on the token count, the two sum over different ranges and n_tokens alone decides.
+ *   vamd_lce_backward_subset_rows takes the whole call's logits cache: logits_rows[i] is the row of token i in
+ *   logits_cache [planned_tokens, vocab] (a token whose row lies outside gets no gradient).  NULL: token i has row i, as in
+ *   vamd_lce_backward_subset.  Same workspace.
  */
 #define VAMD_DW_STORE 0
 #define VAMD_DW_ADD_BF16 1
@@ -195,6 +198,13 @@ int vamd_lce_backward_subset(const void* hidden, const void* weight, const int64
                              float d_entropy_scalar, const float* logits_cache, void* d_hidden, void* d_weight,
                              int d_weight_mode, float* d_weight_acc32, int64_t vocab_chunk, void* workspace,
                              size_t workspace_bytes, void* stream);
+int vamd_lce_backward_subset_rows(const void* hidden, const void* weight, const int64_t* labels, int64_t n_tokens,
+                                  int64_t planned_tokens, int64_t hidden_size, int64_t vocab, float rcp_temperature,
+                                  const float* lse, const float* mean_z, const float* d_logprobs,
+                                  const float* d_entropy, float d_entropy_scalar, const float* logits_cache,
+                                  const int64_t* logits_rows, void* d_hidden, void* d_weight, int d_weight_mode,
+                                  float* d_weight_acc32, int64_t vocab_chunk, void* workspace, size_t workspace_bytes,
+                                  void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Per-token log-prob / entropy from materialised logits: the unfused definitions the actor uses when the

@@ -250,3 +250,23 @@ def test_as_torch_index_agrees_with_the_oracle_restatement():
         got = as_torch_index(case)
         assert got.dtype == torch.long and got.dim() == 1
         assert torch.equal(got, want.cpu()), f"{case!r}: {got.tolist()} vs {want.tolist()}"
+
+
+def test_free_memory_that_may_hold_the_logits(monkeypatch):
+    """What the device has free plus what torch's allocator holds for no tensor, within the process's memory fraction;
+    nothing where another allocator does not say."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    stats = {"reserved_bytes": {"all": {"current": 50}}, "allocated_bytes": {"all": {"current": 30}}}
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (100, 1000))
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", lambda device: stats)
+    monkeypatch.setattr(torch.cuda, "get_per_process_memory_fraction", lambda device: 1.0)
+    assert K._free_device_bytes("cuda:0") == 120
+    monkeypatch.setattr(torch.cuda, "get_per_process_memory_fraction", lambda device: 0.1)
+    assert K._free_device_bytes("cuda:0") == 70
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", lambda device: {})
+    assert K._free_device_bytes("cuda:0") == 0
+
+    def refuse(device):
+        raise RuntimeError("no such query")
+    monkeypatch.setattr(torch.cuda, "mem_get_info", refuse)
+    assert K._free_device_bytes("cuda:0") == 0

@@ -812,3 +812,82 @@ def test_forward_over_few_tokens(dev, n, h, v, T):
     assert (lp - want_lp).abs().max() <= ATOL and (ent - want_ent).abs().max() <= ATOL
     want_pi2 = OM.sum_pi_squared_from_logits(hidden.float() @ weight.float().t() / T)
     assert torch.allclose(pi2, want_pi2, rtol=2e-3, atol=1e-9)
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (1, 128, 16),          # the kernel for few tokens: one workgroup
+    (77, 128, 66000),      # ... ranges of 272 columns: two tiles of 144 and 128
+    (128, 256, 140000),    # ... three tiles
+    (129, 128, 1000),      # splits: the second token tile has one token, the last vocabulary tile 232 columns
+    (777, 256, 33000),     # splits, a ragged vocabulary
+    (2100, 128, 151936),   # bands: 9 token tiles, one full band and a single tile
+    (10999, 128, 33000),   # bands of 8, 2 and 1, shares that cross from band to band
+])
+@pytest.mark.parametrize("T", [1.0, 0.7])
+def test_kept_logits_change_no_bit(dev, monkeypatch, n, h, v, T):
+    """With and without a logits cache, however the forward launch is shared out: the same forward outputs and gradients,
+    over all tokens and where a third of them has no upstream gradient (their logits are then picked by row)."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    hidden, weight, labels = (t.to(dev) for t in _make(n, h, v, seed=n + v))
+    hidden.requires_grad_(), weight.requires_grad_()
+    cache = torch.full((n, v), float("nan"), device=dev)
+    K.efficient_entropy_forward(hidden, weight, labels, 0, T, logits_cache=cache)
+    for lo in range(0, n, 4096):   # fp32 sums of 128 to 256 bf16 products in another order
+        want = hidden.detach()[lo:lo + 4096].float() @ weight.detach().float().t() / T
+        assert (cache[lo:lo + 4096] - want).abs().max() <= 1e-5 * want.abs().max() + 1e-6
+    del cache
+    g = torch.Generator().manual_seed(n)
+    g_lp, g_ent = torch.randn(n, generator=g).to(dev), torch.full((n,), 0.01, device=dev)
+    monkeypatch.setitem(K._ACTIVE_PROBE, "head", None)
+    for keep in (torch.ones(n, device=dev), (torch.arange(n, device=dev) % 3 != 1).float()):
+        outs = []
+        for budget in ("64", "0"):
+            monkeypatch.setenv("VAMD_LCE_LOGITS_CACHE_GB", budget)
+            monkeypatch.setitem(K._ACTIVE_PROBE, "rest", 0)
+            lp, ent = K.linear_cross_entropy(hidden, weight, labels, T)
+            outs.append((lp, ent, *torch.autograd.grad((lp, ent), (hidden, weight), (g_lp * keep, g_ent * keep))))
+        for name, a, b in zip(("logprobs", "entropy", "d_hidden", "d_weight"), *outs):
+            assert torch.equal(a, b), f"{name}: max abs diff {(a.float() - b.float()).abs().max().item():.3e}"
+
+
+def test_rows_of_the_logits_cache_outside_it(dev):
+    """A token whose row lies outside the cache gets no gradient and adds none."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    n, planned, v = 5, 9, 1000
+    hidden, weight, labels = (t.to(dev) for t in _make(planned, 128, v, seed=1))
+    cache = torch.empty((planned, v), device=dev)
+    _, _, lse, mz = K.efficient_entropy_forward(hidden, weight, labels, logits_cache=cache)
+    rows = torch.tensor([2, 0, 8, 3, 4], device=dev)
+    args = [hidden[rows], weight, labels[rows], lse[rows], mz[rows]]
+    ones = torch.ones(n, device=dev)
+    bad = torch.tensor([2, -1, 9, 3, 4], device=dev)
+    dh, dw = K.efficient_entropy_backward(ones, None, *args, planned_tokens=planned, logits_cache=cache, logits_rows=bad)
+    inside = ones * (bad == rows)
+    want_dh, want_dw = K.efficient_entropy_backward(inside, None, *args, planned_tokens=planned, logits_cache=cache,
+                                                    logits_rows=rows)
+    assert torch.equal(dh, want_dh) and torch.equal(dw, want_dw) and not dh[1:3].any() and dh[0].any()
+
+
+def test_logits_are_kept_where_they_are_a_small_part_of_the_free_memory(dev, monkeypatch):
+    """Without a budget in the environment: an eighth of the free memory or less, not under saved-tensor hooks, and
+    released by the backward pass."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    monkeypatch.delenv("VAMD_LCE_LOGITS_CACHE_GB", raising=False)
+    n, h, v = 512, 128, 65536
+    hidden, weight, labels = (t.to(dev) for t in _make(n, h, v, seed=4))
+    weight.requires_grad_()
+
+    def held():
+        before = torch.cuda.memory_allocated(dev)
+        lp, _ = K.linear_cross_entropy(hidden, weight, labels)
+        return lp, torch.cuda.memory_allocated(dev) - before
+
+    lp, bytes_held = held()
+    assert bytes_held >= 4 * n * v
+    lp.sum().backward()
+    assert torch.cuda.memory_allocated(dev) < 4 * n * v + hidden.nbytes + 2 * weight.nbytes + (32 << 20)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert held()[1] < 4 * n * v
+    for free, kept in ((8 * 4 * n * v, True), (8 * 4 * n * v - 1, False)):
+        monkeypatch.setattr(K, "_free_device_bytes", lambda device: free)
+        assert (held()[1] >= 4 * n * v) is kept

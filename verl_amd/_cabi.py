@@ -50,6 +50,10 @@ SIGNATURES = {
     "vamd_lce_backward_subset": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float,
                                          c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
                                          c_int, c_void_p, c_int64, c_void_p, c_size_t, c_void_p]),
+    "vamd_lce_backward_subset_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float,
+                                              c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p,
+                                              c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p, c_size_t,
+                                              c_void_p]),
     "vamd_lce_timing_enable": (c_int, [c_int]),
     "vamd_lce_timing_collect": (c_int, [c_void_p, c_void_p]),
     "vamd_row_softmax_stats": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,

@@ -152,7 +152,7 @@ struct FwdArgs {
   float scale2;      // log2(e) / temperature
   float rcp_t;       // 1 / temperature
   float4* partials;  // [plan.slots()][256] : (max in the log2 domain, sum e, sum e x with x = hidden . weight, label logit)
-  float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward (splits only)
+  float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward
   float* pi2_partials;  // optional [plan.slots()][256] : sum of e^2 relative to the same max
 };
 
@@ -249,52 +249,59 @@ struct FwdSched<true> {
   __device__ __forceinline__ int slabs(int) const { return k_slabs; }
 };
 
-// The epilogues that write matrices hand the accumulators through a 4 KB LDS patch private to the
-// wavefront (the 32 KB the pipeline leaves free), 32 x 32 values at a time (2 x 2 MFMA blocks), so that
+// The epilogues that write matrices hand the accumulators through an LDS patch private to the
+// wavefront (in the 32 KB the pipeline leaves free), ROWS x 32 values at a time (ROWS / 16 x 2 MFMA blocks), so that
 // global accesses are whole 128-byte rows of fp32 (64-byte rows of bf16) touched by 8 consecutive
 // lanes instead of 16-byte pieces of 16 different rows.  After the exchange lane L holds columns
-// 4 (L % 8) .. + 3 of rows 8 i + L / 8 (i = 0..3) of the 32 x 32 patch.  LDS operations of one wavefront
+// 4 (L % 8) .. + 3 of rows 8 i + L / 8 (i < ROWS / 8) of the patch.  LDS operations of one wavefront
 // execute in issue order, so the patch needs no barrier, only the waits that order its writes and reads.
 constexpr int kNB2 = kNB / 2, kMB2 = kMB / 2;  // 32 x 32 patches per wavefront along r and c
+template <int ROWS>
 struct BlockExchange {
+  static constexpr int kRB = ROWS / kBlk, kPatchBytes = ROWS * 128;
   char* stage;  // this wavefront's patch
   int lx, lq, rd_row, rd_chunk;
-  __device__ __forceinline__ void init(char* lds_after_pipeline, const LanePos& p) {
-    stage = lds_after_pipeline + (threadIdx.x >> 6) * 4096;
+  __device__ __forceinline__ void init(char* patches, const LanePos& p) {
+    stage = patches + (threadIdx.x >> 6) * kPatchBytes;
     lx = p.lx;
     lq = p.lq;
     rd_row = (threadIdx.x & 63) >> 3;
     rd_chunk = threadIdx.x & 7;
   }
-  // blk[cb][rb]: the four 16 x 16 blocks of the patch, cb along c, rb along r
-  __device__ __forceinline__ void run(const f32x4 (&blk)[2][2], f32x4 (&out)[4]) const {
+  // blk[cb][rb]: the 16 x 16 blocks of the patch, cb along c, rb along r
+  __device__ __forceinline__ void run(const f32x4 (&blk)[2][kRB], f32x4 (&out)[ROWS / 8]) const {
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
+      for (int rb = 0; rb < kRB; ++rb) {
         const int row = 16 * rb + lx;
         *reinterpret_cast<f32x4*>(stage + row * 128 + (((4 * cb + lq) ^ ((row >> 1) & 7)) << 4)) = blk[cb][rb];
       }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < ROWS / 8; ++i) {
       const int row = 8 * i + rd_row;
       out[i] = *reinterpret_cast<const f32x4*>(stage + row * 128 + ((rd_chunk ^ ((row >> 1) & 7)) << 4));
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
-  // the patch (mb2, nb2) of an accumulator
-  __device__ __forceinline__ void run(const Accum& acc, int mb2, int nb2, f32x4 (&out)[4]) const {
-    const f32x4 blk[2][2] = {{acc.a[2 * mb2][2 * nb2], acc.a[2 * mb2][2 * nb2 + 1]},
-                             {acc.a[2 * mb2 + 1][2 * nb2], acc.a[2 * mb2 + 1][2 * nb2 + 1]}};
-    run(blk, out);
-  }
 };
+using GradExchange = BlockExchange<32>;
+// the patch (mb2, nb2) of an accumulator
+__device__ __forceinline__ void exchange_patch(const GradExchange& ex, const Accum& acc, int mb2, int nb2, f32x4 (&out)[4]) {
+  const f32x4 blk[2][2] = {{acc.a[2 * mb2][2 * nb2], acc.a[2 * mb2][2 * nb2 + 1]},
+                           {acc.a[2 * mb2 + 1][2 * nb2], acc.a[2 * mb2 + 1][2 * nb2 + 1]}};
+  ex.run(blk, out);
+}
 
-constexpr int kCacheStageBytes = (kThreads / 64) * 4096;  // one 32 x 32 fp32 patch per wavefront
-// forward without a cache: two sets of labels, label-logit sums, states of one half of the wavefronts (and squared sums)
+constexpr int kGradStageBytes = kWaves * GradExchange::kPatchBytes;
+// forward: two sets of labels, label-logit sums, states of one half of the wavefronts (and squared sums); with a logits
+// cache, behind them, patches of 16 rows
 static_assert(kLdsBytes % (2 * kTile * 4) == 0, "the sets of labels are told apart by one address bit");
 constexpr int kFwdTokenLds = 2 * kTile * 4 + kThreads * kNB * 4 + kTile * (16 + 4);
+using CacheExchange = BlockExchange<16>;
+constexpr int kFwdCacheLds = kFwdTokenLds + kWaves * CacheExchange::kPatchBytes;
+static_assert(kLdsBytes + kFwdCacheLds <= 160 * 1024 && kFwdTokenLds % 128 == 0, "LDS of a CU");
 
 __device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float m2, float s2, float sy2) {
   const float mm = fmaxf(m, m2);
@@ -321,48 +328,40 @@ __device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float
 // (calculate_sum_pi_squared_from_logits, verl/utils/torch_functional.py:680-694).
 template <bool CACHE, bool PI2, bool BANDS>
 struct FwdEpi {
-  static_assert(!(CACHE && BANDS), "with a logits cache every workgroup has one token tile");
   LanePos p;
   float scale2;
   int vocab;
   // vectors and not arrays: an array here ends up in scratch memory, whose set-up alone is 1 to 2 us of a launch (129 x 896 x
   // 151936 68.4 -> 70.9 us, 400 x 1024 x 32000 32.1 -> 33.2)
   f32x4 m, s, sy, s2;
-  // The labels of the lane's token rows and the label-logit sums live in LDS behind the pipeline's stages when the
-  // kernel has LDS to spare (no logits cache), in registers otherwise: with them in registers the kernel spilled,
-  // and every reload of a spilled value waits out the slab transfers in flight (one counter counts both).
-  f32x4 zl;  // CACHE
-  int lab[kNB];  // CACHE
+  // The labels of the lane's token rows and the label-logit sums live in LDS behind the pipeline's stages: with them in
+  // registers the kernel spilled, and every reload of a spilled value waits out the slab transfers in flight (one
+  // counter counts both).
   unsigned lab_lds, zl_lds, red_lds;  // LDS byte addresses: labels [256] by row, in the set in use of two; sums
                                       // [kThreads][kNB]; states [256] float4, then squared sums [256]
+  char* patches;  // CACHE: the wavefronts' exchange patches
   const FwdArgs* args;
   FwdSched<BANDS> sched;
   int64_t slot;  // where the state of the token tile at hand goes
   float rcp_t;
-  float* z_cache;  // CACHE: [n_tokens][vocab]
-  BlockExchange ex;  // CACHE
-  int tok0;        // CACHE: first token row of the wavefront
-  int n_tokens;
 
   // When the token tile changes: the low dwords of its 256 labels, 64 per wavefront of the first four, straight into LDS;
   // a token past the end reads as label 0, whose sums nobody looks at.  They go into the set that is not in use: other
   // wavefronts may still be in the epilogue that reads this one.
   __device__ __forceinline__ void prefetch(int tile, int r0, int) {
-    if constexpr (!CACHE) {
-      if constexpr (BANDS) {
-        const auto here = sched.at(tile);
-        if (here.slot == slot) return;
-        if (tile > 0) write_state();  // (here no accumulators are alive)
-        slot = here.slot;
-        lab_lds ^= kTile * 4;
-      } else if (tile > 0) {
-        return;
-      }
-      const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-      if (w < 4) {
-        const u32x4 rs = span_rsrc(args->labels, (int64_t)args->n_tokens * 8);
-        load_to_lds_4(rs, ((unsigned)r0 + 64u * w + (threadIdx.x & 63u)) * 8u, lab_lds + 64u * w * 4u);
-      }
+    if constexpr (BANDS) {
+      const auto here = sched.at(tile);
+      if (here.slot == slot) return;
+      if (tile > 0) write_state();  // (here no accumulators are alive)
+      slot = here.slot;
+      lab_lds ^= kTile * 4;
+    } else if (tile > 0) {
+      return;
+    }
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (w < 4) {
+      const u32x4 rs = span_rsrc(args->labels, (int64_t)args->n_tokens * 8);
+      load_to_lds_4(rs, ((unsigned)r0 + 64u * w + (threadIdx.x & 63u)) * 8u, lab_lds + 64u * w * 4u);
     }
   }
 
@@ -444,34 +443,37 @@ struct FwdEpi {
     reset();
   }
 
-  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int /*r0*/, int c0) {
+  // The scaled logits of the tile's valid tokens and columns, in whole 128-byte rows.
+  __device__ __forceinline__ void store_logits(const Accum& acc, int r0, int c0) {
+    const int tok0 = r0 + p.wr * (kNB * kBlk), n_tokens = args->n_tokens;
+    float* const z_cache = args->z_cache;
+    CacheExchange ex;
+    ex.init(patches, p);
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb)
+#pragma unroll
+      for (int mb2 = 0; mb2 < kMB2; ++mb2) {
+        const f32x4 blk[2][1] = {{acc.a[2 * mb2][nb] * rcp_t}, {acc.a[2 * mb2 + 1][nb] * rcp_t}};
+        f32x4 out[2];
+        ex.run(blk, out);
+        const int col = c0 + p.wc * 128 + mb2 * 32 + 4 * ex.rd_chunk;
+        if (col < vocab) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int tok = tok0 + nb * kBlk + 8 * i + ex.rd_row;
+            if (tok < n_tokens)
+              __builtin_nontemporal_store(out[i], reinterpret_cast<f32x4*>(z_cache + (int64_t)tok * vocab + col));
+          }
+        }
+      }
+  }
+
+  __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int r0, int c0) {
     const bool ragged = c0 + kTile > vocab;
     // element (mb, v) of the lane is column 16 mb + v of this: comparing immediates with one register, where a column
     // number per element would be computed ahead of the tile loop and held (or spilled) through it
     const int cols_left = vocab - c0 - p.wc * 128 - 4 * p.lq;
-    if constexpr (CACHE) {
-#pragma unroll
-      for (int nb2 = 0; nb2 < kNB2; ++nb2)
-#pragma unroll
-        for (int mb2 = 0; mb2 < kMB2; ++mb2) {
-          f32x4 blk[2][2];
-#pragma unroll
-          for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) blk[cb][rb] = acc.a[2 * mb2 + cb][2 * nb2 + rb] * rcp_t;
-          f32x4 out[4];
-          ex.run(blk, out);
-          const int col = c0 + p.wc * 128 + mb2 * 32 + 4 * ex.rd_chunk;
-          if (col < vocab) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int tok = tok0 + nb2 * 32 + 8 * i + ex.rd_row;
-              if (tok < n_tokens)
-                __builtin_nontemporal_store(out[i], reinterpret_cast<f32x4*>(z_cache + (int64_t)tok * vocab + col));
-            }
-          }
-        }
-    }
+    if constexpr (CACHE) store_logits(acc, r0, c0);
 #pragma unroll
     for (int nb = 0; nb < kNB; ++nb) {
       // pass 1: tile maximum of the raw products (the vocabulary tail of the last tile replaced in place)
@@ -494,9 +496,7 @@ struct FwdEpi {
       // label logit: only when some lane's label falls in this wavefront's 128 columns
       typedef int __attribute__((address_space(3))) * lds_i32_t;
       typedef float __attribute__((address_space(3))) * lds_f32_t;
-      int label;
-      if constexpr (CACHE) label = lab[nb];
-      else label = *(lds_i32_t)(uintptr_t)(lab_lds + 4u * (unsigned)acc_row(p, nb));
+      const int label = *(lds_i32_t)(uintptr_t)(lab_lds + 4u * (unsigned)acc_row(p, nb));
       const int rel = label - c0 - p.wc * 128;
       if (__any(rel >= 0 && rel < 128)) {
         float add = 0.f;
@@ -508,12 +508,8 @@ struct FwdEpi {
           for (int v = 0; v < 4; ++v) {
             add += mb * kBlk + v == mine ? acc.a[mb][nb][v] * rcp_t : 0.f;
           }
-        if constexpr (CACHE) {
-          zl[nb] += add;
-        } else {
-          const lds_f32_t slot = (lds_f32_t)(uintptr_t)(zl_lds + 4u * (threadIdx.x * kNB + nb));
-          *slot += add;
-        }
+        const lds_f32_t slot = (lds_f32_t)(uintptr_t)(zl_lds + 4u * (threadIdx.x * kNB + nb));
+        *slot += add;
       }
       // pass 2: the running state in the log2 domain, three operations and an exponential per element:
       // e = 2^(x scale2 - m), s += e, sy += e x (the raw product: the 1 / temperature goes on at the very end)
@@ -554,59 +550,17 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   if constexpr (BANDS) epi.slot = -1;
   else epi.slot = sched.slot;
   epi.reset();
-  if constexpr (CACHE) {
+  typedef float __attribute__((address_space(3))) * lds_f32_t;
+  epi.lab_lds = lds_address(lds + kLdsBytes);
+  epi.zl_lds = epi.lab_lds + 2 * kTile * 4;
+  epi.red_lds = epi.zl_lds + kThreads * kNB * 4;
 #pragma unroll
-    for (int nb = 0; nb < kNB; ++nb) {
-      epi.zl[nb] = 0.f;
-      const int tok = sched.tn * kTile + acc_row(epi.p, nb);
-      epi.lab[nb] = tok < a.n_tokens ? (int)a.labels[tok] : -1;
-    }
-    epi.z_cache = a.z_cache;
-    epi.ex.init(lds + kLdsBytes, epi.p);
-    epi.tok0 = sched.tn * kTile + epi.p.wr * (kNB * kBlk);
-    epi.n_tokens = a.n_tokens;
-  } else {
-    typedef float __attribute__((address_space(3))) * lds_f32_t;
-    epi.lab_lds = lds_address(lds + kLdsBytes);
-    epi.zl_lds = epi.lab_lds + 2 * kTile * 4;
-    epi.red_lds = epi.zl_lds + kThreads * kNB * 4;
-#pragma unroll
-    for (int nb = 0; nb < kNB; ++nb) *(lds_f32_t)(uintptr_t)(epi.zl_lds + 4u * (threadIdx.x * kNB + nb)) = 0.f;
-  }
+  for (int nb = 0; nb < kNB; ++nb) *(lds_f32_t)(uintptr_t)(epi.zl_lds + 4u * (threadIdx.x * kNB + nb)) = 0.f;
+  epi.patches = lds + kLdsBytes + kFwdTokenLds;
 
   run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 
-  if constexpr (!CACHE) {
-    if (sched.count() > 0) epi.write_state();
-  } else {  // one token tile per workgroup (splits): its state is written once, at the end
-    epi.merge_lanes(epi.zl, threadIdx.x);
-    // the two wavefronts that share a token quarter, through LDS (once every wavefront's last slab transfers have landed)
-    __syncthreads();
-    float4* red = reinterpret_cast<float4*>(lds);                     // [2][256]
-    float* redq = reinterpret_cast<float*>(lds + 2 * kTile * 16);    // [2][256] squared sums
-    if (epi.p.lq == 0) {
-#pragma unroll
-      for (int nb = 0; nb < kNB; ++nb) {
-        red[epi.p.wc * kTile + acc_row(epi.p, nb)] = make_float4(epi.m[nb], epi.s[nb], epi.sy[nb], epi.zl[nb]);
-        if (PI2) redq[epi.p.wc * kTile + acc_row(epi.p, nb)] = epi.s2[nb];
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < kTile) {
-      const int t = threadIdx.x;
-      float4 x = red[t], y = red[kTile + t];
-      const int64_t slot = sched.slot * kTile + t;
-      if (PI2) {
-        float q = redq[t];
-        merge_state(x.x, x.y, x.z, q, y.x, y.y, y.z, redq[kTile + t]);
-        a.pi2_partials[slot] = q;
-      } else {
-        merge_state(x.x, x.y, x.z, y.x, y.y, y.z);
-      }
-      x.w += y.w;
-      a.partials[slot] = x;
-    }
-  }
+  if (sched.count() > 0) epi.write_state();
 }
 
 // The forward pass over at most kFewTokens tokens.  It is bound by reading the weight: with a 256-token tile the matrix cores
@@ -620,12 +574,14 @@ constexpr int kFewTokens = 128;
 constexpr int kFewStageBytes = (kFewTokens + kTile) * kBK * 2;
 constexpr int kFewStages = 3;
 constexpr int kFewLds = kFewStages * kFewStageBytes;
+constexpr int kFewCacheLds = kFewLds + kWaves * CacheExchange::kPatchBytes;  // with a logits cache
+static_assert(kFewCacheLds <= 160 * 1024, "LDS of a CU");
 constexpr int kFewWavesR = 2, kFewWavesC = 4, kFewMB = kTile / kBlk / kFewWavesC;
 constexpr int kFewLoadsR = kFewTokens * 8 / kThreads;  // transfers per lane of one slab of hidden (2)
 static_assert(kFewLoadsR + kLoads == 6, "the s_waitcnt vmcnt(6) of lce_forward_few_kernel counts the transfers of one slab");
 static_assert(kFewTokens == kFewWavesR * kNB * kBlk, "a wavefront owns kNB blocks of tokens");
 
-template <bool PI2>
+template <bool CACHE, bool PI2>
 __global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int split = xcd_regroup(blockIdx.x, gridDim.x);
@@ -719,6 +675,31 @@ __global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
     // the tile is done: online softmax over its columns, as in FwdEpi
     const int col0 = c_begin + tile * tile_cols + wc * (kFewMB * kBlk) + 4 * lq;  // column of element (0, 0) of the lane
     const int cols_left = tile_end(tile) - col0;
+    if constexpr (CACHE) {
+      LanePos pos{};
+      pos.lx = lx;
+      pos.lq = lq;
+      CacheExchange ex;
+      ex.init(lds + kFewLds, pos);
+#pragma unroll
+      for (int nb = 0; nb < kNB; ++nb)
+#pragma unroll
+        for (int mb2 = 0; mb2 < kFewMB / 2; ++mb2) {
+          const f32x4 blk[2][1] = {{acc[2 * mb2][nb] * a.rcp_t}, {acc[2 * mb2 + 1][nb] * a.rcp_t}};
+          f32x4 out[2];
+          ex.run(blk, out);
+          // 4 columns that exist or do not: vocab % 8 == 0, and tiles end at multiples of kBlk or at the vocabulary
+          const int col = col0 - 4 * lq + 32 * mb2 + 4 * ex.rd_chunk;
+          if (col < tile_end(tile)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const int tok = wr * (kNB * kBlk) + nb * kBlk + 8 * i + ex.rd_row;
+              if (tok < a.n_tokens)
+                __builtin_nontemporal_store(out[i], reinterpret_cast<f32x4*>(a.z_cache + (int64_t)tok * a.vocab + col));
+            }
+          }
+        }
+    }
     ++tile;
 #pragma unroll
     for (int nb = 0; nb < kNB; ++nb) {
@@ -886,7 +867,7 @@ struct RecomputeArgs {
   int n_tokens, vocab_left;  // vocab_left = vocab - chunk_c0
   int chunk_c0;
   int k_slabs, tok_tiles, chunk_tiles;
-  float scale2, rcp_t;
+  float rcp_t;
   uint16_t* dz;  // [tok_tiles*256][dz_ld] bf16
   int dz_ld;
 };
@@ -932,7 +913,7 @@ constexpr int kBf16StageBytes = (kThreads / 64) * 2048;  // one 32 x 32 bf16 pat
 // two sets used in turn so that a tile's transfers never land in what the previous tile's epilogue still reads.
 constexpr int kTokArrays = 5, kTokSetBytes = kTokArrays * kTile * 4;
 constexpr int kRecomputeExtraLds = kBf16StageBytes + 2 * kTokSetBytes;
-static_assert(kRecomputeExtraLds <= kCacheStageBytes, "the recompute kernel is launched with the cache stage's LDS");
+static_assert(kLdsBytes + kRecomputeExtraLds <= 160 * 1024, "LDS of a CU");
 
 struct RecomputeEpi {
   LanePos p;
@@ -982,6 +963,7 @@ struct RecomputeEpi {
   // stored.  PLAIN: a tile inside the matrix with no label in the wavefront's 128 columns -- nothing but the
   // arithmetic, four multiply-adds and an exponential per element; otherwise the one-hot term and the zeros for
   // padding rows and columns come in through two comparisons per element (no branches).
+  // The accumulators hold logits, z = x / T in fp32: the expressions are lce_dlogits_kernel's, bit for bit.
   //   code[rb]: 4 mb + v of the element of row rb that holds the label's column, or -1
   //   lim[rb] : columns of the wavefront's 128 that exist for row rb (0 for a padding row), minus 4 lq
   template <bool PLAIN>
@@ -999,9 +981,9 @@ struct RecomputeEpi {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const int mb = 2 * mb2 + cb;
-            const float x = acc.a[mb][2 * nb2 + rb][v];
-            const float prob = fast_exp2(fmaf(x, A.scale2, -lse2[rb]));
-            const float u = fmaf(u1[rb], x, u0[rb]);  // g_lp/T + g_ent/T * (z - mean_z), z = x / T
+            const float z = acc.a[mb][2 * nb2 + rb][v];
+            const float prob = fast_exp2(fmaf(z, kLog2e, -lse2[rb]));
+            const float u = fmaf(u1[rb], z, u0[rb]);  // g_lp/T + g_ent/T * (z - mean_z)
             if constexpr (PLAIN) {
               d[cb][rb][v] = -prob * u;
             } else {
@@ -1030,10 +1012,19 @@ struct RecomputeEpi {
     parity ^= 1;
     const bool inside = r0 + kTile <= A.n_tokens && c0 + kTile <= A.vocab_left;  // uniform over the workgroup
     const int cols_left = A.vocab_left - c0 - p.wc * 128 - 4 * p.lq;
+    // Rounded to z first, as the logits cache holds it, so that the gradients are the same bits with and without a cache,
+    // which is kept or not by what memory there is (with the scale folded into the exponent they differed in the last bit
+    // of some at T = 0.7).
+    if (A.rcp_t != 1.f) {
+#pragma unroll
+      for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < kNB; ++nb) acc.a[mb][nb] = acc.a[mb][nb] * A.rcp_t;
+    }
 #pragma unroll
     for (int nb2 = 0; nb2 < kNB2; ++nb2) {
       // the lane's two token rows of this 32-row patch
-      // u = u1 x + u0 with u1 = g_ent / T^2 and u0 = g_lp / T - g_ent / T * mean_z: one multiply-add per element
+      // u = u1 z + u0 with u1 = g_ent / T and u0 = g_lp / T - g_ent / T * mean_z: one multiply-add per element
       float lse2[2], u1[2], u0[2], glp[2];
       int code[2], lim[2];
       bool hit = false;
@@ -1042,9 +1033,8 @@ struct RecomputeEpi {
         const int t = acc_row(p, 2 * nb2 + rb);  // row inside the tile
         lse2[rb] = tokf[t] * kLog2e;
         glp[rb] = (A.g_lp ? tokf[2 * kTile + t] : 0.f) * A.rcp_t;
-        const float gent = (A.g_ent ? tokf[4 * kTile + t] : A.g_ent_scalar) * A.rcp_t;
-        u1[rb] = gent * A.rcp_t;
-        u0[rb] = fmaf(-gent, tokf[kTile + t], glp[rb]);
+        u1[rb] = (A.g_ent ? tokf[4 * kTile + t] : A.g_ent_scalar) * A.rcp_t;
+        u0[rb] = fmaf(-u1[rb], tokf[kTile + t], glp[rb]);
         const int rel = toki[3 * kTile + t] - A.chunk_c0 - c0 - p.wc * 128;  // label's column among the wavefront's 128
         const bool here = rel >= 0 && rel < 128;
         hit = hit || here;
@@ -1070,10 +1060,12 @@ __global__ __launch_bounds__(kThreads) void lce_recompute_kernel(RecomputeArgs a
   run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 }
 
-// d_logits panel of one vocabulary chunk from cached logits: the same arithmetic as RecomputeEpi,
+// d_logits panel of one vocabulary chunk from cached logits, to the bits of RecomputeEpi,
 // one thread per 8 consecutive columns of a token, 2048 columns per workgroup.
 struct DLogitsArgs {
-  const float* z_cache;  // [n_tokens][vocab]
+  const float* z_cache;  // [cache_rows][vocab]
+  const int64_t* rows;   // the row of each token, or null: token i has row i
+  int64_t cache_rows;
   const int64_t* labels;
   const float* lse;
   const float* mean_z;
@@ -1091,13 +1083,15 @@ __global__ __launch_bounds__(256) void lce_dlogits_kernel(DLogitsArgs a) {
   if (j >= a.chunk_cols) return;
   u32x4 out = {0u, 0u, 0u, 0u};
   const int col = a.chunk_c0 + j;
-  if (tok < a.n_tokens && col < a.vocab) {  // vocab % 8 == 0: the 8 columns are all in or all out
+  const int64_t row = tok < a.n_tokens && a.rows ? a.rows[tok] : tok;
+  // vocab % 8 == 0: the 8 columns are all in or all out
+  if (tok < a.n_tokens && col < a.vocab && row >= 0 && row < a.cache_rows) {
     const float lse2 = a.lse[tok] * kLog2e;
     const float glp = (a.g_lp ? a.g_lp[tok] : 0.f) * a.rcp_t;
     const float gent = (a.g_ent ? a.g_ent[tok] : a.g_ent_scalar) * a.rcp_t;
-    const float u0 = fmaf(-gent, a.mean_z[tok], glp);  // as in the recompute epilogue, with z in place of x / T
+    const float u0 = fmaf(-gent, a.mean_z[tok], glp);
     const int rel = (int)a.labels[tok] - col;
-    const f32x4* src = reinterpret_cast<const f32x4*>(a.z_cache + (int64_t)tok * a.vocab + col);
+    const f32x4* src = reinterpret_cast<const f32x4*>(a.z_cache + row * a.vocab + col);
     const f32x4 z0 = __builtin_nontemporal_load(src), z1 = __builtin_nontemporal_load(src + 1);
     float d[8];
 #pragma unroll
@@ -1138,7 +1132,7 @@ struct DHiddenEpi {
   LanePos p;
   const GemmOutArgs* a;
   SplitKSched sched;
-  BlockExchange ex;
+  GradExchange ex;
   __device__ __forceinline__ void prefetch(int, int, int) {}
   __device__ __forceinline__ void operator()(Accum& acc, int tile, int r0, int c0) {
     const GemmOutArgs& A = *a;
@@ -1150,7 +1144,7 @@ struct DHiddenEpi {
 #pragma unroll
       for (int mb = 0; mb < kMB2; ++mb) {
         f32x4 v[4];
-        ex.run(acc, mb, nb, v);
+        exchange_patch(ex, acc, mb, nb, v);
         const int col = c0 + p.wc * 128 + mb * 32 + 4 * ex.rd_chunk;
         if (col >= A.c_valid) continue;
         const int row0 = r0 + p.wr * (kNB * kBlk) + nb * 32 + ex.rd_row;
@@ -1179,7 +1173,7 @@ struct DHiddenEpi {
 struct DWeightEpi {
   LanePos p;
   const GemmOutArgs* a;
-  BlockExchange ex;
+  GradExchange ex;
   __device__ __forceinline__ void prefetch(int, int, int) {}
   __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int r0, int c0) {
     const GemmOutArgs& A = *a;
@@ -1188,7 +1182,7 @@ struct DWeightEpi {
 #pragma unroll
       for (int mb = 0; mb < kMB2; ++mb) {
         f32x4 v[4];
-        ex.run(acc, mb, nb, v);
+        exchange_patch(ex, acc, mb, nb, v);
         const int col = c0 + p.wc * 128 + mb * 32 + 4 * ex.rd_chunk;
         if (col >= A.c_valid) continue;
         const int row0 = r0 + p.wr * (kNB * kBlk) + nb * 32 + ex.rd_row;
@@ -1280,12 +1274,16 @@ static int ensure_lds_attributes() {
   if ((s = allow_big_lds(lce_forward_kernel<false, true, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_kernel<false, false, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_kernel<false, true, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, false, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, true, false>, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_few_kernel<false>, kFewLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_few_kernel<true>, kFewLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_dgrad_kernel, kLdsBytes + kCacheStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, false, false>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, true, false>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, false, true>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_kernel<true, true, true>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<false, false>, kFewLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<false, true>, kFewLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<true, false>, kFewCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_forward_few_kernel<true, true>, kFewCacheLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kRecomputeExtraLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_dgrad_kernel, kLdsBytes + kGradStageBytes)) != VAMD_OK) return s;
   done[dev] = true;
   return VAMD_OK;
 }
@@ -1299,7 +1297,7 @@ static inline int64_t dz_pitch(int64_t cv) { return cv + 128; }
 
 // max_slots: most partial states (of 256 tokens each) the caller's buffer holds; the built-in buffer of the entry point that
 // allocates nothing is sized for 256 CUs and must serve a part with more of them too.
-static FwdPlan plan_forward(int64_t n_tokens, int64_t vocab, bool one_tile_only, int64_t max_slots = INT64_MAX) {
+static FwdPlan plan_forward(int64_t n_tokens, int64_t vocab, int64_t max_slots = INT64_MAX) {
   const int64_t cus = device_cu_count(), tok_tiles = ceil_div(n_tokens, kTile), voc_tiles = ceil_div(vocab, kTile);
   FwdPlan p{};
   p.tok_tiles = (int)tok_tiles;
@@ -1309,14 +1307,14 @@ static FwdPlan plan_forward(int64_t n_tokens, int64_t vocab, bool one_tile_only,
   if (sp < 1) sp = 1;
   if (sp > voc_tiles) sp = voc_tiles;
   p.splits = (int)sp;
-  if (n_tokens <= kFewTokens && !one_tile_only) {
+  if (n_tokens <= kFewTokens) {
     // equal ranges of weight rows; 64 rows are the least that is worth a workgroup
     const int64_t even = ceil_div(ceil_div(vocab, cus < max_slots ? cus : max_slots), kBlk) * kBlk;
     p.few_cols = (int)(even < 64 ? 64 : even);
     p.splits = (int)ceil_div(vocab, p.few_cols);
     return p;
   }
-  if (one_tile_only || cus % (8 * kXcds) != 0) return p;
+  if (cus % (8 * kXcds) != 0) return p;
   const int64_t split_rounds = ceil_div(tok_tiles * sp, cus) * ceil_div(voc_tiles, sp);
   FwdPlan b = p;
   b.splits = 0;
@@ -1451,12 +1449,19 @@ extern "C" int vamd_lce_timing_collect(double* ms_by_kernel, int64_t* launches_b
 extern "C" size_t vamd_lce_forward_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab) {
   (void)hidden_size;
   if (n_tokens <= 0 || vocab <= 0) return 0;
-  int64_t slots = 0;  // with a logits cache the launch has one token tile per workgroup
-  for (bool one_tile_only : {false, true}) {
-    const int64_t n = plan_forward(n_tokens, vocab, one_tile_only).slots();
-    if (n > slots) slots = n;
-  }
-  return (size_t)slots * kTile * (sizeof(float4) + sizeof(float));  // state + squared sums
+  return (size_t)plan_forward(n_tokens, vocab).slots() * kTile * (sizeof(float4) + sizeof(float));  // state + squared sums
+}
+
+typedef void (*ForwardKernel)(FwdArgs);
+static ForwardKernel forward_kernel(bool cache, bool pi2, const FwdPlan& plan) {
+  static const ForwardKernel kernels[3][2][2] = {
+      {{lce_forward_few_kernel<false, false>, lce_forward_few_kernel<false, true>},
+       {lce_forward_few_kernel<true, false>, lce_forward_few_kernel<true, true>}},
+      {{lce_forward_kernel<false, false, false>, lce_forward_kernel<false, true, false>},
+       {lce_forward_kernel<true, false, false>, lce_forward_kernel<true, true, false>}},
+      {{lce_forward_kernel<false, false, true>, lce_forward_kernel<false, true, true>},
+       {lce_forward_kernel<true, false, true>, lce_forward_kernel<true, true, true>}}};
+  return kernels[plan.few_cols ? 0 : plan.splits ? 1 : 2][cache][pi2];
 }
 
 // Forward launches shared by the two entry points; `workspace` holds at least
@@ -1473,7 +1478,7 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   a.n_tokens = (int)n_tokens;
   a.vocab = (int)vocab;
   a.k_slabs = (int)(hidden_size / kBK);
-  a.plan = plan_forward(n_tokens, vocab, logits_cache != nullptr, max_slots);
+  a.plan = plan_forward(n_tokens, vocab, max_slots);
   a.scale2 = rcp_temperature * kLog2e;
   a.rcp_t = rcp_temperature;
   a.partials = static_cast<float4*>(workspace);
@@ -1486,19 +1491,9 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
   {
     ScopedTiming tm(kTagForward, s);
     const dim3 grid(a.plan.splits ? a.plan.tok_tiles * a.plan.splits : a.plan.group * kXcds), block(kThreads);
-    auto launch = [&](auto* kernel, size_t lds_bytes) { hipLaunchKernelGGL(kernel, grid, block, lds_bytes, s, a); };
-    const bool pi2 = sum_pi_squared != nullptr;
-    if (logits_cache)
-      launch(pi2 ? lce_forward_kernel<true, true, false> : lce_forward_kernel<true, false, false>,
-             kLdsBytes + kCacheStageBytes);
-    else if (a.plan.few_cols)
-      launch(pi2 ? lce_forward_few_kernel<true> : lce_forward_few_kernel<false>, kFewLds);
-    else if (a.plan.splits)
-      launch(pi2 ? lce_forward_kernel<false, true, false> : lce_forward_kernel<false, false, false>,
-             kLdsBytes + kFwdTokenLds);
-    else
-      launch(pi2 ? lce_forward_kernel<false, true, true> : lce_forward_kernel<false, false, true>,
-             kLdsBytes + kFwdTokenLds);
+    const bool pi2 = sum_pi_squared != nullptr, cache = logits_cache != nullptr;
+    const int lds_bytes = a.plan.few_cols ? (cache ? kFewCacheLds : kFewLds) : kLdsBytes + (cache ? kFwdCacheLds : kFwdTokenLds);
+    hipLaunchKernelGGL(forward_kernel(cache, pi2, a.plan), grid, block, lds_bytes, s, a);
   }
   VAMD_LAUNCH_CHECK();
 
@@ -1653,6 +1648,20 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
                                         const float* logits_cache, void* d_hidden, void* d_weight, int d_weight_mode,
                                         float* d_weight_acc32, int64_t vocab_chunk, void* workspace,
                                         size_t workspace_bytes, void* stream) {
+  return vamd_lce_backward_subset_rows(hidden, weight, labels, n_tokens, planned_tokens, hidden_size, vocab,
+                                       rcp_temperature, lse, mean_z, d_logprobs, d_entropy, d_entropy_scalar,
+                                       logits_cache, nullptr, d_hidden, d_weight, d_weight_mode, d_weight_acc32,
+                                       vocab_chunk, workspace, workspace_bytes, stream);
+}
+
+extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* weight, const int64_t* labels,
+                                             int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size,
+                                             int64_t vocab, float rcp_temperature, const float* lse,
+                                             const float* mean_z, const float* d_logprobs, const float* d_entropy,
+                                             float d_entropy_scalar, const float* logits_cache,
+                                             const int64_t* logits_rows, void* d_hidden, void* d_weight,
+                                             int d_weight_mode, float* d_weight_acc32, int64_t vocab_chunk,
+                                             void* workspace, size_t workspace_bytes, void* stream) {
   int st = check_head_shapes(n_tokens, hidden_size, vocab, logits_cache);
   if (st != VAMD_OK) return st;
   VAMD_REQUIRE(hidden && weight && labels && lse && mean_z, "lce_backward: null pointer");
@@ -1711,6 +1720,8 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     if (logits_cache) {
       DLogitsArgs d;
       d.z_cache = logits_cache;
+      d.rows = logits_rows;
+      d.cache_rows = logits_rows ? planned_tokens : n_tokens;
       d.labels = labels;
       d.lse = lse;
       d.mean_z = mean_z;
@@ -1746,7 +1757,6 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
       r.k_slabs = (int)(hidden_size / kBK);
       r.tok_tiles = tok_tiles;
       r.chunk_tiles = chunk_tiles;
-      r.scale2 = rcp_temperature * kLog2e;
       r.rcp_t = rcp_temperature;
       r.dz = dz;
       r.dz_ld = (int)pitch;
@@ -1755,7 +1765,7 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
         const int grid = tiles < cus ? tiles : cus;
         {
           ScopedTiming tm(kTagRecompute, s);
-          hipLaunchKernelGGL(lce_recompute_kernel, dim3(grid), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, r);
+          hipLaunchKernelGGL(lce_recompute_kernel, dim3(grid), dim3(kThreads), kLdsBytes + kRecomputeExtraLds, s, r);
         }
         VAMD_LAUNCH_CHECK();
       }
@@ -1797,7 +1807,7 @@ extern "C" int vamd_lce_backward_subset(const void* hidden, const void* weight, 
     gw.ld_out = hidden_size;
     {
       ScopedTiming tm(kTagDGrad, s);
-      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kCacheStageBytes, s, gh, gw,
+      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kGradStageBytes, s, gh, gw,
                          plan);
     }
     VAMD_LAUNCH_CHECK();

@@ -4,12 +4,13 @@ Drop-in for ``verl.utils.kernel.linear_cross_entropy`` (reference
 verl/utils/kernel/linear_cross_entropy.py:38-119): same class name, ``forward`` / ``backward``
 signatures, argument checks and return tuple.  The arithmetic runs in ``libverl_amd.so``
 (``vamd_lce_forward`` / ``vamd_lce_backward``): bf16 MFMA logits tiles with an in-register online
-softmax.  The ``[tokens, vocab]`` logits are never materialised: the backward pass recomputes them
-tile by tile, as the reference does.  Opt-in trade for a 288 GB part: with
-``VAMD_LCE_LOGITS_CACHE_GB=<budget>`` in the environment (default 0 = off), a forward pass that a
-backward pass will follow keeps the logits in fp32 when ``4 * tokens * vocab`` bytes fit the budget,
-and the backward pass then skips its logits-recompute GEMM (a quarter of the step's matrix work).
-Results are the same either way up to one fp32 rounding of the logits.
+softmax.  The backward pass needs the ``[tokens, vocab]`` logits again.  A forward pass that a backward pass will
+follow keeps them in fp32 where they are a small part of the memory that is free at that moment
+(``keeps_logits``): on a 288 GB part that is the ordinary case, and it spares the backward pass its
+logits-recompute GEMM, a quarter of the step's matrix work.  Otherwise no such tensor ever exists and the logits are
+recomputed tile by tile, as the reference does.  ``VAMD_LCE_LOGITS_CACHE_GB=<budget>`` in the environment decides
+instead by ``4 * tokens * vocab`` against the budget (0 = never keep them).  The gradients are the same bits
+either way.
 """
 from __future__ import annotations
 
@@ -44,10 +45,54 @@ def _check_inputs(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tens
     )
 
 
-def logits_cache_budget_bytes() -> int:
-    """Largest fp32 logits cache the autograd path may allocate: ``VAMD_LCE_LOGITS_CACHE_GB`` GiB, default 0
-    (no cache: the backward pass recomputes the logits)."""
-    return int(float(os.environ.get("VAMD_LCE_LOGITS_CACHE_GB", "0")) * (1 << 30))
+def logits_cache_budget_bytes() -> int | None:
+    """Largest fp32 logits cache the autograd path may allocate, where ``VAMD_LCE_LOGITS_CACHE_GB`` (GiB) says so; 0: no
+    cache, the backward pass recomputes the logits."""
+    budget = os.environ.get("VAMD_LCE_LOGITS_CACHE_GB")
+    return None if budget is None else int(float(budget) * (1 << 30))
+
+
+# Without a budget the logits are kept while they take no more than this part of the memory that is free.
+_LOGITS_CACHE_SHARE = 8
+
+
+def _free_device_bytes(device) -> int:
+    """Memory that a new tensor of this process can be made of: free on the device or held by torch's allocator for no
+    tensor, and within the process's memory fraction.  0 where the allocator does not say."""
+    try:
+        free, total = torch.cuda.mem_get_info(device)
+        stats = torch.cuda.memory_stats_as_nested_dict(device)
+        held, used = (stats[key]["all"]["current"] for key in ("reserved_bytes", "allocated_bytes"))
+        return min(free + held - used, int(torch.cuda.get_per_process_memory_fraction(device) * total) - used)
+    except (KeyError, RuntimeError):   # another allocator than torch's own
+        return 0
+
+
+def keeps_logits(n_tokens: int, vocab: int, device) -> bool:
+    """Whether a forward pass that a backward pass will follow keeps its logits (``4 * n_tokens * vocab`` bytes).
+
+    Keeping them is quicker at every size (forward and backward, ms: 16384 x 3584 x 152064 50.9 -> 41.7, 777 x 896 x 151936
+    0.960 -> 0.898, 64 x 896 x 151936 0.352 -> 0.312; asking for the free memory takes 15 us of the host's time), so memory
+    alone decides: an eighth of what is free at the moment, so that several micro-batches whose backward passes are still to
+    come, and other users of the device, find room.  Not under stream capture, where a graph would hold the memory for
+    good, nor while saved-tensor hooks are set, which would move the logits off the device or keep them elsewhere."""
+    if vocab % 8 != 0:
+        return False
+    budget = logits_cache_budget_bytes()
+    if budget is not None:
+        return 4 * n_tokens * vocab <= budget
+    if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None or torch.cuda.is_current_stream_capturing():
+        return False
+    return 4 * n_tokens * vocab * _LOGITS_CACHE_SHARE <= _free_device_bytes(device)
+
+
+def _new_logits_cache(n_tokens: int, vocab: int, device) -> torch.Tensor | None:
+    try:
+        return torch.empty((n_tokens, vocab), device=device, dtype=torch.float32)
+    except torch.OutOfMemoryError:   # free, but not in one piece
+        if logits_cache_budget_bytes() is not None:
+            raise
+        return None
 
 
 def efficient_entropy_forward(hidden, weight, labels, reduction: int = 0, temperature: float = 1.0,
@@ -105,7 +150,8 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
                                d_weight_out: torch.Tensor | None = None, vocab_chunk: int = 0,
                                logits_cache: torch.Tensor | None = None,
                                d_weight_acc32: torch.Tensor | None = None, acc32_step: str | None = None,
-                               need_d_hidden: bool = True, need_d_weight: bool = True, planned_tokens: int | None = None):
+                               need_d_hidden: bool = True, need_d_weight: bool = True, planned_tokens: int | None = None,
+                               logits_rows: torch.Tensor | None = None):
     """Host side of the backward kernels (reference kernels.py:1512-1723).
 
     ``dlogprobs`` / ``dentropy`` may be ``None`` (no contribution).  ``d_entropy_scalar`` adds a
@@ -121,6 +167,7 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
     torch backend allocates and accumulates only the gradients its inputs require
     (verl/utils/experimental/torch_functional.py:150-156, :184-187).
     ``planned_tokens``: set when the arguments are some of the tokens of a larger call, to that call's token count.
+    ``logits_rows``: then the rows of the larger call's ``logits_cache`` that belong to them (int64).
     Returns ``(d_hidden, d_weight)`` in ``hidden.dtype``; ``d_weight`` is ``None`` for the "first" and
     "middle" steps of an fp32 accumulation.
     """
@@ -145,9 +192,13 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
         dentropy = dentropy.to(torch.float32).contiguous()
         assert d_entropy_scalar == 0.0, "pass the entropy gradient either as a tensor or as a scalar"
     assert lse.shape == (n,) and mean_z.shape == (n,)
+    planned = n if planned_tokens is None else planned_tokens
     if logits_cache is not None:
-        assert logits_cache.shape == (n, v) and logits_cache.dtype == torch.float32
+        assert logits_cache.shape == (n if logits_rows is None else planned, v) and logits_cache.dtype == torch.float32
         assert logits_cache.is_contiguous() and logits_cache.device == dev
+    if logits_rows is not None:
+        assert logits_rows.shape == (n,) and logits_rows.dtype == torch.int64
+        assert logits_rows.is_contiguous() and logits_rows.device == dev
     if labels.dtype != torch.int64:
         labels = labels.to(torch.int64)
     L = _cabi.lib()
@@ -169,13 +220,12 @@ def efficient_entropy_backward(dlogprobs, dentropy, hidden, weight, labels, lse,
         d_weight = d_weight_out if d_weight_out is not None else torch.empty_like(weight)
     if d_weight is not None:
         assert d_weight.shape == weight.shape and d_weight.dtype == weight.dtype and d_weight.is_contiguous()
-    planned = n if planned_tokens is None else planned_tokens
     with _cabi.device_guard(dev):   # the query as well: it counts the current device's compute units
         ws = _cabi.workspace(L.vamd_lce_backward_subset_workspace_bytes(n, planned, h, v, vocab_chunk), dev)
-        _cabi.check(L.vamd_lce_backward_subset(
+        _cabi.check(L.vamd_lce_backward_subset_rows(
             hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(), n, planned, h, v, 1.0 / temperature,
             lse.data_ptr(), mean_z.data_ptr(), _cabi.ptr(dlogprobs), _cabi.ptr(dentropy), float(d_entropy_scalar),
-            _cabi.ptr(logits_cache), _cabi.ptr(d_hidden), _cabi.ptr(d_weight), mode, _cabi.ptr(d_weight_acc32),
+            _cabi.ptr(logits_cache), _cabi.ptr(logits_rows), _cabi.ptr(d_hidden), _cabi.ptr(d_weight), mode, _cabi.ptr(d_weight_acc32),
             int(vocab_chunk), ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
     return d_hidden, d_weight
 
@@ -224,7 +274,7 @@ def active_token_index(dlogprobs, dentropy, n_tokens: int, weight_shape):
 
 
 def backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels, lse, mean_z, temperature,
-                                need_d_hidden: bool, need_d_weight: bool):
+                                need_d_hidden: bool, need_d_weight: bool, logits_cache=None):
     """``efficient_entropy_backward`` over the rows ``idx`` of its per-token arguments; ``d_hidden`` comes back with
     zero rows for the tokens left out.  ``d_hidden`` rows are the same bits as over all tokens where the backward pass over
     all of them stages ``d_logits`` in one vocabulary chunk (a row depends on its own token only); with several chunks,
@@ -237,7 +287,8 @@ def backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels
     dh, d_weight = efficient_entropy_backward(take(dlogprobs), take(dentropy), take(hidden), weight, take(labels),
                                               take(lse), take(mean_z), 0, temperature,
                                               need_d_hidden=need_d_hidden, need_d_weight=need_d_weight,
-                                              planned_tokens=hidden.shape[0])
+                                              planned_tokens=hidden.shape[0], logits_cache=logits_cache,
+                                              logits_rows=None if logits_cache is None else idx)
     if need_d_hidden:
         d_hidden.index_copy_(0, idx, dh)
     return d_hidden, d_weight
@@ -293,8 +344,8 @@ class LinearCrossEntropy(torch.autograd.Function):
         cache = None
         n_tokens, vocab = hidden.shape[0], weight.shape[0]
         backward_follows = grad_mode and (ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
-        if backward_follows and vocab % 8 == 0 and 4 * n_tokens * vocab <= logits_cache_budget_bytes():
-            cache = torch.empty((n_tokens, vocab), device=hidden.device, dtype=torch.float32)
+        if backward_follows and hidden.is_cuda and keeps_logits(n_tokens, vocab, hidden.device):
+            cache = _new_logits_cache(n_tokens, vocab, hidden.device)
         logprobs, entropy, lse, mean_z = efficient_entropy_forward(
             hidden, weight, labels, REDUCTION, temperature, dist_process_group, logits_cache=cache)
         ctx.save_for_backward(hidden, weight, labels, lse, mean_z, cache)
@@ -317,11 +368,11 @@ class LinearCrossEntropy(torch.autograd.Function):
             dlogprobs = dlogprobs.reshape(-1)
         need_dh, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         idx = None
-        if cache is None and ctx.REDUCTION == 0 and (need_dh or need_dw):
+        if ctx.REDUCTION == 0 and (need_dh or need_dw):
             idx = active_token_index(dlogprobs, dentropy, hidden.shape[0], weight.shape)
         if idx is not None:   # tokens the loss masked out are left out of the backward kernels
             d_hidden, d_weight = backward_over_active_tokens(idx, dlogprobs, dentropy, hidden, weight, labels, lse,
-                                                             mean_z, ctx.temperature, need_dh, need_dw)
+                                                             mean_z, ctx.temperature, need_dh, need_dw, cache)
         else:
             d_hidden, d_weight = efficient_entropy_backward(
                 dlogprobs, dentropy, hidden, weight, labels, lse, mean_z, ctx.REDUCTION, ctx.temperature,

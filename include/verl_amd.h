@@ -570,6 +570,14 @@ int vamd_kl_loss_forward(const float* logprob, const float* ref_logprob, const v
                          float* grad_unscaled, float* coef_out, void* workspace, size_t workspace_bytes,
                          void* stream);
 
+/* ------------------------------------------------------------------------------------------
+ * A few results to the host without a copy and a synchronisation of their own: one wavefront copies `bytes` (a multiple
+ * of 4, at most 4096) from device memory at src to host_values and then stores `number` to host_flag.  Both are device
+ * addresses of coherent host memory (hipHostMalloc); a host thread that reads `number` from the flag (with acquire order)
+ * finds the values in place.  No counterpart in the reference, which reads each metric with .item(). */
+int vamd_write_to_host(const void* src, int64_t bytes, void* host_values, void* host_flag, uint32_t number,
+                       void* stream);
+
 /* ==========================================================================================
  * MEASUREMENT AIDS.  Nothing below is part of the drop-in: none of these entry points has a counterpart in the
  * reference and no caller of the policy math needs them.  They exist so that bench.py and the profiler passes

@@ -2051,3 +2051,93 @@ def test_odd_rows_are_written_to_their_last_column_and_no_further(dev, cols, off
                                             _cabi.stream_ptr(dev)))
     assert torch.equal(out.view(B, cols), x * (0.5 * coef[:, None]))
     assert bool((buf[:guard + offset] == -7.0).all()) and bool((buf[guard + offset + B * cols:] == -7.0).all())
+
+
+def test_fetch_reads_what_the_stream_will_have_written(dev):
+    """A few numbers to the host: both element types, up to and past what a slot holds, behind work that takes longer than
+    the host reads for, and from several threads on streams of their own."""
+    import threading
+    from verl_amd import _cabi
+    fetch = _cabi.ops().fetch
+    for dtype in (torch.float32, torch.float64):
+        for n in (1, 4, 56, 57, 112, 113, 300):
+            x = torch.randn(n, device=dev, dtype=dtype)
+            assert fetch(x) == x.tolist()
+    x = torch.randn(8, device=dev)
+    assert fetch(x[::2]) == x[::2].tolist() and fetch(x[3]) == [x[3].item()] and fetch(x.cpu()) == x.tolist()
+    special = torch.tensor([float("inf"), float("-inf"), -0.0, 1e-45], device=dev)
+    assert fetch(special) == special.tolist() and np.isnan(fetch(x.new_tensor([float("nan")]))[0])
+    a = torch.eye(8192, device=dev)
+    for _ in range(3):
+        a = a @ a          # milliseconds of work in front
+    assert fetch(a.diagonal()[:4].contiguous()) == [1.0] * 4
+    wrong = []
+
+    def work(k):
+        stream = torch.cuda.Stream(dev)
+        with torch.cuda.stream(stream):
+            for i in range(200):
+                y = torch.full((5,), float(1000 * k + i), device=dev)
+                if fetch(y) != [1000.0 * k + i] * 5:
+                    wrong.append((k, i))
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    assert _cabi.ticket_workspace(0, dev).data_ptr() == _cabi.ticket_workspace(4096, torch.device("cuda")).data_ptr()
+
+
+def _native_losses(dev):
+    from verl_amd.trainer.ppo import core_algos as CA
+    B, L = 4, 37
+    mask = (torch.arange(L, device=dev)[None, :] < torch.tensor([37, 20, 1, 36], device=dev)[:, None]).long()
+    old, adv, ref = (torch.randn(B, L, device=dev) for _ in range(3))
+    cfg = type("Cfg", (), {"clip_ratio": 0.2, "clip_ratio_low": None, "clip_ratio_high": None, "global_batch_info": {},
+                           "get": lambda self, key, default=None: default})()
+    return (B, L), {
+        "policy": lambda x: CA.compute_policy_loss_vanilla(old, x, adv, mask, "token-mean", cfg)[0],
+        "value": lambda x: CA.compute_value_loss(x, ref, old, mask, 0.5)[0],
+        "kl": lambda x: CA.compute_kl_loss(x, ref, mask),
+        "agg": lambda x: CA.agg_loss(x, mask, "seq-mean-token-mean"),
+    }
+
+
+@pytest.mark.parametrize("name", ["policy", "value", "kl", "agg"])
+def test_native_loss_nodes_in_autograd(dev, name):
+    """What the losses' autograd nodes share with any other: saved-tensor hooks see what they keep, a graph is used once
+    unless retained, inputs of another form get their gradient back in it, and no gradient is made under no_grad; forward
+    mode and vmap are refused."""
+    shape, losses = _native_losses(dev)
+    fn = losses[name]
+    x = torch.randn(shape, device=dev, requires_grad=True)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.cpu(), lambda t: t.to(dev)):
+        loss = fn(x)
+    assert len(packed) == 2 and shape in packed
+    (want,) = torch.autograd.grad(loss, x, retain_graph=True)
+    (again,) = torch.autograd.grad(loss * 3.0, x, create_graph=True)
+    assert torch.allclose(again, 3.0 * want, rtol=1e-6) and not again.requires_grad
+    torch.autograd.grad(loss, x)          # (create_graph retained it)
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(loss, x)
+    (plain,) = torch.autograd.grad(fn(x), x)
+    assert torch.equal(plain, want)
+    # another layout, another type, another device: the gradient comes back in the input's form
+    xt = x.detach().t().contiguous().requires_grad_()
+    assert torch.equal(torch.autograd.grad(fn(xt.t()), xt)[0].t(), want)
+    xd = x.detach().double().requires_grad_()
+    gd = torch.autograd.grad(fn(xd), xd)[0]
+    assert gd.dtype == torch.float64 and torch.equal(gd.float(), want)
+    xc = x.detach().cpu().requires_grad_()
+    lc = fn(xc)
+    assert lc.device.type == "cpu" and torch.equal(torch.autograd.grad(lc, xc)[0].to(dev), want)
+    with torch.no_grad():
+        assert not fn(x).requires_grad
+    assert not fn(x.detach()).requires_grad
+    import torch.autograd.forward_ad as fwAD
+    with fwAD.dual_level(), pytest.raises(RuntimeError):
+        fn(fwAD.make_dual(x, torch.ones_like(x)))
+    with pytest.raises(RuntimeError):
+        torch.vmap(fn)(x.detach()[None].expand(2, *shape))

@@ -6,15 +6,18 @@ has already mapped (same ``libamdhip64.so.7`` soname) and torch's streams are va
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
-from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_size_t, c_uint64, c_void_p
+from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_size_t, c_uint32, c_uint64, c_void_p
 
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libverl_amd.so")
+_OPS_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_torch_ops.so")
 _lock = threading.Lock()
 _lib = None
+_ops = None
 
 MASK_F32, MASK_I64, MASK_U8, MASK_I32 = 0, 1, 2, 3
 # d_weight_mode of vamd_lce_backward (VAMD_DW_*)
@@ -33,6 +36,7 @@ SIGNATURES = {
     "vamd_last_error": (c_char_p, []),
     "vamd_set_waiting_kernels": (None, [c_int]),
     "vamd_waiting_kernels_enabled": (c_int, []),
+    "vamd_write_to_host": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_uint32, c_void_p]),
     "vamd_copy_bytes": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "vamd_sum4": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "vamd_mfma_yardstick_flops": (c_int64, [c_int, c_int, c_int]),
@@ -174,6 +178,25 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def ops():
+    """The native host side of the ``[B, L]`` entry points (``csrc/torch_ops.cpp``), which calls the same library."""
+    global _ops
+    if _ops is None:
+        lib()
+        with _lock:
+            if _ops is None:
+                if not os.path.exists(_OPS_PATH):
+                    raise RuntimeError(f"{_OPS_PATH} is missing: build it with `python -m verl_amd.csrc.build`")
+                spec = importlib.util.spec_from_file_location("_torch_ops", _OPS_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                if module.abi_version() != ABI_VERSION:
+                    raise RuntimeError(f"{_OPS_PATH} was built for ABI version {module.abi_version()}, these bindings "
+                                       f"are written for {ABI_VERSION}: rebuild it")
+                _ops = module
+    return _ops
+
+
 def check(rc: int) -> None:
     if rc != 0:
         msg = lib().vamd_last_error().decode("utf-8", "replace")
@@ -225,21 +248,11 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
-_ticket_ws: dict[tuple[int, int], torch.Tensor] = {}
-
-
 def ticket_workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     """Scratch for the single-launch reductions.  Their contract: the first VAMD_TICKET_BYTES (arrival
     counters) are zero on entry and zero again on exit, so one zero-initialised buffer per
     (device, stream) is kept and reused; kernels on one stream run in order and never share it."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_ptr(device))
-    need = max(int(nbytes), 4096)
-    with _lock:
-        buf = _ticket_ws.get(key)
-        if buf is None or buf.numel() < need:
-            buf = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device=device)
-            _ticket_ws[key] = buf
-    return buf
+    return ops().ticket_workspace(int(nbytes), device)
 
 
 GAVE_UP_OFFSET = 136  # VAMD_TICKET_GAVE_UP_OFFSET

@@ -113,6 +113,15 @@ __global__ __launch_bounds__(256) void sum4_kernel(const ys_f32x4* __restrict__ 
   }
 }
 
+// One wavefront: its stores to host memory are complete (the fence waits for them) before the flag is stored.
+__global__ __launch_bounds__(64) void write_to_host_kernel(const uint32_t* __restrict__ src, int words, uint32_t* values,
+                                                           uint32_t* flag, uint32_t number) {
+  for (int i = threadIdx.x; i < words; i += 64)
+    __hip_atomic_store(values + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  if (threadIdx.x == 0) __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr int64_t kStreamingBytes = 64ll << 20;  // per tensor: the size from which the [B, L] kernels stream
 
 }  // namespace vamd
@@ -132,6 +141,17 @@ extern "C" int vamd_copy_bytes(const void* src, void* dst, int64_t bytes, void* 
   else
     hipLaunchKernelGGL(copy_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                        (const ys_u32x4*)src, (ys_u32x4*)dst, n16);
+  VAMD_LAUNCH_CHECK();
+  return VAMD_OK;
+}
+
+extern "C" int vamd_write_to_host(const void* src, int64_t bytes, void* host_values, void* host_flag, uint32_t number,
+                                  void* stream) {
+  using namespace vamd;
+  VAMD_REQUIRE(src && host_values && host_flag && bytes >= 0 && bytes <= 4096 && bytes % 4 == 0,
+               "write_to_host: need non-null pointers and at most 4096 bytes, a multiple of 4");
+  hipLaunchKernelGGL(write_to_host_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, static_cast<const uint32_t*>(src),
+                     (int)(bytes / 4), static_cast<uint32_t*>(host_values), static_cast<uint32_t*>(host_flag), number);
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;
 }

@@ -1,0 +1,597 @@
+// Native host side of the [B, L] entry points that an update calls many times a step: argument conversion, allocation,
+// the library call and the autograd nodes, which in Python cost more than the kernels they launch (GRPO, policy loss,
+// entropy aggregation and KL loss with their backward at 512 x 4096: 61 us of kernels in 340 us).  The Python functions
+// in verl_amd/trainer/ppo keep names, arguments and checks of configuration; everything from the tensors on is here.
+//
+// The backward nodes run on autograd's device thread without the interpreter, the losses' results come back through
+// host memory the GPU writes (fetch()), and the counter buffers of the single-launch reductions are kept here, one per
+// (device, stream), for Python's ctypes calls as well.
+#include <ATen/hip/HIPContext.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/extension.h>
+
+#include <atomic>
+#include <chrono>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "../../include/verl_amd.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+
+[[noreturn]] void raise_assertion(const std::string& text) {
+  PyErr_SetString(PyExc_AssertionError, text.c_str());
+  throw py::error_already_set();
+}
+
+void check(int rc) {
+  TORCH_CHECK(rc == 0, "libverl_amd error ", rc, ": ", vamd_last_error());
+}
+
+// Device the kernels run on: the tensors' GPU, or the current GPU for CPU inputs.
+at::Device compute_device(std::initializer_list<const Tensor*> tensors) {
+  for (const Tensor* t : tensors)
+    if (t->defined() && t->is_cuda()) return t->device();
+  if (!at::hasCUDA() || c10::hip::device_count() == 0)
+    throw std::runtime_error("verl_amd needs a ROCm GPU: no device is visible and there is no CPU fallback");
+  at::globalContext().lazyInitDevice(at::kCUDA);
+  return at::Device(at::kCUDA, c10::hip::current_device());
+}
+
+void* stream_of(const at::Device& dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+// fp32, contiguous, on `dev`
+Tensor as_f32(const Tensor& t, const at::Device& dev) {
+  Tensor x = t;
+  if (x.device() != dev || x.scalar_type() != at::kFloat) x = x.to(dev, at::kFloat);
+  return x.is_contiguous() ? x : x.contiguous();
+}
+
+std::string shape_text(const Tensor& t) {
+  std::string s = "(";
+  for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+  return s + (t.dim() == 1 ? ",)" : ")");
+}
+
+Tensor matrix(const Tensor& t, const at::Device& dev) {
+  Tensor x = as_f32(t, dev);
+  if (x.dim() == 1) x = x.view({1, -1});
+  if (x.dim() != 2) raise_assertion("expected a (batch, length) tensor, got shape " + shape_text(t));
+  return x;
+}
+
+// Contiguous mask on `dev` in one of the element types the kernels read, with its VAMD_MASK_* code.
+struct Mask {
+  Tensor t;
+  int code;
+};
+Mask mask_of(const Tensor& mask, const at::Device& dev) {
+  Mask m{mask.device() == dev ? mask : mask.to(dev), 0};
+  switch (mask.scalar_type()) {
+    case at::kFloat: m.code = VAMD_MASK_F32; break;
+    case at::kLong: m.code = VAMD_MASK_I64; break;
+    case at::kBool:
+    case at::kByte: m.code = VAMD_MASK_U8; break;
+    case at::kInt: m.code = VAMD_MASK_I32; break;
+    default:  // fp16 / bf16 / fp64 / int8 / int16: exact in fp32 for 0/1 masks
+      m.t = m.t.to(at::kFloat);
+      m.code = VAMD_MASK_F32;
+  }
+  if (!m.t.is_contiguous()) m.t = m.t.contiguous();
+  return m;
+}
+Mask mask_matrix(const Tensor& mask, const at::Device& dev, const Tensor& like) {
+  Mask m = mask_of(mask, dev);
+  if (m.t.dim() == 1) m.t = m.t.view({1, -1});
+  if (m.t.sizes() != like.sizes())
+    raise_assertion("mask shape " + shape_text(mask) + " does not match " + shape_text(like));
+  return m;
+}
+
+const float* f32(const Tensor& t) { return t.defined() ? t.const_data_ptr<float>() : nullptr; }
+float* f32_out(const Tensor& t) { return t.defined() ? t.mutable_data_ptr<float>() : nullptr; }
+
+Tensor new_f32(at::IntArrayRef shape, const at::Device& dev) {
+  return at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(dev));
+}
+
+// Scratch of the single-launch reductions: its first VAMD_TICKET_BYTES are arrival counters that are zero on entry and
+// zero again on completion, so one zeroed buffer per (device, stream) is kept; kernels on one stream run in order and
+// never share it.  Never destroyed: at exit the runtime may be gone first.
+Tensor ticket_workspace(size_t bytes, const at::Device& dev) {
+  static std::mutex mu;
+  static auto* buffers = new std::map<std::pair<int, void*>, Tensor>;
+  const int64_t need = bytes < 4096 ? 4096 : (int64_t)bytes;
+  std::lock_guard<std::mutex> lock(mu);
+  Tensor& buf = (*buffers)[{(int)dev.index(), stream_of(dev)}];
+  if (!buf.defined() || buf.numel() < need)
+    buf = at::zeros({need < (1 << 20) ? (1 << 20) : need}, at::TensorOptions().dtype(at::kByte).device(dev));
+  return buf;
+}
+
+bool wants_gradient(const Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }
+
+struct Aggregation {
+  int mode;
+  double dp_size, batch_num_tokens, global_batch_size, loss_scale_factor;
+};
+
+// A loss node saves the gradient per unit upstream gradient, which the forward pass wrote, and the rows' coefficients;
+// what else its backward needs to hand the gradient back in the input's form is kept only where that is not
+// (batch, length) fp32 on the compute device.
+void save_form(AutogradContext* ctx, const Tensor& input, const at::Device& dev) {
+  if (input.dim() == 2 && input.scalar_type() == at::kFloat && input.device() == dev) return;
+  ctx->saved_data["shape"] = input.sizes().vec();
+  ctx->saved_data["device"] = input.device();
+  ctx->saved_data["dtype"] = (int64_t)input.scalar_type();
+}
+Tensor in_saved_form(AutogradContext* ctx, Tensor g) {
+  auto it = ctx->saved_data.find("shape");
+  if (it == ctx->saved_data.end()) return g;
+  return g.view(it->second.toIntVector())
+      .to(ctx->saved_data["device"].toDevice(), (at::ScalarType)ctx->saved_data["dtype"].toInt());
+}
+
+Tensor upstream(const Tensor& d_loss, const at::Device& dev) { return as_f32(d_loss, dev).reshape({1}); }
+
+// The gradient of a loss whose forward pass left it per unit upstream gradient.
+variable_list scaled_gradient(AutogradContext* ctx, const variable_list& grads, float extra_scale, size_t inputs) {
+  at::AutoGradMode no_grad(false);
+  variable_list result(inputs);
+  const auto saved = ctx->get_saved_variables();
+  TORCH_CHECK(saved.size() == 2, "the forward pass was not asked for a gradient of this input");
+  if (!grads[0].defined()) return result;
+  const Tensor &g = saved[0], &coef = saved[1];
+  const at::Device dev = g.device();
+  const c10::DeviceGuard guard(dev);
+  const Tensor d = upstream(grads[0], dev);
+  const Tensor out = at::empty_like(g);
+  check(vamd_scale_rows(f32(g), f32(coef), f32(d), extra_scale, g.size(0), g.size(1), f32_out(out), stream_of(dev)));
+  result[0] = in_saved_form(ctx, out);
+  return result;
+}
+
+// ---- policy loss ---------------------------------------------------------------------------------------------
+struct PolicyArgs {
+  int variant;
+  double clip_low, clip_high, clip_c, tau_pos, tau_neg;
+  Aggregation agg;
+};
+struct LossResult {
+  Tensor loss, out, grad, coef;
+  at::Device dev;
+};
+
+LossResult policy_forward(const Tensor& log_prob, const Tensor& old_log_prob, const Tensor& advantages,
+                          const Tensor& mask, const std::optional<Tensor>& is_weights, const PolicyArgs& a,
+                          bool need_grad) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&log_prob, &old_log_prob, &advantages, &mask});
+  const Tensor lp = matrix(log_prob, dev), old = matrix(old_log_prob, dev), adv = matrix(advantages, dev);
+  if (lp.sizes() != old.sizes() || old.sizes() != adv.sizes()) raise_assertion("");
+  const Mask m = mask_matrix(mask, dev, lp);
+  const Tensor isw = is_weights ? matrix(*is_weights, dev) : Tensor();
+  const int64_t rows = lp.size(0), cols = lp.size(1);
+  const c10::DeviceGuard guard(dev);
+  // one allocation for the four result floats and the per-row coefficients (16-byte aligned both)
+  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 4), coef = buf.narrow(0, 4, rows);
+  const Tensor g = need_grad ? at::empty_like(lp) : Tensor();
+  const Tensor ws = ticket_workspace(vamd_policy_loss_variant_workspace_bytes(rows, cols), dev);
+  check(vamd_policy_loss_variant_forward(a.variant, f32(old), f32(lp), f32(adv), m.t.const_data_ptr(), m.code, f32(isw),
+                                         rows, cols, (float)a.clip_low, (float)a.clip_high, (float)a.clip_c,
+                                         (float)a.tau_pos, (float)a.tau_neg, a.agg.mode, a.agg.dp_size,
+                                         a.agg.batch_num_tokens, a.agg.global_batch_size, a.agg.loss_scale_factor,
+                                         f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(), ws.numel(),
+                                         stream_of(dev)));
+  // the loss is a view: it shares the floats the kernel wrote with the metrics
+  const Tensor result = log_prob.device() == dev ? out : out.to(log_prob.device());
+  return {result.select(0, 0), result, g, coef, dev};
+}
+
+class PolicyLoss : public torch::autograd::Function<PolicyLoss> {
+ public:
+  static variable_list forward(AutogradContext* ctx, const Tensor& log_prob, const Tensor& old_log_prob,
+                               const Tensor& advantages, const Tensor& mask,
+                               const std::optional<Tensor>& is_weights, const PolicyArgs& args) {
+    const LossResult r = policy_forward(log_prob, old_log_prob, advantages, mask, is_weights, args, true);
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({r.grad, r.coef});
+    save_form(ctx, log_prob, r.dev);
+    ctx->mark_non_differentiable({r.out});
+    return {r.loss, r.out};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    return scaled_gradient(ctx, grads, 1.f, 6);
+  }
+};
+
+std::pair<Tensor, Tensor> policy_loss(const Tensor& log_prob, const Tensor& old_log_prob, const Tensor& advantages,
+                                      const Tensor& mask, const std::optional<Tensor>& is_weights, double clip_low,
+                                      double clip_high, double clip_c, int mode, double dp_size, double bnt, double gbs,
+                                      double lsf, int variant, double tau_pos, double tau_neg) {
+  const PolicyArgs a{variant, clip_low, clip_high, clip_c, tau_pos, tau_neg, {mode, dp_size, bnt, gbs, lsf}};
+  if (wants_gradient(log_prob)) {
+    const auto r = PolicyLoss::apply(log_prob, old_log_prob, advantages, mask, is_weights, a);
+    return {r[0], r[1]};
+  }
+  const LossResult r = policy_forward(log_prob, old_log_prob, advantages, mask, is_weights, a, false);
+  return {r.loss, r.out};
+}
+
+// ---- value loss ----------------------------------------------------------------------------------------------
+LossResult value_forward(const Tensor& vpreds, const Tensor& returns, const Tensor& values, const Tensor& mask,
+                         double clip, int mode, bool need_grad) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&vpreds, &returns, &values, &mask});
+  const Tensor vp = matrix(vpreds, dev), ret = matrix(returns, dev), val = matrix(values, dev);
+  if (vp.sizes() != ret.sizes() || ret.sizes() != val.sizes()) raise_assertion("");
+  const Mask m = mask_matrix(mask, dev, vp);
+  const int64_t rows = vp.size(0), cols = vp.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 2), coef = buf.narrow(0, 4, rows);
+  const Tensor g = need_grad ? at::empty_like(vp) : Tensor();
+  const Tensor ws = ticket_workspace(vamd_value_loss_workspace_bytes(rows, cols), dev);
+  check(vamd_value_loss_forward(f32(vp), f32(ret), f32(val), m.t.const_data_ptr(), m.code, rows, cols, (float)clip, mode,
+                                f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(), ws.numel(),
+                                stream_of(dev)));
+  const Tensor result = vpreds.device() == dev ? out : out.to(vpreds.device());
+  return {result.select(0, 0), result, g, coef, dev};
+}
+
+class ValueLoss : public torch::autograd::Function<ValueLoss> {
+ public:
+  static variable_list forward(AutogradContext* ctx, const Tensor& vpreds, const Tensor& returns, const Tensor& values,
+                               const Tensor& mask, double clip, int mode) {
+    const LossResult r = value_forward(vpreds, returns, values, mask, clip, mode, true);
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({r.grad, r.coef});
+    save_form(ctx, vpreds, r.dev);
+    ctx->mark_non_differentiable({r.out});
+    return {r.loss, r.out};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    return scaled_gradient(ctx, grads, 0.5f, 6);
+  }
+};
+
+// (loss, clip fraction)
+std::pair<Tensor, Tensor> value_loss(const Tensor& vpreds, const Tensor& returns, const Tensor& values,
+                                     const Tensor& mask, double clip, int mode) {
+  if (wants_gradient(vpreds)) {
+    const auto r = ValueLoss::apply(vpreds, returns, values, mask, clip, mode);
+    return {r[0], r[1].select(0, 1)};
+  }
+  const LossResult r = value_forward(vpreds, returns, values, mask, clip, mode, false);
+  return {r.loss, r.out.select(0, 1)};
+}
+
+// ---- KL loss -------------------------------------------------------------------------------------------------
+struct KlArgs {
+  int kind, straight_through;
+  Aggregation agg;
+};
+LossResult kl_forward(const Tensor& logprob, const Tensor& ref_logprob, const Tensor& mask, const KlArgs& a,
+                      bool need_grad) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&logprob, &ref_logprob, &mask});
+  const Tensor lp = matrix(logprob, dev), ref = matrix(ref_logprob, dev);
+  if (lp.sizes() != ref.sizes()) raise_assertion("");
+  const Mask m = mask_matrix(mask, dev, lp);
+  const int64_t rows = lp.size(0), cols = lp.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 1), coef = buf.narrow(0, 4, rows);
+  const Tensor g = need_grad ? at::empty_like(lp) : Tensor();
+  const Tensor ws = ticket_workspace(vamd_kl_loss_workspace_bytes(rows, cols), dev);
+  check(vamd_kl_loss_forward(f32(lp), f32(ref), m.t.const_data_ptr(), m.code, rows, cols, a.kind, a.straight_through,
+                             a.agg.mode, a.agg.dp_size, a.agg.batch_num_tokens, a.agg.global_batch_size,
+                             a.agg.loss_scale_factor, f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(),
+                             ws.numel(), stream_of(dev)));
+  const Tensor loss = out.select(0, 0);
+  return {logprob.device() == dev ? loss : loss.to(logprob.device()), Tensor(), g, coef, dev};
+}
+
+class KlLoss : public torch::autograd::Function<KlLoss> {
+ public:
+  static Tensor forward(AutogradContext* ctx, const Tensor& logprob, const Tensor& ref_logprob, const Tensor& mask,
+                        const KlArgs& args) {
+    const bool need_grad = logprob.requires_grad();
+    const LossResult r = kl_forward(logprob, ref_logprob, mask, args, need_grad);
+    ctx->set_materialize_grads(false);
+    if (need_grad) ctx->save_for_backward({r.grad, r.coef});
+    save_form(ctx, logprob, r.dev);
+    return r.loss;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    return scaled_gradient(ctx, grads, 1.f, 4);
+  }
+};
+
+Tensor kl_loss(const Tensor& logprob, const Tensor& ref_logprob, const Tensor& mask, int kind, bool straight_through,
+               int mode, double dp_size, double bnt, double gbs, double lsf) {
+  const KlArgs a{kind, straight_through, {mode, dp_size, bnt, gbs, lsf}};
+  if (wants_gradient(logprob) || wants_gradient(ref_logprob)) return KlLoss::apply(logprob, ref_logprob, mask, a);
+  return kl_forward(logprob, ref_logprob, mask, a, false).loss;
+}
+
+// ---- agg_loss ------------------------------------------------------------------------------------------------
+struct AggResult {
+  Tensor loss, coef, mask;
+  int code;
+  at::Device dev;
+};
+AggResult agg_forward(const Tensor& loss_mat, const Tensor& mask, const Aggregation& a) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&loss_mat, &mask});
+  const Tensor x = matrix(loss_mat, dev);
+  const Mask m = mask_matrix(mask, dev, x);
+  const int64_t rows = x.size(0), cols = x.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor buf = new_f32({4 + rows}, dev), out = buf.select(0, 0), coef = buf.narrow(0, 4, rows);
+  const Tensor ws = ticket_workspace(vamd_agg_loss_workspace_bytes(rows, cols), dev);
+  check(vamd_agg_loss_forward(f32(x), m.t.const_data_ptr(), m.code, rows, cols, a.mode, a.dp_size, a.batch_num_tokens,
+                              a.global_batch_size, a.loss_scale_factor, f32_out(out), f32_out(coef),
+                              ws.mutable_data_ptr(), ws.numel(), stream_of(dev)));
+  return {loss_mat.device() == dev ? out : out.to(loss_mat.device()), coef, m.t, m.code, dev};
+}
+
+class AggLoss : public torch::autograd::Function<AggLoss> {
+ public:
+  static Tensor forward(AutogradContext* ctx, const Tensor& loss_mat, const Tensor& mask, const Aggregation& args) {
+    const AggResult r = agg_forward(loss_mat, mask, args);
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({r.coef, r.mask});
+    ctx->saved_data["code"] = (int64_t)r.code;
+    save_form(ctx, loss_mat, r.dev);
+    return r.loss;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    at::AutoGradMode no_grad(false);
+    variable_list result(3);
+    const auto saved = ctx->get_saved_variables();
+    if (!grads[0].defined()) return result;
+    const Tensor &coef = saved[0], &mask = saved[1];
+    const at::Device dev = coef.device();
+    const c10::DeviceGuard guard(dev);
+    const Tensor d = upstream(grads[0], dev), g = new_f32(mask.sizes(), dev);
+    check(vamd_agg_loss_backward(f32(d), f32(coef), mask.const_data_ptr(), (int)ctx->saved_data["code"].toInt(),
+                                 mask.size(0), mask.size(1), f32_out(g), stream_of(dev)));
+    result[0] = in_saved_form(ctx, g);
+    return result;
+  }
+};
+
+Tensor agg_loss(const Tensor& loss_mat, const Tensor& mask, int mode, double dp_size, double bnt, double gbs,
+                double lsf) {
+  const Aggregation a{mode, dp_size, bnt, gbs, lsf};
+  if (wants_gradient(loss_mat) || wants_gradient(mask)) return AggLoss::apply(loss_mat, mask, a);
+  return agg_forward(loss_mat, mask, a).loss;
+}
+
+// ---- advantages and statistics -------------------------------------------------------------------------------
+Tensor in_form_of(const Tensor& x, const Tensor& input) {
+  const Tensor y = x.sizes() == input.sizes() ? x : x.view(input.sizes());
+  return y.device() == input.device() ? y : y.to(input.device());
+}
+
+// (advantages, the counter buffer the call used)
+std::pair<Tensor, Tensor> grpo_advantage(const Tensor& rewards, const Tensor& mask, const Tensor& ids, int64_t groups,
+                                         double epsilon, bool norm_by_std, int std_mode) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&rewards, &mask});
+  const Tensor r = matrix(rewards, dev);
+  const Mask m = mask_matrix(mask, dev, r);
+  const int64_t rows = r.size(0), cols = r.size(1);
+  TORCH_CHECK_VALUE(ids.numel() == rows, "index has ", ids.numel(), " entries for a batch of ", rows);
+  const c10::DeviceGuard guard(dev);
+  const Tensor adv = at::empty_like(r);
+  const Tensor ws = ticket_workspace(vamd_grpo_workspace_bytes(rows, cols, groups), dev);
+  check(vamd_grpo_advantage(f32(r), m.t.const_data_ptr(), m.code, ids.const_data_ptr<int64_t>(), rows, cols, groups,
+                            (float)epsilon, norm_by_std, std_mode, f32_out(adv), nullptr, ws.mutable_data_ptr(),
+                            ws.numel(), stream_of(dev)));
+  return {in_form_of(adv, rewards), ws};
+}
+
+// (advantages, returns, moments)
+std::tuple<Tensor, Tensor, Tensor> gae(const Tensor& rewards, const Tensor& values, const Tensor& mask, double gamma,
+                                       double lam, int whiten) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&rewards, &values, &mask});
+  const Tensor r = matrix(rewards, dev), v = matrix(values, dev);
+  if (r.sizes() != v.sizes()) raise_assertion("");
+  const Mask m = mask_matrix(mask, dev, r);
+  const int64_t rows = r.size(0), cols = r.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor adv = at::empty_like(r), ret = at::empty_like(r);
+  const Tensor mom = at::empty({5}, at::TensorOptions().dtype(at::kDouble).device(dev));
+  const Tensor ws = ticket_workspace(vamd_gae_workspace_bytes(rows, cols), dev);
+  check(vamd_gae(f32(r), f32(v), m.t.const_data_ptr(), m.code, rows, cols, (float)gamma, (float)lam, whiten,
+                 f32_out(adv), f32_out(ret), mom.mutable_data_ptr<double>(), ws.mutable_data_ptr(), ws.numel(),
+                 stream_of(dev)));
+  return {in_form_of(adv, rewards), in_form_of(ret, rewards), mom};
+}
+
+// (token-level rewards, mean KL [1])
+std::pair<Tensor, Tensor> kl_rewards(const Tensor& scores, const Tensor& logprob, const Tensor& ref_logprob,
+                                     const Tensor& mask, int kind, double beta) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&scores, &logprob, &ref_logprob, &mask});
+  const Tensor sc = matrix(scores, dev), lp = matrix(logprob, dev), rf = matrix(ref_logprob, dev);
+  if (sc.sizes() != lp.sizes() || lp.sizes() != rf.sizes()) raise_assertion("");
+  const Mask m = mask_matrix(mask, dev, sc);
+  const int64_t rows = sc.size(0), cols = sc.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor out = at::empty_like(sc), kl = new_f32({1}, dev);
+  const Tensor ws = ticket_workspace(vamd_apply_kl_penalty_workspace_bytes(rows, cols), dev);
+  check(vamd_apply_kl_penalty(f32(sc), f32(lp), f32(rf), m.t.const_data_ptr(), m.code, rows, cols, kind, (float)beta,
+                              f32_out(out), f32_out(kl), ws.mutable_data_ptr(), ws.numel(), stream_of(dev)));
+  return {in_form_of(out, scores), kl};
+}
+
+Tensor scratch(size_t bytes, const at::Device& dev) {
+  return at::empty({bytes < 256 ? 256 : (int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(dev));
+}
+
+// (weights or None, metrics)
+std::pair<std::optional<Tensor>, Tensor> rollout_correction(const Tensor& old_log_prob,
+                                                            const std::optional<Tensor>& rollout_log_prob,
+                                                            const Tensor& mask, int level, double threshold,
+                                                            bool batch_normalize, int64_t slots) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&old_log_prob, &mask});
+  Tensor old = as_f32(old_log_prob, dev);
+  if (old.dim() == 1) old = old.view({1, -1});
+  if (old.dim() != 2) raise_assertion("expected (batch, length) log-probabilities, got " + shape_text(old_log_prob));
+  const Tensor roll = rollout_log_prob ? as_f32(*rollout_log_prob, dev).view(old.sizes()) : Tensor();
+  Mask m = mask_of(mask, dev);
+  m.t = m.t.view(old.sizes());
+  const int64_t rows = old.size(0), cols = old.size(1);
+  const c10::DeviceGuard guard(dev);
+  const Tensor weights = level ? at::empty_like(old) : Tensor();
+  const Tensor out = at::empty({slots}, at::TensorOptions().dtype(at::kDouble).device(dev));
+  const Tensor ws = scratch(vamd_rollout_correction_workspace_bytes(rows, cols), dev);
+  check(vamd_rollout_correction(f32(old), f32(roll), m.t.const_data_ptr(), m.code, rows, cols, level, (float)threshold,
+                                batch_normalize, f32_out(weights), out.mutable_data_ptr<double>(),
+                                ws.mutable_data_ptr(), ws.numel(), stream_of(dev)));
+  if (!level) return {std::nullopt, out};
+  return {in_form_of(weights, old_log_prob), out};
+}
+
+Tensor data_metrics(const Tensor& scores, const Tensor& rewards, const Tensor& advantages, const Tensor& returns,
+                    const std::optional<Tensor>& values, const Tensor& response_mask, const Tensor& attention_mask,
+                    int64_t width, int64_t slots) {
+  at::AutoGradMode no_grad(false);
+  const at::Device dev = compute_device({&scores, &response_mask, &attention_mask});
+  const Tensor sc = as_f32(scores, dev);
+  if (sc.dim() != 2 || sc.size(1) != width)
+    raise_assertion("token_level_scores " + shape_text(sc) + " vs response width " + std::to_string(width));
+  const Tensor rw = as_f32(rewards, dev), adv = as_f32(advantages, dev), ret = as_f32(returns, dev);
+  const Tensor val = values ? as_f32(*values, dev) : Tensor();
+  for (const Tensor* t : {&rw, &adv, &ret, &val})
+    if (t->defined() && t->sizes() != sc.sizes()) raise_assertion("");
+  const Mask m = mask_of(response_mask, dev), att = mask_of(attention_mask, dev);
+  const int64_t rows = sc.size(0);
+  if (m.t.sizes() != sc.sizes() || att.t.size(0) != rows || att.t.size(1) < width) raise_assertion("");
+  const c10::DeviceGuard guard(dev);
+  const Tensor out = at::empty({slots}, at::TensorOptions().dtype(at::kDouble).device(dev));
+  const Tensor ws = scratch(vamd_data_metrics_workspace_bytes(rows, width), dev);
+  check(vamd_data_metrics(f32(sc), f32(rw), f32(adv), f32(ret), f32(val), m.t.const_data_ptr(), m.code,
+                          att.t.const_data_ptr(), att.code, rows, att.t.size(1) - width, width,
+                          out.mutable_data_ptr<double>(), ws.mutable_data_ptr(), ws.numel(), stream_of(dev)));
+  return out;
+}
+
+// ---- a few numbers to the host -------------------------------------------------------------------------------
+// What a copy and a synchronisation take 13 us for on an idle stream: a kernel of one wavefront writes the numbers and
+// then a sequence number into host memory, which this thread reads until it sees it.  Slots are taken for the length of a
+// call; a call that finds none left, or numbers that do not fit, goes through a copy.
+constexpr int kSlots = 32, kSlotBytes = 512, kFlagBytes = 64;
+struct Slots {
+  std::mutex mu;
+  char* base = nullptr;
+  bool failed = false;
+  uint32_t sequence = 0;
+  std::vector<int> free;
+
+  // index of a slot and the sequence number to wait for, or -1
+  int take(uint32_t& number) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!base && !failed) {
+      void* p = nullptr;
+      failed = hipHostMalloc(&p, kSlots * kSlotBytes, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess;
+      if (!failed) {
+        base = static_cast<char*>(p);
+        for (int i = 0; i < kSlots; ++i) {
+          *reinterpret_cast<uint32_t*>(base + i * kSlotBytes) = 0;
+          free.push_back(i);
+        }
+      } else {
+        (void)hipGetLastError();
+      }
+    }
+    if (free.empty()) return -1;
+    const int slot = free.back();
+    free.pop_back();
+    number = ++sequence ? sequence : ++sequence;  // never 0
+    return slot;
+  }
+  void give_back(int slot) {
+    std::lock_guard<std::mutex> lock(mu);
+    free.push_back(slot);
+  }
+};
+
+// The values of a contiguous fp32 or fp64 vector as Python floats.
+std::vector<double> fetch(const Tensor& t) {
+  static auto* slots = new Slots;  // never destroyed: at exit the runtime may be gone first
+  const bool f64 = t.scalar_type() == at::kDouble;
+  const int64_t n = t.numel(), bytes = n * (f64 ? 8 : 4);
+  std::vector<double> values(n);
+  auto read = [&](const void* p) {
+    for (int64_t i = 0; i < n; ++i)
+      values[i] = f64 ? static_cast<const double*>(p)[i] : (double)static_cast<const float*>(p)[i];
+  };
+  py::gil_scoped_release no_gil;
+  if (t.is_cuda() && t.is_contiguous() && bytes <= kSlotBytes - kFlagBytes) {
+    const c10::DeviceGuard guard(t.device());
+    const hipStream_t stream = (hipStream_t)stream_of(t.device());
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    uint32_t number = 0;
+    int slot = -1;
+    if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone)
+      slot = slots->take(number);
+    if (slot >= 0) {
+      char* const at = slots->base + slot * kSlotBytes;
+      const int rc = vamd_write_to_host(t.const_data_ptr(), bytes, at + kFlagBytes, at, number, stream);
+      hipError_t err = hipSuccess;
+      if (rc == 0) {
+        // Reads for as long as a step's small kernels may take, then waits for the stream, which does not keep a core busy.
+        const auto* flag = reinterpret_cast<const std::atomic<uint32_t>*>(at);
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while (flag->load(std::memory_order_acquire) != number) {
+          if (std::chrono::steady_clock::now() < until) continue;
+          err = hipStreamSynchronize(stream);
+          break;
+        }
+        if (err == hipSuccess && flag->load(std::memory_order_acquire) == number) read(at + kFlagBytes);
+        else if (err == hipSuccess) err = hipErrorUnknown;
+      }
+      // after an error the kernel may still write the slot: it is not used again
+      if (rc != 0 || err == hipSuccess) slots->give_back(slot);
+      check(rc);
+      TORCH_CHECK(err == hipSuccess, "libverl_amd: results could not be read: ", hipGetErrorString(err));
+      return values;
+    }
+  }
+  const Tensor host = t.detach().to(at::kCPU).contiguous();
+  read(host.const_data_ptr());
+  return values;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("abi_version", [] { return VAMD_ABI_VERSION; });
+  m.def("ticket_workspace", [](int64_t bytes, at::Device dev) {
+    if (!dev.has_index()) dev.set_index(c10::hip::current_device());
+    return ticket_workspace((size_t)(bytes < 0 ? 0 : bytes), dev);
+  });
+  m.def("policy_loss", &policy_loss);
+  m.def("value_loss", &value_loss);
+  m.def("kl_loss", &kl_loss);
+  m.def("agg_loss", &agg_loss);
+  m.def("grpo_advantage", &grpo_advantage);
+  m.def("gae", &gae);
+  m.def("kl_rewards", &kl_rewards);
+  m.def("rollout_correction", &rollout_correction);
+  m.def("data_metrics", &data_metrics);
+  m.def("fetch", &fetch);
+}

@@ -166,43 +166,28 @@ def compute_gae_advantage_return(token_level_rewards: torch.Tensor, values: torc
     ``no_grad``.  The recurrence is evaluated as a parallel scan of affine maps, so results agree
     with the sequential fp32 loop to rounding, not bit for bit.
     """
-    with torch.no_grad():
-        dev = _cabi.compute_device(token_level_rewards, values, response_mask)
-        r = _matrix(token_level_rewards, dev)
-        v = _matrix(values, dev)
-        assert r.shape == v.shape
-        m, code = _mask_matrix(response_mask, dev, r.shape)
-        B, Lc = r.shape
-        adv = torch.empty_like(r)
-        ret = torch.empty_like(r)
-        mom = torch.empty(5, dtype=torch.float64, device=dev)
-        Lb = _cabi.lib()
-        ws = _cabi.ticket_workspace(Lb.vamd_gae_workspace_bytes(B, Lc), dev)
-        # 1: one launch whose workgroups meet once (the library itself takes the two-launch form when waiting kernels
-        # are switched off); 2: two launches, nobody waits.  Once the meeting has timed out in this process (a GPU
-        # shared with long-running kernels) the waiting kernels are switched off for the whole library -- GRPO and the
-        # sequence-level losses included: a time-out costs about a second of polling, and the conditions that caused it
-        # rarely go away between two calls.
-        for whiten in (1, 2):
-            with _cabi.device_guard(dev):
-                _cabi.check(Lb.vamd_gae(r.data_ptr(), v.data_ptr(), m.data_ptr(), code, B, Lc, float(gamma),
-                                        float(lam), whiten, adv.data_ptr(), ret.data_ptr(), mom.data_ptr(),
-                                        ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
-            mom_host = mom.tolist()
-            if mom_host[4] == 0.0:
-                break
-            # the workgroups' bounded wait for each other ran out (a GPU shared with long-running kernels): the
-            # advantages were left unwhitened; do it again without waiting
-            Lb.vamd_set_waiting_kernels(0)
-            _warn_once("vamd_gae: the one-launch estimator timed out waiting for its workgroups; kernels that wait "
-                       "inside a launch are switched off from now on (set VAMD_WAITING_KERNELS=0 to make that the "
-                       "rule from the start)")
-        verl_F._raise_on_tiny_mask(mom_host[0])
-        if mom_host[4] != 0.0:
-            raise RuntimeError("vamd_gae: the workgroups' bounded wait for the whitening statistics ran out; "
-                               "the advantages were left unwhitened")
-        out_dev = token_level_rewards.device
-        return adv.view(token_level_rewards.shape).to(out_dev), ret.view(token_level_rewards.shape).to(out_dev)
+    ops = _cabi.ops()
+    # 1: one launch whose workgroups meet once (the library itself takes the two-launch form when waiting kernels
+    # are switched off); 2: two launches, nobody waits.  Once the meeting has timed out in this process (a GPU
+    # shared with long-running kernels) the waiting kernels are switched off for the whole library -- GRPO and the
+    # sequence-level losses included: a time-out costs about a second of polling, and the conditions that caused it
+    # rarely go away between two calls.
+    for whiten in (1, 2):
+        adv, ret, moments = ops.gae(token_level_rewards, values, response_mask, float(gamma), float(lam), whiten)
+        moments = ops.fetch(moments)
+        if moments[4] == 0.0:
+            break
+        # the workgroups' bounded wait for each other ran out (a GPU shared with long-running kernels): the
+        # advantages were left unwhitened; do it again without waiting
+        _cabi.lib().vamd_set_waiting_kernels(0)
+        _warn_once("vamd_gae: the one-launch estimator timed out waiting for its workgroups; kernels that wait "
+                   "inside a launch are switched off from now on (set VAMD_WAITING_KERNELS=0 to make that the "
+                   "rule from the start)")
+    verl_F._raise_on_tiny_mask(moments[0])
+    if moments[4] != 0.0:
+        raise RuntimeError("vamd_gae: the workgroups' bounded wait for the whitening statistics ran out; "
+                           "the advantages were left unwhitened")
+    return adv, ret
 
 
 # GRPO and the sequence-level losses recover from a wait that ran out inside their kernels and tell nobody; the
@@ -258,25 +243,12 @@ def _group_ids_on_device(index, vectorized: bool, dev: torch.device):
 
 
 def _grpo(token_level_rewards, response_mask, index, epsilon, norm_adv_by_std_in_grpo, std_mode):
-    with torch.no_grad():
-        dev = _cabi.compute_device(token_level_rewards, response_mask)
-        r = _matrix(token_level_rewards, dev)
-        m, code = _mask_matrix(response_mask, dev, r.shape)
-        B, Lc = r.shape
-        ids, G = _group_ids_on_device(index, std_mode == 1, dev)
-        if ids.numel() != B:
-            raise ValueError(f"index has {ids.numel()} entries for a batch of {B}")
-        adv = torch.empty_like(r)
-        Lb = _cabi.lib()
-        ws = _cabi.ticket_workspace(Lb.vamd_grpo_workspace_bytes(B, Lc, G), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_grpo_advantage(r.data_ptr(), m.data_ptr(), code, ids.data_ptr(), B, Lc, G,
-                                               float(epsilon), int(bool(norm_adv_by_std_in_grpo)), std_mode,
-                                               adv.data_ptr(), None, ws.data_ptr(), ws.numel(),
-                                               _cabi.stream_ptr(dev)))
-        _watch_waiting_kernels(ws)
-        out = adv.view(token_level_rewards.shape).to(token_level_rewards.device)
-        return out, out
+    dev = _cabi.compute_device(token_level_rewards, response_mask)
+    ids, G = _group_ids_on_device(index, std_mode == 1, dev)
+    adv, ws = _cabi.ops().grpo_advantage(token_level_rewards, response_mask, ids, G, float(epsilon),
+                                         bool(norm_adv_by_std_in_grpo), std_mode)
+    _watch_waiting_kernels(ws)
+    return adv, adv
 
 
 @register_adv_est(AdvantageEstimator.GRPO)
@@ -546,42 +518,6 @@ def _opt(x) -> float:
     return float(x.item()) if isinstance(x, torch.Tensor) else float(x)
 
 
-class _AggLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, loss_mat, loss_mask, mode, dp_size, bnt, gbs, lsf):
-        dev = _cabi.compute_device(loss_mat, loss_mask)
-        x = _matrix(loss_mat, dev)
-        m, code = _mask_matrix(loss_mask, dev, x.shape)
-        rows, cols = x.shape
-        Lb = _cabi.lib()
-        out = torch.empty((), dtype=torch.float32, device=dev)
-        coef = torch.empty(rows, dtype=torch.float32, device=dev)
-        ws = _cabi.ticket_workspace(Lb.vamd_agg_loss_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_agg_loss_forward(x.data_ptr(), m.data_ptr(), code, rows, cols, mode, dp_size, bnt,
-                                                 gbs, lsf, out.data_ptr(), coef.data_ptr(), ws.data_ptr(),
-                                                 ws.numel(), _cabi.stream_ptr(dev)))
-        ctx.save_for_backward(coef, m)
-        ctx.code = code
-        ctx.in_shape = loss_mat.shape
-        ctx.in_device = loss_mat.device
-        ctx.in_dtype = loss_mat.dtype
-        return out.to(loss_mat.device)
-
-    @staticmethod
-    def backward(ctx, d_loss):
-        coef, m = ctx.saved_tensors
-        dev = coef.device
-        rows, cols = m.shape
-        g = torch.empty((rows, cols), dtype=torch.float32, device=dev)
-        d = _cabi.as_f32(d_loss, dev).reshape(1)
-        with _cabi.device_guard(dev):
-            _cabi.check(_cabi.lib().vamd_agg_loss_backward(d.data_ptr(), coef.data_ptr(), m.data_ptr(), ctx.code,
-                                                           rows, cols, g.data_ptr(), _cabi.stream_ptr(dev)))
-        g = g.view(ctx.in_shape).to(device=ctx.in_device, dtype=ctx.in_dtype)
-        return g, None, None, None, None, None, None
-
-
 def agg_loss(loss_mat: torch.Tensor, loss_mask: torch.Tensor, loss_agg_mode: str, dp_size: int = 1,
              batch_num_tokens: Optional[int] = None, global_batch_size: Optional[int] = None,
              loss_scale_factor: Optional[int] = None):
@@ -590,79 +526,21 @@ def agg_loss(loss_mat: torch.Tensor, loss_mask: torch.Tensor, loss_agg_mode: str
     ``seq-mean-token-sum-norm``; any other mode raises ``ValueError``.  Differentiable with
     respect to ``loss_mat``."""
     mode = _agg_mode(loss_agg_mode)
-    return _AggLoss.apply(loss_mat, loss_mask, mode, float(dp_size), _opt(batch_num_tokens),
-                          _opt(global_batch_size), _opt(loss_scale_factor))
+    return _cabi.ops().agg_loss(loss_mat, loss_mask, mode, float(dp_size), _opt(batch_num_tokens),
+                                _opt(global_batch_size), _opt(loss_scale_factor))
 
 
 # ---------------------------------------------------------------------------------------------
-class _NoGradContext:
-    """What a loss Function's ``forward`` sees in place of an autograd context when nothing asks for a gradient."""
-    needs_input_grad = (False,) * 16
-
-    def save_for_backward(self, *tensors):
-        pass
-
-    def mark_non_differentiable(self, *tensors):
-        pass
-
-
-def _apply_loss(fn, differentiable_input, *rest):
-    """``fn.apply`` when the one differentiable input requires a gradient; otherwise ``fn.forward`` called directly,
-    which skips the Function machinery (argument wrapping, context, output bookkeeping: about 5 us of a 40 us
-    call)."""
-    if torch.is_grad_enabled() and differentiable_input.requires_grad:
-        return fn.apply(differentiable_input, *rest)
-    return fn.forward(_NoGradContext(), differentiable_input, *rest)
-
-
-class _PolicyLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low, clip_high, clip_c,
-                mode, dp_size, bnt, gbs, lsf, variant=0, tau_pos=1.0, tau_neg=1.0):
-        dev = _cabi.compute_device(log_prob, old_log_prob, advantages, response_mask)
-        lp = _matrix(log_prob, dev)
-        old = _matrix(old_log_prob, dev)
-        adv = _matrix(advantages, dev)
-        assert lp.shape == old.shape == adv.shape
-        m, code = _mask_matrix(response_mask, dev, lp.shape)
-        isw = _matrix(is_weights, dev) if is_weights is not None else None
-        rows, cols = lp.shape
-        need_grad = ctx.needs_input_grad[0]
-        Lb = _cabi.lib()
-        # one allocation for the four result floats and the per-row coefficients (16-byte aligned both)
-        buf = torch.empty(4 + rows, dtype=torch.float32, device=dev)
-        out, coef = buf[:4], buf[4:]
-        g = torch.empty_like(lp) if need_grad else None
-        ws = _cabi.ticket_workspace(Lb.vamd_policy_loss_variant_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_policy_loss_variant_forward(variant, old.data_ptr(), lp.data_ptr(), adv.data_ptr(),
-                                                            m.data_ptr(), code, _cabi.ptr(isw), rows, cols, clip_low,
-                                                            clip_high, clip_c, tau_pos, tau_neg, mode, dp_size, bnt,
-                                                            gbs, lsf, out.data_ptr(), _cabi.ptr(g), coef.data_ptr(),
-                                                            ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
-        if variant in (_PL["gspo"], _PL["geo_mean"]):
-            _watch_waiting_kernels(ws)
-        if need_grad:
-            ctx.save_for_backward(g, coef)
-        ctx.in_shape = log_prob.shape
-        ctx.in_device = log_prob.device
-        ctx.in_dtype = log_prob.dtype
-        out = out.to(log_prob.device)
-        ctx.mark_non_differentiable(out)
-        return out[0], out   # a view: the loss and the metrics share the floats the kernel wrote
-
-    @staticmethod
-    def backward(ctx, d_loss, _d_out):
-        g, coef = ctx.saved_tensors
-        dev = g.device
-        rows, cols = g.shape
-        d = _cabi.as_f32(d_loss, dev).reshape(1)
-        res = torch.empty_like(g)
-        with _cabi.device_guard(dev):
-            _cabi.check(_cabi.lib().vamd_scale_rows(g.data_ptr(), coef.data_ptr(), d.data_ptr(), 1.0, rows, cols,
-                                                    res.data_ptr(), _cabi.stream_ptr(dev)))
-        res = res.view(ctx.in_shape).to(device=ctx.in_device, dtype=ctx.in_dtype)
-        return (res,) + (None,) * 15
+def _policy_loss(log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low, clip_high, clip_c, mode, dp_size,
+                 bnt, gbs, lsf, variant=0, tau_pos=1.0, tau_neg=1.0):
+    """``(loss, metrics)`` of one policy loss; the metrics as Python floats, which is the one wait for the GPU."""
+    ops = _cabi.ops()
+    pg_loss, out = ops.policy_loss(log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low, clip_high,
+                                   clip_c, mode, dp_size, bnt, gbs, lsf, variant, tau_pos, tau_neg)
+    if variant in (_PL["gspo"], _PL["geo_mean"]):
+        _watch_waiting_kernels(_cabi.ticket_workspace(0, out.device if out.is_cuda else _cabi.compute_device(out)))
+    vals = ops.fetch(out)
+    return pg_loss, {"actor/pg_clipfrac": vals[1], "actor/ppo_kl": vals[2], "actor/pg_clipfrac_lower": vals[3]}
 
 
 def _cfg_get(config, key, default=None):
@@ -697,17 +575,10 @@ def compute_policy_loss_vanilla(old_log_prob: torch.Tensor, log_prob: torch.Tens
     )
     info = dict(getattr(config, "global_batch_info", None) or {})
     mode = _agg_mode(loss_agg_mode)
-    pg_loss, out = _apply_loss(
-        _PolicyLoss, log_prob, old_log_prob, advantages, response_mask, rollout_is_weights, float(clip_ratio_low),
+    return _policy_loss(
+        log_prob, old_log_prob, advantages, response_mask, rollout_is_weights, float(clip_ratio_low),
         float(clip_ratio_high), float(clip_ratio_c), mode, float(info.get("dp_size", 1)),
         _opt(info.get("batch_num_tokens")), _opt(info.get("global_batch_size")), _opt(info.get("loss_scale_factor")))
-    vals = out.detach().tolist()
-    pg_metrics = {
-        "actor/pg_clipfrac": vals[1],
-        "actor/ppo_kl": vals[2],
-        "actor/pg_clipfrac_lower": vals[3],
-    }
-    return pg_loss, pg_metrics
 
 
 _PL = {"vanilla": 0, "gpg": 1, "cispo": 2, "sapo": 3, "gspo": 4, "reinforce": 5, "geo_mean": 6}
@@ -723,14 +594,12 @@ def _policy_loss_variant(variant, old_log_prob, log_prob, advantages, response_m
         clip_low = low if low is not None else clip_ratio
         clip_high = high if high is not None else clip_ratio
     info = dict(getattr(config, "global_batch_info", None) or {})
-    pg_loss, out = _apply_loss(
-        _PolicyLoss, log_prob, old_log_prob, advantages, response_mask, rollout_is_weights, float(clip_low),
+    return _policy_loss(
+        log_prob, old_log_prob, advantages, response_mask, rollout_is_weights, float(clip_low),
         float(clip_high), 3.0, _agg_mode(loss_agg_mode), float(info.get("dp_size", 1)),
         _opt(info.get("batch_num_tokens")),
         _opt(info.get("global_batch_size")), _opt(info.get("loss_scale_factor")), _PL[variant], float(tau_pos),
         float(tau_neg))
-    vals = out.detach().tolist()
-    return pg_loss, {"actor/pg_clipfrac": vals[1], "actor/ppo_kl": vals[2], "actor/pg_clipfrac_lower": vals[3]}
 
 
 @register_policy_loss("gspo")
@@ -984,64 +853,19 @@ def compute_policy_loss(old_log_prob, log_prob, advantages, response_mask, clipr
         cliprange_low = cliprange
     if cliprange_high is None:
         cliprange_high = cliprange
-    pg_loss, out = _apply_loss(_PolicyLoss, log_prob, old_log_prob, advantages, response_mask, None,
-                               float(cliprange_low), float(cliprange_high), float(clip_ratio_c),
-                               _agg_mode(loss_agg_mode), 1.0, -1.0, -1.0, -1.0)
+    pg_loss, out = _cabi.ops().policy_loss(log_prob, old_log_prob, advantages, response_mask, None, float(cliprange_low),
+                                           float(cliprange_high), float(clip_ratio_c), _agg_mode(loss_agg_mode), 1.0,
+                                           -1.0, -1.0, -1.0, _PL["vanilla"], 1.0, 1.0)
     return pg_loss, out[1], out[2], out[3]
 
 
 # ---------------------------------------------------------------------------------------------
-class _ValueLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, vpreds, returns, values, response_mask, cliprange_value, mode):
-        dev = _cabi.compute_device(vpreds, returns, values, response_mask)
-        vp = _matrix(vpreds, dev)
-        ret = _matrix(returns, dev)
-        val = _matrix(values, dev)
-        assert vp.shape == ret.shape == val.shape
-        m, code = _mask_matrix(response_mask, dev, vp.shape)
-        rows, cols = vp.shape
-        need_grad = ctx.needs_input_grad[0]
-        Lb = _cabi.lib()
-        buf = torch.empty(4 + rows, dtype=torch.float32, device=dev)   # results and per-row coefficients together
-        out, coef = buf[:2], buf[4:]
-        g = torch.empty_like(vp) if need_grad else None
-        ws = _cabi.ticket_workspace(Lb.vamd_value_loss_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_value_loss_forward(vp.data_ptr(), ret.data_ptr(), val.data_ptr(), m.data_ptr(), code,
-                                                   rows, cols, cliprange_value, mode, out.data_ptr(), _cabi.ptr(g),
-                                                   coef.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                   _cabi.stream_ptr(dev)))
-        if need_grad:
-            ctx.save_for_backward(g, coef)
-        ctx.in_shape = vpreds.shape
-        ctx.in_device = vpreds.device
-        ctx.in_dtype = vpreds.dtype
-        out = out.to(vpreds.device)
-        ctx.mark_non_differentiable(out)
-        return out[0], out   # a view: the loss and the metrics share the floats the kernel wrote
-
-    @staticmethod
-    def backward(ctx, d_loss, _d_out):
-        g, coef = ctx.saved_tensors
-        dev = g.device
-        rows, cols = g.shape
-        d = _cabi.as_f32(d_loss, dev).reshape(1)
-        res = torch.empty_like(g)
-        with _cabi.device_guard(dev):
-            _cabi.check(_cabi.lib().vamd_scale_rows(g.data_ptr(), coef.data_ptr(), d.data_ptr(), 0.5, rows, cols,
-                                                    res.data_ptr(), _cabi.stream_ptr(dev)))
-        res = res.view(ctx.in_shape).to(device=ctx.in_device, dtype=ctx.in_dtype)
-        return res, None, None, None, None, None
-
-
 def compute_value_loss(vpreds: torch.Tensor, returns: torch.Tensor, values: torch.Tensor,
                        response_mask: torch.Tensor, cliprange_value: float, loss_agg_mode: str = "token-mean"):
     """Clipped value loss (reference core_algos.py:1799-1838): returns ``(vf_loss, vf_clipfrac)``,
     ``vf_loss`` differentiable with respect to ``vpreds``."""
-    vf_loss, out = _apply_loss(_ValueLoss, vpreds, returns, values, response_mask, float(cliprange_value),
-                                    _agg_mode(loss_agg_mode))
-    return vf_loss, out[1]
+    return _cabi.ops().value_loss(vpreds, returns, values, response_mask, float(cliprange_value),
+                                  _agg_mode(loss_agg_mode))
 
 
 # ---- PF-PPO data reweighting -----------------------------------------------------------------------
@@ -1149,47 +973,6 @@ def kl_penalty(logprob: torch.Tensor, ref_logprob: torch.Tensor, kl_penalty) -> 
     return kl_penalty_forward(logprob, ref_logprob, kl_penalty)
 
 
-class _KlLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logprob, ref_logprob, response_mask, kind, straight_through, mode, dp, bnt, gbs, lsf):
-        dev = _cabi.compute_device(logprob, ref_logprob, response_mask)
-        lp = _matrix(logprob, dev)
-        ref = _matrix(ref_logprob, dev)
-        assert lp.shape == ref.shape
-        m, code = _mask_matrix(response_mask, dev, lp.shape)
-        rows, cols = lp.shape
-        need_grad = ctx.needs_input_grad[0]
-        Lb = _cabi.lib()
-        out = torch.empty(1, dtype=torch.float32, device=dev)
-        coef = torch.empty(rows, dtype=torch.float32, device=dev)
-        g = torch.empty_like(lp) if need_grad else None
-        ws = _cabi.ticket_workspace(Lb.vamd_kl_loss_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_kl_loss_forward(lp.data_ptr(), ref.data_ptr(), m.data_ptr(), code, rows, cols, kind,
-                                                int(straight_through), mode, dp, bnt, gbs, lsf, out.data_ptr(),
-                                                _cabi.ptr(g), coef.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                _cabi.stream_ptr(dev)))
-        if need_grad:
-            ctx.save_for_backward(g, coef)
-        ctx.in_shape = logprob.shape
-        ctx.in_device = logprob.device
-        ctx.in_dtype = logprob.dtype
-        return out[0].to(logprob.device)
-
-    @staticmethod
-    def backward(ctx, d_loss):
-        g, coef = ctx.saved_tensors
-        dev = g.device
-        rows, cols = g.shape
-        d = _cabi.as_f32(d_loss, dev).reshape(1)
-        res = torch.empty_like(g)
-        with _cabi.device_guard(dev):
-            _cabi.check(_cabi.lib().vamd_scale_rows(g.data_ptr(), coef.data_ptr(), d.data_ptr(), 1.0, rows, cols,
-                                                    res.data_ptr(), _cabi.stream_ptr(dev)))
-        res = res.view(ctx.in_shape).to(device=ctx.in_device, dtype=ctx.in_dtype)
-        return (res,) + (None,) * 9
-
-
 def compute_kl_loss(logprob: torch.Tensor, ref_logprob: torch.Tensor, response_mask: torch.Tensor,
                     kl_penalty: str = "low_var_kl", loss_agg_mode: str = "token-mean", dp_size: int = 1,
                     batch_num_tokens=None, global_batch_size=None, loss_scale_factor=None,
@@ -1200,9 +983,9 @@ def compute_kl_loss(logprob: torch.Tensor, ref_logprob: torch.Tensor, response_m
     single function of the reference does both steps; this one exists so that the pair costs one
     read of the inputs.  ``straight_through=True`` keeps the estimator's value and uses the k2
     gradient, the behaviour the reference documents for the ``"+"`` names."""
-    return _KlLoss.apply(logprob, ref_logprob, response_mask, _kl_kind(kl_penalty), bool(straight_through),
-                         _agg_mode(loss_agg_mode), float(dp_size), _opt(batch_num_tokens), _opt(global_batch_size),
-                         _opt(loss_scale_factor))
+    return _cabi.ops().kl_loss(logprob, ref_logprob, response_mask, _kl_kind(kl_penalty), bool(straight_through),
+                               _agg_mode(loss_agg_mode), float(dp_size), _opt(batch_num_tokens), _opt(global_batch_size),
+                               _opt(loss_scale_factor))
 
 
 def kl_penalised_rewards(token_level_scores: torch.Tensor, old_log_probs: torch.Tensor, ref_log_prob: torch.Tensor,
@@ -1211,24 +994,9 @@ def kl_penalised_rewards(token_level_scores: torch.Tensor, old_log_probs: torch.
     ``kld = kl_penalty(old_log_probs, ref_log_prob) * response_mask``, ``token_level_rewards =
     token_level_scores - beta * kld`` and ``current_kl = mean_i masked_mean(kld_i, mask_i)``.  Returns
     ``(token_level_rewards, current_kl)`` with ``current_kl`` a 0-d device tensor (no host sync here)."""
-    with torch.no_grad():
-        dev = _cabi.compute_device(token_level_scores, old_log_probs, ref_log_prob, response_mask)
-        sc = _matrix(token_level_scores, dev)
-        lp = _matrix(old_log_probs, dev)
-        rf = _matrix(ref_log_prob, dev)
-        assert sc.shape == lp.shape == rf.shape
-        m, code = _mask_matrix(response_mask, dev, sc.shape)
-        rows, cols = sc.shape
-        out = torch.empty_like(sc)
-        kl = torch.empty(1, dtype=torch.float32, device=dev)
-        Lb = _cabi.lib()
-        ws = _cabi.ticket_workspace(Lb.vamd_apply_kl_penalty_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_apply_kl_penalty(sc.data_ptr(), lp.data_ptr(), rf.data_ptr(), m.data_ptr(), code,
-                                                 rows, cols, _kl_kind(kl_penalty), float(beta), out.data_ptr(),
-                                                 kl.data_ptr(), ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
-        out_dev = token_level_scores.device
-        return out.view(token_level_scores.shape).to(out_dev), kl[0].to(out_dev)
+    rewards, kl = _cabi.ops().kl_rewards(token_level_scores, old_log_probs, ref_log_prob, response_mask,
+                                         _kl_kind(kl_penalty), float(beta))
+    return rewards, kl[0].to(token_level_scores.device)
 
 
 def compute_rewards(token_level_scores, old_log_prob, ref_log_prob, kl_ratio):

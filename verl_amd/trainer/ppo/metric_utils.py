@@ -46,28 +46,11 @@ def compute_data_metrics(batch, use_critic: bool = True) -> dict[str, Any]:
     """
     b = batch.batch
     scores = b["token_level_scores"]
-    dev = _cabi.compute_device(scores, b["response_mask"], b["attention_mask"])
-    width = b["responses"].shape[-1]
-    sc = _cabi.as_f32(scores, dev)
-    rows = sc.shape[0]
-    assert sc.dim() == 2 and sc.shape[1] == width, f"token_level_scores {tuple(sc.shape)} vs response width {width}"
-    tensors = [sc] + [_cabi.as_f32(b[k], dev) for k in ("token_level_rewards", "advantages", "returns")]
-    values = _cabi.as_f32(b["values"], dev) if use_critic else None
-    for t in tensors + ([values] if use_critic else []):
-        assert t.shape == sc.shape
-    mask, mcode = _cabi.mask_code(b["response_mask"].detach().to(dev))
-    attention, acode = _cabi.mask_code(b["attention_mask"].detach().to(dev))
-    assert tuple(mask.shape) == tuple(sc.shape) and attention.shape[0] == rows and attention.shape[1] >= width
-    prompt = attention.shape[1] - width
-    out = torch.empty(len(_SLOTS), dtype=torch.float64, device=dev)
-    Lb = _cabi.lib()
-    ws = _cabi.workspace(Lb.vamd_data_metrics_workspace_bytes(rows, width), dev)
-    with _cabi.device_guard(dev):
-        _cabi.check(Lb.vamd_data_metrics(tensors[0].data_ptr(), tensors[1].data_ptr(), tensors[2].data_ptr(),
-                                         tensors[3].data_ptr(), _cabi.ptr(values), mask.data_ptr(), mcode,
-                                         attention.data_ptr(), acode, rows, prompt, width, out.data_ptr(),
-                                         ws.data_ptr(), ws.numel(), _cabi.stream_ptr(dev)))
-    got = dict(zip(_SLOTS, out.cpu().tolist()))          # the one host sync of the function
+    ops = _cabi.ops()
+    out = ops.data_metrics(scores, b["token_level_rewards"], b["advantages"], b["returns"],
+                           b["values"] if use_critic else None, b["response_mask"], b["attention_mask"],
+                           b["responses"].shape[-1], len(_SLOTS))
+    got = dict(zip(_SLOTS, ops.fetch(out)))              # the one wait for the GPU of the function
     if got.pop("_non_aborted") == 0:
         raise ValueError("All samples are aborted, this should not happen.")
     if got.pop("_valid_tokens") == 0:

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 from typing import Any, Optional
 
+from ... import _cabi
 from . import core_algos
 from .core_algos import AdvantageEstimator
 
@@ -33,7 +34,7 @@ def apply_kl_penalty(data, kl_ctrl, kl_penalty: str = "kl"):
     rewards, current_kl = core_algos.kl_penalised_rewards(
         data.batch["token_level_scores"], data.batch["old_log_probs"], data.batch["ref_log_prob"],
         data.batch["response_mask"], beta, kl_penalty)
-    current_kl = current_kl.item()
+    current_kl = _cabi.ops().fetch(current_kl)[0]
     kl_ctrl.update(current_kl=current_kl, n_steps=_batch_size(data))
     data.batch["token_level_rewards"] = rewards
     return data, {"actor/reward_kl_penalty": current_kl, "actor/reward_kl_penalty_coeff": beta}

@@ -35,31 +35,10 @@ _SLOTS = _OFFPOLICY + _IS + ("_valid_tokens",)
 
 def _run(old_log_prob, rollout_log_prob, response_mask, level, threshold, batch_normalize):
     """One pass: ``(weights or None, {name: float})`` with every slot of the metric vector."""
-    with torch.no_grad():
-        dev = _cabi.compute_device(old_log_prob, response_mask)
-        old = _cabi.as_f32(old_log_prob, dev)
-        if old.dim() == 1:
-            old = old.view(1, -1)
-        assert old.dim() == 2, f"expected (batch, length) log-probabilities, got {tuple(old_log_prob.shape)}"
-        roll = None
-        if rollout_log_prob is not None:
-            roll = _cabi.as_f32(rollout_log_prob, dev).view(old.shape)
-        mask, code = _cabi.mask_code(_cabi.on_device(response_mask, dev))
-        mask = mask.view(old.shape)
-        rows, cols = old.shape
-        weights = torch.empty_like(old) if level else None
-        out = torch.empty(len(_SLOTS), dtype=torch.float64, device=dev)
-        Lb = _cabi.lib()
-        ws = _cabi.workspace(Lb.vamd_rollout_correction_workspace_bytes(rows, cols), dev)
-        with _cabi.device_guard(dev):
-            _cabi.check(Lb.vamd_rollout_correction(old.data_ptr(), _cabi.ptr(roll), mask.data_ptr(), code, rows, cols,
-                                                   level, float(threshold or 0.0), int(bool(batch_normalize)),
-                                                   _cabi.ptr(weights), out.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                   _cabi.stream_ptr(dev)))
-        values = dict(zip(_SLOTS, out.cpu().tolist()))       # the one host sync
-        if weights is not None:
-            weights = weights.view(old_log_prob.shape).to(old_log_prob.device)
-        return weights, values
+    ops = _cabi.ops()
+    weights, out = ops.rollout_correction(old_log_prob, rollout_log_prob, response_mask, level, float(threshold or 0.0),
+                                          bool(batch_normalize), len(_SLOTS))
+    return weights, dict(zip(_SLOTS, ops.fetch(out)))        # the one wait for the GPU
 
 
 def _check_level(rollout_is, rollout_is_threshold):

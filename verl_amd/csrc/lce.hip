@@ -1061,7 +1061,9 @@ __global__ __launch_bounds__(kThreads) void lce_recompute_kernel(RecomputeArgs a
 }
 
 // d_logits panel of one vocabulary chunk from cached logits, to the bits of RecomputeEpi,
-// one thread per 8 consecutive columns of a token, 2048 columns per workgroup.
+// one thread per 8 consecutive columns of a token, 2048 columns per workgroup.  Bound by memory (5.7 TB/s at 777 x 151936).
+// Rows of the panel past the last token are not written: the gradient products read them as zero without fetching them
+// (filling the last 256-token tile took 64 x 151936 from 15.5 to 22.4 us, 777 x 151936 from 128 to 137).
 struct DLogitsArgs {
   const float* z_cache;  // [cache_rows][vocab]
   const int64_t* rows;   // the row of each token, or null: token i has row i
@@ -1083,9 +1085,9 @@ __global__ __launch_bounds__(256) void lce_dlogits_kernel(DLogitsArgs a) {
   if (j >= a.chunk_cols) return;
   u32x4 out = {0u, 0u, 0u, 0u};
   const int col = a.chunk_c0 + j;
-  const int64_t row = tok < a.n_tokens && a.rows ? a.rows[tok] : tok;
+  const int64_t row = a.rows ? a.rows[tok] : tok;
   // vocab % 8 == 0: the 8 columns are all in or all out
-  if (tok < a.n_tokens && col < a.vocab && row >= 0 && row < a.cache_rows) {
+  if (col < a.vocab && row >= 0 && row < a.cache_rows) {
     const float lse2 = a.lse[tok] * kLog2e;
     const float glp = (a.g_lp ? a.g_lp[tok] : 0.f) * a.rcp_t;
     const float gent = (a.g_ent ? a.g_ent[tok] : a.g_ent_scalar) * a.rcp_t;
@@ -1737,7 +1739,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
       d.dz_ld = (int)pitch;
       {
         ScopedTiming tm(kTagDLogits, s);
-        hipLaunchKernelGGL(lce_dlogits_kernel, dim3((unsigned)n_pad, (unsigned)ceil_div(d.chunk_cols, 2048)), dim3(256),
+        hipLaunchKernelGGL(lce_dlogits_kernel, dim3((unsigned)n_tokens, (unsigned)ceil_div(d.chunk_cols, 2048)), dim3(256),
                            0, s, d);
       }
       VAMD_LAUNCH_CHECK();
@@ -1773,7 +1775,8 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
 
     // d_hidden: k runs over the chunk's vocabulary columns (staged zeros beyond `cols`)
     GemmOutArgs gh;
-    gh.R = Operand{dz, pitch, (int)n_pad, (int)cv};
+    // (the panel has no rows past n_tokens: they read as zero through the operand's bounds)
+    gh.R = Operand{dz, pitch, (int)n_tokens, (int)cv};
     gh.C = Operand{wgt + c0 * hidden_size, hidden_size, (int)hidden_size, (int)left};
     gh.k_slabs = (int)ceil_div(cols, kBK);
     gh.r_tiles = d_hidden ? tok_tiles : 0;  // an input that needs no gradient leaves its GEMM an empty tile list
@@ -1794,7 +1797,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     gh.ld_out = hidden_size;
     // d_weight rows of this chunk: k runs over tokens (staged zeros beyond n_tokens)
     GemmOutArgs gw;
-    gw.R = Operand{dz, pitch, (int)(ceil_div(cols, 8) * 8), (int)n_pad};
+    gw.R = Operand{dz, pitch, (int)(ceil_div(cols, 8) * 8), (int)n_tokens};
     gw.C = Operand{hid, hidden_size, (int)hidden_size, (int)n_tokens};
     gw.k_slabs = (int)ceil_div(n_tokens, kBK);
     gw.r_tiles = want_dw ? chunk_tiles : 0;

@@ -1709,6 +1709,13 @@ def test_rollout_correction_weights_and_metrics(dev, shape, level, spread, norma
     assert torch.equal(w.cpu()[mask == 0], torch.zeros_like(w.cpu()[mask == 0]))
 
 
+@pytest.mark.parametrize("rows", [63, 64, 65, 129, 16385])   # a row per lane, 64 per workgroup, 256 workgroups, then a second trip
+def test_statistics_fold_edges(dev, rows):
+    test_data_metrics(dev, (rows, 9), 4, torch.int64, True)
+    test_rollout_correction_weights_and_metrics(dev, (rows, 9), "token", 0.5, False, torch.int64)
+    test_rollout_correction_weights_and_metrics(dev, (rows, 9), "sequence", 0.02, True, torch.float32)
+
+
 def test_rollout_correction_reference_literals_and_entry_points(dev):
     from verl_amd.trainer.ppo import rollout_corr_helper as RC
     case = GOLDEN["rollout_corr_mask_mode"]

@@ -3,10 +3,10 @@
 // compute_data_metrics (verl/trainer/ppo/metric_utils.py:81-225) derives about thirty scalars from
 // six tensors with one masked_select / reduction / .item() each.  Here one launch reads every
 // tensor once: each (row, 4096-column chunk) workgroup leaves a record of partial sums and
-// extrema.  A second, single-workgroup launch folds the records into per-row quantities (sequence
+// extrema.  A second, small launch folds the records into per-row quantities (sequence
 // score and reward, prompt and response length) and then into the output vector, so the host
 // reads the whole set with a single copy.  The fold is a launch of its own because its registers
-// (a 17-slot record per row in flight, 32 running statistics) would otherwise be charged to every
+// (a 17-slot record in flight, 32 running statistics) would otherwise be charged to every
 // wavefront of the streaming kernel.
 #include "rowchunk.h"
 
@@ -24,6 +24,7 @@ enum {
   kDmRec
 };
 constexpr int kDmSums = kDmAdvMax;  // slots [0, kDmSums) add, the rest are extrema
+constexpr int kDmFoldValues = 32;   // 16 sums and 16 maxima of the fold launch
 
 // Maximum of NV doubles per thread over the workgroup; result valid in thread 0.
 template <int NV, int NT>
@@ -37,7 +38,7 @@ struct DmArgs {
   int chunks;       // records per row: spans of `span` 4096-column chunks
   int span;
   double* records;  // kDmRec slots per (row, span) workgroup, slot-major
-  double* shares;   // per workgroup of the fold launch: its 16 sums and 16 maxima
+  double* shares;   // per workgroup of the fold launch: its kDmFoldValues totals
   unsigned* fold_counter;  // arrivals of the fold launch's workgroups; the streaming pass clears it
   double* out;      // [VAMD_DM_COUNT]
 };
@@ -127,73 +128,56 @@ __global__ __launch_bounds__(kRcThreads) void data_metrics_kernel(DmArgs a, cons
   }
 }
 
-constexpr int kFoldRows = 4;          // rows per thread and trip of the fold launch
-constexpr int kDmFoldThreads = 128;   // a workgroup of the fold launch takes up to kFoldRows * kDmFoldThreads rows
-
-// records -> per-row quantities -> the output vector: one row per thread, the workgroups' totals combined by the
-// last of them to finish.
-template <int NT>
-__global__ __launch_bounds__(NT) void data_metrics_fold_kernel(DmArgs a) {
+// records -> per-row quantities -> the output vector, a row per lane and trip.
+__global__ __launch_bounds__(kStatsFoldThreads) void data_metrics_fold_kernel(DmArgs a) {
   const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  __shared__ double stage[(NT / 64) * 16 * kWidePitch];
-  // ---- fold: thread-strided over rows -------------------------------------------------------------
+  __shared__ double stage[kDmFoldValues * kWidePitch];
+  // ---- fold: lane-strided over rows -------------------------------------------------------------
   // sums: 0 n_non_aborted 1 score 2 reward 3 resp_len 4 resp_len==cols 5 resp_len (non-aborted)
   //       6 resp_len==cols (non-aborted) 7 prompt_len 8 prompt_len==prompt
   //       9.. the valid-element sums kDmValid .. kDmDiff2
   constexpr int kElem = kDmSums - kDmValid;  // 7
-  double t[9 + kElem];
+  double lane_t[9 + kElem];
 #pragma unroll
-  for (int i = 0; i < 9 + kElem; ++i) t[i] = 0;
+  for (int i = 0; i < 9 + kElem; ++i) lane_t[i] = 0;
   // maxima (minima negated): 0/1 score, 2/3 reward, 4/5 resp_len, 6/7 resp_len non-aborted, 8/9 prompt_len,
   //                          10..15 adv, ret, val
-  double x[16];
+  double lane_x[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) x[i] = -inf;
-  // kFoldRows rows per thread and trip, their records in flight together: few wavefronts keep the workgroup
-  // reductions below short, and the loads of a trip are one round trip to memory whatever their number
-  for (int64_t r0 = (int64_t)blockIdx.x * NT * kFoldRows + threadIdx.x; r0 < a.rows;
-       r0 += (int64_t)gridDim.x * NT * kFoldRows) {
-    int64_t rr[kFoldRows];
-    bool have[kFoldRows];
+  for (int i = 0; i < 16; ++i) lane_x[i] = -inf;
+  for (int64_t r = (int64_t)blockIdx.x * kStatsFoldThreads + threadIdx.x; r < a.rows; r += (int64_t)gridDim.x * kStatsFoldThreads) {
+    const int64_t rr[1] = {r};
+    const bool have[1] = {true};
+    double rec[1][kDmRec];
+    fold_row_records<kDmRec, kDmSums, 1, false, 1>(a.records, rr, have, a.rows, a.chunks, rec);
+    const double* row_s = rec[0];
 #pragma unroll
-    for (int k = 0; k < kFoldRows; ++k) {
-      rr[k] = r0 + (int64_t)k * NT;
-      have[k] = rr[k] < a.rows;
-    }
-    double rec[kFoldRows][kDmRec];
-    fold_row_records<kDmRec, kDmSums, kFoldRows, false, 1>(a.records, rr, have, a.rows, a.chunks, rec);
+    for (int i = 0; i < kElem; ++i) lane_t[9 + i] += rec[0][kDmValid + i];
 #pragma unroll
-    for (int k = 0; k < kFoldRows; ++k) {
-      if (!have[k]) break;
-      const double* row_s = rec[k];
-#pragma unroll
-      for (int i = 0; i < kElem; ++i) t[9 + i] += rec[k][kDmValid + i];
-#pragma unroll
-      for (int i = 0; i < 6; ++i) x[10 + i] = fmax(x[10 + i], rec[k][kDmSums + i]);
-      const double score = (double)(float)row_s[kDmScore], reward = (double)(float)row_s[kDmReward];
-      const double rl = row_s[kDmRespLen], pl = row_s[kDmPromptLen];
-      t[3] += rl;
-      t[4] += rl == (double)a.cols ? 1.0 : 0.0;
-      x[4] = fmax(x[4], rl); x[5] = fmax(x[5], -rl);
-      t[7] += pl;
-      t[8] += pl == (double)a.prompt ? 1.0 : 0.0;
-      x[8] = fmax(x[8], pl); x[9] = fmax(x[9], -pl);
-      if (rl != 0.0) {  // not aborted (:119-120)
-        t[0] += 1.0;
-        t[1] += score;
-        t[2] += reward;
-        x[0] = fmax(x[0], score); x[1] = fmax(x[1], -score);
-        x[2] = fmax(x[2], reward); x[3] = fmax(x[3], -reward);
-        t[5] += rl;
-        t[6] += rl == (double)a.cols ? 1.0 : 0.0;
-        x[6] = fmax(x[6], rl); x[7] = fmax(x[7], -rl);
-      }
+    for (int i = 0; i < 6; ++i) lane_x[10 + i] = fmax(lane_x[10 + i], rec[0][kDmSums + i]);
+    const double score = (double)(float)row_s[kDmScore], reward = (double)(float)row_s[kDmReward];
+    const double rl = row_s[kDmRespLen], pl = row_s[kDmPromptLen];
+    lane_t[3] += rl;
+    lane_t[4] += rl == (double)a.cols ? 1.0 : 0.0;
+    lane_x[4] = fmax(lane_x[4], rl); lane_x[5] = fmax(lane_x[5], -rl);
+    lane_t[7] += pl;
+    lane_t[8] += pl == (double)a.prompt ? 1.0 : 0.0;
+    lane_x[8] = fmax(lane_x[8], pl); lane_x[9] = fmax(lane_x[9], -pl);
+    if (rl != 0.0) {  // not aborted (:119-120)
+      lane_t[0] += 1.0;
+      lane_t[1] += score;
+      lane_t[2] += reward;
+      lane_x[0] = fmax(lane_x[0], score); lane_x[1] = fmax(lane_x[1], -score);
+      lane_x[2] = fmax(lane_x[2], reward); lane_x[3] = fmax(lane_x[3], -reward);
+      lane_t[5] += rl;
+      lane_t[6] += rl == (double)a.cols ? 1.0 : 0.0;
+      lane_x[6] = fmax(lane_x[6], rl); lane_x[7] = fmax(lane_x[7], -rl);
     }
   }
-  block_reduce_wide<9 + kElem, NT>(t, stage, SumOp());
-  block_reduce_wide<16, NT>(x, stage, MaxOp());
-  if (!fold_across_workgroups<9 + kElem, 16, NT>(t, x, a.shares, a.fold_counter, stage)) return;
+  static_assert(9 + kElem + 16 == kDmFoldValues, "the staging area and the shares are sized for these");
+  if (!fold_launch_totals(lane_t, lane_x, a.shares, a.fold_counter, stage)) return;
   if (threadIdx.x == 0) {
+    const double *t = stage, *x = stage + 9 + kElem;
     double* o = a.out;
     const double B = (double)a.rows, na = t[0];
     const double n = t[9 + 0], s_adv = t[9 + 1], s_ret = t[9 + 2], s_ret2 = t[9 + 3], s_val = t[9 + 4],
@@ -273,13 +257,6 @@ __global__ __launch_bounds__(kRcThreads) void variance_proxy_rows_kernel(const f
 
 using namespace vamd;
 
-// workgroups of the fold launch (at most 256)
-static unsigned dm_fold_workgroups(int64_t batch) {
-  const int64_t per = (int64_t)kFoldRows * kDmFoldThreads;
-  const int64_t n = (batch + per - 1) / per;
-  return (unsigned)(n < 1 ? 1 : (n > 256 ? 256 : n));
-}
-
 extern "C" int vamd_variance_proxy_rows(const float* advantages, const float* old_log_probs,
                                         const float* sum_pi_squared, const float* is_weights, const void* mask,
                                         int mask_dtype, int64_t batch, int64_t length, double* records,
@@ -308,7 +285,7 @@ extern "C" int vamd_variance_proxy_rows(const float* advantages, const float* ol
 extern "C" size_t vamd_data_metrics_workspace_bytes(int64_t batch, int64_t response_length) {
   if (batch <= 0 || response_length <= 0) return 0;
   return align_up((size_t)batch * chunks_of(response_length) * kDmRec * sizeof(double), 256) +
-         align_up((size_t)dm_fold_workgroups(batch) * 32 * sizeof(double), 256) + 256;
+         align_up((size_t)fold_workgroups(batch) * kDmFoldValues * sizeof(double), 256) + 256;
 }
 
 extern "C" int vamd_data_metrics(const float* token_level_scores, const float* token_level_rewards,
@@ -332,7 +309,7 @@ extern "C" int vamd_data_metrics(const float* token_level_scores, const float* t
   a.chunks = ((int)chunks_of(response_length) + a.span - 1) / a.span;
   Carver carve(workspace);
   a.records = carve.take<double>((size_t)batch * a.chunks * kDmRec);
-  a.shares = carve.take<double>((size_t)dm_fold_workgroups(batch) * 32);
+  a.shares = carve.take<double>((size_t)fold_workgroups(batch) * kDmFoldValues);
   a.fold_counter = carve.take<unsigned>(1);
   a.out = out;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -361,8 +338,7 @@ extern "C" int vamd_data_metrics(const float* token_level_scores, const float* t
     default: set_error("unknown mask dtype code %d", attention_dtype); return VAMD_EINVAL;
   }
 #undef VAMD_DM
-  hipLaunchKernelGGL(data_metrics_fold_kernel<kDmFoldThreads>, dim3(dm_fold_workgroups(batch)), dim3(kDmFoldThreads),
-                     0, s, a);
+  hipLaunchKernelGGL(data_metrics_fold_kernel, dim3(fold_workgroups(batch)), dim3(kStatsFoldThreads), 0, s, a);
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;
 }

@@ -4,7 +4,7 @@
 // (verl/trainer/ppo/rollout_corr_helper.py:481-712, 835-937) evaluate about thirty masked reductions
 // over old_log_prob, rollout_log_prob and the response mask, each followed by .item().  Here every
 // (row, 4096-column chunk) workgroup reads the three tensors once, writes the truncated token-level
-// weights if those are asked for, and leaves a record of partial sums; a single-workgroup launch then
+// weights if those are asked for, and leaves a record of partial sums; a small launch then
 // folds the records into per-sequence quantities and the metric vector (a launch of its own, so that
 // the fold's registers are not charged to every wavefront of the streaming kernel).  Sequence-level
 // weights (one per row, known only after the fold) are broadcast by a further small launch, as is the
@@ -45,7 +45,7 @@ struct RcArgs {
   float* weights;      // [rows][cols] or null
   double* records;     // kRcRec slots per (row, chunk) workgroup, slot-major
   float* row_weight;   // [rows]: sequence-level weight, truncated (the broadcast divides by `factor`)
-  double* shares;      // per workgroup of the fold launch: its 26 sums and 9 maxima
+  double* shares;      // per workgroup of the fold launch: its kRcFoldValues totals
   unsigned* fold_counter;  // arrivals of the fold launch's workgroups; the streaming pass clears it
   float* factor;       // [1]: batch-normalisation divisor for the token-level weights (1 when not applied)
   double* out;         // [VAMD_RC_COUNT]
@@ -129,15 +129,11 @@ __global__ __launch_bounds__(kRcThreads) void rollout_stats_kernel(RcArgs a, con
   }
 }
 
-constexpr int kFoldRows = 4;          // rows per thread and trip of the fold launch
-constexpr int kRcFoldThreads = 128;   // a workgroup of the fold launch takes up to kFoldRows * kRcFoldThreads rows
-
-// records -> per-sequence quantities -> the metric vector (and the per-row weights): one row per thread, the
-// workgroups' totals combined by the last of them to finish.
-template <int NT>
-__global__ __launch_bounds__(NT) void rollout_fold_kernel(RcArgs a) {
+// records -> per-sequence quantities -> the metric vector (and the per-row weights), a row per lane and trip.
+constexpr int kRcFoldValues = 26 + 9;  // sums and maxima of the fold launch
+__global__ __launch_bounds__(kStatsFoldThreads) void rollout_fold_kernel(RcArgs a) {
   const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  __shared__ double stage[(NT / 64) * 26 * kWidePitch];
+  __shared__ double stage[kRcFoldValues * kWidePitch];
   enum {
     tM = 0, tD, tK3, tRho2, tW, tC, tC2, tTrunc, tHigh, tLow,         // token totals
     tTrainPpl, tTrainLog, tRollPpl, tRollLog, tGap, tGapAbs, tRatio, tChiSeq,  // sums over rows
@@ -147,86 +143,72 @@ __global__ __launch_bounds__(NT) void rollout_fold_kernel(RcArgs a) {
     tN
   };
   enum { xGap = 0, xGapMinNeg, xW, xWMinNeg, xSeq, xSeqMinNeg, xDev, xLog, xLogMinNeg, xN };
-  double t[tN], x[xN];
+  double lane_t[tN], lane_x[xN];
 #pragma unroll
-  for (int i = 0; i < tN; ++i) t[i] = 0;
+  for (int i = 0; i < tN; ++i) lane_t[i] = 0;
 #pragma unroll
-  for (int i = 0; i < xN; ++i) x[i] = -inf;
+  for (int i = 0; i < xN; ++i) lane_x[i] = -inf;
   const float log_hi = logf(a.thr), log_lo = logf(a.lower);
   const bool seq_level = a.level == VAMD_IS_SEQUENCE;
-  // kFoldRows rows per thread and trip, their records in flight together: few wavefronts keep the workgroup
-  // reductions below short, and the loads of a trip are one round trip to memory whatever their number
-  for (int64_t r0 = (int64_t)blockIdx.x * NT * kFoldRows + threadIdx.x; r0 < a.rows;
-       r0 += (int64_t)gridDim.x * NT * kFoldRows) {
-    int64_t rr[kFoldRows];
-    bool have[kFoldRows];
-#pragma unroll
-    for (int k = 0; k < kFoldRows; ++k) {
-      rr[k] = r0 + (int64_t)k * NT;
-      have[k] = rr[k] < a.rows;
+  for (int64_t r = (int64_t)blockIdx.x * kStatsFoldThreads + threadIdx.x; r < a.rows; r += (int64_t)gridDim.x * kStatsFoldThreads) {
+    const int64_t rr[1] = {r};
+    const bool have[1] = {true};
+    double rec[1][kRcRec];
+    fold_row_records<kRcRec, kRcSums, 1, false, 1>(a.records, rr, have, a.rows, a.chunks, rec);
+    const double* f = rec[0];
+    lane_x[xW] = fmax(lane_x[xW], rec[0][kRcWMax]);
+    lane_x[xWMinNeg] = fmax(lane_x[xWMinNeg], rec[0][kRcWMinNeg]);
+    const float Mi = (float)f[kRcM];
+    const float train = (float)f[kRcOld] / (Mi + 1e-8f);  // masked_mean(., axis=-1)
+    lane_t[tM] += f[kRcM]; lane_t[tD] += f[kRcD]; lane_t[tK3] += f[kRcK3]; lane_t[tRho2] += f[kRcRho2];
+    lane_t[tTrainPpl] += (double)expf(-train);
+    lane_t[tTrainLog] += (double)(-train);
+    if (Mi > 0.f) lane_t[tAlive] += 1.0;
+    if (!a.roll_lp) continue;
+    const float roll = (float)f[kRcRoll] / (Mi + 1e-8f);
+    const float gap = roll - train;
+    const float dsum = (float)f[kRcD];
+    const float dsafe = fminf(fmaxf(dsum, -kSafetyBound), kSafetyBound);
+    lane_t[tRollPpl] += (double)expf(-roll);
+    lane_t[tRollLog] += (double)(-roll);
+    lane_t[tGap] += (double)gap;
+    lane_t[tGapAbs] += (double)fabsf(gap);
+    lane_t[tRatio] += (double)expf(gap);
+    lane_t[tChiSeq] += (double)expf(2.f * dsafe);
+    lane_x[xGap] = fmax(lane_x[xGap], (double)gap);
+    lane_x[xGapMinNeg] = fmax(lane_x[xGapMinNeg], -(double)gap);
+    float seq = 0.f;  // masked_mean(weights, axis=-1) of the untruncated weights
+    if (a.level == VAMD_IS_TOKEN) {
+      lane_t[tW] += f[kRcW]; lane_t[tC] += f[kRcC]; lane_t[tC2] += f[kRcC2]; lane_t[tTrunc] += f[kRcTrunc];
+      lane_t[tHigh] += f[kRcHigh]; lane_t[tLow] += f[kRcLow];
+      seq = (float)f[kRcW] / (Mi + 1e-8f);
+    } else if (seq_level) {
+      const float w = expf(dsafe);
+      const float c = fminf(fmaxf(w, a.lower), a.thr);
+      const float tr = fminf(w, a.thr);
+      lane_t[tW] += (double)w * f[kRcM]; lane_t[tC] += (double)c * f[kRcM]; lane_t[tC2] += (double)c * (double)c * f[kRcM];
+      lane_t[tLogHigh] += dsum > log_hi ? 1.0 : 0.0;
+      lane_t[tLogLow] += dsum < log_lo ? 1.0 : 0.0;
+      lane_x[xLog] = fmax(lane_x[xLog], (double)dsum);
+      lane_x[xLogMinNeg] = fmax(lane_x[xLogMinNeg], -(double)dsum);
+      seq = w * Mi / (Mi + 1e-8f);
+      if (Mi > 0.f) lane_t[tSeqTrunc] += (double)(tr * Mi / (Mi + 1e-8f));
+      a.row_weight[r] = tr;
     }
-    double rec[kFoldRows][kRcRec];
-    fold_row_records<kRcRec, kRcSums, kFoldRows, false, 1>(a.records, rr, have, a.rows, a.chunks, rec);
-#pragma unroll
-    for (int k = 0; k < kFoldRows; ++k) {
-      if (!have[k]) break;
-      const int64_t r = rr[k];
-      const double* f = rec[k];
-      x[xW] = fmax(x[xW], rec[k][kRcWMax]);
-      x[xWMinNeg] = fmax(x[xWMinNeg], rec[k][kRcWMinNeg]);
-      const float Mi = (float)f[kRcM];
-      const float train = (float)f[kRcOld] / (Mi + 1e-8f);  // masked_mean(., axis=-1)
-      t[tM] += f[kRcM]; t[tD] += f[kRcD]; t[tK3] += f[kRcK3]; t[tRho2] += f[kRcRho2];
-      t[tTrainPpl] += (double)expf(-train);
-      t[tTrainLog] += (double)(-train);
-      if (Mi > 0.f) t[tAlive] += 1.0;
-      if (!a.roll_lp) continue;
-      const float roll = (float)f[kRcRoll] / (Mi + 1e-8f);
-      const float gap = roll - train;
-      const float dsum = (float)f[kRcD];
-      const float dsafe = fminf(fmaxf(dsum, -kSafetyBound), kSafetyBound);
-      t[tRollPpl] += (double)expf(-roll);
-      t[tRollLog] += (double)(-roll);
-      t[tGap] += (double)gap;
-      t[tGapAbs] += (double)fabsf(gap);
-      t[tRatio] += (double)expf(gap);
-      t[tChiSeq] += (double)expf(2.f * dsafe);
-      x[xGap] = fmax(x[xGap], (double)gap);
-      x[xGapMinNeg] = fmax(x[xGapMinNeg], -(double)gap);
-      float seq = 0.f;  // masked_mean(weights, axis=-1) of the untruncated weights
-      if (a.level == VAMD_IS_TOKEN) {
-        t[tW] += f[kRcW]; t[tC] += f[kRcC]; t[tC2] += f[kRcC2]; t[tTrunc] += f[kRcTrunc];
-        t[tHigh] += f[kRcHigh]; t[tLow] += f[kRcLow];
-        seq = (float)f[kRcW] / (Mi + 1e-8f);
-      } else if (seq_level) {
-        const float w = expf(dsafe);
-        const float c = fminf(fmaxf(w, a.lower), a.thr);
-        const float tr = fminf(w, a.thr);
-        t[tW] += (double)w * f[kRcM]; t[tC] += (double)c * f[kRcM]; t[tC2] += (double)c * (double)c * f[kRcM];
-        t[tLogHigh] += dsum > log_hi ? 1.0 : 0.0;
-        t[tLogLow] += dsum < log_lo ? 1.0 : 0.0;
-        x[xLog] = fmax(x[xLog], (double)dsum);
-        x[xLogMinNeg] = fmax(x[xLogMinNeg], -(double)dsum);
-        seq = w * Mi / (Mi + 1e-8f);
-        if (Mi > 0.f) t[tSeqTrunc] += (double)(tr * Mi / (Mi + 1e-8f));
-        a.row_weight[r] = tr;
-      }
-      if (a.level != VAMD_IS_NONE) {
-        t[tSeq] += (double)seq;
-        t[tSeq2] += (double)seq * (double)seq;
-        t[tSeqHigh] += seq > a.thr ? 1.0 : 0.0;
-        t[tSeqLow] += seq < a.lower ? 1.0 : 0.0;
-        x[xSeq] = fmax(x[xSeq], (double)seq);
-        x[xSeqMinNeg] = fmax(x[xSeqMinNeg], -(double)seq);
-        x[xDev] = fmax(x[xDev], (double)fabsf(seq - 1.f));
-      }
+    if (a.level != VAMD_IS_NONE) {
+      lane_t[tSeq] += (double)seq;
+      lane_t[tSeq2] += (double)seq * (double)seq;
+      lane_t[tSeqHigh] += seq > a.thr ? 1.0 : 0.0;
+      lane_t[tSeqLow] += seq < a.lower ? 1.0 : 0.0;
+      lane_x[xSeq] = fmax(lane_x[xSeq], (double)seq);
+      lane_x[xSeqMinNeg] = fmax(lane_x[xSeqMinNeg], -(double)seq);
+      lane_x[xDev] = fmax(lane_x[xDev], (double)fabsf(seq - 1.f));
     }
   }
-  static_assert(tN <= 26 && xN <= 26, "the staging area is sized for 26 values");
-  block_reduce_wide<tN, NT>(t, stage, SumOp());
-  block_reduce_wide<xN, NT>(x, stage, MaxOp());
-  if (!fold_across_workgroups<tN, xN, NT>(t, x, a.shares, a.fold_counter, stage)) return;
+  static_assert(tN + xN == kRcFoldValues, "the staging area and the shares are sized for these");
+  if (!fold_launch_totals(lane_t, lane_x, a.shares, a.fold_counter, stage)) return;
   if (threadIdx.x == 0) {
+    const double *t = stage, *x = stage + tN;
     double* o = a.out;
     const double B = (double)a.rows, Mt = t[tM];
     const double den = (double)((float)Mt + 1e-8f);  // masked_mean over everything
@@ -315,19 +297,11 @@ __global__ __launch_bounds__(256) void rollout_divide_kernel(float* __restrict__
 
 using namespace vamd;
 
-// workgroups of the fold launch (at most 256), each leaving 26 sums and 9 maxima
-constexpr size_t kRcShareSlots = 26 + 9;
-static unsigned rc_fold_workgroups(int64_t batch) {
-  const int64_t per = (int64_t)kFoldRows * kRcFoldThreads;
-  const int64_t n = (batch + per - 1) / per;
-  return (unsigned)(n < 1 ? 1 : (n > 256 ? 256 : n));
-}
-
 extern "C" size_t vamd_rollout_correction_workspace_bytes(int64_t batch, int64_t length) {
   if (batch <= 0 || length <= 0) return 0;
   return align_up((size_t)batch * chunks_of(length) * kRcRec * sizeof(double), 256) +
          align_up((size_t)batch * sizeof(float), 256) + 256 +
-         align_up((size_t)rc_fold_workgroups(batch) * kRcShareSlots * sizeof(double), 256) + 256;
+         align_up((size_t)fold_workgroups(batch) * kRcFoldValues * sizeof(double), 256) + 256;
 }
 
 extern "C" int vamd_rollout_correction(const float* old_log_prob, const float* rollout_log_prob, const void* mask,
@@ -357,7 +331,7 @@ extern "C" int vamd_rollout_correction(const float* old_log_prob, const float* r
   a.records = carve.take<double>((size_t)batch * a.chunks * kRcRec);
   a.row_weight = carve.take<float>((size_t)batch);
   a.factor = carve.take<float>(1);
-  a.shares = carve.take<double>((size_t)rc_fold_workgroups(batch) * kRcShareSlots);
+  a.shares = carve.take<double>((size_t)fold_workgroups(batch) * kRcFoldValues);
   a.fold_counter = carve.take<unsigned>(1);
   a.out = metrics;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -371,8 +345,7 @@ extern "C" int vamd_rollout_correction(const float* old_log_prob, const float* r
       hipLaunchKernelGGL((rollout_stats_kernel<true, M>), grid, block, 0, s, a, mk);
     else
       hipLaunchKernelGGL((rollout_stats_kernel<false, M>), grid, block, 0, s, a, mk);
-    hipLaunchKernelGGL(rollout_fold_kernel<kRcFoldThreads>, dim3(rc_fold_workgroups(batch)), dim3(kRcFoldThreads), 0,
-                       s, a);
+    hipLaunchKernelGGL(rollout_fold_kernel, dim3(fold_workgroups(batch)), dim3(kStatsFoldThreads), 0, s, a);
     if (level == VAMD_IS_SEQUENCE) {
       if (vec)
         hipLaunchKernelGGL((rollout_broadcast_kernel<true, M>), cols_grid, block, 0, s, a.row_weight, a.factor, mk,

@@ -216,7 +216,8 @@ int vamd_lce_backward_subset_rows(const void* hidden, const void* weight, const 
  *   backward pass (the reference's gather would fault on it; 0 is what flash-attn's cross_entropy_loss returns
  *   for its ignore index).
  *   logprobs = z[label] - lse(z); entropy = lse(z) - sum softmax(z) z; lse and mean_z (= sum softmax(z) z) are
- *   what the backward pass needs.  Every output is fp32 [n_rows] and may be NULL if not wanted.
+ *   what the backward pass needs.  Every output is fp32 [n_rows] and may be NULL if not wanted;
+ *   vamd_row_softmax_stats_as writes logprobs and entropy as out_dtype, VAMD_DT_F32 or the logits' type (rounded once).
  * One pass over the logits (online softmax), no workspace. */
 #define VAMD_DT_F32 0
 #define VAMD_DT_BF16 1
@@ -224,14 +225,21 @@ int vamd_lce_backward_subset_rows(const void* hidden, const void* weight, const 
 int vamd_row_softmax_stats(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
                            const int64_t* labels, float* logprobs, float* entropy, float* lse, float* mean_z,
                            void* stream);
+int vamd_row_softmax_stats_as(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
+                              const int64_t* labels, void* logprobs, void* entropy, int out_dtype, float* lse,
+                              float* mean_z, void* stream);
 /* d_logits = d_logprobs (onehot(label) - p) - d_entropy p (z - mean_z), p = exp(z - lse): what autograd hands back
  * through log_softmax + gather (logprobs_from_logits_naive) and through logsumexp - sum softmax * z
- * (entropy_from_logits).  d_logprobs / d_entropy: fp32 [n_rows], either may be NULL (no contribution);
+ * (entropy_from_logits).  d_logprobs / d_entropy: fp32 [n_rows] (_as: grad_dtype, VAMD_DT_F32 or the logits' type),
+ * either may be NULL (no contribution);
  * d_logits has the element type of logits and row pitch ld_out, and may be the logits buffer itself (in place, the
  * reference's inplace_backward). */
 int vamd_row_softmax_backward(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
                               const int64_t* labels, const float* lse, const float* mean_z, const float* d_logprobs,
                               const float* d_entropy, void* d_logits, int64_t ld_out, void* stream);
+int vamd_row_softmax_backward_as(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
+                                 const int64_t* labels, const float* lse, const float* mean_z, const void* d_logprobs,
+                                 const void* d_entropy, int grad_dtype, void* d_logits, int64_t ld_out, void* stream);
 /* clip_by_value (verl/utils/torch_functional.py:203-221): out = max(min(x, hi), lo) over n fp32 elements, and its
  * gradients with torch's rule for binary min / max (the selected operand takes the gradient, equal operands half
  * each); d_x / d_lo / d_hi may be NULL.  A NaN in x, lo or hi gives a NaN output, as torch.min / torch.max of two

@@ -430,3 +430,24 @@ def test_model_forward_backends_roll_labels_and_call_the_head(dev):
     out_t = model(input_ids=ids, return_dict=True, temperature=1.3)
     assert out_t.log_probs.dtype == torch.bfloat16 and out_t.log_probs.shape == (b, s)
     assert torch.equal(out_t.log_probs, want_lp.bfloat16())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 2, 5])
+@pytest.mark.parametrize("offset", [0, 1])          # the gradient's first element in the lower or upper half of a word
+def test_row_values_in_the_type_of_the_logits(dev, dtype, rows, offset):
+    """Results rounded in the kernel are the rounded fp32 results, and upstream gradients read in 16 bits give the bits
+    that their fp32 copies give."""
+    import verl_amd.utils.torch_functional as F
+    v = 2056
+    z, labels = _logits(rows, v, dtype, seed=rows)
+    z, lab = z.to(dev), labels.to(dev)
+    lp32, ent32, lse, mean_z = F._row_stats(z, v, lab, True, True, True)
+    lp, ent, _, _ = F._row_stats(z, v, lab, True, True, True, dtype)
+    assert torch.equal(lp, lp32.to(dtype)) and torch.equal(ent, ent32.to(dtype))
+    g = torch.randn(2, rows + 3, generator=torch.Generator().manual_seed(rows)).to(dtype).to(dev)
+    g_lp, g_ent = g[0, offset:offset + rows], g[1, offset:offset + rows]
+    for a, b in ((g_lp, g_ent), (g_lp, None), (None, g_ent)):
+        up = lambda t: None if t is None else t.float()
+        got = F._row_backward(z, v, lab, lse, mean_z, a, b, False)
+        assert torch.equal(got, F._row_backward(z, v, lab, lse, mean_z, up(a), up(b), False))

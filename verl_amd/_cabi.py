@@ -64,6 +64,10 @@ SIGNATURES = {
                                        c_void_p, c_void_p, c_void_p]),
     "vamd_row_softmax_backward": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                           c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "vamd_row_softmax_stats_as": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+                                          c_int, c_void_p, c_void_p, c_void_p]),
+    "vamd_row_softmax_backward_as": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+                                             c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p]),
     "vamd_clip_by_value": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "vamd_clip_by_value_backward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
                                             c_void_p, c_void_p]),

@@ -96,11 +96,34 @@ struct StatsArgs {
   int64_t ld;
   const int64_t* labels;
   int64_t cols;
-  float* logprobs;
-  float* entropy;
+  void* logprobs;  // element type of the logits or fp32
+  void* entropy;   // likewise
+  bool typed;      // they have the element type of the logits
   float* lse;
   float* mean_z;
 };
+
+// Element r of a per-row vector whose elements are D's (typed) or fp32.  16-bit callers' results leave and their upstream
+// gradients arrive in their own type: conversions around these kernels were four launches of 5 us of a pass, and more than
+// that in host time (log-probs, entropy and their gradients at 300 x 151936 bf16 206 -> 180 us, 800 x 152064 387 -> 376,
+// 1500 x 152064 679 -> 669, 3001 x 152064 1321 -> 1312).
+template <class D>
+__device__ __forceinline__ void store_row_value(void* p, bool typed, int64_t r, float x) {
+  if (typed) static_cast<typename D::type*>(p)[r] = from_float(x, D());
+  else static_cast<float*>(p)[r] = x;
+}
+// A 16-bit element is taken out of its aligned word, which a scalar load fetches (r is uniform); a load of 16 bits is a vector
+// load, whose round trip in front of everything else made the backward kernel 40 us slower at 3001 x 152064.
+template <class D, bool TYPED>
+__device__ __forceinline__ float load_row_value(const void* p, int64_t r) {
+  if (!TYPED || sizeof(typename D::type) == 4) return static_cast<const float*>(p)[r];
+  const unsigned odd = ((unsigned)reinterpret_cast<uintptr_t>(p) >> 1) & 1u;  // p sits in the upper half of a word
+  const uint64_t half = (uint64_t)r + odd;
+  const unsigned word = reinterpret_cast<const unsigned*>(static_cast<const uint16_t*>(p) - odd)[half >> 1];
+  const uint16_t bits = (uint16_t)((half & 1) ? word >> 16 : word);
+  if constexpr (std::is_same_v<D, BF16>) return __uint_as_float((unsigned)bits << 16);
+  else return (float)__builtin_bit_cast(_Float16, bits);
+}
 
 template <class D, bool VEC, int NT>
 __global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
@@ -177,11 +200,11 @@ __global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
     const float mz = sz / s;
     if (a.lse) a.lse[r] = lse;
     if (a.mean_z) a.mean_z[r] = mz;
-    if (a.entropy) a.entropy[r] = lse - mz;
+    if (a.entropy) store_row_value<D>(a.entropy, a.typed, r, lse - mz);
     if (a.logprobs) {
       // a label outside [0, cols) (an ignore index such as -100, a padding id) reads nothing and yields 0
       const int64_t lab = a.labels[r];
-      a.logprobs[r] = (lab >= 0 && lab < a.cols) ? to_float(row[lab], D()) - lse : 0.f;
+      store_row_value<D>(a.logprobs, a.typed, r, (lab >= 0 && lab < a.cols) ? to_float(row[lab], D()) - lse : 0.f);
     }
   }
 }
@@ -192,8 +215,8 @@ struct BackwardArgs {
   const int64_t* labels;  // needed with d_logprobs
   const float* lse;
   const float* mean_z;    // needed with d_entropy
-  const float* d_logprobs;
-  const float* d_entropy;
+  const void* d_logprobs;  // element type of the logits or fp32
+  const void* d_entropy;   // likewise
   void* d_logits;
   int64_t ld_out;
   int64_t cols;
@@ -206,7 +229,9 @@ struct BackwardArgs {
 // walks the items and requests the next one before it stores).  What counts is the elements per workgroup, about
 // 2048: one load per thread for 16-bit logits (bf16, steady state: 461 us with four loads, 404 with two, 378 with
 // one), two for fp32 (828 us; 863 with one).  Trimming the arithmetic per element changed nothing measurable.
-template <class D, bool VEC>
+// TYPED: d_logprobs and d_entropy have the element type of the logits (a kernel of its own: every one of its many small
+// workgroups would start with the choice).
+template <class D, bool VEC, bool TYPED>
 __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(BackwardArgs a) {
   using T = typename D::type;
   constexpr int G = D::kVec, F = D::kBackwardLoads;
@@ -214,22 +239,24 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(Backw
   const int chunk = blockIdx.x % a.chunks;
   const T* __restrict__ row = static_cast<const T*>(a.logits) + r * a.ld;
   T* __restrict__ out = static_cast<T*>(a.d_logits) + r * a.ld_out;
-  const float lse2 = a.lse[r] * kLog2e;
-  const float glp = a.d_logprobs ? a.d_logprobs[r] : 0.f;
-  const float gent = a.d_entropy ? a.d_entropy[r] : 0.f;
-  const float mz = a.d_entropy ? a.mean_z[r] : 0.f;
-  const float t0 = fmaf(-gent, mz, glp);  // g_lp + g_ent (z - mean_z) = g_ent z + t0
-  const int64_t label = a.d_logprobs ? a.labels[r] : -1;
   const int64_t stride = (int64_t)kRowThreads * G;
   const int64_t c0 = (int64_t)chunk * stride * F + (int64_t)threadIdx.x * G;
-  // every whole 16-byte group is requested before anything else happens (the ragged last group of a row, if any,
-  // is fetched element by element when its turn comes)
+  // Every whole 16-byte group is requested before anything else happens (the ragged last group of a row, if any,
+  // is fetched element by element when its turn comes): the row's values come in by scalar loads, a chain of three trips
+  // at the start of every one of many small workgroups.
   u32x4_t raw[F];
 #pragma unroll
   for (int u = 0; u < F; ++u) {
     const int64_t c = c0 + u * stride;
     if (c + G <= a.cols) raw[u] = load_whole<D, VEC>(row + c);
   }
+  __builtin_amdgcn_sched_barrier(0);
+  const float lse2 = a.lse[r] * kLog2e;
+  const float glp = a.d_logprobs ? load_row_value<D, TYPED>(a.d_logprobs, r) : 0.f;
+  const float gent = a.d_entropy ? load_row_value<D, TYPED>(a.d_entropy, r) : 0.f;
+  const float mz = a.d_entropy ? a.mean_z[r] : 0.f;
+  const float t0 = fmaf(-gent, mz, glp);  // g_lp + g_ent (z - mean_z) = g_ent z + t0
+  const int64_t label = a.d_logprobs ? a.labels[r] : -1;
   float x[F][G];
 #pragma unroll
   for (int u = 0; u < F; ++u) {
@@ -336,11 +363,20 @@ using namespace vamd;
 extern "C" int vamd_row_softmax_stats(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
                                       const int64_t* labels, float* logprobs, float* entropy, float* lse,
                                       float* mean_z, void* stream) {
+  return vamd_row_softmax_stats_as(logits, dtype, n_rows, vocab, ld, labels, logprobs, entropy, VAMD_DT_F32, lse, mean_z,
+                                   stream);
+}
+
+extern "C" int vamd_row_softmax_stats_as(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
+                                         const int64_t* labels, void* logprobs, void* entropy, int out_dtype, float* lse,
+                                         float* mean_z, void* stream) {
   int st = check_rows("row_softmax_stats", logits, dtype, n_rows, vocab, ld);
   if (st != VAMD_OK) return st;
+  VAMD_REQUIRE(out_dtype == VAMD_DT_F32 || out_dtype == dtype,
+               "row_softmax_stats: outputs are fp32 or of the logits' type, not of type %d", out_dtype);
   VAMD_REQUIRE((logprobs == nullptr) || labels, "row_softmax_stats: logprobs need labels");
   VAMD_REQUIRE(logprobs || entropy || lse || mean_z, "row_softmax_stats: no output requested");
-  StatsArgs a{logits, ld, labels, vocab, logprobs, entropy, lse, mean_z};
+  StatsArgs a{logits, ld, labels, vocab, logprobs, entropy, out_dtype == dtype, lse, mean_z};
   hipStream_t s = static_cast<hipStream_t>(stream);
   VAMD_DTYPE_DISPATCH(dtype, D, {
     if (rows_vectorizable<D>(logits, ld)) launch_stats<D, true>(a, n_rows, s);
@@ -354,8 +390,18 @@ extern "C" int vamd_row_softmax_backward(const void* logits, int dtype, int64_t 
                                          const int64_t* labels, const float* lse, const float* mean_z,
                                          const float* d_logprobs, const float* d_entropy, void* d_logits,
                                          int64_t ld_out, void* stream) {
+  return vamd_row_softmax_backward_as(logits, dtype, n_rows, vocab, ld, labels, lse, mean_z, d_logprobs, d_entropy,
+                                      VAMD_DT_F32, d_logits, ld_out, stream);
+}
+
+extern "C" int vamd_row_softmax_backward_as(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
+                                            const int64_t* labels, const float* lse, const float* mean_z,
+                                            const void* d_logprobs, const void* d_entropy, int grad_dtype,
+                                            void* d_logits, int64_t ld_out, void* stream) {
   int st = check_rows("row_softmax_backward", logits, dtype, n_rows, vocab, ld);
   if (st != VAMD_OK) return st;
+  VAMD_REQUIRE(grad_dtype == VAMD_DT_F32 || grad_dtype == dtype,
+               "row_softmax_backward: upstream gradients are fp32 or of the logits' type, not of type %d", grad_dtype);
   VAMD_REQUIRE(d_logits && ld_out >= vocab && lse, "row_softmax_backward: bad output or missing lse");
   VAMD_REQUIRE(d_logprobs || d_entropy, "row_softmax_backward: no upstream gradient");
   VAMD_REQUIRE(!d_logprobs || labels, "row_softmax_backward: d_logprobs needs labels");
@@ -367,10 +413,15 @@ extern "C" int vamd_row_softmax_backward(const void* logits, int dtype, int64_t 
     VAMD_REQUIRE(n_rows * chunks < (1ll << 31), "row_softmax_backward: too many workgroups");
     BackwardArgs a{logits, ld, labels, lse, mean_z, d_logprobs, d_entropy, d_logits, ld_out, vocab, (int)chunks};
     const dim3 grid((unsigned)(n_rows * chunks));
-    if (rows_vectorizable<D>(logits, ld) && rows_vectorizable<D>(d_logits, ld_out))
-      hipLaunchKernelGGL((row_softmax_backward_kernel<D, true>), grid, dim3(kRowThreads), 0, s, a);
-    else
-      hipLaunchKernelGGL((row_softmax_backward_kernel<D, false>), grid, dim3(kRowThreads), 0, s, a);
+    const bool vec = rows_vectorizable<D>(logits, ld) && rows_vectorizable<D>(d_logits, ld_out);
+    constexpr bool kSmall = sizeof(typename D::type) < 4;
+    if (kSmall && grad_dtype == dtype) {
+      if (vec) hipLaunchKernelGGL((row_softmax_backward_kernel<D, true, kSmall>), grid, dim3(kRowThreads), 0, s, a);
+      else hipLaunchKernelGGL((row_softmax_backward_kernel<D, false, kSmall>), grid, dim3(kRowThreads), 0, s, a);
+    } else {
+      if (vec) hipLaunchKernelGGL((row_softmax_backward_kernel<D, true, false>), grid, dim3(kRowThreads), 0, s, a);
+      else hipLaunchKernelGGL((row_softmax_backward_kernel<D, false, false>), grid, dim3(kRowThreads), 0, s, a);
+    }
   });
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;

@@ -33,15 +33,18 @@ def _logit_rows(logits: torch.Tensor):
     return rows, (rows.stride(0) if rows.shape[0] > 1 else vocab)
 
 
-def _row_stats(rows, ld, labels, want_logprobs: bool, want_entropy: bool, want_mean_z: bool):
+def _row_stats(rows, ld, labels, want_logprobs: bool, want_entropy: bool, want_mean_z: bool,
+               dtype=torch.float32):
+    """Log-probs and entropies come in ``dtype`` (fp32 or that of the logits), the backward pass's values in fp32."""
     n, vocab = rows.shape
     dev = rows.device
-    f = lambda want: torch.empty(n, dtype=torch.float32, device=dev) if want else None
-    logprobs, entropy, lse, mean_z = f(want_logprobs), f(want_entropy), f(True), f(want_mean_z)
+    f = lambda want, kind: torch.empty(n, dtype=kind, device=dev) if want else None
+    logprobs, entropy = f(want_logprobs, dtype), f(want_entropy, dtype)
+    lse, mean_z = f(True, torch.float32), f(want_mean_z, torch.float32)
     with _cabi.device_guard(dev):
-        _cabi.check(_cabi.lib().vamd_row_softmax_stats(
+        _cabi.check(_cabi.lib().vamd_row_softmax_stats_as(
             rows.data_ptr(), _ROW_DTYPES[rows.dtype], n, vocab, ld, _cabi.ptr(labels), _cabi.ptr(logprobs),
-            _cabi.ptr(entropy), lse.data_ptr(), _cabi.ptr(mean_z), _cabi.stream_ptr(dev)))
+            _cabi.ptr(entropy), _ROW_DTYPES[dtype], lse.data_ptr(), _cabi.ptr(mean_z), _cabi.stream_ptr(dev)))
     return logprobs, entropy, lse, mean_z
 
 
@@ -50,12 +53,14 @@ def _row_backward(rows, ld, labels, lse, mean_z, d_logprobs, d_entropy, in_place
     dev = rows.device
     out = rows if in_place else torch.empty((n, vocab), dtype=rows.dtype, device=dev)
     ld_out = ld if in_place else vocab
-    g = lambda t: None if t is None else t.detach().reshape(-1).to(device=dev, dtype=torch.float32).contiguous()
+    given = [t for t in (d_logprobs, d_entropy) if t is not None]
+    dtype = rows.dtype if all(t.dtype == rows.dtype for t in given) else torch.float32
+    g = lambda t: None if t is None else t.detach().reshape(-1).to(device=dev, dtype=dtype).contiguous()
     d_logprobs, d_entropy = g(d_logprobs), g(d_entropy)
     with _cabi.device_guard(dev):
-        _cabi.check(_cabi.lib().vamd_row_softmax_backward(
+        _cabi.check(_cabi.lib().vamd_row_softmax_backward_as(
             rows.data_ptr(), _ROW_DTYPES[rows.dtype], n, vocab, ld, _cabi.ptr(labels), lse.data_ptr(),
-            _cabi.ptr(mean_z), _cabi.ptr(d_logprobs), _cabi.ptr(d_entropy), out.data_ptr(), ld_out,
+            _cabi.ptr(mean_z), _cabi.ptr(d_logprobs), _cabi.ptr(d_entropy), _ROW_DTYPES[dtype], out.data_ptr(), ld_out,
             _cabi.stream_ptr(dev)))
     return out
 
@@ -66,13 +71,13 @@ class _LogProbsFromLogits(torch.autograd.Function):
         assert labels.shape == logits.shape[:-1], f"labels {tuple(labels.shape)} do not match logits {tuple(logits.shape)}"
         rows, ld = _logit_rows(logits)
         lab = labels.reshape(-1).to(device=rows.device, dtype=torch.int64).contiguous()
-        logprobs, _, lse, _ = _row_stats(rows, ld, lab, True, False, False)
+        logprobs, _, lse, _ = _row_stats(rows, ld, lab, True, False, False, logits.dtype)
         ctx.save_for_backward(rows, lab, lse)
         ctx.ld, ctx.shape = ld, logits.shape
         # writing the gradient over the logits needs the rows to BE the caller's storage
         ctx.in_place = (bool(inplace_backward) and rows.data_ptr() == logits.data_ptr() and logits.is_contiguous()
                         and not (logits.is_leaf and logits.requires_grad))   # never overwrite a parameter
-        return logprobs.to(logits.dtype).view(logits.shape[:-1])
+        return logprobs.view(logits.shape[:-1])
 
     @staticmethod
     @torch.autograd.function.once_differentiable
@@ -94,11 +99,10 @@ class _EntropyFromLogits(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, fp32_output: bool):
         rows, ld = _logit_rows(logits)
-        _, entropy, lse, mean_z = _row_stats(rows, ld, None, False, True, True)
+        _, entropy, lse, mean_z = _row_stats(rows, ld, None, False, True, True,
+                                             torch.float32 if fp32_output else logits.dtype)
         ctx.save_for_backward(rows, lse, mean_z)
         ctx.ld, ctx.shape = ld, logits.shape
-        if not fp32_output:
-            entropy = entropy.to(logits.dtype)
         return entropy.view(logits.shape[:-1])
 
     @staticmethod

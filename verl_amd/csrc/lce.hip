@@ -1060,10 +1060,15 @@ __global__ __launch_bounds__(kThreads) void lce_recompute_kernel(RecomputeArgs a
   run_tiles<false, false>(a.hidden, a.weight, sched, epi, lds);
 }
 
-// d_logits panel of one vocabulary chunk from cached logits, to the bits of RecomputeEpi,
-// one thread per 8 consecutive columns of a token, 2048 columns per workgroup.  Bound by memory (5.7 TB/s at 777 x 151936).
+// d_logits panel of one vocabulary chunk from cached logits, to the bits of RecomputeEpi.  Bound by memory.
+// A workgroup takes kPanelCols columns of a token, two groups of 4 per thread, each group's loads and stores contiguous across the
+// wavefront; workgroups walk along a row.  With 8 consecutive columns per thread an instruction touched half of every line,
+// and tokens as the fast index made neighbouring workgroups a row of the cache apart: 16384 x 152064 2695 -> 2470 us (6.1 TB/s),
+// 4096 x 151936 717 -> 600, 777 x 151936 127 -> 115.  One group per thread 2913, four 2549, cached instead of non-temporal loads
+// 2682, non-temporal stores 2499.
 // Rows of the panel past the last token are not written: the gradient products read them as zero without fetching them
-// (filling the last 256-token tile took 64 x 151936 from 15.5 to 22.4 us, 777 x 151936 from 128 to 137).
+// (filling the last 256-token tile took 64 x 151936 from 15.5 to 22.4 us).
+constexpr int kPanelCols = 2048;
 struct DLogitsArgs {
   const float* z_cache;  // [cache_rows][vocab]
   const int64_t* rows;   // the row of each token, or null: token i has row i
@@ -1080,33 +1085,42 @@ struct DLogitsArgs {
 };
 
 __global__ __launch_bounds__(256) void lce_dlogits_kernel(DLogitsArgs a) {
-  const int tok = blockIdx.x;
-  const int j = (blockIdx.y * 256 + threadIdx.x) * 8;  // column inside the chunk
-  if (j >= a.chunk_cols) return;
-  u32x4 out = {0u, 0u, 0u, 0u};
-  const int col = a.chunk_c0 + j;
+  const int blocks = (a.chunk_cols + kPanelCols - 1) / kPanelCols, tok = blockIdx.x / blocks;
+  const int j0 = (int)(blockIdx.x % blocks) * kPanelCols + threadIdx.x * 4;  // column inside the chunk
   const int64_t row = a.rows ? a.rows[tok] : tok;
-  // vocab % 8 == 0: the 8 columns are all in or all out
-  if (col < a.vocab && row >= 0 && row < a.cache_rows) {
-    const float lse2 = a.lse[tok] * kLog2e;
-    const float glp = (a.g_lp ? a.g_lp[tok] : 0.f) * a.rcp_t;
-    const float gent = (a.g_ent ? a.g_ent[tok] : a.g_ent_scalar) * a.rcp_t;
-    const float u0 = fmaf(-gent, a.mean_z[tok], glp);
-    const int rel = (int)a.labels[tok] - col;
-    const f32x4* src = reinterpret_cast<const f32x4*>(a.z_cache + row * a.vocab + col);
-    const f32x4 z0 = __builtin_nontemporal_load(src), z1 = __builtin_nontemporal_load(src + 1);
-    float d[8];
+  const int cols = row >= 0 && row < a.cache_rows ? a.vocab - a.chunk_c0 : 0;  // columns that exist
+  const float lse2 = a.lse[tok] * kLog2e;
+  const float glp = (a.g_lp ? a.g_lp[tok] : 0.f) * a.rcp_t;
+  const float gent = (a.g_ent ? a.g_ent[tok] : a.g_ent_scalar) * a.rcp_t;
+  const float u0 = fmaf(-gent, a.mean_z[tok], glp);
+  const int label = (int)a.labels[tok] - a.chunk_c0;
+  f32x4 z[2];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float z = e < 4 ? z0[e] : z1[e - 4];
-      const float prob = fast_exp2(fmaf(z, kLog2e, -lse2));
-      const float u = fmaf(gent, z, u0);
-      d[e] = fmaf(-prob, u, (e == rel) ? glp : 0.f);
-    }
-    const u32x2 lo = pack_bf16x4(d[0], d[1], d[2], d[3]), hi = pack_bf16x4(d[4], d[5], d[6], d[7]);
-    out = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  for (int g = 0; g < 2; ++g) {
+    const int j = j0 + g * (kPanelCols / 2);
+    z[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // vocab % 8 == 0: the 4 columns are all in or all out
+    if (j < a.chunk_cols && j < cols)
+      z[g] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(a.z_cache + row * a.vocab + a.chunk_c0 + j));
   }
-  *reinterpret_cast<u32x4*>(a.dz + (int64_t)tok * a.dz_ld + j) = out;
+  u32x2 out[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int j = j0 + g * (kPanelCols / 2);
+    float d[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float prob = fast_exp2(fmaf(z[g][e], kLog2e, -lse2));
+      const float u = fmaf(gent, z[g][e], u0);
+      d[e] = fmaf(-prob, u, (j + e == label) ? glp : 0.f);
+    }
+    out[g] = j < cols ? pack_bf16x4(d[0], d[1], d[2], d[3]) : u32x2{0u, 0u};
+  }
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int j = j0 + g * (kPanelCols / 2);
+    if (j < a.chunk_cols) *reinterpret_cast<u32x2*>(a.dz + (int64_t)tok * a.dz_ld + j) = out[g];
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1739,7 +1753,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
       d.dz_ld = (int)pitch;
       {
         ScopedTiming tm(kTagDLogits, s);
-        hipLaunchKernelGGL(lce_dlogits_kernel, dim3((unsigned)n_tokens, (unsigned)ceil_div(d.chunk_cols, 2048)), dim3(256),
+        hipLaunchKernelGGL(lce_dlogits_kernel, dim3((unsigned)(n_tokens * ceil_div(d.chunk_cols, kPanelCols))), dim3(256),
                            0, s, d);
       }
       VAMD_LAUNCH_CHECK();

@@ -1387,14 +1387,19 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
 // 7339 x 3584 have 406 on 256 CUs (87 % of the launch busy).  So a tile's k range is cut into pieces of equal length,
 // each summed in fp32 into an accumulator of its own, and the d_weight tiles are shared out so that the workgroups
 // with a piece more get correspondingly fewer tiles.  The number of pieces is the one whose slowest workgroup is
-// quickest, counting in slabs (1.4 us each): a tile's epilogue about 2, and the accumulators' way to memory and back.
-constexpr int kEpilogueSlabs = 2, kMaxSplits = 64, kMinPieceSlabs = 32;
+// quickest, counting in slabs (1.4 us each): a d_hidden unit's epilogue about 2, a d_weight tile's, all of whose 128 KB go to
+// memory, 3, and a d_weight tile of few slabs 7 in all: with every CU storing, 128 KB take 6 us.  Gradient products with
+// 2 and no least, and as it is: 64 x 896 x 151936 207 -> 163 us, 128 tokens 206 -> 165, 777 467 -> 464; 64 x 3584 x 152064
+// 700 -> 553, 128 tokens 701 -> 590, 300 tokens 980 -> 938, 777 tokens 1620 -> 1590 (256 tokens 675 -> 693); from 1300
+// tokens on within 1 %.
+constexpr int kEpilogueSlabs = 2, kTileEpilogueSlabs = 3, kLeastTileSlabs = 7, kMaxSplits = 64, kMinPieceSlabs = 32;
 constexpr int64_t kMaxPieceBytes = 256ll << 20;  // bound on the pieces' accumulators
 static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t cols, bool want_dh, bool want_dw,
                                int cus, int fixed_pieces = 0) {
   const int64_t h_tiles = ceil_div(hidden_size, kTile);
   const int64_t th = want_dh ? ceil_div(n_tokens, kTile) * h_tiles : 0, kh = ceil_div(cols, kBK);
-  const int64_t tw = want_dw ? ceil_div(cols, kTile) * h_tiles : 0, cost_w = ceil_div(n_tokens, kBK) + kEpilogueSlabs;
+  const int64_t tw = want_dw ? ceil_div(cols, kTile) * h_tiles : 0, tile_slabs = ceil_div(n_tokens, kBK) + kTileEpilogueSlabs;
+  const int64_t cost_w = tile_slabs > kLeastTileSlabs ? tile_slabs : kLeastTileSlabs;
   const int64_t piece_bytes = n_tokens * hidden_size * 4;
   GradPlan best;
   best.split_slabs = (int)kh;

@@ -1709,6 +1709,41 @@ def test_rollout_correction_weights_and_metrics(dev, shape, level, spread, norma
     assert torch.equal(w.cpu()[mask == 0], torch.zeros_like(w.cpu()[mask == 0]))
 
 
+@pytest.mark.parametrize("shape", [(2049, 5), (2304, 5), (3200, 9), (1100, 4099), (2050, 8)])   # records beyond 2048: workgroups walk
+@pytest.mark.parametrize("agg", ["token-mean", "seq-mean-token-sum-norm"])
+def test_losses_whose_workgroups_walk_several_chunks(dev, shape, agg):
+    """Losses and gradients of launches with more chunks than the device holds workgroups, against fp64 sums."""
+    from verl_amd.trainer.ppo import core_algos as CA
+    B, L = shape
+    g = torch.Generator().manual_seed(B + L)
+    mask, _ = _prefix_mask(B, L, g, lo=1)
+    old, ref, adv = (torch.randn(B, L, generator=g) * 0.3 for _ in range(3))
+    new = old + torch.randn(B, L, generator=g) * 0.2
+    norm = mask.double().sum() if agg == "token-mean" else float(L)
+    x = new.double().requires_grad_()
+    ratio = torch.exp(x - old.double())
+    a = adv.double()
+    pl = torch.maximum(-a * ratio, -a * ratio.clamp(0.8, 1.2))
+    pl = torch.where(a < 0, torch.minimum(-a * 3.0, pl), pl)
+    d = ref.double() - x
+    want = ((pl * mask).sum() / norm, ((torch.exp(d) - d - 1) * mask).sum() / norm, (x * mask).sum() / norm)
+    cuda = lambda t: t.to(dev)
+    lp = cuda(new).requires_grad_()
+    m = cuda(mask)
+    cfg = types.SimpleNamespace(clip_ratio=0.2, clip_ratio_low=None, clip_ratio_high=None, clip_ratio_c=3.0,
+                                global_batch_info={}, get=lambda k, default=None: default)
+    got = (CA.compute_policy_loss_vanilla(cuda(old), lp, cuda(adv), m, agg, cfg)[0],
+           CA.compute_kl_loss(lp, cuda(ref), m, "low_var_kl", agg), CA.agg_loss(lp, m, agg))
+    for loss, ref_loss in zip(got, want):
+        (gd,) = torch.autograd.grad(loss, lp, retain_graph=True)
+        (wd,) = torch.autograd.grad(ref_loss, x, retain_graph=True)
+        # fp32 arithmetic per token, fp64 sums: 2^-20 relative to the mean magnitude of what is summed
+        scale = float((mask.double().sum() / norm).clamp(min=1.0)) if agg != "token-mean" else 1.0
+        assert abs(loss.item() - ref_loss.item()) <= 2e-6 * max(scale, 1.0), (loss.item(), ref_loss.item())
+        err = (gd.cpu().double() - wd).abs().max().item()
+        assert err <= 4e-6 * wd.abs().max().item(), err
+
+
 @pytest.mark.parametrize("rows", [63, 64, 65, 129, 16385])   # a row per lane, 64 per workgroup, 256 workgroups, then a second trip
 def test_statistics_fold_edges(dev, rows):
     test_data_metrics(dev, (rows, 9), 4, torch.int64, True)

@@ -20,6 +20,22 @@ struct Work {
   int totals;        // loss kernels built without the fold: take the launch totals here (totals_epilogue)
 };
 
+// A workgroup of the policy, value and KL losses takes the (row, chunk) items b, b + gridDim.x, ...  One each where the per-row sums are needed or
+// the launch is small; where the launch totals are all that is wanted, a large launch has as many workgroups as the device
+// holds at once (loss_grid), so that the workgroup reduction, the record and the arrival, during which a workgroup's registers
+// stream nothing, come once per workgroup and not once per item.  1000 x 11999 (3000 items) with an int64 mask: policy loss
+// with gradient 64.6 -> 57.3 us, KL loss with gradient 46.9 -> 43.2; 760 x 11999 fp32: 42.9 -> 38.7, 30.7 -> 28.3; 2048 x 16384
+// bool (8192 items): KL loss 84.5 -> 78.2.  The policy and value losses walk only in launches that do not stream past the
+// caches (and where rows are not aligned): 2048 x 16384 takes 115.5 us walking, 112.8 with a workgroup per item.  agg_loss,
+// whose workgroups are light enough for eight to a CU, does not: with the loop 1000 x 11999 took 29.7 us, without it 28.0.
+__device__ __forceinline__ bool walks_several(int64_t rows, int chunks) { return (int64_t)gridDim.x != rows * chunks; }
+template <int NV>
+__device__ __forceinline__ void store_loss_record(const Work& wk, unsigned item, int64_t rows, int chunks,
+                                                  const double (&acc)[NV]) {
+  if (walks_several(rows, chunks)) store_record<NV>(wk.partials, blockIdx.x, 0, gridDim.x, 1, acc);
+  else store_record<NV>(wk.partials, item / (unsigned)chunks, (int)(item % (unsigned)chunks), rows, chunks, acc);
+}
+
 // The loss kernels of a large launch carry no fold of their own (FOLD = false).  Two of the four agg_loss modes,
 // token-mean and seq-mean-token-sum-norm, need nothing but the launch totals, and those come cheaply in two
 // levels (sum_all_records: a few dozen registers, no per-row pass), so such a launch finishes here; the per-row
@@ -29,7 +45,8 @@ __device__ __forceinline__ void totals_epilogue(const Work& wk, int64_t rows, in
                                                 const AggParams& ap, float* __restrict__ coef,
                                                 float* __restrict__ out, double* smem) {
   double tot[NV];
-  if (!sum_all_records<NV>(wk.ticket, wk.partials, rows, chunks, tot, smem)) return;
+  const bool walks = walks_several(rows, chunks);
+  if (!sum_all_records<NV>(wk.ticket, wk.partials, walks ? (int64_t)gridDim.x : rows, walks ? 1 : chunks, tot, smem)) return;
   __shared__ float c_all;
   if (threadIdx.x == 0) {
     double loss, c;
@@ -53,6 +70,13 @@ __device__ __forceinline__ void totals_epilogue(const Work& wk, int64_t rows, in
     for (int64_t r = threadIdx.x; r < rows; r += kRcThreads) coef[r] = c_all;
   ticket_reset(wk.ticket);
 }
+// Workgroups of a loss launch; per_cu: how many of the kernel a CU holds (measured one less and one more as well: policy loss
+// at 1000 x 11999 62.6, 59.0, 68.3 us with 2, 3, 4; KL loss 44.6, 42.5, 42.4 with 3, 4, 5).
+inline unsigned loss_grid(int64_t items, bool walks, int per_cu) {
+  const int64_t resident = (int64_t)device_cu_count() * per_cu;
+  return (unsigned)(walks && items > kInlineFoldRecords ? balanced_waiting_grid(items, resident) : items);
+}
+constexpr int kPolicyPerCu = 3, kValuePerCu = 3, kKlPerCu = 4;
 __host__ __device__ inline bool totals_suffice(int mode) {
   return mode == VAMD_AGG_TOKEN_MEAN || mode == VAMD_AGG_SEQ_MEAN_TOKEN_SUM_NORM;
 }
@@ -492,127 +516,135 @@ __global__ __launch_bounds__(kRcThreads) void policy_kernel(
     const M* __restrict__ mask, const float* __restrict__ isw, int64_t rows, int64_t cols, int chunks,
     PolicyParams pp, AggParams ap, Work wk, float* __restrict__ out, float* __restrict__ grad,
     float* __restrict__ coef) {
-  const int64_t row = blockIdx.x / chunks;
-  const int chunk = blockIdx.x % chunks;
-  const ChunkPos pos(row, chunk, cols);
-  float o[kGroups][4], n[kGroups][4], a[kGroups][4], w[kGroups][4], iw[kGroups][4], gr[kGroups][4];
-  load_groups<VEC>(old_lp, pos, o);
-  load_groups<VEC>(lp, pos, n);
-  load_groups<VEC>(adv, pos, a);
-  load_mask_groups<VEC>(mask, pos, w);
-  if (ISW) load_groups<VEC>(isw, pos, iw);
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
-  float seq_lr = 0.f;
   const int variant = VARIANT >= 0 ? VARIANT : pp.variant;
   __shared__ double smem[(5 + 3) * 4];
-  double r[4] = {0, 0, 0, 0};  // the row's four sums (GSPO, GEO_MEAN)
-  if constexpr (ROWS) {
-    __shared__ double row_sums[4];
-    double own[4];
-    row_presums<ISW>(variant, pos, o, n, a, w, iw, pp.nkl_lo, pp.nkl_hi, own);
-    block_sum<4, kRcThreads>(own, smem);  // valid in thread 0
-    bool open = true;
-    if (chunks > 1) {
-      if (threadIdx.x == 0) {
-        double* mine = pp.row_partials + (row * chunks + chunk) * 4;
+  const unsigned items = (unsigned)(rows * chunks);
+  const bool streaming = items >= kStreamingGrid;
+  double acc[5] = {0, 0, 0, 0, 0};
+  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
+    const int64_t row = item / (unsigned)chunks;
+    const int chunk = (int)(item % (unsigned)chunks);
+    const ChunkPos pos(row, chunk, cols);
+    float o[kGroups][4], n[kGroups][4], a[kGroups][4], w[kGroups][4], iw[kGroups][4], gr[kGroups][4];
+    load_groups<VEC>(old_lp, pos, o, streaming);
+    load_groups<VEC>(lp, pos, n, streaming);
+    load_groups<VEC>(adv, pos, a, streaming);
+    load_mask_groups<VEC>(mask, pos, w, streaming);
+    if (ISW) load_groups<VEC>(isw, pos, iw, streaming);
+    float seq_lr = 0.f;
+    double r[4] = {0, 0, 0, 0};  // the row's four sums (GSPO, GEO_MEAN)
+    if constexpr (ROWS) {
+      __shared__ double row_sums[4];
+      double own[4];
+      row_presums<ISW>(variant, pos, o, n, a, w, iw, pp.nkl_lo, pp.nkl_hi, own);
+      block_sum<4, kRcThreads>(own, smem);  // valid in thread 0
+      bool open = true;
+      if (chunks > 1) {
+        if (threadIdx.x == 0) {
+          double* mine = pp.row_partials + (row * chunks + chunk) * 4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) peer_store(mine + i, own[i]);
-        ready_byte_set(wk.ticket, row * chunks + chunk);
+          for (int i = 0; i < 4; ++i) peer_store(mine + i, own[i]);
+          ready_byte_set(wk.ticket, row * chunks + chunk);
+        }
+        bool ready = true;
+        unsigned polls = 0;
+        if ((int)threadIdx.x < chunks && (int)threadIdx.x != chunk)
+          ready = ready_byte_wait(wk.ticket, row * chunks + threadIdx.x, polls, pp.spin_limit);
+        open = __syncthreads_and(ready) != 0;
+        if (!open && threadIdx.x == 0) note_gave_up(wk.ticket);
       }
-      bool ready = true;
-      unsigned polls = 0;
-      if ((int)threadIdx.x < chunks && (int)threadIdx.x != chunk)
-        ready = ready_byte_wait(wk.ticket, row * chunks + threadIdx.x, polls, pp.spin_limit);
-      open = __syncthreads_and(ready) != 0;
-      if (!open && threadIdx.x == 0) note_gave_up(wk.ticket);
-    }
-    if (open) {
-      if (threadIdx.x == 0) {
+      if (open) {
+        if (threadIdx.x == 0) {
+          for (int c = 0; c < chunks; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              r[i] += c == chunk ? own[i] : peer_load(pp.row_partials + (row * chunks + c) * 4 + i);
+        }
+      } else {
+        for (int c = 0; c < chunks; ++c) {  // uniform over the workgroup
+          double part[4];
+          if (c != chunk) {
+            const ChunkPos p2(row, c, cols);
+            float o2[kGroups][4], n2[kGroups][4], a2[kGroups][4], w2[kGroups][4], iw2[kGroups][4];
+            load_groups<VEC>(old_lp, p2, o2);
+            load_groups<VEC>(lp, p2, n2);
+            load_groups<VEC>(adv, p2, a2);
+            load_mask_groups<VEC>(mask, p2, w2);
+            if (ISW) load_groups<VEC>(isw, p2, iw2);
+            row_presums<ISW>(variant, p2, o2, n2, a2, w2, iw2, pp.nkl_lo, pp.nkl_hi, part);
+            block_sum<4, kRcThreads>(part, smem);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] += c == chunk ? own[i] : part[i];  // thread 0's are the sums
+        }
+      }
+      if (threadIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) row_sums[i] = r[i];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = row_sums[i];
+    } else {
+      if (variant == VAMD_PL_GSPO) {
+        r[0] = pp.row_moments[row * 4];
+        r[1] = pp.row_moments[row * 4 + 1];
+      }
+      if (variant == VAMD_PL_GEO_MEAN)
         for (int c = 0; c < chunks; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            r[i] += c == chunk ? own[i] : peer_load(pp.row_partials + (row * chunks + c) * 4 + i);
-      }
-    } else {
-      for (int c = 0; c < chunks; ++c) {  // uniform over the workgroup
-        double part[4];
-        if (c != chunk) {
-          const ChunkPos p2(row, c, cols);
-          float o2[kGroups][4], n2[kGroups][4], a2[kGroups][4], w2[kGroups][4], iw2[kGroups][4];
-          load_groups<VEC>(old_lp, p2, o2);
-          load_groups<VEC>(lp, p2, n2);
-          load_groups<VEC>(adv, p2, a2);
-          load_mask_groups<VEC>(mask, p2, w2);
-          if (ISW) load_groups<VEC>(isw, p2, iw2);
-          row_presums<ISW>(variant, p2, o2, n2, a2, w2, iw2, pp.nkl_lo, pp.nkl_hi, part);
-          block_sum<4, kRcThreads>(part, smem);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] += c == chunk ? own[i] : part[i];  // thread 0's are the sums
-      }
+          for (int i = 0; i < 4; ++i) r[i] += pp.row_moments[(row * chunks + c) * 4 + i];
     }
-    if (threadIdx.x == 0)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) row_sums[i] = r[i];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = row_sums[i];
-  } else {
-    if (variant == VAMD_PL_GSPO) {
-      r[0] = pp.row_moments[row * 4];
-      r[1] = pp.row_moments[row * 4 + 1];
+    if (variant == VAMD_PL_GSPO)  // sum((lp - old) m) / clamp(sum(m), min = 1)
+      seq_lr = (float)r[1] / fmaxf((float)r[0], 1.f);
+    if (variant == VAMD_PL_GEO_MEAN) {
+      const float den = (float)r[0] + 1e-8f;
+      const float ratio = expf((float)r[1] / den);
+      const float a_seq = (float)r[2] / den;
+      const float w_seq = expf((float)r[3] / den);  // 1 when no importance weights were given (sum of logs = 0)
+      seq_lr = -a_seq * ratio * w_seq / den;
     }
-    if (variant == VAMD_PL_GEO_MEAN)
-      for (int c = 0; c < chunks; ++c)
+    // GMPO's importance weights enter through the sequence weight above, not token by token
+    const bool isw_per_token = ISW && variant != VAMD_PL_GEO_MEAN;
+    float s_loss = 0, s_m = 0, s_kl = 0, s_cf = 0, s_cfl = 0;
+    // a kernel built for every variant (VARIANT = -1) picks the variant once, here, and runs that variant's copy of
+    // the token loop: chosen per token, the sixteen tokens of a thread were sixteen seven-way switches
+    with_policy_variant<VARIANT>(variant, [&](auto which) {
+      constexpr int V = decltype(which)::value;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] += pp.row_moments[(row * chunks + c) * 4 + i];
-  }
-  if (variant == VAMD_PL_GSPO)  // sum((lp - old) m) / clamp(sum(m), min = 1)
-    seq_lr = (float)r[1] / fmaxf((float)r[0], 1.f);
-  if (variant == VAMD_PL_GEO_MEAN) {
-    const float den = (float)r[0] + 1e-8f;
-    const float ratio = expf((float)r[1] / den);
-    const float a_seq = (float)r[2] / den;
-    const float w_seq = expf((float)r[3] / den);  // 1 when no importance weights were given (sum of logs = 0)
-    seq_lr = -a_seq * ratio * w_seq / den;
-  }
-  // GMPO's importance weights enter through the sequence weight above, not token by token
-  const bool isw_per_token = ISW && variant != VAMD_PL_GEO_MEAN;
-  float s_loss = 0, s_m = 0, s_kl = 0, s_cf = 0, s_cfl = 0;
-  // a kernel built for every variant (VARIANT = -1) picks the variant once, here, and runs that variant's copy of
-  // the token loop: chosen per token, the sixteen tokens of a thread were sixteen seven-way switches
-  with_policy_variant<VARIANT>(variant, [&](auto which) {
-    constexpr int V = decltype(which)::value;
+      for (int g = 0; g < kGroups; ++g)
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const TokenLoss t = token_loss<V>(pp, o[g][e], n[g][e], a[g][e], seq_lr);
-        float loss = t.loss;
-        if (isw_per_token) loss *= iw[g][e];
-        const float we = w[g][e];
-        const bool in = we != 0.f;
-        // Elements past the end of the row were loaded as zeros with weight zero and add nothing, so the test is
-        // redundant.  The small launches (FOLD) are faster without its sixteen branches (512 x 4096: 16.1 -> 15.8
-        // us with the gradient); the large ones are faster with it (2048 x 16384: 115 against 117 us), where the
-        // compiler then holds all of a thread's loads in registers at once.
-        if (FOLD || e < pos.valid[g]) {
-          s_loss += ((token_mean && !in) ? 0.f : loss) * we;
-          s_m += we;
-          s_kl += in ? t.kl * we : 0.f;
-          s_cf += in ? t.cf * we : 0.f;
-          s_cfl += in ? t.cfl * we : 0.f;
+        for (int e = 0; e < 4; ++e) {
+          const TokenLoss t = token_loss<V>(pp, o[g][e], n[g][e], a[g][e], seq_lr);
+          float loss = t.loss;
+          if (isw_per_token) loss *= iw[g][e];
+          const float we = w[g][e];
+          const bool in = we != 0.f;
+          // Elements past the end of the row were loaded as zeros with weight zero and add nothing, so the test is
+          // redundant.  The small launches (FOLD) are faster without its sixteen branches (512 x 4096: 16.1 -> 15.8
+          // us with the gradient); the large ones are faster with it (2048 x 16384: 115 against 117 us), where the
+          // compiler then holds all of a thread's loads in registers at once.
+          if (FOLD || e < pos.valid[g]) {
+            s_loss += ((token_mean && !in) ? 0.f : loss) * we;
+            s_m += we;
+            s_kl += in ? t.kl * we : 0.f;
+            s_cf += in ? t.cf * we : 0.f;
+            s_cfl += in ? t.cfl * we : 0.f;
+          }
+          if (GRAD) gr[g][e] = (isw_per_token ? t.dloss * iw[g][e] : t.dloss) * we;
         }
-        if (GRAD) gr[g][e] = (isw_per_token ? t.dloss * iw[g][e] : t.dloss) * we;
-      }
-  });
-  if (GRAD) store_groups<VEC>(grad, pos, gr);
+    });
+    if (GRAD) store_groups<VEC>(grad, pos, gr, streaming);
+    acc[0] += (double)s_loss;
+    acc[1] += (double)s_m;
+    acc[2] += (double)s_kl;
+    acc[3] += (double)s_cf;
+    acc[4] += (double)s_cfl;
+    if constexpr (!FOLD) break;  // one item per workgroup
+  }
   static_assert(!ROWS || FOLD, "a launch that sets ready bytes has a last workgroup that clears them");
-  double acc[5] = {s_loss, s_m, s_kl, s_cf, s_cfl};
   block_sum<5, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) {
-    store_record<5>(wk.partials, row, chunk, rows, chunks, acc);
-  }
+  if (threadIdx.x == 0) store_loss_record<5>(wk, blockIdx.x, rows, chunks, acc);
   if constexpr (FOLD) {
     if (!ROWS && totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
       totals_epilogue<5, kEpiPolicy>(wk, rows, chunks, cols, ap, coef, out, smem);
@@ -706,48 +738,52 @@ __global__ __launch_bounds__(kRcThreads) void value_kernel(
     const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
     const M* __restrict__ mask, int64_t rows, int64_t cols, int chunks, float clip, AggParams ap, Work wk,
     float* __restrict__ out, float* __restrict__ grad, float* __restrict__ coef) {
-  const int64_t row = blockIdx.x / chunks;
-  const int chunk = blockIdx.x % chunks;
-  const ChunkPos pos(row, chunk, cols);
-  float vp[kGroups][4], R[kGroups][4], v[kGroups][4], w[kGroups][4], gr[kGroups][4];
-  load_groups<VEC>(vpreds, pos, vp);
-  load_groups<VEC>(returns, pos, R);
-  load_groups<VEC>(values, pos, v);
-  load_mask_groups<VEC>(mask, pos, w);
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
-  float s_loss = 0, s_m = 0, s_cf = 0;
+  const unsigned items = (unsigned)(rows * chunks);
+  const bool streaming = items >= kStreamingGrid;
+  double acc[3] = {0, 0, 0};
+  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
+    const ChunkPos pos(item / (unsigned)chunks, (int)(item % (unsigned)chunks), cols);
+    float vp[kGroups][4], R[kGroups][4], v[kGroups][4], w[kGroups][4], gr[kGroups][4];
+    load_groups<VEC>(vpreds, pos, vp, streaming);
+    load_groups<VEC>(returns, pos, R, streaming);
+    load_groups<VEC>(values, pos, v, streaming);
+    load_mask_groups<VEC>(mask, pos, w, streaming);
+    float s_loss = 0, s_m = 0, s_cf = 0;
 #pragma unroll
-  for (int g = 0; g < kGroups; ++g)
+    for (int g = 0; g < kGroups; ++g)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float lo = v[g][e] - clip, hi = v[g][e] + clip;
-      const float inner = fminf(vp[g][e], hi);
-      const float vc = fmaxf(inner, lo);
-      const float d1 = vp[g][e] - R[g][e], d2 = vc - R[g][e];
-      const float e1 = d1 * d1, e2 = d2 * d2;
-      const float loss = fmaxf(e1, e2);
-      const float we = w[g][e];
-      const bool in = we != 0.f;
-      if (FOLD || e < pos.valid[g]) {  // redundant (zeros with weight zero past the end); see policy_kernel
-        s_loss += ((token_mean && !in) ? 0.f : loss) * we;
-        s_m += we;
-        s_cf += (in && e2 > e1) ? we : 0.f;
+      for (int e = 0; e < 4; ++e) {
+        const float lo = v[g][e] - clip, hi = v[g][e] + clip;
+        const float inner = fminf(vp[g][e], hi);
+        const float vc = fmaxf(inner, lo);
+        const float d1 = vp[g][e] - R[g][e], d2 = vc - R[g][e];
+        const float e1 = d1 * d1, e2 = d2 * d2;
+        const float loss = fmaxf(e1, e2);
+        const float we = w[g][e];
+        const bool in = we != 0.f;
+        if (FOLD || e < pos.valid[g]) {  // redundant (zeros with weight zero past the end); see policy_kernel
+          s_loss += ((token_mean && !in) ? 0.f : loss) * we;
+          s_m += we;
+          s_cf += (in && e2 > e1) ? we : 0.f;
+        }
+        if (GRAD) {
+          const float ga = vp[g][e] < hi ? 1.f : (vp[g][e] == hi ? 0.5f : 0.f);
+          const float gb = inner > lo ? 1.f : (inner == lo ? 0.5f : 0.f);
+          const float g1 = e1 > e2 ? 1.f : (e1 == e2 ? 0.5f : 0.f);
+          const float g2 = e2 > e1 ? 1.f : (e1 == e2 ? 0.5f : 0.f);
+          gr[g][e] = (g1 * 2.f * d1 + g2 * 2.f * d2 * ga * gb) * we;
+        }
       }
-      if (GRAD) {
-        const float ga = vp[g][e] < hi ? 1.f : (vp[g][e] == hi ? 0.5f : 0.f);
-        const float gb = inner > lo ? 1.f : (inner == lo ? 0.5f : 0.f);
-        const float g1 = e1 > e2 ? 1.f : (e1 == e2 ? 0.5f : 0.f);
-        const float g2 = e2 > e1 ? 1.f : (e1 == e2 ? 0.5f : 0.f);
-        gr[g][e] = (g1 * 2.f * d1 + g2 * 2.f * d2 * ga * gb) * we;
-      }
-    }
-  if (GRAD) store_groups<VEC>(grad, pos, gr);
-  __shared__ double smem[(3 + 3) * 4];
-  double acc[3] = {s_loss, s_m, s_cf};
-  block_sum<3, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) {
-    store_record<3>(wk.partials, row, chunk, rows, chunks, acc);
+    if (GRAD) store_groups<VEC>(grad, pos, gr, streaming);
+    acc[0] += (double)s_loss;
+    acc[1] += (double)s_m;
+    acc[2] += (double)s_cf;
+    if constexpr (!FOLD) break;  // one item per workgroup
   }
+  __shared__ double smem[(3 + 3) * 4];
+  block_sum<3, kRcThreads>(acc, smem);
+  if (threadIdx.x == 0) store_loss_record<3>(wk, blockIdx.x, rows, chunks, acc);
   if constexpr (FOLD) {
     if (totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
       totals_epilogue<3, kEpiValue>(wk, rows, chunks, cols, ap, coef, out, smem);
@@ -828,38 +864,40 @@ __global__ __launch_bounds__(kRcThreads) void kl_loss_kernel(
     const float* __restrict__ logprob, const float* __restrict__ ref, const M* __restrict__ mask, int64_t rows,
     int64_t cols, int chunks, int kind, int straight, AggParams ap, Work wk, float* __restrict__ out,
     float* __restrict__ grad, float* __restrict__ coef) {
-  const int64_t row = blockIdx.x / chunks;
-  const int chunk = blockIdx.x % chunks;
-  const ChunkPos pos(row, chunk, cols);
-  float lp[kGroups][4], rf[kGroups][4], w[kGroups][4], gr[kGroups][4];
-  load_groups<VEC>(logprob, pos, lp);
-  load_groups<VEC>(ref, pos, rf);
-  load_mask_groups<VEC>(mask, pos, w);
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
-  float s_loss = 0, s_m = 0;
-  with_kl_kind(kind, [&](auto which) {
-    constexpr int KIND = decltype(which)::value;
+  const unsigned items = (unsigned)(rows * chunks);
+  const bool streaming = items >= kStreamingGrid;
+  double acc[2] = {0, 0};
+  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
+    const ChunkPos pos(item / (unsigned)chunks, (int)(item % (unsigned)chunks), cols);
+    float lp[kGroups][4], rf[kGroups][4], w[kGroups][4], gr[kGroups][4];
+    load_groups<VEC>(logprob, pos, lp, streaming);
+    load_groups<VEC>(ref, pos, rf, streaming);
+    load_mask_groups<VEC>(mask, pos, w, streaming);
+    float s_loss = 0, s_m = 0;
+    with_kl_kind(kind, [&](auto which) {
+      constexpr int KIND = decltype(which)::value;
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g)
+      for (int g = 0; g < kGroups; ++g)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float kld, dk;
-        kl_point<KIND>(kind, straight != 0, lp[g][e], rf[g][e], kld, dk);
-        const float we = w[g][e];
-        if (FOLD || e < pos.valid[g]) {  // redundant (zeros with weight zero past the end); see policy_kernel
-          s_loss += ((token_mean && we == 0.f) ? 0.f : kld) * we;
-          s_m += we;
+        for (int e = 0; e < 4; ++e) {
+          float kld, dk;
+          kl_point<KIND>(kind, straight != 0, lp[g][e], rf[g][e], kld, dk);
+          const float we = w[g][e];
+          if (FOLD || e < pos.valid[g]) {  // redundant (zeros with weight zero past the end); see policy_kernel
+            s_loss += ((token_mean && we == 0.f) ? 0.f : kld) * we;
+            s_m += we;
+          }
+          if (GRAD) gr[g][e] = dk * we;
         }
-        if (GRAD) gr[g][e] = dk * we;
-      }
-  });
-  if (GRAD) store_groups<VEC>(grad, pos, gr);
-  __shared__ double smem[(2 + 3) * 4];
-  double acc[2] = {s_loss, s_m};
-  block_sum<2, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) {
-    store_record<2>(wk.partials, row, chunk, rows, chunks, acc);
+    });
+    if (GRAD) store_groups<VEC>(grad, pos, gr, streaming);
+    acc[0] += (double)s_loss;
+    acc[1] += (double)s_m;
   }
+  __shared__ double smem[(2 + 3) * 4];
+  block_sum<2, kRcThreads>(acc, smem);
+  if (threadIdx.x == 0) store_loss_record<2>(wk, blockIdx.x, rows, chunks, acc);
   if constexpr (FOLD) {
     if (totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
       totals_epilogue<2, kEpiKl>(wk, rows, chunks, cols, ap, coef, out, smem);
@@ -1820,7 +1858,7 @@ extern "C" int vamd_policy_loss_variant_forward(int variant, const float* old_lo
   double* const row_area =
       reinterpret_cast<double*>(static_cast<char*>(workspace) + reduce_workspace_bytes(rows, cols, 5));
   AggParams ap = make_agg(mode, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor);
-  const dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
+  dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
   const float* token_weights = is_weights;  // what the per-token pass multiplies by
   if (variant == VAMD_PL_GEO_MEAN) {
     // the loss is the plain mean of the per-sequence losses over all rows (:1706): every valid token carries its
@@ -1914,7 +1952,9 @@ extern "C" int vamd_policy_loss_variant_forward(int variant, const float* old_lo
     const bool vec = can_vectorize(cols, {old_log_prob, log_prob, advantages, token_weights, grad_unscaled}, mask,
                                    sizeof(M));
     const M* mk = static_cast<const M*>(mask);
-    sep = sep && vec;
+    const bool walks = totals_suffice(ap.mode) && !rows_inline && (!vec || rows * chunks < kStreamingGrid);
+    grid.x = loss_grid(rows * chunks, walks, kPolicyPerCu);
+    sep = sep && vec && !walks;
     if (sep) { VAMD_PL_GW(true, false) }
     else if (vec) { VAMD_PL_GW(true, true) }
     else { VAMD_PL_GW(false, true) }
@@ -1951,7 +1991,7 @@ extern "C" int vamd_value_loss_forward(const float* vpreds, const float* returns
   const int chunks = (int)chunks_of(cols);
   Work wk = carve_work(workspace);
   const AggParams ap = make_agg(mode, 1.0, -1.0, -1.0, -1.0);
-  const dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
+  dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
   bool sep = rows * chunks > kInlineFoldRecords;
   wk.totals = sep && totals_suffice(mode);
 #define VAMD_VL(V, G, F)                                                                                     \
@@ -1960,7 +2000,9 @@ extern "C" int vamd_value_loss_forward(const float* vpreds, const float* returns
   VAMD_MASK_DISPATCH(mask_dtype, M, {
     const bool vec = can_vectorize(cols, {vpreds, returns, values, grad_unscaled}, mask, sizeof(M));
     const M* mk = static_cast<const M*>(mask);
-    sep = sep && vec;
+    const bool walks = totals_suffice(mode) && (!vec || rows * chunks < kStreamingGrid);
+    grid.x = loss_grid(rows * chunks, walks, kValuePerCu);
+    sep = sep && vec && !walks;
     if (sep) { if (grad_unscaled) VAMD_VL(true, true, false); else VAMD_VL(true, false, false); }
     else if (vec) { if (grad_unscaled) VAMD_VL(true, true, true); else VAMD_VL(true, false, true); }
     else { if (grad_unscaled) VAMD_VL(false, true, true); else VAMD_VL(false, false, true); }
@@ -2009,7 +2051,7 @@ extern "C" int vamd_kl_loss_forward(const float* logprob, const float* ref_logpr
   const int chunks = (int)chunks_of(cols);
   Work wk = carve_work(workspace);
   const AggParams ap = make_agg(mode, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor);
-  const dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
+  const dim3 grid(loss_grid(rows * chunks, totals_suffice(mode), kKlPerCu)), block(kRcThreads);
   bool sep = rows * chunks > kInlineFoldRecords;
   wk.totals = sep && totals_suffice(mode);
 #define VAMD_KL(V, G, F)                                                                                       \

@@ -1186,6 +1186,37 @@ struct DHiddenEpi {
   }
 };
 
+// Hand-over of a result that is stored as bf16 and not added to anything: 32 rows x 64 columns, rounded before the exchange, so
+// that a wavefront's store instruction covers 8 whole 128-byte lines (as 8 bytes per lane of 32-column patches it covered the
+// halves of 8).  Gradient products 777 x 896 x 151936 467 -> 453 us, 777 x 3584 x 152064 1625 -> 1497, 64 tokens 562 -> 475,
+// 16384 tokens 25.82 -> 25.69 ms.  16-byte chunk c of row r lives at position c ^ ((r >> 1) & 7) of the wavefront's patch,
+// which is that of GradExchange.
+typedef unsigned u32x4_at8 __attribute__((ext_vector_type(4), aligned(8)));  // d_weight's alignment is the caller's
+struct LineExchange {
+  char* stage;
+  int lx, lq, rd_row, rd_chunk;
+  __device__ __forceinline__ explicit LineExchange(const GradExchange& e)
+      : stage(e.stage), lx(e.lx), lq(e.lq), rd_row(e.rd_row), rd_chunk(e.rd_chunk) {}
+  // the patch (mb4, nb2) of an accumulator; lane L gets columns 8 (L % 8) .. + 7 of rows 8 i + L / 8
+  __device__ __forceinline__ void run(const Accum& acc, int mb4, int nb2, u32x4 (&out)[4]) const {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        const f32x4& v = acc.a[4 * mb4 + cb][2 * nb2 + rb];
+        const int row = 16 * rb + lx, chunk = (2 * cb + (lq >> 1)) ^ ((row >> 1) & 7);
+        *reinterpret_cast<u32x2*>(stage + row * 128 + chunk * 16 + (lq & 1) * 8) = pack_bf16x4(v[0], v[1], v[2], v[3]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 8 * i + rd_row;
+      out[i] = *reinterpret_cast<const u32x4*>(stage + row * 128 + ((rd_chunk ^ ((row >> 1) & 7)) << 4));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+};
+
 struct DWeightEpi {
   LanePos p;
   const GemmOutArgs* a;
@@ -1193,6 +1224,23 @@ struct DWeightEpi {
   __device__ __forceinline__ void prefetch(int, int, int) {}
   __device__ __forceinline__ void operator()(Accum& acc, int /*tile*/, int r0, int c0) {
     const GemmOutArgs& A = *a;
+    if (A.mode == VAMD_DW_STORE) {
+      const LineExchange line(ex);
+#pragma unroll
+      for (int nb = 0; nb < kNB2; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < kMB / 4; ++mb) {
+          u32x4 v[4];
+          line.run(acc, mb, nb, v);
+          const int col = c0 + p.wc * 128 + mb * 64 + 8 * line.rd_chunk;  // c_valid % 128 == 0: 8 columns are all in or all out
+          const int row0 = r0 + p.wr * (kNB * kBlk) + nb * 32 + line.rd_row;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (col < A.c_valid && row0 + 8 * i < A.r_valid)
+              *reinterpret_cast<u32x4_at8*>(A.out + (int64_t)(row0 + 8 * i) * A.ld_out + col) = v[i];
+        }
+      return;
+    }
 #pragma unroll
     for (int nb = 0; nb < kNB2; ++nb)
 #pragma unroll
@@ -1387,19 +1435,18 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
 // 7339 x 3584 have 406 on 256 CUs (87 % of the launch busy).  So a tile's k range is cut into pieces of equal length,
 // each summed in fp32 into an accumulator of its own, and the d_weight tiles are shared out so that the workgroups
 // with a piece more get correspondingly fewer tiles.  The number of pieces is the one whose slowest workgroup is
-// quickest, counting in slabs (1.4 us each): a d_hidden unit's epilogue about 2, a d_weight tile's, all of whose 128 KB go to
-// memory, 3, and a d_weight tile of few slabs 7 in all: with every CU storing, 128 KB take 6 us.  Gradient products with
-// 2 and no least, and as it is: 64 x 896 x 151936 207 -> 163 us, 128 tokens 206 -> 165, 777 467 -> 464; 64 x 3584 x 152064
-// 700 -> 553, 128 tokens 701 -> 590, 300 tokens 980 -> 938, 777 tokens 1620 -> 1590 (256 tokens 675 -> 693); from 1300
-// tokens on within 1 %.
-constexpr int kEpilogueSlabs = 2, kTileEpilogueSlabs = 3, kLeastTileSlabs = 7, kMaxSplits = 64, kMinPieceSlabs = 32;
+// quickest, counting in slabs (1.4 us each): an epilogue about 2, and a d_weight tile of up to 3 slabs 7 in all: with every CU
+// storing, its 128 KB take 6 us, and a slab or three more hardly show.  Gradient products over few tokens with 2 for every
+// epilogue, and as it is: 64 x 3584 x 152064 623 -> 490 us, 93 tokens 645 -> 487, 150 tokens 681 -> 588; 128 x 4096 x 128256
+// 600 -> 523; 7 for four slabs as well: 256 x 3584 643 -> 680.
+constexpr int kEpilogueSlabs = 2, kFewTileSlabs = 3, kFewTileCost = 7, kMaxSplits = 64, kMinPieceSlabs = 32;
 constexpr int64_t kMaxPieceBytes = 256ll << 20;  // bound on the pieces' accumulators
 static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t cols, bool want_dh, bool want_dw,
                                int cus, int fixed_pieces = 0) {
   const int64_t h_tiles = ceil_div(hidden_size, kTile);
   const int64_t th = want_dh ? ceil_div(n_tokens, kTile) * h_tiles : 0, kh = ceil_div(cols, kBK);
-  const int64_t tw = want_dw ? ceil_div(cols, kTile) * h_tiles : 0, tile_slabs = ceil_div(n_tokens, kBK) + kTileEpilogueSlabs;
-  const int64_t cost_w = tile_slabs > kLeastTileSlabs ? tile_slabs : kLeastTileSlabs;
+  const int64_t tw = want_dw ? ceil_div(cols, kTile) * h_tiles : 0, tile_slabs = ceil_div(n_tokens, kBK);
+  const int64_t cost_w = tile_slabs <= kFewTileSlabs ? kFewTileCost : tile_slabs + kEpilogueSlabs;
   const int64_t piece_bytes = n_tokens * hidden_size * 4;
   GradPlan best;
   best.split_slabs = (int)kh;

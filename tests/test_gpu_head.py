@@ -891,3 +891,32 @@ def test_logits_are_kept_where_they_are_a_small_part_of_the_free_memory(dev, mon
     for free, kept in ((8 * 4 * n * v, True), (8 * 4 * n * v - 1, False)):
         monkeypatch.setattr(K, "_free_device_bytes", lambda device: free)
         assert (held()[1] >= 4 * n * v) is kept
+
+
+@pytest.mark.parametrize("n,h,v", [(1, 128, 8), (65, 384, 257), (64, 128, 250), (200, 640, 300), (300, 256, 1031), (130, 896, 512)])
+@pytest.mark.parametrize("offset", [0, 4])          # elements: d_weight on an 8-byte boundary only
+def test_weight_gradient_stored_in_whole_lines(dev, n, h, v, offset):
+    """Stored in bf16 it is the same bits as added to zeros, at ragged vocabularies and hidden sizes that end in half a
+    tile, and nothing outside it is written."""
+    from verl_amd import _cabi
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    g = torch.Generator().manual_seed(n + h + v)
+    hidden = ((torch.rand(n, h, generator=g) - 0.5) * 2).bfloat16().to(dev)
+    weight = ((torch.rand(v, h, generator=g) - 0.5) * 0.2).bfloat16().to(dev)
+    labels = torch.randint(0, v, (n,), generator=g).to(dev)
+    d_logprobs = torch.randn(n, generator=g).to(dev)
+    _, _, lse, mean_z = K.efficient_entropy_forward(hidden, weight, labels)
+    want_h, want = K.efficient_entropy_backward(d_logprobs, None, hidden, weight, labels, lse, mean_z,
+                                                d_weight_out=torch.zeros(v, h, dtype=torch.bfloat16, device=dev))
+    guard = 64
+    buf = torch.full((guard + offset + v * h + guard,), 77.0, dtype=torch.bfloat16, device=dev)
+    out = buf[guard + offset:guard + offset + v * h].view(v, h)
+    d_hidden = torch.empty_like(hidden)
+    L = _cabi.lib()
+    size = L.vamd_lce_backward_workspace_bytes(n, h, v, 0)
+    ws = torch.empty(size, dtype=torch.uint8, device=dev)
+    P = lambda t: t.data_ptr()
+    _cabi.check(L.vamd_lce_backward(P(hidden), P(weight), P(labels), n, h, v, 1.0, P(lse), P(mean_z), P(d_logprobs), None, 0.0,
+                                    None, P(d_hidden), P(out), 0, None, 0, P(ws), size, _cabi.stream_ptr(hidden.device)))
+    assert torch.equal(out, want) and torch.equal(d_hidden, want_h)
+    assert (buf[:guard + offset] == 77).all() and (buf[guard + offset + v * h:] == 77).all()

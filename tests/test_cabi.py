@@ -270,3 +270,21 @@ def test_free_memory_that_may_hold_the_logits(monkeypatch):
         raise RuntimeError("no such query")
     monkeypatch.setattr(torch.cuda, "mem_get_info", refuse)
     assert K._free_device_bytes("cuda:0") == 0
+
+
+@pytest.mark.parametrize("name,at", [(name, at) for name, count in (("policy", 4), ("value", 4), ("kl", 3), ("agg", 2))
+                                     for at in range(count)])
+def test_losses_refuse_a_tangent_on_any_input(name, at):
+    """A dual tensor needs no ``requires_grad`` and carries its tangent under ``no_grad`` too; a loss returned without one
+    would read as a derivative of zero.  (Refused before a device is looked for.)"""
+    import torch.autograd.forward_ad as fwAD
+    from verl_amd.trainer.ppo import core_algos as CA
+    count, fn = {"policy": (4, lambda x, old, adv, mask: CA.compute_policy_loss(old, x, adv, mask, 0.2)),
+                 "value": (4, lambda v, ret, val, mask: CA.compute_value_loss(v, ret, val, mask, 0.5)),
+                 "kl": (3, CA.compute_kl_loss), "agg": (2, lambda x, mask: CA.agg_loss(x, mask, "token-mean"))}[name]
+    for grad_mode in (True, False):
+        with fwAD.dual_level(), torch.set_grad_enabled(grad_mode):
+            inputs = [torch.ones(2, 8) for _ in range(count)]
+            inputs[at] = fwAD.make_dual(inputs[at], torch.ones(2, 8))
+            with pytest.raises(NotImplementedError, match="forward mode"):
+                fn(*inputs)

@@ -120,6 +120,14 @@ Tensor ticket_workspace(size_t bytes, const at::Device& dev) {
 
 bool wants_gradient(const Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }
 
+// The losses have no forward-mode derivative.  Asked before the choice between a node and a plain call: a dual tensor needs
+// no requires_grad, and a loss without a tangent would read as a derivative of zero.
+void refuse_tangents(const char* loss, std::initializer_list<const Tensor*> inputs) {
+  for (const Tensor* t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), loss,
+                                " cannot be differentiated in forward mode");
+}
+
 struct Aggregation {
   int mode;
   double dp_size, batch_num_tokens, global_batch_size, loss_scale_factor;
@@ -219,6 +227,8 @@ std::pair<Tensor, Tensor> policy_loss(const Tensor& log_prob, const Tensor& old_
                                       double clip_high, double clip_c, int mode, double dp_size, double bnt, double gbs,
                                       double lsf, int variant, double tau_pos, double tau_neg) {
   const PolicyArgs a{variant, clip_low, clip_high, clip_c, tau_pos, tau_neg, {mode, dp_size, bnt, gbs, lsf}};
+  const Tensor weights = is_weights ? *is_weights : Tensor();
+  refuse_tangents("the policy loss", {&log_prob, &old_log_prob, &advantages, &mask, &weights});
   if (wants_gradient(log_prob)) {
     const auto r = PolicyLoss::apply(log_prob, old_log_prob, advantages, mask, is_weights, a);
     return {r[0], r[1]};
@@ -266,6 +276,7 @@ class ValueLoss : public torch::autograd::Function<ValueLoss> {
 // (loss, clip fraction)
 std::pair<Tensor, Tensor> value_loss(const Tensor& vpreds, const Tensor& returns, const Tensor& values,
                                      const Tensor& mask, double clip, int mode) {
+  refuse_tangents("the value loss", {&vpreds, &returns, &values, &mask});
   if (wants_gradient(vpreds)) {
     const auto r = ValueLoss::apply(vpreds, returns, values, mask, clip, mode);
     return {r[0], r[1].select(0, 1)};
@@ -318,6 +329,7 @@ class KlLoss : public torch::autograd::Function<KlLoss> {
 Tensor kl_loss(const Tensor& logprob, const Tensor& ref_logprob, const Tensor& mask, int kind, bool straight_through,
                int mode, double dp_size, double bnt, double gbs, double lsf) {
   const KlArgs a{kind, straight_through, {mode, dp_size, bnt, gbs, lsf}};
+  refuse_tangents("the KL loss", {&logprob, &ref_logprob, &mask});
   if (wants_gradient(logprob) || wants_gradient(ref_logprob)) return KlLoss::apply(logprob, ref_logprob, mask, a);
   return kl_forward(logprob, ref_logprob, mask, a, false).loss;
 }
@@ -372,6 +384,7 @@ class AggLoss : public torch::autograd::Function<AggLoss> {
 Tensor agg_loss(const Tensor& loss_mat, const Tensor& mask, int mode, double dp_size, double bnt, double gbs,
                 double lsf) {
   const Aggregation a{mode, dp_size, bnt, gbs, lsf};
+  refuse_tangents("agg_loss", {&loss_mat, &mask});
   if (wants_gradient(loss_mat) || wants_gradient(mask)) return AggLoss::apply(loss_mat, mask, a);
   return agg_forward(loss_mat, mask, a).loss;
 }

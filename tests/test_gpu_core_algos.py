@@ -2183,3 +2183,35 @@ def test_native_loss_nodes_in_autograd(dev, name):
         fn(fwAD.make_dual(x, torch.ones_like(x)))
     with pytest.raises(RuntimeError):
         torch.vmap(fn)(x.detach()[None].expand(2, *shape))
+
+
+@pytest.mark.parametrize("name", ["policy", "value", "kl", "agg"])
+def test_native_losses_may_be_changed_in_place(dev, name):
+    """A loss is a tensor of its own: scaled or added to in place it stays differentiable, and changing the detached loss
+    (a mean over ranks for the log) leaves what its node has saved alone."""
+    shape, losses = _native_losses(dev)
+    fn = losses[name]
+    for where in (dev, torch.device("cpu")):
+        x = torch.randn(shape, device=dev).to(where).requires_grad_()
+        plain = fn(x)
+        value = plain.item()
+        (want,) = torch.autograd.grad(plain, x)
+        loss = fn(x)
+        loss *= 2.0
+        loss += 1.0
+        assert loss.item() == pytest.approx(2.0 * value + 1.0, rel=1e-6)
+        assert torch.equal(torch.autograd.grad(loss, x)[0], 2.0 * want)      # a power of two: the same bits
+        loss = fn(x)
+        loss.detach().mul_(3.0)
+        assert torch.equal(torch.autograd.grad(loss, x)[0], want)
+        loss = fn(x)
+        loss.unsqueeze_(0)
+        assert loss.shape == (1,)
+        # without a gradient: a term that requires one is added in place, with grad mode on again
+        term = torch.ones((), device=where, requires_grad=True)
+        with torch.no_grad():
+            under = fn(x)
+        for loss in (fn(x.detach()), under):
+            assert not loss.requires_grad
+            loss += term
+            assert torch.autograd.grad(loss, term)[0].item() == 1.0 and loss.item() == pytest.approx(value + 1.0, rel=1e-6)

@@ -104,6 +104,17 @@ Tensor new_f32(at::IntArrayRef shape, const at::Device& dev) {
   return at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(dev));
 }
 
+// Parts of a call's one result allocation as tensors of their own, not views of it to autograd: a loss may be changed in place
+// (`loss /= n`, `loss.detach().mul_(s)`), and the version of what a node has saved is not that of the loss beside it.
+Tensor part(const Tensor& t, int64_t first, int64_t count) {
+  at::AutoDispatchBelowADInplaceOrView no_view;
+  return t.narrow(0, first, count);
+}
+Tensor scalar_part(const Tensor& t, int64_t i) {
+  at::AutoDispatchBelowADInplaceOrView no_view;
+  return t.select(0, i);
+}
+
 // Scratch of the single-launch reductions: its first VAMD_TICKET_BYTES are arrival counters that are zero on entry and
 // zero again on completion, so one zeroed buffer per (device, stream) is kept; kernels on one stream run in order and
 // never share it.  Never destroyed: at exit the runtime may be gone first.
@@ -191,7 +202,7 @@ LossResult policy_forward(const Tensor& log_prob, const Tensor& old_log_prob, co
   const int64_t rows = lp.size(0), cols = lp.size(1);
   const c10::DeviceGuard guard(dev);
   // one allocation for the four result floats and the per-row coefficients (16-byte aligned both)
-  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 4), coef = buf.narrow(0, 4, rows);
+  const Tensor buf = new_f32({4 + rows}, dev), out = part(buf, 0, 4), coef = part(buf, 4, rows);
   const Tensor g = need_grad ? at::empty_like(lp) : Tensor();
   const Tensor ws = ticket_workspace(vamd_policy_loss_variant_workspace_bytes(rows, cols), dev);
   check(vamd_policy_loss_variant_forward(a.variant, f32(old), f32(lp), f32(adv), m.t.const_data_ptr(), m.code, f32(isw),
@@ -200,9 +211,9 @@ LossResult policy_forward(const Tensor& log_prob, const Tensor& old_log_prob, co
                                          a.agg.batch_num_tokens, a.agg.global_batch_size, a.agg.loss_scale_factor,
                                          f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(), ws.numel(),
                                          stream_of(dev)));
-  // the loss is a view: it shares the floats the kernel wrote with the metrics
+  // the loss shares the floats the kernel wrote with the metrics
   const Tensor result = log_prob.device() == dev ? out : out.to(log_prob.device());
-  return {result.select(0, 0), result, g, coef, dev};
+  return {scalar_part(result, 0), result, g, coef, dev};
 }
 
 class PolicyLoss : public torch::autograd::Function<PolicyLoss> {
@@ -247,14 +258,14 @@ LossResult value_forward(const Tensor& vpreds, const Tensor& returns, const Tens
   const Mask m = mask_matrix(mask, dev, vp);
   const int64_t rows = vp.size(0), cols = vp.size(1);
   const c10::DeviceGuard guard(dev);
-  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 2), coef = buf.narrow(0, 4, rows);
+  const Tensor buf = new_f32({4 + rows}, dev), out = part(buf, 0, 2), coef = part(buf, 4, rows);
   const Tensor g = need_grad ? at::empty_like(vp) : Tensor();
   const Tensor ws = ticket_workspace(vamd_value_loss_workspace_bytes(rows, cols), dev);
   check(vamd_value_loss_forward(f32(vp), f32(ret), f32(val), m.t.const_data_ptr(), m.code, rows, cols, (float)clip, mode,
                                 f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(), ws.numel(),
                                 stream_of(dev)));
   const Tensor result = vpreds.device() == dev ? out : out.to(vpreds.device());
-  return {result.select(0, 0), result, g, coef, dev};
+  return {scalar_part(result, 0), result, g, coef, dev};
 }
 
 class ValueLoss : public torch::autograd::Function<ValueLoss> {
@@ -299,15 +310,14 @@ LossResult kl_forward(const Tensor& logprob, const Tensor& ref_logprob, const Te
   const Mask m = mask_matrix(mask, dev, lp);
   const int64_t rows = lp.size(0), cols = lp.size(1);
   const c10::DeviceGuard guard(dev);
-  const Tensor buf = new_f32({4 + rows}, dev), out = buf.narrow(0, 0, 1), coef = buf.narrow(0, 4, rows);
+  const Tensor buf = new_f32({4 + rows}, dev), out = scalar_part(buf, 0), coef = part(buf, 4, rows);
   const Tensor g = need_grad ? at::empty_like(lp) : Tensor();
   const Tensor ws = ticket_workspace(vamd_kl_loss_workspace_bytes(rows, cols), dev);
   check(vamd_kl_loss_forward(f32(lp), f32(ref), m.t.const_data_ptr(), m.code, rows, cols, a.kind, a.straight_through,
                              a.agg.mode, a.agg.dp_size, a.agg.batch_num_tokens, a.agg.global_batch_size,
                              a.agg.loss_scale_factor, f32_out(out), f32_out(g), f32_out(coef), ws.mutable_data_ptr(),
                              ws.numel(), stream_of(dev)));
-  const Tensor loss = out.select(0, 0);
-  return {logprob.device() == dev ? loss : loss.to(logprob.device()), Tensor(), g, coef, dev};
+  return {logprob.device() == dev ? out : out.to(logprob.device()), Tensor(), g, coef, dev};
 }
 
 class KlLoss : public torch::autograd::Function<KlLoss> {
@@ -347,7 +357,7 @@ AggResult agg_forward(const Tensor& loss_mat, const Tensor& mask, const Aggregat
   const Mask m = mask_matrix(mask, dev, x);
   const int64_t rows = x.size(0), cols = x.size(1);
   const c10::DeviceGuard guard(dev);
-  const Tensor buf = new_f32({4 + rows}, dev), out = buf.select(0, 0), coef = buf.narrow(0, 4, rows);
+  const Tensor buf = new_f32({4 + rows}, dev), out = scalar_part(buf, 0), coef = part(buf, 4, rows);
   const Tensor ws = ticket_workspace(vamd_agg_loss_workspace_bytes(rows, cols), dev);
   check(vamd_agg_loss_forward(f32(x), m.t.const_data_ptr(), m.code, rows, cols, a.mode, a.dp_size, a.batch_num_tokens,
                               a.global_batch_size, a.loss_scale_factor, f32_out(out), f32_out(coef),

@@ -2215,3 +2215,18 @@ def test_native_losses_may_be_changed_in_place(dev, name):
             assert not loss.requires_grad
             loss += term
             assert torch.autograd.grad(loss, term)[0].item() == 1.0 and loss.item() == pytest.approx(value + 1.0, rel=1e-6)
+
+
+@pytest.mark.parametrize("requires_grad", [True, False])
+@pytest.mark.parametrize("name", ["policy", "value", "kl", "agg"])
+def test_native_losses_traced(dev, name, requires_grad):
+    """A traced program computes the loss, and its gradient, of the inputs it is run on."""
+    shape, losses = _native_losses(dev)
+    fn = losses[name]
+    traced = torch.jit.trace(fn, (torch.randn(shape, device=dev).requires_grad_(requires_grad),), check_trace=False)
+    for _ in range(2):
+        x = torch.randn(shape, device=dev).requires_grad_(requires_grad)
+        got, want = traced(x), fn(x)
+        assert torch.equal(got, want) and got.requires_grad == requires_grad
+        if requires_grad:
+            assert torch.equal(torch.autograd.grad(got * 2.0, x)[0], torch.autograd.grad(want * 2.0, x)[0])

@@ -518,6 +518,36 @@ def _opt(x) -> float:
     return float(x.item()) if isinstance(x, torch.Tensor) else float(x)
 
 
+class _TracedLoss(torch.autograd.Function):
+    """A native loss while ``torch.jit.trace`` records: one Python operation, which a traced program runs on its own
+    inputs.  Called as outside a trace, the loss would leave its result's allocation in the recording and nothing of the
+    library call that fills it."""
+
+    @staticmethod
+    def forward(ctx, name, x, *rest):
+        with torch.enable_grad():
+            ctx.x = x.detach().requires_grad_(ctx.needs_input_grad[1])
+            result = getattr(_cabi.ops(), name)(ctx.x, *rest)
+        ctx.loss, *others = result if isinstance(result, tuple) else (result,)
+        ctx.mark_non_differentiable(*others)
+        ctx.rest = len(rest)
+        loss = ctx.loss.detach().clone()
+        return (loss, *others) if others else loss
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, d_loss, *_):
+        d = torch.autograd.grad(ctx.loss, ctx.x, d_loss, retain_graph=True)[0] if ctx.needs_input_grad[1] else None
+        return (None, d) + (None,) * ctx.rest
+
+
+def _native_loss(name: str, x: torch.Tensor, *rest):
+    """The loss ``name`` of the native host side, differentiable with respect to ``x``."""
+    if torch._C._get_tracing_state() is not None:
+        return _TracedLoss.apply(name, x, *rest)
+    return getattr(_cabi.ops(), name)(x, *rest)
+
+
 def agg_loss(loss_mat: torch.Tensor, loss_mask: torch.Tensor, loss_agg_mode: str, dp_size: int = 1,
              batch_num_tokens: Optional[int] = None, global_batch_size: Optional[int] = None,
              loss_scale_factor: Optional[int] = None):
@@ -526,20 +556,19 @@ def agg_loss(loss_mat: torch.Tensor, loss_mask: torch.Tensor, loss_agg_mode: str
     ``seq-mean-token-sum-norm``; any other mode raises ``ValueError``.  Differentiable with
     respect to ``loss_mat``."""
     mode = _agg_mode(loss_agg_mode)
-    return _cabi.ops().agg_loss(loss_mat, loss_mask, mode, float(dp_size), _opt(batch_num_tokens),
-                                _opt(global_batch_size), _opt(loss_scale_factor))
+    return _native_loss("agg_loss", loss_mat, loss_mask, mode, float(dp_size), _opt(batch_num_tokens),
+                        _opt(global_batch_size), _opt(loss_scale_factor))
 
 
 # ---------------------------------------------------------------------------------------------
 def _policy_loss(log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low, clip_high, clip_c, mode, dp_size,
                  bnt, gbs, lsf, variant=0, tau_pos=1.0, tau_neg=1.0):
     """``(loss, metrics)`` of one policy loss; the metrics as Python floats, which is the one wait for the GPU."""
-    ops = _cabi.ops()
-    pg_loss, out = ops.policy_loss(log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low, clip_high,
-                                   clip_c, mode, dp_size, bnt, gbs, lsf, variant, tau_pos, tau_neg)
+    pg_loss, out = _native_loss("policy_loss", log_prob, old_log_prob, advantages, response_mask, is_weights, clip_low,
+                                clip_high, clip_c, mode, dp_size, bnt, gbs, lsf, variant, tau_pos, tau_neg)
     if variant in (_PL["gspo"], _PL["geo_mean"]):
         _watch_waiting_kernels(_cabi.ticket_workspace(0, out.device if out.is_cuda else _cabi.compute_device(out)))
-    vals = ops.fetch(out)
+    vals = _cabi.ops().fetch(out)
     return pg_loss, {"actor/pg_clipfrac": vals[1], "actor/ppo_kl": vals[2], "actor/pg_clipfrac_lower": vals[3]}
 
 
@@ -853,9 +882,9 @@ def compute_policy_loss(old_log_prob, log_prob, advantages, response_mask, clipr
         cliprange_low = cliprange
     if cliprange_high is None:
         cliprange_high = cliprange
-    pg_loss, out = _cabi.ops().policy_loss(log_prob, old_log_prob, advantages, response_mask, None, float(cliprange_low),
-                                           float(cliprange_high), float(clip_ratio_c), _agg_mode(loss_agg_mode), 1.0,
-                                           -1.0, -1.0, -1.0, _PL["vanilla"], 1.0, 1.0)
+    pg_loss, out = _native_loss("policy_loss", log_prob, old_log_prob, advantages, response_mask, None,
+                                float(cliprange_low), float(cliprange_high), float(clip_ratio_c),
+                                _agg_mode(loss_agg_mode), 1.0, -1.0, -1.0, -1.0, _PL["vanilla"], 1.0, 1.0)
     return pg_loss, out[1], out[2], out[3]
 
 
@@ -864,8 +893,8 @@ def compute_value_loss(vpreds: torch.Tensor, returns: torch.Tensor, values: torc
                        response_mask: torch.Tensor, cliprange_value: float, loss_agg_mode: str = "token-mean"):
     """Clipped value loss (reference core_algos.py:1799-1838): returns ``(vf_loss, vf_clipfrac)``,
     ``vf_loss`` differentiable with respect to ``vpreds``."""
-    return _cabi.ops().value_loss(vpreds, returns, values, response_mask, float(cliprange_value),
-                                  _agg_mode(loss_agg_mode))
+    return _native_loss("value_loss", vpreds, returns, values, response_mask, float(cliprange_value),
+                        _agg_mode(loss_agg_mode))
 
 
 # ---- PF-PPO data reweighting -----------------------------------------------------------------------
@@ -983,9 +1012,9 @@ def compute_kl_loss(logprob: torch.Tensor, ref_logprob: torch.Tensor, response_m
     single function of the reference does both steps; this one exists so that the pair costs one
     read of the inputs.  ``straight_through=True`` keeps the estimator's value and uses the k2
     gradient, the behaviour the reference documents for the ``"+"`` names."""
-    return _cabi.ops().kl_loss(logprob, ref_logprob, response_mask, _kl_kind(kl_penalty), bool(straight_through),
-                               _agg_mode(loss_agg_mode), float(dp_size), _opt(batch_num_tokens), _opt(global_batch_size),
-                               _opt(loss_scale_factor))
+    return _native_loss("kl_loss", logprob, ref_logprob, response_mask, _kl_kind(kl_penalty), bool(straight_through),
+                        _agg_mode(loss_agg_mode), float(dp_size), _opt(batch_num_tokens), _opt(global_batch_size),
+                        _opt(loss_scale_factor))
 
 
 def kl_penalised_rewards(token_level_scores: torch.Tensor, old_log_probs: torch.Tensor, ref_log_prob: torch.Tensor,

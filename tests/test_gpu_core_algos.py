@@ -1744,6 +1744,69 @@ def test_losses_whose_workgroups_walk_several_chunks(dev, shape, agg):
         assert err <= 4e-6 * wd.abs().max().item(), err
 
 
+# aligned and unaligned rows, below the size from which launches stream past the caches and from it on
+@pytest.mark.parametrize("shape", [(2304, 8), (2100, 4099), (4200, 9), (4200, 12)])
+@pytest.mark.parametrize("mask_dtype", [torch.float32, torch.int64, torch.bool])
+@pytest.mark.parametrize("name", ["vanilla", "cispo", "gspo", "geo_mean", "value", "kl"])
+def test_large_launches_that_walk_and_that_do_not(dev, monkeypatch, name, mask_dtype, shape):
+    """More chunks than a launch folds records of, in the modes that want its totals: which kernels walk depends on loss, mask
+    type, gradient, alignment and importance weights.  Against the oracle's mathematics in fp64 on the device."""
+    import oracle.losses as OL
+    from verl_amd import _cabi
+    from verl_amd.trainer.ppo import core_algos as CA
+    B, L = shape
+    g = torch.Generator(device=dev).manual_seed(B + L)
+    randn = lambda: torch.randn(B, L, device=dev, generator=g)
+    old, a, b = randn() * 0.5 - 1, randn(), randn()
+    x = old + randn() * 0.2
+    mask = torch.rand(B, L, device=dev, generator=g) < 0.8
+    mask[:, 0] = True
+    m, w64 = mask.to(mask_dtype), mask.double()
+    weights = torch.rand(B, L, device=dev, generator=g) + 0.5 if name not in ("value", "kl") else None
+    # the mode of GSPO is fixed in Python, not in the library
+    plain = OL.agg_loss
+    monkeypatch.setattr(OL, "agg_loss", lambda mat, mk, mode, **kw: plain(mat, mk, "token-mean"))
+
+    def native(x, weights):
+        if name == "value":
+            return CA.compute_value_loss(x, a, b, m, 0.5)
+        if name == "kl":
+            return CA.compute_kl_loss(x, old, m), None
+        loss, out = _cabi.ops().policy_loss(x, old, a, m, weights, 0.2, 0.28, 3.0, _cabi.AGG_MODES["token-mean"], 1.0, -1.0,
+                                            -1.0, -1.0, CA._PL[name], 1.0, 1.0)
+        return loss, out[1]
+
+    def wanted(x, weights):
+        args = (old.double(), x, a.double(), w64)
+        w = None if weights is None else weights.double()
+        if name == "value":
+            return OL.value_loss(x, a.double(), b.double(), w64, 0.5)
+        if name == "kl":
+            return OL.agg_loss(OL.kl_penalty(x, old.double(), "k3"), w64, "token-mean"), None
+        if name == "vanilla":
+            return OL.policy_loss_vanilla(*args, "token-mean", 0.2, 0.28, 3.0, w)[:2]
+        if name == "cispo":
+            return OL.policy_loss_cispo(*args, "token-mean", 0.2, 0.28, w)[:2]
+        return getattr(OL, "policy_loss_" + name)(*args, 0.2, 0.28, w)[:2]
+
+    for wts in {id(weights): weights, id(None): None}.values():
+        xd = x.double().requires_grad_()
+        want, share = wanted(xd, wts)
+        (wd,) = torch.autograd.grad(want, xd)
+        xg = x.clone().requires_grad_()
+        loss, got_share = native(xg, wts)
+        (gd,) = torch.autograd.grad(loss, xg)
+        quiet, _ = native(x, wts)
+        # fp32 per token and for the sixteen tokens of a thread, fp64 sums: terms of magnitude 1 to 2^-20
+        assert abs(loss.item() - want.item()) <= 2e-6 and abs(quiet.item() - want.item()) <= 2e-6, (loss, quiet, want)
+        if share is not None:   # tokens whose fp32 ratio falls on the other side of a bound: a few in 10^7
+            assert abs(got_share.item() - share.item()) <= 1e-5
+        # The clip bounds are compared in fp32: such a token takes the other branch's gradient.  All others agree to the 8 ulp
+        # of an exponential of a sum of up to 4099 terms.
+        off = (gd.double() - wd).abs() > 4e-6 * wd.abs().max()
+        assert off.double().mean().item() <= 1e-5 and not gd[~mask].any()
+
+
 @pytest.mark.parametrize("rows", [63, 64, 65, 129, 16385])   # a row per lane, 64 per workgroup, 256 workgroups, then a second trip
 def test_statistics_fold_edges(dev, rows):
     test_data_metrics(dev, (rows, 9), 4, torch.int64, True)

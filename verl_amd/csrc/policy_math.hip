@@ -20,32 +20,43 @@ struct Work {
   int totals;        // loss kernels built without the fold: take the launch totals here (totals_epilogue)
 };
 
-// A workgroup of the policy, value and KL losses takes the (row, chunk) items b, b + gridDim.x, ...  One each where the per-row sums are needed or
-// the launch is small; where the launch totals are all that is wanted, a large launch has as many workgroups as the device
-// holds at once (loss_grid), so that the workgroup reduction, the record and the arrival, during which a workgroup's registers
-// stream nothing, come once per workgroup and not once per item.  1000 x 11999 (3000 items) with an int64 mask: policy loss
-// with gradient 64.6 -> 57.3 us, KL loss with gradient 46.9 -> 43.2; 760 x 11999 fp32: 42.9 -> 38.7, 30.7 -> 28.3; 2048 x 16384
-// bool (8192 items): KL loss 84.5 -> 78.2.  The policy and value losses walk only in launches that do not stream past the
-// caches (and where rows are not aligned): 2048 x 16384 takes 115.5 us walking, 112.8 with a workgroup per item.  agg_loss,
-// whose workgroups are light enough for eight to a CU, does not: with the loop 1000 x 11999 took 29.7 us, without it 28.0.
-__device__ __forceinline__ bool walks_several(int64_t rows, int chunks) { return (int64_t)gridDim.x != rows * chunks; }
-template <int NV>
-__device__ __forceinline__ void store_loss_record(const Work& wk, unsigned item, int64_t rows, int chunks,
-                                                  const double (&acc)[NV]) {
-  if (walks_several(rows, chunks)) store_record<NV>(wk.partials, blockIdx.x, 0, gridDim.x, 1, acc);
-  else store_record<NV>(wk.partials, item / (unsigned)chunks, (int)(item % (unsigned)chunks), rows, chunks, acc);
+// Policy, value and KL losses: the (row, chunk) items of a workgroup.  One, its own; or, in a kernel built to LOOP, the items
+// b, b + gridDim.x, ...: a large launch that wants nothing but the launch totals then has as many workgroups as the device
+// holds at once (walking_grid), and the workgroup reduction, the record and the arrival, during which a workgroup's registers
+// stream nothing, come once per workgroup and not once per item.  Kernels of their own: the loop in every kernel cost small
+// launches 3 to 8 % (512 x 4096 fp32 mask, with gradient: policy loss 14.4 -> 15.0 us, GSPO 15.8 -> 17.0).  agg_loss, whose
+// workgroups are light enough for eight to a CU, does not walk: with the loop 1000 x 11999 took 29.7 us, without it 28.0.
+template <bool LOOP>
+struct OwnItems {
+  unsigned items;  // of the launch
+  int chunks;
+  bool streaming;
+  __device__ __forceinline__ OwnItems(int64_t rows, int chunks_)
+      : items((unsigned)(rows * chunks_)), chunks(chunks_), streaming(LOOP ? items >= kStreamingGrid : launch_streams_past_caches()) {}
+  __device__ __forceinline__ bool more(unsigned item) const { return !LOOP || item < items; }
+  __device__ __forceinline__ int64_t row(unsigned item) const { return item / (unsigned)chunks; }
+  __device__ __forceinline__ int chunk(unsigned item) const { return (int)(item % (unsigned)chunks); }
+};
+template <bool LOOP>
+__device__ __forceinline__ bool walks_several(int64_t rows, int chunks) {
+  return LOOP && (int64_t)gridDim.x != rows * chunks;
+}
+template <bool LOOP, int NV>
+__device__ __forceinline__ void store_loss_record(const Work& wk, int64_t rows, int chunks, const double (&acc)[NV]) {
+  if (walks_several<LOOP>(rows, chunks)) store_record<NV>(wk.partials, blockIdx.x, 0, gridDim.x, 1, acc);
+  else store_record<NV>(wk.partials, blockIdx.x / chunks, (int)(blockIdx.x % chunks), rows, chunks, acc);
 }
 
 // The loss kernels of a large launch carry no fold of their own (FOLD = false).  Two of the four agg_loss modes,
 // token-mean and seq-mean-token-sum-norm, need nothing but the launch totals, and those come cheaply in two
 // levels (sum_all_records: a few dozen registers, no per-row pass), so such a launch finishes here; the per-row
 // modes leave their records to fold_loss_kernel.  Same formulas as finalize_agg.
-template <int NV, int EPI>
+template <int NV, int EPI, bool LOOP = false>
 __device__ __forceinline__ void totals_epilogue(const Work& wk, int64_t rows, int chunks, int64_t cols,
                                                 const AggParams& ap, float* __restrict__ coef,
                                                 float* __restrict__ out, double* smem) {
   double tot[NV];
-  const bool walks = walks_several(rows, chunks);
+  const bool walks = walks_several<LOOP>(rows, chunks);
   if (!sum_all_records<NV>(wk.ticket, wk.partials, walks ? (int64_t)gridDim.x : rows, walks ? 1 : chunks, tot, smem)) return;
   __shared__ float c_all;
   if (threadIdx.x == 0) {
@@ -70,13 +81,10 @@ __device__ __forceinline__ void totals_epilogue(const Work& wk, int64_t rows, in
     for (int64_t r = threadIdx.x; r < rows; r += kRcThreads) coef[r] = c_all;
   ticket_reset(wk.ticket);
 }
-// Workgroups of a loss launch; per_cu: how many of the kernel a CU holds (measured one less and one more as well: policy loss
-// at 1000 x 11999 62.6, 59.0, 68.3 us with 2, 3, 4; KL loss 44.6, 42.5, 42.4 with 3, 4, 5).
-inline unsigned loss_grid(int64_t items, bool walks, int per_cu) {
-  const int64_t resident = (int64_t)device_cu_count() * per_cu;
-  return (unsigned)(walks && items > kInlineFoldRecords ? balanced_waiting_grid(items, resident) : items);
+// Workgroups of a loss launch that walks: as many as the device holds of this kernel, each with the same number of items.
+inline unsigned walking_grid(int64_t items, const void* kernel) {
+  return (unsigned)balanced_waiting_grid(items, resident_workgroups(kernel, kRcThreads));
 }
-constexpr int kPolicyPerCu = 3, kValuePerCu = 3, kKlPerCu = 4;
 __host__ __device__ inline bool totals_suffice(int mode) {
   return mode == VAMD_AGG_TOKEN_MEAN || mode == VAMD_AGG_SEQ_MEAN_TOKEN_SUM_NORM;
 }
@@ -510,7 +518,7 @@ __global__ __launch_bounds__(kRcThreads) void geo_rows_kernel(const float* __res
 // have the neighbouring ids and start together with it.  A workgroup whose wait ran out computes the missing chunks'
 // sums itself, to the same bits, so the result does not depend on what the device lets run at the same time.  The
 // launch's last workgroup clears the ready bytes (ROWS launches always fold their own records).
-template <bool VEC, class M, bool GRAD, bool ISW, bool FOLD, int VARIANT, bool ROWS = false>
+template <bool VEC, class M, bool GRAD, bool ISW, bool FOLD, int VARIANT, bool ROWS = false, bool LOOP = false>
 __global__ __launch_bounds__(kRcThreads) void policy_kernel(
     const float* __restrict__ old_lp, const float* __restrict__ lp, const float* __restrict__ adv,
     const M* __restrict__ mask, const float* __restrict__ isw, int64_t rows, int64_t cols, int chunks,
@@ -519,12 +527,13 @@ __global__ __launch_bounds__(kRcThreads) void policy_kernel(
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
   const int variant = VARIANT >= 0 ? VARIANT : pp.variant;
   __shared__ double smem[(5 + 3) * 4];
-  const unsigned items = (unsigned)(rows * chunks);
-  const bool streaming = items >= kStreamingGrid;
+  __shared__ double row_sums[4];  // ROWS
   double acc[5] = {0, 0, 0, 0, 0};
-  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
-    const int64_t row = item / (unsigned)chunks;
-    const int chunk = (int)(item % (unsigned)chunks);
+  const OwnItems<LOOP> own_items(rows, chunks);
+  const bool streaming = own_items.streaming;
+  for (unsigned item = blockIdx.x; own_items.more(item); item += gridDim.x) {
+    const int64_t row = own_items.row(item);
+    const int chunk = own_items.chunk(item);
     const ChunkPos pos(row, chunk, cols);
     float o[kGroups][4], n[kGroups][4], a[kGroups][4], w[kGroups][4], iw[kGroups][4], gr[kGroups][4];
     load_groups<VEC>(old_lp, pos, o, streaming);
@@ -535,7 +544,6 @@ __global__ __launch_bounds__(kRcThreads) void policy_kernel(
     float seq_lr = 0.f;
     double r[4] = {0, 0, 0, 0};  // the row's four sums (GSPO, GEO_MEAN)
     if constexpr (ROWS) {
-      __shared__ double row_sums[4];
       double own[4];
       row_presums<ISW>(variant, pos, o, n, a, w, iw, pp.nkl_lo, pp.nkl_hi, own);
       block_sum<4, kRcThreads>(own, smem);  // valid in thread 0
@@ -640,14 +648,14 @@ __global__ __launch_bounds__(kRcThreads) void policy_kernel(
     acc[2] += (double)s_kl;
     acc[3] += (double)s_cf;
     acc[4] += (double)s_cfl;
-    if constexpr (!FOLD) break;  // one item per workgroup
+    if constexpr (!LOOP) break;
   }
-  static_assert(!ROWS || FOLD, "a launch that sets ready bytes has a last workgroup that clears them");
+  static_assert(!ROWS || (FOLD && !LOOP), "a launch that sets ready bytes has a last workgroup that clears them");
   block_sum<5, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) store_loss_record<5>(wk, blockIdx.x, rows, chunks, acc);
+  if (threadIdx.x == 0) store_loss_record<LOOP>(wk, rows, chunks, acc);
   if constexpr (FOLD) {
     if (!ROWS && totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
-      totals_epilogue<5, kEpiPolicy>(wk, rows, chunks, cols, ap, coef, out, smem);
+      totals_epilogue<5, kEpiPolicy, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
       return;
     }
     if (!last_block_arrives(wk.ticket)) return;
@@ -657,7 +665,7 @@ __global__ __launch_bounds__(kRcThreads) void policy_kernel(
     ticket_reset(wk.ticket);
     if (ROWS && chunks > 1) ready_bytes_clear<kRcThreads>(wk.ticket, rows * chunks);
   } else {
-    if (wk.totals) totals_epilogue<5, kEpiPolicy>(wk, rows, chunks, cols, ap, coef, out, smem);
+    if (wk.totals) totals_epilogue<5, kEpiPolicy, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
   }
 }
 
@@ -733,17 +741,19 @@ __global__ __launch_bounds__(kWholeRowThreads) void policy_whole_row_kernel(
 // =============================================================================================
 // value loss (compute_value_loss, core_algos.py:1799-1838)
 // =============================================================================================
-template <bool VEC, class M, bool GRAD, bool FOLD>
+template <bool VEC, class M, bool GRAD, bool FOLD, bool LOOP>
 __global__ __launch_bounds__(kRcThreads) void value_kernel(
     const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
     const M* __restrict__ mask, int64_t rows, int64_t cols, int chunks, float clip, AggParams ap, Work wk,
     float* __restrict__ out, float* __restrict__ grad, float* __restrict__ coef) {
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
-  const unsigned items = (unsigned)(rows * chunks);
-  const bool streaming = items >= kStreamingGrid;
   double acc[3] = {0, 0, 0};
-  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
-    const ChunkPos pos(item / (unsigned)chunks, (int)(item % (unsigned)chunks), cols);
+  const OwnItems<LOOP> own_items(rows, chunks);
+  const bool streaming = own_items.streaming;
+  for (unsigned item = blockIdx.x; own_items.more(item); item += gridDim.x) {
+    const int64_t row = own_items.row(item);
+    const int chunk = own_items.chunk(item);
+    const ChunkPos pos(row, chunk, cols);
     float vp[kGroups][4], R[kGroups][4], v[kGroups][4], w[kGroups][4], gr[kGroups][4];
     load_groups<VEC>(vpreds, pos, vp, streaming);
     load_groups<VEC>(returns, pos, R, streaming);
@@ -779,14 +789,14 @@ __global__ __launch_bounds__(kRcThreads) void value_kernel(
     acc[0] += (double)s_loss;
     acc[1] += (double)s_m;
     acc[2] += (double)s_cf;
-    if constexpr (!FOLD) break;  // one item per workgroup
+    if constexpr (!LOOP) break;
   }
   __shared__ double smem[(3 + 3) * 4];
   block_sum<3, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) store_loss_record<3>(wk, blockIdx.x, rows, chunks, acc);
+  if (threadIdx.x == 0) store_loss_record<LOOP>(wk, rows, chunks, acc);
   if constexpr (FOLD) {
     if (totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
-      totals_epilogue<3, kEpiValue>(wk, rows, chunks, cols, ap, coef, out, smem);
+      totals_epilogue<3, kEpiValue, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
       return;
     }
     if (!last_block_arrives(wk.ticket)) return;
@@ -795,7 +805,7 @@ __global__ __launch_bounds__(kRcThreads) void value_kernel(
     if (threadIdx.x == 0) loss_epilogue<kEpiValue>(loss, msum, extra, out);
     ticket_reset(wk.ticket);
   } else {
-    if (wk.totals) totals_epilogue<3, kEpiValue>(wk, rows, chunks, cols, ap, coef, out, smem);
+    if (wk.totals) totals_epilogue<3, kEpiValue, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
   }
 }
 
@@ -859,17 +869,19 @@ __global__ __launch_bounds__(256) void kl_elementwise_kernel(const float* __rest
 
 // agg_loss(kl_penalty(logprob, ref), mask, mode) in one pass, with the per-element gradient
 // (times the mask weight, before the per-row agg_loss coefficient) on request.
-template <bool VEC, class M, bool GRAD, bool FOLD>
+template <bool VEC, class M, bool GRAD, bool FOLD, bool LOOP>
 __global__ __launch_bounds__(kRcThreads) void kl_loss_kernel(
     const float* __restrict__ logprob, const float* __restrict__ ref, const M* __restrict__ mask, int64_t rows,
     int64_t cols, int chunks, int kind, int straight, AggParams ap, Work wk, float* __restrict__ out,
     float* __restrict__ grad, float* __restrict__ coef) {
   const bool token_mean = ap.mode == VAMD_AGG_TOKEN_MEAN;
-  const unsigned items = (unsigned)(rows * chunks);
-  const bool streaming = items >= kStreamingGrid;
   double acc[2] = {0, 0};
-  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
-    const ChunkPos pos(item / (unsigned)chunks, (int)(item % (unsigned)chunks), cols);
+  const OwnItems<LOOP> own_items(rows, chunks);
+  const bool streaming = own_items.streaming;
+  for (unsigned item = blockIdx.x; own_items.more(item); item += gridDim.x) {
+    const int64_t row = own_items.row(item);
+    const int chunk = own_items.chunk(item);
+    const ChunkPos pos(row, chunk, cols);
     float lp[kGroups][4], rf[kGroups][4], w[kGroups][4], gr[kGroups][4];
     load_groups<VEC>(logprob, pos, lp, streaming);
     load_groups<VEC>(ref, pos, rf, streaming);
@@ -894,13 +906,14 @@ __global__ __launch_bounds__(kRcThreads) void kl_loss_kernel(
     if (GRAD) store_groups<VEC>(grad, pos, gr, streaming);
     acc[0] += (double)s_loss;
     acc[1] += (double)s_m;
+    if constexpr (!LOOP) break;
   }
   __shared__ double smem[(2 + 3) * 4];
   block_sum<2, kRcThreads>(acc, smem);
-  if (threadIdx.x == 0) store_loss_record<2>(wk, blockIdx.x, rows, chunks, acc);
+  if (threadIdx.x == 0) store_loss_record<LOOP>(wk, rows, chunks, acc);
   if constexpr (FOLD) {
     if (totals_suffice(ap.mode)) {  // no per-row pass: the launch totals are all these modes need
-      totals_epilogue<2, kEpiKl>(wk, rows, chunks, cols, ap, coef, out, smem);
+      totals_epilogue<2, kEpiKl, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
       return;
     }
     if (!last_block_arrives(wk.ticket)) return;
@@ -909,7 +922,7 @@ __global__ __launch_bounds__(kRcThreads) void kl_loss_kernel(
     if (threadIdx.x == 0) loss_epilogue<kEpiKl>(loss, msum, extra, out);
     ticket_reset(wk.ticket);
   } else {
-    if (wk.totals) totals_epilogue<2, kEpiKl>(wk, rows, chunks, cols, ap, coef, out, smem);
+    if (wk.totals) totals_epilogue<2, kEpiKl, LOOP>(wk, rows, chunks, cols, ap, coef, out, smem);
   }
 }
 
@@ -1938,30 +1951,45 @@ extern "C" int vamd_policy_loss_variant_forward(int variant, const float* old_lo
   bool sep = rows * chunks > kInlineFoldRecords;  // fold the records in a launch of their own
   wk.totals = sep && totals_suffice(ap.mode);     // ... unless the launch totals are all the mode needs
   // the clipped PPO loss gets kernels of its own, the other variants share one with a per-token switch
-#define VAMD_PL_LAUNCH(V, G, W, F, K, R)                                                                              \
-  hipLaunchKernelGGL((policy_kernel<V, M, G, W, F, K, (R) && (V) && (F)>), grid, block, 0, s, old_log_prob, log_prob, advantages, mk, \
-                     token_weights, rows, cols, chunks, pp, ap, wk, out, grad_unscaled, coef_out)
-#define VAMD_PL(V, G, W, F)                                                           \
-  if (variant == VAMD_PL_VANILLA) VAMD_PL_LAUNCH(V, G, W, F, VAMD_PL_VANILLA, false); \
-  else if (rows_inline) VAMD_PL_LAUNCH(V, G, W, F, -1, true); /* rows_inline implies 16-byte accesses */ \
-  else VAMD_PL_LAUNCH(V, G, W, F, -1, false)
-#define VAMD_PL_GW(V, F)                                                                             \
-  if (grad_unscaled) { if (token_weights) { VAMD_PL(V, true, true, F); } else { VAMD_PL(V, true, false, F); } } \
-  else { if (token_weights) { VAMD_PL(V, false, true, F); } else { VAMD_PL(V, false, false, F); } }
+#define VAMD_PL_LAUNCH(V, G, W, F, K, R, L)                                                                              \
+  {                                                                                                                      \
+    const auto kernel = policy_kernel<V, M, G, W, F, K, (R) && (V) && (F) && !(L), L>;                                   \
+    if (L) grid.x = walking_grid(rows * chunks, reinterpret_cast<const void*>(kernel));                                  \
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, old_log_prob, log_prob, advantages, mk, token_weights, rows, cols,     \
+                       chunks, pp, ap, wk, out, grad_unscaled, coef_out);                                                \
+  }
+#define VAMD_PL(V, G, W, F, L)                                                          \
+  if (variant == VAMD_PL_VANILLA) VAMD_PL_LAUNCH(V, G, W, F, VAMD_PL_VANILLA, false, L) \
+  else if (rows_inline) VAMD_PL_LAUNCH(V, G, W, F, -1, true, L) /* rows_inline implies 16-byte accesses */ \
+  else VAMD_PL_LAUNCH(V, G, W, F, -1, false, L)
+#define VAMD_PL_GW(V, F)                                                                                         \
+  if (grad_unscaled) { if (token_weights) { VAMD_PL(V, true, true, F, false) } else { VAMD_PL(V, true, false, F, false) } } \
+  else { if (token_weights) { VAMD_PL(V, false, true, F, false) } else { VAMD_PL(V, false, false, F, false) } }
+#define VAMD_PL_WALK(V) \
+  if (grad_unscaled) { VAMD_PL(V, true, false, true, true) } else { VAMD_PL(V, false, false, true, true) }
   VAMD_MASK_DISPATCH(mask_dtype, M, {
     const bool vec = can_vectorize(cols, {old_log_prob, log_prob, advantages, token_weights, grad_unscaled}, mask,
                                    sizeof(M));
     const M* mk = static_cast<const M*>(mask);
-    const bool walks = totals_suffice(ap.mode) && !rows_inline && (!vec || rows * chunks < kStreamingGrid);
-    grid.x = loss_grid(rows * chunks, walks, kPolicyPerCu);
+    // The launch is large and wants only its totals; how much it gains depends on what it reads per token (us, a workgroup per
+    // item -> walking; gradient, buffers not in the caches).  int64 mask: 2100 x 4096 52.1 -> 48.3, CISPO 58.4 -> 46.2; one-byte
+    // mask: 44.9 -> 39.8, 2200 x 8190 81.6 -> 72.7.  From kStreamingGrid items only rows that are not aligned walk (2048 x 16384
+    // 112.8 -> 115.5).  With a 4-byte mask and a gradient the clipped PPO loss lost more than it gained (3900 x 4096 67.9 ->
+    // 71.3, 2100 x 4096 41.8 -> 40.7); the other variants gained (1200 x 6000 46.6 -> 39.4) below the streaming size
+    // (2200 x 8190 75.2 -> 78.0).  With importance weights nothing was measured: a workgroup per item.
+    const bool big = rows * cols >= (int64_t)kStreamingGrid * 4096;
+    const bool walks = wk.totals && !rows_inline && !token_weights && (!vec || rows * chunks < kStreamingGrid) &&
+                       !(sizeof(M) == 4 && grad_unscaled && (variant == VAMD_PL_VANILLA || big));
     sep = sep && vec && !walks;
-    if (sep) { VAMD_PL_GW(true, false) }
+    if (walks) { if (vec) { VAMD_PL_WALK(true) } else { VAMD_PL_WALK(false) } }
+    else if (sep) { VAMD_PL_GW(true, false) }
     else if (vec) { VAMD_PL_GW(true, true) }
     else { VAMD_PL_GW(false, true) }
   });
   if (sep && !wk.totals)
     hipLaunchKernelGGL((fold_loss_kernel<5, kEpiPolicy>), dim3(1), dim3(kFoldThreads), 0, s, wk.partials, rows,
                        chunks, cols, ap, coef_out, out);
+#undef VAMD_PL_WALK
 #undef VAMD_PL_GW
 #undef VAMD_PL
 #undef VAMD_PL_LAUNCH
@@ -1994,18 +2022,26 @@ extern "C" int vamd_value_loss_forward(const float* vpreds, const float* returns
   dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
   bool sep = rows * chunks > kInlineFoldRecords;
   wk.totals = sep && totals_suffice(mode);
-#define VAMD_VL(V, G, F)                                                                                     \
-  hipLaunchKernelGGL((value_kernel<V, M, G, F>), grid, block, 0, s, vpreds, returns, values, mk, rows, cols, \
-                     chunks, cliprange_value, ap, wk, out, grad_unscaled, coef_out)
+#define VAMD_VL(V, G, F, L)                                                                                          \
+  {                                                                                                                  \
+    const auto kernel = value_kernel<V, M, G, F, L>;                                                                 \
+    if (L) grid.x = walking_grid(rows * chunks, reinterpret_cast<const void*>(kernel));                              \
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, vpreds, returns, values, mk, rows, cols, chunks, cliprange_value, \
+                       ap, wk, out, grad_unscaled, coef_out);                                                        \
+  }
   VAMD_MASK_DISPATCH(mask_dtype, M, {
     const bool vec = can_vectorize(cols, {vpreds, returns, values, grad_unscaled}, mask, sizeof(M));
     const M* mk = static_cast<const M*>(mask);
-    const bool walks = totals_suffice(mode) && (!vec || rows * chunks < kStreamingGrid);
-    grid.x = loss_grid(rows * chunks, walks, kValuePerCu);
+    // as policy_kernel, but only with a one-byte mask and a gradient: 2100 x 4096 41.4 -> 35.7, 1000 x 11999 50.9 -> 46.7 us.
+    // Elsewhere what one size gained another lost (int64: 2100 x 4096 48.7 -> 44.9, 1000 x 11999 62.4 -> 65.1; fp32: 38.9 ->
+    // 37.7, 50.5 -> 51.8; without gradient 2100 x 4099 35.0 -> 36.7).
+    const bool walks = wk.totals && sizeof(M) == 1 && grad_unscaled && (!vec || rows * chunks < kStreamingGrid);
     sep = sep && vec && !walks;
-    if (sep) { if (grad_unscaled) VAMD_VL(true, true, false); else VAMD_VL(true, false, false); }
-    else if (vec) { if (grad_unscaled) VAMD_VL(true, true, true); else VAMD_VL(true, false, true); }
-    else { if (grad_unscaled) VAMD_VL(false, true, true); else VAMD_VL(false, false, true); }
+    if (walks) {
+      if constexpr (sizeof(M) == 1) { if (vec) VAMD_VL(true, true, true, true) else VAMD_VL(false, true, true, true) }
+    } else if (sep) { if (grad_unscaled) VAMD_VL(true, true, false, false) else VAMD_VL(true, false, false, false) }
+    else if (vec) { if (grad_unscaled) VAMD_VL(true, true, true, false) else VAMD_VL(true, false, true, false) }
+    else { if (grad_unscaled) VAMD_VL(false, true, true, false) else VAMD_VL(false, false, true, false) }
   });
   if (sep && !wk.totals)
     hipLaunchKernelGGL((fold_loss_kernel<3, kEpiValue>), dim3(1), dim3(kFoldThreads), 0, s, wk.partials, rows, chunks,
@@ -2051,23 +2087,35 @@ extern "C" int vamd_kl_loss_forward(const float* logprob, const float* ref_logpr
   const int chunks = (int)chunks_of(cols);
   Work wk = carve_work(workspace);
   const AggParams ap = make_agg(mode, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor);
-  const dim3 grid(loss_grid(rows * chunks, totals_suffice(mode), kKlPerCu)), block(kRcThreads);
+  dim3 grid((unsigned)(rows * chunks)), block(kRcThreads);
   bool sep = rows * chunks > kInlineFoldRecords;
   wk.totals = sep && totals_suffice(mode);
-#define VAMD_KL(V, G, F)                                                                                       \
-  hipLaunchKernelGGL((kl_loss_kernel<V, M, G, F>), grid, block, 0, s, logprob, ref_logprob, mk, rows, cols, chunks, \
-                     kind, straight_through, ap, wk, out, grad_unscaled, coef_out)
+#define VAMD_KL(V, G, F, L)                                                                                          \
+  {                                                                                                                  \
+    const auto kernel = kl_loss_kernel<V, M, G, F, L>;                                                               \
+    if (walks) grid.x = walking_grid(rows * chunks, reinterpret_cast<const void*>(kernel));                          \
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, logprob, ref_logprob, mk, rows, cols, chunks, kind,                \
+                       straight_through, ap, wk, out, grad_unscaled, coef_out);                                      \
+  }
+#define VAMD_KL_G(V, F) \
+  if (grad_unscaled) VAMD_KL(V, true, F, true) else if (walks) VAMD_KL(V, false, F, true) else VAMD_KL(V, false, F, false)
   VAMD_MASK_DISPATCH(mask_dtype, M, {
     const bool vec = can_vectorize(cols, {logprob, ref_logprob, grad_unscaled}, mask, sizeof(M));
     const M* mk = static_cast<const M*>(mask);
+    // One-byte masks at every size (2100 x 4096 33.8 -> 30.0, 2048 x 16384 82.7 -> 76.3 us with gradient; 2100 x 4099 28.7 ->
+    // 24.4 without); int64 masks with a gradient below the streaming size (2100 x 4096 42.0 -> 38.2, 2048 x 16384 115.1 ->
+    // 117.9); other launches lost (1200 x 6000 fp32 31.5 -> 32.9, without gradient 20.2 -> 21.9).  With a gradient the kernel
+    // with the loop is the quicker one for a single item too (1000 x 11999 fp32 43.1 -> 41.0).
+    const bool walks = wk.totals && (sizeof(M) == 1 || (sizeof(M) == 8 && grad_unscaled && rows * chunks < kStreamingGrid));
     sep = sep && vec;
-    if (sep) { if (grad_unscaled) VAMD_KL(true, true, false); else VAMD_KL(true, false, false); }
-    else if (vec) { if (grad_unscaled) VAMD_KL(true, true, true); else VAMD_KL(true, false, true); }
-    else { if (grad_unscaled) VAMD_KL(false, true, true); else VAMD_KL(false, false, true); }
+    if (sep) { VAMD_KL_G(true, false) }
+    else if (vec) { VAMD_KL_G(true, true) }
+    else { VAMD_KL_G(false, true) }
   });
   if (sep && !wk.totals)
     hipLaunchKernelGGL((fold_loss_kernel<2, kEpiKl>), dim3(1), dim3(kFoldThreads), 0, s, wk.partials, rows, chunks,
                        cols, ap, coef_out, out);
+#undef VAMD_KL_G
 #undef VAMD_KL
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;

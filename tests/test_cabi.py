@@ -288,3 +288,15 @@ def test_losses_refuse_a_tangent_on_any_input(name, at):
             inputs[at] = fwAD.make_dual(inputs[at], torch.ones(2, 8))
             with pytest.raises(NotImplementedError, match="forward mode"):
                 fn(*inputs)
+
+
+def test_group_ids_of_an_object_array_that_is_refilled():
+    """The kept results are found by the addresses of the label objects.  Refilling a two-entry array comes back to the
+    same three addresses every third time, here with equal labels where there were different ones."""
+    from verl_amd.trainer.ppo.core_algos import _group_ids_on_device
+    index = np.empty(2, dtype=object)
+    for i in range(60):
+        for k in range(2):
+            index[k] = f"prompt-{(i if i % 2 else 2 * i + k) + 1000}".ljust(300)   # a size nothing else here has
+        ids, groups = _group_ids_on_device(index, False, torch.device("cpu"))
+        assert groups == (1 if i % 2 else 2) and ids.tolist() == [0, groups - 1], (i, ids, groups)

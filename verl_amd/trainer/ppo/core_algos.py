@@ -223,7 +223,7 @@ def _group_ids_on_device(index, vectorized: bool, dev: torch.device):
     ``uid`` array to every estimator call of a step, and factorising the labels plus copying 4 KB to the device
     costs more than the advantage kernel itself, so the last few results are kept, keyed by the labels' content
     (numpy arrays: dtype, shape and raw bytes -- for object arrays the bytes are the addresses of the label
-    objects, which the kept array keeps alive).  Anything else is factorised afresh."""
+    objects, which are kept alive with the result).  Anything else is factorised afresh."""
     key = None
     if isinstance(index, np.ndarray):
         # the bytes themselves, not their hash: a dictionary compares keys in full, so two label arrays can never
@@ -233,10 +233,13 @@ def _group_ids_on_device(index, vectorized: bool, dev: torch.device):
         if hit is not None:
             _GROUP_ID_CACHE.move_to_end(key)
             return hit[0], hit[1]
+    # the labels themselves: the array is the caller's, who may put other objects into it, and new labels at the addresses
+    # of freed ones would find this entry
+    labels = index.ravel().tolist() if key is not None and index.dtype.hasobject else None
     ids, G = contiguous_group_ids(index, vectorized=vectorized)
     ids = ids.to(dev)
     if key is not None:
-        _GROUP_ID_CACHE[key] = (ids, G, index)
+        _GROUP_ID_CACHE[key] = (ids, G, labels)
         while len(_GROUP_ID_CACHE) > _GROUP_ID_CACHE_SIZE:
             _GROUP_ID_CACHE.popitem(last=False)
     return ids, G

@@ -300,3 +300,30 @@ def test_group_ids_of_an_object_array_that_is_refilled():
             index[k] = f"prompt-{(i if i % 2 else 2 * i + k) + 1000}".ljust(300)   # a size nothing else here has
         ids, groups = _group_ids_on_device(index, False, torch.device("cpu"))
         assert groups == (1 if i % 2 else 2) and ids.tolist() == [0, groups - 1], (i, ids, groups)
+
+
+def test_group_ids_from_several_threads():
+    """Threads that push each other's results out of the kept ones."""
+    import sys
+    import threading
+    from verl_amd.trainer.ppo.core_algos import _group_ids_on_device
+    wrong, interval = [], sys.getswitchinterval()
+
+    def work(k):
+        try:
+            for i in range(400):
+                ids, groups = _group_ids_on_device(np.array([0, (k + i) % 12, 0]), False, torch.device("cpu"))
+                if groups != (1 if (k + i) % 12 == 0 else 2):
+                    wrong.append((k, i))
+        except Exception as e:   # noqa: BLE001 (a thread's exception is not the test's)
+            wrong.append(e)
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not wrong, wrong[0]

@@ -270,6 +270,18 @@ def test_grpo_group_ids_follow_the_labels_when_the_array_is_reused(dev):
     assert torch.equal(a, b) and torch.equal(a, first)
 
 
+def test_grpo_group_ids_are_kept_per_stream(dev):
+    from verl_amd.trainer.ppo.core_algos import _group_ids_on_device
+    index = np.repeat(np.arange(9), 7)
+    here, _ = _group_ids_on_device(index, False, dev)
+    other = torch.cuda.Stream(dev)
+    with torch.cuda.stream(other):
+        there, _ = _group_ids_on_device(index, False, dev)
+        assert _group_ids_on_device(index, False, dev)[0] is there
+    assert _group_ids_on_device(index, False, dev)[0] is here and there is not here
+    assert torch.equal(here.cpu(), there.cpu())
+
+
 @pytest.mark.parametrize("B,L", [(512, 4096), (3000, 300), (2400, 4500), (64, 40000)])
 def test_grpo_single_launch_bounded_wait_runs_out_without_hanging(dev, monkeypatch, B, L):
     """The one-launch GRPO estimator with its poll limit forced to zero, on both ways of waiting (one meeting of the

@@ -12,6 +12,7 @@ from __future__ import annotations
 import collections
 
 from enum import Enum
+import threading
 import warnings
 from typing import Any, Callable, Optional
 
@@ -216,6 +217,7 @@ def _watch_waiting_kernels(ticket_ws: torch.Tensor) -> None:
 
 _GROUP_ID_CACHE: "collections.OrderedDict" = collections.OrderedDict()
 _GROUP_ID_CACHE_SIZE = 8
+_GROUP_ID_LOCK = threading.Lock()
 
 
 def _group_ids_on_device(index, vectorized: bool, dev: torch.device):
@@ -223,25 +225,29 @@ def _group_ids_on_device(index, vectorized: bool, dev: torch.device):
     ``uid`` array to every estimator call of a step, and factorising the labels plus copying 4 KB to the device
     costs more than the advantage kernel itself, so the last few results are kept, keyed by the labels' content
     (numpy arrays: dtype, shape and raw bytes -- for object arrays the bytes are the addresses of the label
-    objects, which are kept alive with the result).  Anything else is factorised afresh."""
+    objects, which are kept alive with the result) and by the stream the ids were copied on: a result that drops out
+    gives its memory back to that stream.  Anything else is factorised afresh."""
     key = None
     if isinstance(index, np.ndarray):
         # the bytes themselves, not their hash: a dictionary compares keys in full, so two label arrays can never
         # be taken for each other
-        key = (index.dtype.str, index.shape, index.tobytes(), bool(vectorized), dev)
-        hit = _GROUP_ID_CACHE.get(key)
-        if hit is not None:
-            _GROUP_ID_CACHE.move_to_end(key)
-            return hit[0], hit[1]
+        stream = _cabi.stream_ptr(dev) if dev.type == "cuda" else 0
+        key = (index.dtype.str, index.shape, index.tobytes(), bool(vectorized), dev, stream)
+        with _GROUP_ID_LOCK:
+            hit = _GROUP_ID_CACHE.get(key)
+            if hit is not None:
+                _GROUP_ID_CACHE.move_to_end(key)
+                return hit[0], hit[1]
     # the labels themselves: the array is the caller's, who may put other objects into it, and new labels at the addresses
     # of freed ones would find this entry
     labels = index.ravel().tolist() if key is not None and index.dtype.hasobject else None
     ids, G = contiguous_group_ids(index, vectorized=vectorized)
     ids = ids.to(dev)
     if key is not None:
-        _GROUP_ID_CACHE[key] = (ids, G, labels)
-        while len(_GROUP_ID_CACHE) > _GROUP_ID_CACHE_SIZE:
-            _GROUP_ID_CACHE.popitem(last=False)
+        with _GROUP_ID_LOCK:
+            _GROUP_ID_CACHE[key] = (ids, G, labels)
+            while len(_GROUP_ID_CACHE) > _GROUP_ID_CACHE_SIZE:
+                _GROUP_ID_CACHE.popitem(last=False)
     return ids, G
 
 

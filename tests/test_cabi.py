@@ -327,3 +327,23 @@ def test_group_ids_from_several_threads():
     finally:
         sys.setswitchinterval(interval)
     assert not wrong, wrong[0]
+
+
+@pytest.mark.parametrize("capturing,kept", [(0, True), (1, False)])
+def test_logits_are_not_kept_while_their_device_captures(monkeypatch, capturing, kept):
+    """The stream that is asked is that of the tensors' device (1), not of the current one (0)."""
+    import contextlib
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    current = [0]
+
+    @contextlib.contextmanager
+    def device(d):
+        current.append(d.index)
+        yield
+        current.pop()
+    monkeypatch.delenv("VAMD_LCE_LOGITS_CACHE_GB", raising=False)
+    monkeypatch.setattr(K, "_free_device_bytes", lambda d: 1 << 40)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current[-1])
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[-1] == capturing)
+    assert K.keeps_logits(64, 1024, torch.device("cuda", 1)) == kept and current == [0]

@@ -81,8 +81,11 @@ def keeps_logits(n_tokens: int, vocab: int, device) -> bool:
     budget = logits_cache_budget_bytes()
     if budget is not None:
         return 4 * n_tokens * vocab <= budget
-    if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None or torch.cuda.is_current_stream_capturing():
+    if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
         return False
+    with _cabi.device_guard(device):   # the question is asked of the current device's stream
+        if torch.cuda.is_current_stream_capturing():
+            return False
     return 4 * n_tokens * vocab * _LOGITS_CACHE_SHARE <= _free_device_bytes(device)
 
 

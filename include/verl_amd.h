@@ -230,8 +230,8 @@ int vamd_row_softmax_stats_as(const void* logits, int dtype, int64_t n_rows, int
                               float* mean_z, void* stream);
 /* d_logits = d_logprobs (onehot(label) - p) - d_entropy p (z - mean_z), p = exp(z - lse): what autograd hands back
  * through log_softmax + gather (logprobs_from_logits_naive) and through logsumexp - sum softmax * z
- * (entropy_from_logits).  d_logprobs / d_entropy: fp32 [n_rows] (_as: grad_dtype, VAMD_DT_F32 or the logits' type),
- * either may be NULL (no contribution);
+ * (entropy_from_logits).  d_logprobs / d_entropy: fp32 [n_rows] (_as: grad_dtype, VAMD_DT_F32 or the logits' type; 16-bit
+ * ones 2-byte aligned), either may be NULL (no contribution);
  * d_logits has the element type of logits and row pitch ld_out, and may be the logits buffer itself (in place, the
  * reference's inplace_backward). */
 int vamd_row_softmax_backward(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,

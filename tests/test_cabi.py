@@ -79,6 +79,13 @@ def test_a_call_over_more_tokens_than_planned_is_refused(lib):
         assert rc == -1 and b"tokens are no part of" in lib.vamd_last_error()
 
 
+def test_unaligned_16_bit_row_gradients_are_refused(lib):
+    at = 4096                                                # never read: the call is refused on the host
+    for d_logprobs, d_entropy in ((at + 1, None), (at, at + 1)):
+        rc = lib.vamd_row_softmax_backward_as(at, 1, 4, 256, 256, at, at, at, d_logprobs, d_entropy, 1, at, 128, None)
+        assert rc == -1 and b"2-byte aligned" in lib.vamd_last_error()
+
+
 def test_head_size_queries_are_asked_on_the_tensors_device(monkeypatch):
     """The head's workspaces depend on the compute units of the current device, so the query belongs inside the guard that
     makes the tensors' device current for the call itself (devices need not be alike)."""

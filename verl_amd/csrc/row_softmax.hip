@@ -105,22 +105,28 @@ struct StatsArgs {
 
 // Element r of a per-row vector whose elements are D's (typed) or fp32.  16-bit callers' results leave and their upstream
 // gradients arrive in their own type: conversions around these kernels were four launches of 5 us of a pass, and more than
-// that in host time (log-probs, entropy and their gradients at 300 x 151936 bf16 206 -> 180 us, 800 x 152064 387 -> 376,
-// 1500 x 152064 679 -> 669, 3001 x 152064 1321 -> 1312).
+// that in host time (log-probs, entropy and their gradients at 300 x 151936 bf16 206 -> 180 us, 800 x 152064 387 -> 376; at
+// 3001 rows they are within the noise).
 template <class D>
 __device__ __forceinline__ void store_row_value(void* p, bool typed, int64_t r, float x) {
   if (typed) static_cast<typename D::type*>(p)[r] = from_float(x, D());
   else static_cast<float*>(p)[r] = x;
 }
 // A 16-bit element is taken out of its aligned word, which a scalar load fetches (r is uniform); a load of 16 bits is a vector
-// load, whose round trip in front of everything else made the backward kernel 40 us slower at 3001 x 152064.
+// load, whose round trip in front of everything else made the backward kernel 40 us slower at 3001 x 152064.  It is left to
+// the first or last of the n elements where the word reaches past them (the test takes 1 of 286 us).
 template <class D, bool TYPED>
-__device__ __forceinline__ float load_row_value(const void* p, int64_t r) {
+__device__ __forceinline__ float load_row_value(const void* p, unsigned r, unsigned n) {
   if (!TYPED || sizeof(typename D::type) == 4) return static_cast<const float*>(p)[r];
-  const unsigned odd = ((unsigned)reinterpret_cast<uintptr_t>(p) >> 1) & 1u;  // p sits in the upper half of a word
-  const uint64_t half = (uint64_t)r + odd;
-  const unsigned word = reinterpret_cast<const unsigned*>(static_cast<const uint16_t*>(p) - odd)[half >> 1];
-  const uint16_t bits = (uint16_t)((half & 1) ? word >> 16 : word);
+  const uint16_t* const q = static_cast<const uint16_t*>(p) + r;
+  const unsigned upper = ((unsigned)reinterpret_cast<uintptr_t>(q) >> 1) & 1u;  // the element is the upper half of its word
+  uint16_t bits;
+  if (__builtin_expect(r - upper < n - 1, 1)) {  // (r - upper wraps round for an upper half in front)
+    const unsigned word = *reinterpret_cast<const unsigned*>(q - upper);
+    bits = (uint16_t)(upper ? word >> 16 : word);
+  } else {
+    bits = *q;
+  }
   if constexpr (std::is_same_v<D, BF16>) return __uint_as_float((unsigned)bits << 16);
   else return (float)__builtin_bit_cast(_Float16, bits);
 }
@@ -217,6 +223,7 @@ struct BackwardArgs {
   const float* mean_z;    // needed with d_entropy
   const void* d_logprobs;  // element type of the logits or fp32
   const void* d_entropy;   // likewise
+  unsigned rows;           // elements of each
   void* d_logits;
   int64_t ld_out;
   int64_t cols;
@@ -252,8 +259,8 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(Backw
   }
   __builtin_amdgcn_sched_barrier(0);
   const float lse2 = a.lse[r] * kLog2e;
-  const float glp = a.d_logprobs ? load_row_value<D, TYPED>(a.d_logprobs, r) : 0.f;
-  const float gent = a.d_entropy ? load_row_value<D, TYPED>(a.d_entropy, r) : 0.f;
+  const float glp = a.d_logprobs ? load_row_value<D, TYPED>(a.d_logprobs, (unsigned)r, a.rows) : 0.f;
+  const float gent = a.d_entropy ? load_row_value<D, TYPED>(a.d_entropy, (unsigned)r, a.rows) : 0.f;
   const float mz = a.d_entropy ? a.mean_z[r] : 0.f;
   const float t0 = fmaf(-gent, mz, glp);  // g_lp + g_ent (z - mean_z) = g_ent z + t0
   const int64_t label = a.d_logprobs ? a.labels[r] : -1;
@@ -402,6 +409,8 @@ extern "C" int vamd_row_softmax_backward_as(const void* logits, int dtype, int64
   if (st != VAMD_OK) return st;
   VAMD_REQUIRE(grad_dtype == VAMD_DT_F32 || grad_dtype == dtype,
                "row_softmax_backward: upstream gradients are fp32 or of the logits' type, not of type %d", grad_dtype);
+  VAMD_REQUIRE(grad_dtype == VAMD_DT_F32 || ((reinterpret_cast<uintptr_t>(d_logprobs) | reinterpret_cast<uintptr_t>(d_entropy)) & 1) == 0,
+               "row_softmax_backward: 16-bit upstream gradients must be 2-byte aligned");
   VAMD_REQUIRE(d_logits && ld_out >= vocab && lse, "row_softmax_backward: bad output or missing lse");
   VAMD_REQUIRE(d_logprobs || d_entropy, "row_softmax_backward: no upstream gradient");
   VAMD_REQUIRE(!d_logprobs || labels, "row_softmax_backward: d_logprobs needs labels");
@@ -411,7 +420,7 @@ extern "C" int vamd_row_softmax_backward_as(const void* logits, int dtype, int64
     const int64_t per_wg = (int64_t)kRowThreads * D::kVec * D::kBackwardLoads;
     const int64_t chunks = (vocab + per_wg - 1) / per_wg;
     VAMD_REQUIRE(n_rows * chunks < (1ll << 31), "row_softmax_backward: too many workgroups");
-    BackwardArgs a{logits, ld, labels, lse, mean_z, d_logprobs, d_entropy, d_logits, ld_out, vocab, (int)chunks};
+    BackwardArgs a{logits, ld, labels, lse, mean_z, d_logprobs, d_entropy, (unsigned)n_rows, d_logits, ld_out, vocab, (int)chunks};
     const dim3 grid((unsigned)(n_rows * chunks));
     const bool vec = rows_vectorizable<D>(logits, ld) && rows_vectorizable<D>(d_logits, ld_out);
     constexpr bool kSmall = sizeof(typename D::type) < 4;

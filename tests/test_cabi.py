@@ -39,6 +39,25 @@ def test_every_declared_symbol_is_exported_and_bound(lib):
     assert f"#define VAMD_ABI_VERSION {_cabi.ABI_VERSION}\n" in header
 
 
+def test_stale_binaries_are_told_to_be_rebuilt(monkeypatch):
+    """A library from before an entry point was added, and a host module linked with such a library."""
+    import types
+    older = lambda: _cabi.ABI_VERSION - 1
+    with monkeypatch.context() as m:
+        m.setattr(ctypes, "CDLL", lambda path: types.SimpleNamespace(vamd_abi_version=older))
+        with pytest.raises(RuntimeError, match="rebuild"):
+            _cabi.load_library()
+    current = lambda: _cabi.ABI_VERSION
+    for compiled, linked in ((older, current), (current, older)):
+        module = types.SimpleNamespace(abi_version=compiled, library_abi_version=linked)
+        monkeypatch.setattr(_cabi, "_ops", None)
+        monkeypatch.setattr(_cabi.importlib.util, "module_from_spec", lambda spec: module)
+        monkeypatch.setattr(_cabi.importlib.util, "spec_from_file_location",
+                            lambda *a: types.SimpleNamespace(loader=types.SimpleNamespace(exec_module=lambda m: None)))
+        with pytest.raises(RuntimeError, match="rebuild"):
+            _cabi.ops()
+
+
 def test_workspace_queries(lib):
     assert lib.vamd_lce_forward_workspace_bytes(16384, 3584, 152064) > 0
     assert lib.vamd_lce_forward_workspace_bytes(0, 3584, 152064) == 0

@@ -151,7 +151,7 @@ def lib_path() -> str:
     return _LIB_PATH
 
 
-ABI_VERSION = 5  # VAMD_ABI_VERSION of include/verl_amd.h
+ABI_VERSION = 6  # VAMD_ABI_VERSION of include/verl_amd.h
 
 
 def load_library(path: str | None = None) -> ctypes.CDLL:
@@ -163,13 +163,13 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
             "verl_amd has no CPU fallback."
         )
     lib = ctypes.CDLL(path)
+    if lib.vamd_abi_version() != ABI_VERSION:   # before the symbols: an older library lacks some of them
+        raise RuntimeError(f"{path} reports ABI version {lib.vamd_abi_version()}, these bindings are written for "
+                           f"{ABI_VERSION}: rebuild it with `python -m verl_amd.csrc.build`")
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError names the missing symbol
         fn.restype = res
         fn.argtypes = args
-    if lib.vamd_abi_version() != ABI_VERSION:
-        raise RuntimeError(f"{path} reports ABI version {lib.vamd_abi_version()}, these bindings are written for "
-                           f"{ABI_VERSION}: rebuild it with `python -m verl_amd.csrc.build`")
     return lib
 
 
@@ -194,9 +194,11 @@ def ops():
                 spec = importlib.util.spec_from_file_location("_torch_ops", _OPS_PATH)
                 module = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(module)
-                if module.abi_version() != ABI_VERSION:
-                    raise RuntimeError(f"{_OPS_PATH} was built for ABI version {module.abi_version()}, these bindings "
-                                       f"are written for {ABI_VERSION}: rebuild it")
+                # what it was compiled against, and what the library reports that the dynamic linker gave it
+                for version in (module.abi_version(), module.library_abi_version()):
+                    if version != ABI_VERSION:
+                        raise RuntimeError(f"{_OPS_PATH} is built for or linked with ABI version {version}, these bindings "
+                                           f"are written for {ABI_VERSION}: rebuild it with `python -m verl_amd.csrc.build`")
                 _ops = module
     return _ops
 

@@ -603,6 +603,7 @@ std::vector<double> fetch(const Tensor& t) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("abi_version", [] { return VAMD_ABI_VERSION; });
+  m.def("library_abi_version", [] { return vamd_abi_version(); });
   m.def("ticket_workspace", [](int64_t bytes, at::Device dev) {
     if (!dev.has_index()) dev.set_index(c10::hip::current_device());
     return ticket_workspace((size_t)(bytes < 0 ? 0 : bytes), dev);

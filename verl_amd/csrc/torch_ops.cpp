@@ -122,11 +122,18 @@ Tensor ticket_workspace(size_t bytes, const at::Device& dev) {
   static std::mutex mu;
   static auto* buffers = new std::map<std::pair<int, void*>, Tensor>;
   const int64_t need = bytes < 4096 ? 4096 : (int64_t)bytes;
-  std::lock_guard<std::mutex> lock(mu);
-  Tensor& buf = (*buffers)[{(int)dev.index(), stream_of(dev)}];
-  if (!buf.defined() || buf.numel() < need)
-    buf = at::zeros({need < (1 << 20) ? (1 << 20) : need}, at::TensorOptions().dtype(at::kByte).device(dev));
-  return buf;
+  const std::pair<int, void*> key{(int)dev.index(), stream_of(dev)};
+  const auto kept = [&](const Tensor& fresh) {
+    std::lock_guard<std::mutex> lock(mu);
+    Tensor& buf = (*buffers)[key];
+    if (fresh.defined() && (!buf.defined() || buf.numel() < need)) buf = fresh;
+    return buf;
+  };
+  const Tensor buf = kept(Tensor());
+  if (buf.defined() && buf.numel() >= need) return buf;
+  // Without the lock: an allocation may run Python (a dispatch mode), which may let a thread run that comes here, holding the
+  // interpreter.
+  return kept(at::zeros({need < (1 << 20) ? (1 << 20) : need}, at::TensorOptions().dtype(at::kByte).device(dev)));
 }
 
 bool wants_gradient(const Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }

@@ -274,8 +274,8 @@ struct Frags {
 // The body is 64 slots "one MFMA + at most two memory instruction groups", each closed by a scheduling barrier so
 // the compiler keeps the order.  Slot j = 4 G + n multiplies block (mb = G % 8, nb) of k-step G / 8, with nb = n in even
 // groups and 3 - n in odd ones: from one MFMA to the next exactly one of the two operands changes, which on a board at its
-// power limit is speed (register-only loop on normal data 2020 -> 2049 TFLOP/s, with both changing every time 1960;
-// 16384 x 3584 x 152064 forward and backward 50.61 -> 50.36 ms, 21503 x 4096 x 128256 forward 15.47 -> 15.43).
+// power limit is speed in a register-only loop on normal data (2020 -> 2049 TFLOP/s, with both changing every time 1960); in
+// the head's kernels the gain is no larger than what two runs differ by.
 //
 //   slots  0..51 : the C fragment of group G + 3 is read from `cur` in the first slot of group G (its ring slot was
 //                  last used by group G - 1); the R fragments of k-step 1 are read in groups 1..4

@@ -1438,7 +1438,10 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
 // quickest, counting in slabs (1.4 us each): an epilogue about 2, and a d_weight tile of up to 3 slabs 7 in all: with every CU
 // storing, its 128 KB take 6 us, and a slab or three more hardly show.  Gradient products over few tokens with 2 for every
 // epilogue, and as it is: 64 x 3584 x 152064 623 -> 490 us, 93 tokens 645 -> 487, 150 tokens 681 -> 588; 128 x 4096 x 128256
-// 600 -> 523; 7 for four slabs as well: 256 x 3584 643 -> 680.
+// 600 -> 523.  The 7 and where it ends are a fit, not a law: four slabs stay at 4 + 2 = 6, below three, because 7 is slower
+// there (256 tokens, with 6 and 7, us: 896 192 and 201, 3584 646 and 675, 4096 585 and 613), while 6 for all four is quicker at
+// some sizes and slower at others (192 x 896 177 and 184, 128 x 3584 567 and 593; 64 x 3584 524 and 477, 128 x 4096 555 and
+// 522).  Results in fp32 or added to what is there, which move two to four times the bytes, are counted alike: not measured.
 constexpr int kEpilogueSlabs = 2, kFewTileSlabs = 3, kFewTileCost = 7, kMaxSplits = 64, kMinPieceSlabs = 32;
 constexpr int64_t kMaxPieceBytes = 256ll << 20;  // bound on the pieces' accumulators
 static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t cols, bool want_dh, bool want_dw,

@@ -2206,34 +2206,6 @@ def test_fetch_reads_what_the_stream_will_have_written(dev):
     assert _cabi.ticket_workspace(0, dev).data_ptr() == _cabi.ticket_workspace(4096, torch.device("cuda")).data_ptr()
 
 
-def test_counter_buffers_are_allocated_without_a_lock(dev):
-    """The allocation runs a dispatch mode's Python, during which another thread asks for a buffer of its own."""
-    import threading
-    from torch.utils._python_dispatch import TorchDispatchMode
-    from verl_amd import _cabi
-    inside, done = threading.Event(), threading.Event()
-
-    class Mode(TorchDispatchMode):
-        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-            inside.set()
-            assert done.wait(30)
-            return func(*args, **(kwargs or {}))
-
-    def other():
-        inside.wait(30)
-        with torch.cuda.stream(torch.cuda.Stream(dev)):
-            assert _cabi.ticket_workspace(65 << 20, dev).numel() >= 65 << 20
-        done.set()
-    thread = threading.Thread(target=other)
-    thread.start()
-    with torch.cuda.stream(torch.cuda.Stream(dev)):
-        with Mode():
-            mine = _cabi.ticket_workspace(66 << 20, dev)
-        thread.join()
-        assert done.is_set() and mine.numel() >= 66 << 20 and not mine.any()
-        assert _cabi.ticket_workspace(0, dev).data_ptr() == mine.data_ptr()
-
-
 def _native_losses(dev):
     from verl_amd.trainer.ppo import core_algos as CA
     B, L = 4, 37

@@ -451,3 +451,31 @@ def test_row_values_in_the_type_of_the_logits(dev, dtype, rows, offset):
         up = lambda t: None if t is None else t.float()
         got = F._row_backward(z, v, lab, lse, mean_z, a, b, False)
         assert torch.equal(got, F._row_backward(z, v, lab, lse, mean_z, up(a), up(b), False))
+
+
+def test_counter_buffers_are_allocated_without_a_lock(dev):
+    """The allocation runs a dispatch mode's Python, during which another thread asks for a buffer of its own."""
+    import threading
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from verl_amd import _cabi
+    inside, done = threading.Event(), threading.Event()
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            inside.set()
+            assert done.wait(30)
+            return func(*args, **(kwargs or {}))
+
+    def other():
+        inside.wait(30)
+        with torch.cuda.stream(torch.cuda.Stream(dev)):
+            assert _cabi.ticket_workspace((1 << 20) + 1, dev).numel() >= (1 << 20) + 1
+        done.set()
+    thread = threading.Thread(target=other)
+    thread.start()
+    with torch.cuda.stream(torch.cuda.Stream(dev)):
+        with Mode():
+            mine = _cabi.ticket_workspace((1 << 20) + 1, dev)
+        thread.join()
+        assert done.is_set() and mine.numel() >= (1 << 20) + 1 and not mine.any()
+        assert _cabi.ticket_workspace(0, dev).data_ptr() == mine.data_ptr()

@@ -613,7 +613,7 @@ int vamd_mfma_yardstick(int shape, const void* seed, float* out, int workgroups,
  * launch of the process is bracketed by HIP events on its stream.  vamd_lce_timing_collect
  * waits for them and adds up milliseconds and launch counts per kernel, indexed
  * 0 forward, 1 merge, 2 d_logits panel from recomputed logits (the recompute GEMM), 3 gradient GEMMs
- * (d_hidden + d_weight) and, where d_hidden's k range was cut into pieces, the launch that sums them, 4 d_logits panel from cached logits (arrays of VAMD_LCE_TIMING_KERNELS). */
+ * (d_hidden + d_weight, over few tokens in a launch each) and, where d_hidden's k range was cut into pieces, the launch that sums them, 4 d_logits panel from cached logits (arrays of VAMD_LCE_TIMING_KERNELS). */
 #define VAMD_LCE_TIMING_KERNELS 5
 int vamd_lce_timing_enable(int on);
 int vamd_lce_timing_collect(double* ms_by_kernel_host, int64_t* launches_by_kernel_host);

@@ -920,3 +920,30 @@ def test_weight_gradient_stored_in_whole_lines(dev, n, h, v, offset):
                                     None, P(d_hidden), P(out), 0, None, 0, P(ws), size, _cabi.stream_ptr(hidden.device)))
     assert torch.equal(out, want) and torch.equal(d_hidden, want_h)
     assert (buf[:guard + offset] == 77).all() and (buf[guard + offset + v * h:] == 77).all()
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (1, 128, 1024),       # two pieces of 8 slabs
+    (64, 384, 1023),      # below the few-token kernel's smallest vocabulary
+    (127, 640, 1032),     # a third piece of one ragged slab, half a column tile
+    (128, 896, 33001),    # most tokens, last piece shorter, ragged vocabulary
+    (129, 896, 33001),    # one token too many
+    (65, 3584, 115000),   # a weight that is read with the non-temporal hint
+])
+def test_d_hidden_over_few_tokens(dev, n, h, v):
+    """Up to 128 tokens d_hidden has a kernel of its own: the fp32 ground truth with the bound for d_logits staged in bf16, the
+    same bits without d_weight, and for some of the tokens the bits that they have among all."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    hidden, weight, labels = _make(n, h, v, seed=n + v, dist="normal")
+    g_lp = torch.randn(n, generator=torch.Generator().manual_seed(n))
+    hd, wd, ld, gd = (t.to(dev) for t in (hidden, weight, labels, g_lp))
+    _, _, lse, mz = K.efficient_entropy_forward(hd, wd, ld, 0, 0.9)
+    dh, dw = K.efficient_entropy_backward(gd, None, hd, wd, ld, lse, mz, 0, 0.9)
+    alone, _ = K.efficient_entropy_backward(gd, None, hd, wd, ld, lse, mz, 0, 0.9, need_d_weight=False)
+    assert torch.equal(dh, alone)
+    some = torch.arange(0, n, 2, device=dev)
+    part, _ = K.efficient_entropy_backward(gd[some], None, hd[some], wd, ld[some], lse[some], mz[some], 0, 0.9, planned_tokens=n)
+    assert torch.equal(part, dh[some])
+    _, _, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)
+    _close_bf16(dh, want_dh, "d_hidden", e_dh)
+    _close_bf16(dw, want_dw, "d_weight", e_dw)

@@ -156,11 +156,19 @@ __device__ __forceinline__ unsigned lds_address(const char* p) {
 // lds_base + 16 L (lds_base is wave-uniform and travels in M0).  Written as inline assembly so
 // that the compiler's wait-count bookkeeping does not see an outstanding LDS write and fence
 // every later LDS read against it; the engine waits for its transfers itself, once per slab.
+// STREAM: with the non-temporal hint, for data that one workgroup reads and nobody reads again soon.
+template <bool STREAM>
 __device__ __forceinline__ void load_to_lds_16(const u32x4& rsrc, unsigned voff, unsigned soff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
-               : "memory", "m0");
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 :
+                 : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :
+                 : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
+                 : "memory", "m0");
 }
 
 // The same for 4 bytes per lane: lane L's dword lands at lds_base + 4 L (256 consecutive bytes per instruction).
@@ -211,8 +219,9 @@ struct SlabDma {
   }
 
   // slab_lds: LDS byte address of the operand's slab in the stage being filled
+  template <bool STREAM = false>
   __device__ __forceinline__ void issue_one(int i, const SlabSrc& src, unsigned slab_lds) const {
-    load_to_lds_16(src.rsrc, voff, src.soff + (unsigned)i * step, slab_lds + lds_wave + (unsigned)i * (kWaves * 1024u));
+    load_to_lds_16<STREAM>(src.rsrc, voff, src.soff + (unsigned)i * step, slab_lds + lds_wave + (unsigned)i * (kWaves * 1024u));
   }
 };
 

@@ -154,6 +154,7 @@ struct FwdArgs {
   float4* partials;  // [plan.slots()][256] : (max in the log2 domain, sum e, sum e x with x = hidden . weight, label logit)
   float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward
   float* pi2_partials;  // optional [plan.slots()][256] : sum of e^2 relative to the same max
+  int stream_weight;    // lce_forward_few_kernel: streams_weight()
 };
 
 // The tiles of one workgroup.  The two ways of sharing out are kernels of their own: with both in one kernel the split
@@ -571,6 +572,12 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
 // 93 x 3584 x 152064 5.4 TB/s, 93 x 4096 x 128256 5.7 TB/s.  From 129 tokens on the 256-token tile's padding is less than half.  A wavefront owns 64 tokens
 // x 64 columns (2 x 4 wavefronts) and keeps the softmax state of its tokens in registers to the end.
 constexpr int kFewTokens = 128;
+// The few-token kernels read every piece of the weight in one workgroup.  From three times the 256 MB memory-side cache on, when
+// little of the weight can still be there in the next pass, they read it with the non-temporal hint, which also leaves the caches to
+// the logits and the panel.  Forward pass over 64 tokens at 151936 columns, without and with it, us: hidden size 896 (272 MB)
+// 52.7 and 57.2, 1536 (467 MB) 96 and 90, 2560 (778 MB) 152 and 146; 4096 x 128256 (1.05 GB) 187 and 170; with the backward pass
+// 896 203 and 211, 2048 (622 MB) 392 and 405, 2560 480 and 473, 3584 x 152064 621 and 617, 128 tokens 716 and 689.
+constexpr int64_t kStreamWeightBytes = 768ll << 20;
 constexpr int kFewStageBytes = (kFewTokens + kTile) * kBK * 2;
 constexpr int kFewStages = 3;
 constexpr int kFewLds = kFewStages * kFewStageBytes;
@@ -580,6 +587,18 @@ constexpr int kFewWavesR = 2, kFewWavesC = 4, kFewMB = kTile / kBlk / kFewWavesC
 constexpr int kFewLoadsR = kFewTokens * 8 / kThreads;  // transfers per lane of one slab of hidden (2)
 static_assert(kFewLoadsR + kLoads == 6, "the s_waitcnt vmcnt(6) of lce_forward_few_kernel counts the transfers of one slab");
 static_assert(kFewTokens == kFewWavesR * kNB * kBlk, "a wavefront owns kNB blocks of tokens");
+
+// the weight's slab of a stage; `stream` is the same for the whole launch
+template <bool KMAJOR>
+__device__ __forceinline__ void few_fetch_weight(const SlabDma<KMAJOR>& dma, const SlabSrc& src, unsigned slab_lds, int stream) {
+  if (stream) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) dma.template issue_one<true>(i, src, slab_lds);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) dma.template issue_one<false>(i, src, slab_lds);
+  }
+}
 
 template <bool CACHE, bool PI2>
 __global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
@@ -627,8 +646,7 @@ __global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
     const unsigned base = lds_address(lds) + (unsigned)fill * kFewStageBytes;
 #pragma unroll
     for (int i = 0; i < kFewLoadsR; ++i) dma.issue_one(i, r, base);
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) dma.issue_one(i, c, base + kFewTokens * kBK * 2);
+    few_fetch_weight(dma, c, base + kFewTokens * kBK * 2, a.stream_weight);
     fill = fill == kFewStages - 1 ? 0 : fill + 1;
     if (t2 == tiles - 1 && k2 == a.k_slabs - 1) return;
     if (++k2 == a.k_slabs) {
@@ -1234,10 +1252,14 @@ struct DWeightEpi {
           line.run(acc, mb, nb, v);
           const int col = c0 + p.wc * 128 + mb * 64 + 8 * line.rd_chunk;  // c_valid % 128 == 0: 8 columns are all in or all out
           const int row0 = r0 + p.wr * (kNB * kBlk) + nb * 32 + line.rd_row;
+          // Non-temporal: a large d_weight left behind in the memory-side cache is written back while the next pass reads the
+          // weight (128 x 3584 x 152064 forward and backward 858 -> 817 us, 300 x 896 x 151936 424 -> 407; the forward pass
+          // behind a d_weight of 1.09 GB 260 -> 205; sizes from 777 tokens on and small heads the same within 1 %).
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             if (col < A.c_valid && row0 + 8 * i < A.r_valid)
-              *reinterpret_cast<u32x4_at8*>(A.out + (int64_t)(row0 + 8 * i) * A.ld_out + col) = v[i];
+              __builtin_nontemporal_store(
+                  v[i], reinterpret_cast<u32x4_at8*>(A.out + (int64_t)(row0 + 8 * i) * A.ld_out + col));
         }
       return;
     }
@@ -1302,13 +1324,106 @@ __global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, Gem
   }
 }
 
+// d_hidden over at most kFewTokens tokens: the k range (the vocabulary) is cut into pieces, each summed into an fp32
+// accumulator of its own by one workgroup per 256 hidden columns.  Bound by reading the weight, as the forward pass over few
+// tokens is, and built like it: 128 token rows, so that the MFMAs of a slab of the weight take half as long as the slab takes
+// out of HBM, and three LDS stages, so that two slabs are in flight while one is multiplied.  As pieces of 256-token tiles
+// in lce_dgrad_kernel, with one slab in flight and half of the MFMAs on padding, and as here (with the launch that sums the
+// pieces): 64 x 896 x 151936 125 -> 75 us, 64 x 3584 x 152064 247 -> 202 (5.6 TB/s), 128 x 3584 x 152064 340 -> 230,
+// 128 x 1024 x 8192 51 -> 25.
+struct FewHiddenArgs {
+  Operand dz;      // R: [n_tokens][panel pitch], k = panel column
+  Operand weight;  // C: K-major, [vocab][hidden]
+  int k_slabs, split_slabs, col_tiles;
+  int stream_weight;
+  float* acc32;  // [pieces][n_tokens][hidden]
+  int n_tokens, hidden;
+};
+
+__global__ __launch_bounds__(kThreads) void lce_dhidden_few_kernel(FewHiddenArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  // the workgroups of a piece are neighbours: they read the same columns of the panel
+  const int wg = xcd_regroup(blockIdx.x, gridDim.x), piece = wg / a.col_tiles, c0 = (wg - piece * a.col_tiles) * kTile;
+  const int k_begin = piece * a.split_slabs, left = a.k_slabs - k_begin;
+  const int slabs = left < a.split_slabs ? left : a.split_slabs;  // > 0
+  const int w = threadIdx.x >> 6, lx = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
+  const int wr = w % kFewWavesR, wc = w / kFewWavesR;
+
+  SlabDma<false> dma_r;
+  SlabDma<true> dma_c;
+  dma_r.init(a.dz);
+  dma_c.init(a.weight);
+  FragAddr<false> fr;
+  FragAddr<true> fc;
+  fr.init(wr * kNB, kNB);
+  fc.init(wc * kFewMB, kFewMB);
+
+  // fetch cursor; past the end it stays on the last slab
+  const u32x4 rs_r = tile_rsrc<false>(a.dz, 0), rs_c = tile_rsrc<true>(a.weight, c0);
+  int k2 = 0, fill = 0;
+  auto fetch = [&]() {
+    const int k0 = (k_begin + k2) * kBK;
+    const SlabSrc r{rs_r, slab_soff<false>(a.dz, k0)}, c{rs_c, slab_soff<true>(a.weight, k0)};
+    const unsigned base = lds_address(lds) + (unsigned)fill * kFewStageBytes;
+#pragma unroll
+    for (int i = 0; i < kFewLoadsR; ++i) dma_r.issue_one(i, r, base);
+    few_fetch_weight(dma_c, c, base + kFewTokens * kBK * 2, a.stream_weight);
+    fill = fill == kFewStages - 1 ? 0 : fill + 1;
+    if (k2 < slabs - 1) ++k2;
+  };
+  fetch();
+  fetch();
+
+  f32x4 acc[kFewMB][kNB];
+#pragma unroll
+  for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < kNB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int stage = 0;
+  for (int it = 0; it < slabs; ++it) {
+    // as in lce_forward_few_kernel: slab `it` has landed, and the stage before it takes slab it + 2
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    fetch();
+    const char* cur = lds + stage * kFewStageBytes;
+    stage = stage == kFewStages - 1 ? 0 : stage + 1;
+    bf16x8 r[kSteps][kNB], c[kSteps][kFewMB];
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) {
+#pragma unroll
+      for (int nb = 0; nb < kNB; ++nb) r[ks][nb] = fr.read(cur, ks, nb);
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb) c[ks][mb] = fc.read(cur + kFewTokens * kBK * 2, ks, mb);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+      for (int mb = 0; mb < kFewMB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < kNB; ++nb)
+          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[ks][mb], r[ks][nb], acc[mb][nb], 0, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into LDS is left when the workgroup ends
+
+  float* const out = a.acc32 + (int64_t)piece * a.n_tokens * a.hidden;
+#pragma unroll
+  for (int nb = 0; nb < kNB; ++nb) {
+    const int tok = wr * (kNB * kBlk) + nb * kBlk + lx;
+#pragma unroll
+    for (int mb = 0; mb < kFewMB; ++mb) {
+      const int col = c0 + wc * (kFewMB * kBlk) + mb * kBlk + 4 * lq;  // hidden % 128 == 0: 4 columns are all in or all out
+      if (tok < a.n_tokens && col < a.hidden)
+        *reinterpret_cast<f32x4*>(out + (int64_t)tok * a.hidden + col) = acc[mb][nb];
+    }
+  }
+}
+
 // d_hidden = sum of the pieces' fp32 accumulators, rounded once.
 __global__ __launch_bounds__(256) void lce_dhidden_sum_kernel(const float* acc32, int pieces, int64_t elements,
                                                               uint16_t* out) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= elements) return;
   f32x4 s = *reinterpret_cast<const f32x4*>(acc32 + i);
-#pragma unroll 4
+#pragma unroll 16
   for (int k = 1; k < pieces; ++k) s = s + *reinterpret_cast<const f32x4*>(acc32 + (int64_t)k * elements + i);
   *reinterpret_cast<u32x2*>(out + i) = pack_bf16x4(s[0], s[1], s[2], s[3]);
 }
@@ -1347,6 +1462,7 @@ static int ensure_lds_attributes() {
   if ((s = allow_big_lds(lce_forward_few_kernel<true, false>, kFewCacheLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_few_kernel<true, true>, kFewCacheLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kRecomputeExtraLds)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_dhidden_few_kernel, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_dgrad_kernel, kLdsBytes + kGradStageBytes)) != VAMD_OK) return s;
   done[dev] = true;
   return VAMD_OK;
@@ -1484,6 +1600,26 @@ static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t co
   return best;
 }
 
+// Whether d_hidden is formed by lce_dhidden_few_kernel: over few tokens, in one vocabulary chunk (it starts its accumulators
+// afresh).  It gains at every vocabulary measured (64 x 1024 x 2048, both gradients: 44 -> 29 us); below two pieces of
+// kFewMinSlabs slabs there is nothing to share out.
+constexpr int kFewMinSlabs = 8, kFewMinVocab = 2 * kFewMinSlabs * kBK;
+static bool few_hidden(int64_t planned_tokens, int64_t chunk, int64_t vocab) {
+  return planned_tokens <= kFewTokens && vocab >= kFewMinVocab && chunk >= vocab;
+}
+
+// Its workgroups: as many pieces as fill one round over the CUs.
+static GradPlan plan_few_hidden(int64_t hidden_size, int64_t vocab, int cus) {
+  const int64_t slabs = ceil_div(vocab, kBK), pieces = cus / ceil_div(hidden_size, kTile);
+  GradPlan p;
+  p.split_slabs = (int)ceil_div(slabs, pieces < 1 ? 1 : pieces);
+  if (p.split_slabs < kFewMinSlabs) p.split_slabs = kFewMinSlabs;
+  p.splits = (int)ceil_div(slabs, p.split_slabs);
+  return p;
+}
+
+static bool streams_weight(int64_t hidden_size, int64_t vocab) { return vocab * hidden_size * 2 >= kStreamWeightBytes; }
+
 }  // namespace vamd
 
 using namespace vamd;
@@ -1558,6 +1694,7 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
                                                   (size_t)a.plan.slots() * kTile * sizeof(float4))
                        : nullptr;
   a.z_cache = logits_cache;
+  a.stream_weight = streams_weight(hidden_size, vocab);
   hipStream_t s = static_cast<hipStream_t>(stream);
   {
     ScopedTiming tm(kTagForward, s);
@@ -1670,17 +1807,28 @@ extern "C" int vamd_lce_forward_static(const void* hidden, const void* weight, c
 }
 
 namespace vamd {
-// Pieces of a d_hidden tile's k range.  Decided as if both gradients were asked for, whichever are, so that d_hidden is the
-// same bits either way; the first (widest) vocabulary chunk decides for all chunks.  For some of the tokens of a larger call
-// they are that call's pieces, so that its bits come out, where it has one vocabulary chunk.  With several chunks it sums
+// How d_hidden is formed: the pieces of its k range.  Decided as if both gradients were asked for, whichever are, so that
+// d_hidden is the same bits either way; the first (widest) vocabulary chunk decides for all chunks.  For some of the tokens of
+// a larger call it is that call's way, so that its bits come out, where it has one vocabulary chunk.  With several chunks it sums
 // over other ranges anyway: there the tokens at hand decide (1000 of 11290 x 3584 x 152064 would run as 56 whole tiles).
-static int d_hidden_pieces(int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size, int64_t vocab,
-                           int64_t vocab_chunk) {
+struct HiddenPlan {
+  bool few;         // lce_dhidden_few_kernel
+  int pieces;
+  int split_slabs;  // few: slabs of a piece
+  int accumulators(int64_t chunk, int64_t vocab) const {  // fp32 [n_tokens][hidden] each
+    return few || pieces > 1 || chunk < vocab ? pieces : 0;
+  }
+};
+static HiddenPlan plan_hidden(int64_t n_tokens, int64_t planned_tokens, int64_t hidden_size, int64_t vocab,
+                              int64_t vocab_chunk) {
   const int64_t cv = default_vocab_chunk(n_tokens, hidden_size, vocab, vocab_chunk);
   const bool same_ranges =
       planned_tokens > n_tokens && default_vocab_chunk(planned_tokens, hidden_size, vocab, vocab_chunk) >= vocab;
-  return plan_gradients(same_ranges ? planned_tokens : n_tokens, hidden_size, cv < vocab ? cv : vocab, true, true,
-                        device_cu_count()).splits;
+  const int64_t planned = same_ranges ? planned_tokens : n_tokens;
+  const bool few = few_hidden(planned, cv, vocab);
+  const GradPlan p = few ? plan_few_hidden(hidden_size, vocab, device_cu_count())
+                         : plan_gradients(planned, hidden_size, cv < vocab ? cv : vocab, true, true, device_cu_count());
+  return HiddenPlan{few, p.splits, p.split_slabs};
 }
 }  // namespace vamd
 
@@ -1689,11 +1837,9 @@ extern "C" size_t vamd_lce_backward_subset_workspace_bytes(int64_t n_tokens, int
   if (n_tokens <= 0 || vocab <= 0 || hidden_size <= 0) return 0;
   const int64_t n_pad = ceil_div(n_tokens, kTile) * kTile;
   const int64_t cv = default_vocab_chunk(n_tokens, hidden_size, vocab, vocab_chunk);
-  size_t bytes = align_up((size_t)n_pad * dz_pitch(cv) * 2, 256);
-  const int pieces = d_hidden_pieces(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk);
-  if (pieces > 1 || cv < ceil_div(vocab, kTile) * kTile)
-    bytes += align_up((size_t)pieces * n_tokens * hidden_size * 4, 256);
-  return bytes;
+  const int accumulators =
+      plan_hidden(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk).accumulators(cv, vocab);
+  return align_up((size_t)n_pad * dz_pitch(cv) * 2, 256) + align_up((size_t)accumulators * n_tokens * hidden_size * 4, 256);
 }
 
 extern "C" size_t vamd_lce_backward_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab,
@@ -1774,10 +1920,11 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
   Carver carve(workspace);
   const int64_t pitch = dz_pitch(cv);
   uint16_t* dz = carve.take<uint16_t>((size_t)n_pad * pitch);
-  // a narrower last chunk may fill fewer pieces than the first
-  const int pieces = d_hidden ? d_hidden_pieces(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk) : 1;
-  float* acc32 = (d_hidden && (n_chunks > 1 || pieces > 1)) ? carve.take<float>((size_t)pieces * n_tokens * hidden_size)
-                                                            : nullptr;
+  // (a narrower last chunk may fill fewer pieces than the first)
+  const HiddenPlan hp = plan_hidden(n_tokens, planned_tokens, hidden_size, vocab, vocab_chunk);
+  const int pieces = d_hidden ? hp.pieces : 1, accumulators = d_hidden ? hp.accumulators(cv, vocab) : 0;
+  const bool few = d_hidden && hp.few;
+  float* acc32 = accumulators ? carve.take<float>((size_t)accumulators * n_tokens * hidden_size) : nullptr;
   const uint16_t* hid = static_cast<const uint16_t*>(hidden);
   const uint16_t* wgt = static_cast<const uint16_t*>(weight);
   const int h_tiles = (int)ceil_div(hidden_size, kTile);
@@ -1848,15 +1995,14 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     gh.R = Operand{dz, pitch, (int)n_tokens, (int)cv};
     gh.C = Operand{wgt + c0 * hidden_size, hidden_size, (int)hidden_size, (int)left};
     gh.k_slabs = (int)ceil_div(cols, kBK);
-    gh.r_tiles = d_hidden ? tok_tiles : 0;  // an input that needs no gradient leaves its GEMM an empty tile list
+    gh.r_tiles = d_hidden && !few ? tok_tiles : 0;  // an input that needs no gradient leaves its GEMM an empty tile list
     gh.c_tiles = h_tiles;
     gh.r_valid = (int)n_tokens;
     gh.c_valid = (int)hidden_size;
     // No more workgroups than pieces and tiles: with one on every CU, idle or not, and the tiles planned for all of them,
     // the backward of small heads took 85 instead of 73 us (2239 x 896 x 2000: 68 tiles), 44.5 instead of 42.1 (1209 x 128 x 1000).
-    const int64_t units = (int64_t)h_tiles * ((d_hidden ? (int64_t)tok_tiles * pieces : 0) + (want_dw ? chunk_tiles : 0));
+    const int64_t units = (int64_t)h_tiles * ((gh.r_tiles ? (int64_t)tok_tiles * pieces : 0) + (want_dw ? chunk_tiles : 0));
     const int workgroups = (int)(units < cus ? units : cus);
-    const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, d_hidden != nullptr, want_dw, workgroups, pieces);
     if (n_chunks == 1 && pieces == 1) gh.mode = kFinalBf16;
     else if (ci == 0) gh.mode = kStoreF32;
     else if (ci == n_chunks - 1 && pieces == 1) gh.mode = kFinalBf16AddPrev;
@@ -1877,14 +2023,25 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     gw.acc32 = d_weight_acc32 ? d_weight_acc32 + c0 * hidden_size : nullptr;
     gw.out = d_weight ? static_cast<uint16_t*>(d_weight) + c0 * hidden_size : nullptr;
     gw.ld_out = hidden_size;
-    {
-      ScopedTiming tm(kTagDGrad, s);
-      hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kGradStageBytes, s, gh, gw,
-                         plan);
+    if (few) {
+      const FewHiddenArgs f{gh.R, gh.C, gh.k_slabs, hp.split_slabs, h_tiles,
+                            streams_weight(hidden_size, vocab), acc32, (int)n_tokens, (int)hidden_size};
+      {
+        ScopedTiming tm(kTagDGrad, s);
+        hipLaunchKernelGGL(lce_dhidden_few_kernel, dim3(h_tiles * pieces), dim3(kThreads), kFewLds, s, f);
+      }
+      VAMD_LAUNCH_CHECK();
     }
-    VAMD_LAUNCH_CHECK();
+    if (workgroups > 0) {
+      const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, gh.r_tiles > 0, want_dw, workgroups, few ? 1 : pieces);
+      {
+        ScopedTiming tm(kTagDGrad, s);
+        hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kGradStageBytes, s, gh, gw, plan);
+      }
+      VAMD_LAUNCH_CHECK();
+    }
   }
-  if (pieces > 1) {
+  if (pieces > 1 || few) {
     const int64_t elements = n_tokens * hidden_size;
     {
       ScopedTiming tm(kTagDGrad, s);

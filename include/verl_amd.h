@@ -84,7 +84,7 @@ extern "C" {
 
 /* Bumped whenever an entry point is added or changes its signature, or a workspace its layout; a binding compares it
  * with the header it was written against. */
-#define VAMD_ABI_VERSION 6
+#define VAMD_ABI_VERSION 7
 int vamd_abi_version(void);
 const char* vamd_last_error(void);
 
@@ -240,6 +240,11 @@ int vamd_row_softmax_backward(const void* logits, int dtype, int64_t n_rows, int
 int vamd_row_softmax_backward_as(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
                                  const int64_t* labels, const float* lse, const float* mean_z, const void* d_logprobs,
                                  const void* d_entropy, int grad_dtype, void* d_logits, int64_t ld_out, void* stream);
+/* The same added to the gradient that d_logits holds, which is not the logits buffer: the sum of the gradients of two
+ * functions of the same logits, rounded to the element type once. */
+int vamd_row_softmax_backward_add(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld,
+                                  const int64_t* labels, const float* lse, const float* mean_z, const void* d_logprobs,
+                                  const void* d_entropy, int grad_dtype, void* d_logits, int64_t ld_out, void* stream);
 /* clip_by_value (verl/utils/torch_functional.py:203-221): out = max(min(x, hi), lo) over n fp32 elements, and its
  * gradients with torch's rule for binary min / max (the selected operand takes the gradient, equal operands half
  * each); d_x / d_lo / d_hi may be NULL.  A NaN in x, lo or hi gives a NaN output, as torch.min / torch.max of two
@@ -540,6 +545,9 @@ int vamd_policy_loss_cov_forward(int kind, const float* old_log_prob, const floa
                                  void* workspace, size_t workspace_bytes, void* stream);
 int vamd_scale_rows(const float* g, const float* coef, const float* d_loss, float extra_scale, int64_t rows,
                     int64_t cols, float* out, void* stream);
+/* The same added to a gradient that is there already (16-byte loads and stores where both buffers allow them). */
+int vamd_scale_rows_add(const float* g, const float* coef, const float* d_loss, float extra_scale, int64_t rows,
+                        int64_t cols, float* sum, void* stream);
 
 /* compute_value_loss (core_algos.py:1799-1838): out[0] = vf_loss, out[1] = vf_clipfrac;
  * grad_unscaled as above (d per-token loss / d vpreds * mask, before the 0.5 and agg_loss row

@@ -2305,3 +2305,51 @@ def test_native_losses_traced(dev, name, requires_grad):
         assert torch.equal(got, want) and got.requires_grad == requires_grad
         if requires_grad:
             assert torch.equal(torch.autograd.grad(got * 2.0, x)[0], torch.autograd.grad(want * 2.0, x)[0])
+
+
+@pytest.mark.parametrize("cols", [1, 3, 1024, 4097, 8190])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_scaled_rows_are_added_to_their_last_column_and_no_further(dev, cols, offset):
+    from verl_amd import _cabi
+    B, guard = 4, 8
+    x = _at_offset(torch.arange(B * cols, dtype=torch.float32, device=dev).view(B, cols), offset)
+    buf = torch.full((guard + offset + B * cols + guard,), -7.0, device=dev)
+    out = buf[guard + offset:guard + offset + B * cols]
+    coef = torch.tensor([1.0, 2.0, 4.0, 8.0], device=dev)
+    one = torch.ones(1, device=dev)
+    run = lambda p: _cabi.lib().vamd_scale_rows_add(x.data_ptr(), coef.data_ptr(), one.data_ptr(), 0.5, B, cols, p,
+                                                    _cabi.stream_ptr(dev))
+    _cabi.check(run(out.data_ptr()))
+    assert torch.equal(out.view(B, cols), x * (0.5 * coef[:, None]) - 7.0)
+    assert bool((buf[:guard + offset] == -7.0).all()) and bool((buf[guard + offset + B * cols:] == -7.0).all())
+    with pytest.raises(RuntimeError, match="scale_rows_add"):
+        _cabi.check(run(x.data_ptr()))
+
+
+@pytest.mark.parametrize("names", [("policy", "kl"), ("kl", "policy"), ("policy", "policy"), ("policy", "kl", "value"), ("kl", "agg")])
+def test_gradients_of_several_losses_are_summed(dev, names):
+    """Losses of the same tensor: the second node adds to the first one's gradient, to the bits of autograd's own sum; inputs in
+    another form and retained graphs come out the same."""
+    shape, losses = _native_losses(dev)
+    x = torch.randn(shape, device=dev, requires_grad=True)
+    scales = (1.0, 0.001, 3.0)
+
+    def total(t):
+        return sum(s * losses[n](t) for s, n in zip(scales, names))
+
+    alone = [torch.autograd.grad(s * losses[n](x), x)[0] for s, n in zip(scales, names)]
+    want = alone[-1]
+    for g in reversed(alone[:-1]):          # nodes run from the last to the first
+        want = want + g
+    loss = total(x)
+    for retain in (True, False):
+        assert torch.equal(torch.autograd.grad(loss, x, retain_graph=retain)[0], want)
+    y = x * 1.0
+    assert torch.equal(torch.autograd.grad(total(y), y)[0], want)
+    (created,) = torch.autograd.grad(total(x), x, create_graph=True)
+    assert torch.equal(created.detach(), want)
+    xd = x.detach().double().requires_grad_()
+    assert torch.allclose(torch.autograd.grad(total(xd), xd)[0].float(), want, rtol=1e-6, atol=1e-9)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        loss = total(x)
+    assert torch.equal(torch.autograd.grad(loss, x)[0], want)

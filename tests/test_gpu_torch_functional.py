@@ -479,3 +479,128 @@ def test_counter_buffers_are_allocated_without_a_lock(dev):
         thread.join()
         assert done.is_set() and mine.numel() >= (1 << 20) + 1 and not mine.any()
         assert _cabi.ticket_workspace(0, dev).data_ptr() == mine.data_ptr()
+
+
+def _summed(F, z, labels, order, third=None):
+    """log-probs and entropies of the same logits, in the order given (a gradient of 2 z before, between or after them)."""
+    parts = {"lp": lambda: F.logprobs_from_logits(z, labels, inplace_backward=False).float().sum(),
+             "ent": lambda: F.entropy_from_logits(z).float().sum(), "third": lambda: (2 * z).float().sum()}
+    names = list(order)
+    if third is not None:
+        names.insert(third, "third")
+    return sum(parts[n]() for n in names)
+
+
+@pytest.mark.parametrize("dtype,n,v", [(torch.float32, 3, 1001), (torch.float32, 2, 2048), (torch.bfloat16, 3, 7),
+                                       (torch.bfloat16, 5, 4096), (torch.bfloat16, 300, 2051), (torch.float16, 2, 2050)])
+@pytest.mark.parametrize("order", [("lp", "ent"), ("ent", "lp")])
+def test_gradients_of_two_functions_of_the_logits_are_summed(dev, dtype, n, v, order):
+    """The second node adds its gradient to the first one's, rounded once: within half a unit in the last place of the first
+    gradient and one of the sum of the fp64 value; the same through a leaf, a non-leaf, and a graph that is kept."""
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(n, v, dtype, seed=n + v)
+    z64 = z.double().requires_grad_()
+    parts = [torch.autograd.grad(f.sum(), z64)[0] for f in (OM.logprobs_from_logits(z64, labels), OM.entropy_from_logits(z64))]
+    want, lab = sum(parts), labels.to(dev)
+    zd = z.to(dev).requires_grad_()
+    loss = _summed(F, zd, lab, order)
+    first, = torch.autograd.grad(loss, zd, retain_graph=True)
+    slack = 1e-5 + HALF_ULP[dtype] * max(p.abs().max().item() for p in parts)
+    _assert_close(first, want, dtype, "sum", atol=slack)
+    again, = torch.autograd.grad(loss, zd)
+    loss = _summed(F, zd, lab, order)
+    loss.backward()
+    inner = zd * 1.0
+    inner.retain_grad()
+    _summed(F, inner, lab, order).backward()
+    assert torch.equal(again, first) and torch.equal(inner.grad, first)
+    # zd.grad: the sum of two passes
+    assert torch.equal(zd.grad, first + first)
+
+
+def test_summed_gradients_need_no_second_buffer(dev):
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(64, 65536, torch.float32, seed=1)
+    zd, lab = z.to(dev).requires_grad_(), labels.to(dev)
+    loss = _summed(F, zd, lab, ("lp", "ent"))
+    torch.cuda.reset_peak_memory_stats(dev)
+    before = torch.cuda.memory_allocated(dev)
+    got, = torch.autograd.grad(loss, zd)
+    assert got.nbytes <= torch.cuda.max_memory_allocated(dev) - before < 1.5 * got.nbytes
+
+
+def test_gradients_are_summed_apart_where_somebody_sees_them(dev):
+    """A third gradient, hooks, a graph of the gradients, a receiver on another stream, a caller that keeps the first gradient."""
+    import verl_amd.utils.torch_functional as F
+    n, v = 9, 1032
+    z, labels = _logits(n, v, torch.float32, seed=2)
+    zd, lab = z.to(dev).requires_grad_(), labels.to(dev)
+    alone = {k: torch.autograd.grad(_summed(F, zd, lab, (k,)), zd)[0] for k in ("lp", "ent")}
+    want = alone["ent"] + alone["lp"]
+    for order in (("lp", "ent"), ("ent", "lp")):
+        for third in (0, 1, 2):
+            y = zd * 1.0
+            got, = torch.autograd.grad(_summed(F, y, lab, order, third), y)
+            assert (got - want - 2).abs().max() <= 4 * 2.0 ** -23 * 3
+    for hooked in ("lp", "ent"):
+        lp, ent = F.logprobs_from_logits(zd, lab, inplace_backward=False), F.entropy_from_logits(zd)
+        seen = []
+        (lp if hooked == "lp" else ent).grad_fn.register_hook(lambda ins, outs: seen.append(ins[0].clone()))
+        got, = torch.autograd.grad(lp.sum() + ent.sum(), zd)
+        assert torch.equal(seen[0], alone[hooked]) and torch.equal(got, want)
+    kept = []
+    y = zd * 1.0
+    y.register_hook(lambda g: kept.append(g.clone()))          # sees the sum
+    got, = torch.autograd.grad(_summed(F, y, lab, ("lp", "ent")), y)
+    assert torch.equal(kept[0], want) and torch.equal(got, want)
+    got, = torch.autograd.grad(_summed(F, zd, lab, ("lp", "ent")), zd, create_graph=True)
+    assert torch.equal(got.detach(), want)
+    with torch.autograd.detect_anomaly(check_nan=True):
+        got, = torch.autograd.grad(_summed(F, zd, lab, ("lp", "ent")), zd)
+    assert torch.equal(got, want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ent = F.entropy_from_logits(zd)
+    torch.cuda.current_stream().wait_stream(side)
+    got, = torch.autograd.grad(F.logprobs_from_logits(zd, lab, inplace_backward=False).sum() + ent.sum(), zd)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    # over the logits: a gradient in their storage is nobody's to add to
+    y = zd * 1.0
+    lp, ent = F.logprobs_from_logits(y, lab, inplace_backward=True), F.entropy_from_logits(y)
+    got, = torch.autograd.grad(lp.sum() + ent.sum(), y)
+    assert torch.equal(got, want) and torch.equal(y.detach(), alone["lp"])
+
+
+def test_row_functions_traced_and_transformed(dev):
+    """A trace runs them on its own inputs; forward-mode differentiation and functorch's transforms are refused, a second
+    derivative raises."""
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(6, 300, torch.float32, seed=3)
+    zd, lab = z.to(dev), labels.to(dev)
+    f = lambda x, y: (F.logprobs_from_logits(x, y, inplace_backward=False), F.entropy_from_logits(x))
+    traced = torch.jit.trace(f, (torch.zeros_like(zd), lab), check_trace=False)
+    for a, b in zip(traced(zd, lab), f(zd, lab)):
+        assert torch.equal(a, b)
+    for fn in (F.entropy_from_logits, lambda x: F.logprobs_from_logits(x, lab)):
+        with pytest.raises(NotImplementedError), torch.autograd.forward_ad.dual_level():
+            fn(torch.autograd.forward_ad.make_dual(zd, torch.ones_like(zd)))
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda x: fn(x).sum())(zd)
+        with pytest.raises(RuntimeError):
+            torch.vmap(fn)(zd[None])
+    x = zd.clone().requires_grad_()
+    d, = torch.autograd.grad(F.logprobs_from_logits(x, lab, inplace_backward=False).sum(), x, create_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        d.sum().backward()
+
+
+def test_row_gradient_is_not_added_to_the_logits(dev):
+    from verl_amd import _cabi
+    z = torch.randn(2, 64, device=dev)
+    lse = torch.logsumexp(z, -1)
+    with pytest.raises(RuntimeError, match="added to the logits"):
+        _cabi.check(_cabi.lib().vamd_row_softmax_backward_add(
+            z.data_ptr(), 0, 2, 64, 64, None, lse.data_ptr(), lse.data_ptr(), None, lse.data_ptr(), 0, z.data_ptr(), 64,
+            _cabi.stream_ptr(z.device)))

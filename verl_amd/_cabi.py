@@ -68,6 +68,8 @@ SIGNATURES = {
                                           c_int, c_void_p, c_void_p, c_void_p]),
     "vamd_row_softmax_backward_as": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                              c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p]),
+    "vamd_row_softmax_backward_add": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+                                             c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p]),
     "vamd_clip_by_value": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "vamd_clip_by_value_backward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
                                             c_void_p, c_void_p]),
@@ -136,6 +138,7 @@ SIGNATURES = {
                                                  c_double, c_double, c_double, c_double, c_void_p, c_void_p,
                                                  c_void_p, c_void_p, c_size_t, c_void_p]),
     "vamd_scale_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int64, c_void_p, c_void_p]),
+    "vamd_scale_rows_add": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int64, c_void_p, c_void_p]),
     "vamd_kl_penalty": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "vamd_kl_loss_workspace_bytes": (c_size_t, [c_int64, c_int64]),
     "vamd_kl_loss_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_int,
@@ -151,7 +154,7 @@ def lib_path() -> str:
     return _LIB_PATH
 
 
-ABI_VERSION = 6  # VAMD_ABI_VERSION of include/verl_amd.h
+ABI_VERSION = 7  # VAMD_ABI_VERSION of include/verl_amd.h
 
 
 def load_library(path: str | None = None) -> ctypes.CDLL:

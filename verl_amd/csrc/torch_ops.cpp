@@ -11,8 +11,12 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/anomaly_mode.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/extension.h>
 
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <map>
@@ -169,8 +173,87 @@ Tensor in_saved_form(AutogradContext* ctx, Tensor g) {
 
 Tensor upstream(const Tensor& d_loss, const at::Device& dev) { return as_f32(d_loss, dev).reshape({1}); }
 
+// ---- sums of gradients ---------------------------------------------------------------------------------------
+// Two nodes that differentiate the same tensor (entropy and log-probs of the logits, KL loss and policy loss of the
+// log-probs) each hand autograd a gradient, which it adds up in a pass of its own: two tensors read and one written.  The
+// node that runs second may add its gradient to the first one's instead, in the kernel that forms it, and hand back none.
+// Both gradients go to the same input of the same node of one running backward pass, which cannot read the sum before both
+// have arrived, so the only thing to make sure of is that the first gradient is as its node left it and is held by autograd
+// alone: a weak reference to it is kept, per thread, and it is joined only if
+//   - the same backward pass (its id is never used again) still runs, on this thread, and records no graph of its own;
+//   - one reference to the tensor and one to its storage are left, and its version is that of then: nobody else (a hook, a
+//     third gradient that was added to it or that it was added to) has it or has had it;
+//   - neither node has hooks, which would see the gradients apart, and anomaly detection, which looks at each, is off;
+//   - both kernels run on the stream on which the node that receives the sum runs.
+// Otherwise the second node hands back a gradient of its own, as ever.  (Figures: scale_rows_add_kernel and
+// row_softmax_backward_kernel.)
+using torch::autograd::Edge;
+struct Summand {
+  int pass = -1;  // id of the backward pass
+  torch::autograd::Node* receiver = nullptr;
+  uint32_t input = 0, version = 0;
+  std::optional<c10::weak_intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>> grad;
+};
+constexpr int kSummands = 4;  // the newest gradients of a thread
+struct Summands {
+  std::array<Summand, kSummands> list;
+  int next = 0;
+};
+Summands& summands() {
+  static thread_local Summands s;
+  return s;
+}
+
+// Where the running node's gradient of its input 0 goes, if that may be summed here.
+std::optional<Edge> sum_edge(const at::Device& dev) {
+  if (torch::autograd::get_current_graph_task_id() < 0 || at::GradMode::is_enabled() ||
+      torch::autograd::AnomalyMode::is_enabled())
+    return std::nullopt;
+  const auto node = torch::autograd::get_current_node();
+  if (!node || node->num_outputs() == 0 || !node->post_hooks().empty()) return std::nullopt;
+  const Edge edge = node->next_edge(0);
+  if (!edge.is_valid()) return std::nullopt;
+  const auto stream = edge.function->stream();
+  const auto mine = c10::hip::getCurrentHIPStream(dev.index());
+  if (!stream || stream->device_index() != mine.device_index() || stream->id() != mine.id()) return std::nullopt;
+  return edge;
+}
+
+// The gradient that the running node may add its own to (and then return none), or an undefined tensor.
+Tensor gradient_to_join(at::IntArrayRef shape, at::ScalarType dtype, const at::Device& dev) {
+  const auto edge = sum_edge(dev);
+  if (!edge) return Tensor();
+  const int pass = torch::autograd::get_current_graph_task_id();
+  for (Summand& s : summands().list) {
+    if (s.pass != pass || s.receiver != edge->function.get() || s.input != edge->input_nr || !s.grad) continue;
+    auto held = s.grad->lock();
+    if (!held || held.use_count() != 2) continue;  // autograd's reference and this one
+    const Tensor sum(std::move(held));
+    if (sum._version() == s.version && sum.storage().use_count() == 1 && sum.sizes() == shape &&
+        sum.scalar_type() == dtype && sum.device() == dev)
+      return sum;
+  }
+  return Tensor();
+}
+
+// The running node is about to return `grad`, which it made itself, as its gradient of input 0.
+void gradient_returned(const Tensor& grad) {
+  if (!grad.defined() || !grad.is_cuda() || !grad.is_contiguous()) return;
+  const auto edge = sum_edge(grad.device());
+  if (!edge) return;
+  Summands& all = summands();
+  Summand& s = all.list[all.next];
+  all.next = (all.next + 1) % kSummands;
+  s.pass = torch::autograd::get_current_graph_task_id();
+  s.receiver = edge->function.get();  // compared, never followed
+  s.input = edge->input_nr;
+  s.version = grad._version();
+  s.grad.emplace(grad.getIntrusivePtr());
+}
+
 // The gradient of a loss whose forward pass left it per unit upstream gradient.
 variable_list scaled_gradient(AutogradContext* ctx, const variable_list& grads, float extra_scale, size_t inputs) {
+  const bool records = at::GradMode::is_enabled();
   at::AutoGradMode no_grad(false);
   variable_list result(inputs);
   const auto saved = ctx->get_saved_variables();
@@ -180,10 +263,159 @@ variable_list scaled_gradient(AutogradContext* ctx, const variable_list& grads, 
   const at::Device dev = g.device();
   const c10::DeviceGuard guard(dev);
   const Tensor d = upstream(grads[0], dev);
+  const bool may_join = !records && ctx->saved_data.find("shape") == ctx->saved_data.end();
+  const Tensor sum = may_join ? gradient_to_join(g.sizes(), at::kFloat, dev) : Tensor();
+  if (sum.defined()) {
+    check(vamd_scale_rows_add(f32(g), f32(coef), f32(d), extra_scale, g.size(0), g.size(1), f32_out(sum), stream_of(dev)));
+    return result;
+  }
   const Tensor out = at::empty_like(g);
   check(vamd_scale_rows(f32(g), f32(coef), f32(d), extra_scale, g.size(0), g.size(1), f32_out(out), stream_of(dev)));
   result[0] = in_saved_form(ctx, out);
+  if (may_join) gradient_returned(out);
   return result;
+}
+
+// ---- log-probs and entropies of materialised logits ----------------------------------------------------------
+// Nodes in C++ because two of them on the same logits sum their gradients (a gradient that Python has seen is never autograd's
+// alone), and because up to a few hundred rows the host is what a call waits for.
+struct Rows {
+  Tensor t;     // [rows, vocab], unit stride along the vocabulary
+  int64_t ld;   // row pitch
+  int type;     // VAMD_DT_*
+  const void* data() const { return t.const_data_ptr(); }
+  int64_t n() const { return t.size(0); }
+  int64_t vocab() const { return t.size(1); }
+};
+int row_type(at::ScalarType type) {
+  return type == at::kFloat ? VAMD_DT_F32 : type == at::kBFloat16 ? VAMD_DT_BF16 : type == at::kHalf ? VAMD_DT_F16 : -1;
+}
+Rows logit_rows(const Tensor& logits) {
+  if (!logits.is_cuda()) raise_assertion("the logits must live on the GPU: there is no CPU fallback");
+  const int type = row_type(logits.scalar_type());
+  if (type < 0) raise_assertion(std::string("logits must be fp32, bf16 or fp16, got ") + c10::toString(logits.scalar_type()));
+  if (logits.dim() < 1 || logits.numel() == 0) raise_assertion("");
+  const int64_t vocab = logits.size(-1);
+  Tensor rows = logits.reshape({-1, vocab});
+  if (rows.stride(1) != 1 || (rows.size(0) > 1 && rows.stride(0) < vocab)) rows = rows.contiguous();
+  return {rows, rows.size(0) > 1 ? rows.stride(0) : vocab, type};
+}
+Tensor label_rows(const Tensor& labels, const Tensor& logits) {
+  if (logits.dim() < 1 || labels.sizes() != logits.sizes().slice(0, logits.dim() - 1))
+    raise_assertion("labels " + shape_text(labels) + " do not match logits " + shape_text(logits));
+  return labels.reshape({-1}).to(logits.device(), at::kLong).contiguous();
+}
+
+struct RowStats {
+  Tensor value, lse, mean_z;  // log-prob or entropy in `type`; what the backward pass needs, in fp32
+};
+// log-probs of `labels`, or without labels entropies
+RowStats row_stats(const Tensor& logits, const Rows& r, const Tensor& labels, at::ScalarType type, bool need_grad) {
+  const at::Device dev = logits.device();
+  const c10::DeviceGuard guard(dev);
+  const bool entropy = !labels.defined();
+  const Tensor value = at::empty(logits.sizes().slice(0, logits.dim() - 1), at::TensorOptions().dtype(type).device(dev));
+  const Tensor kept = need_grad ? new_f32({entropy ? 2 : 1, r.n()}, dev) : Tensor();
+  const Tensor lse = need_grad ? kept.select(0, 0) : Tensor(), mean_z = need_grad && entropy ? kept.select(0, 1) : Tensor();
+  void* const out = value.mutable_data_ptr();
+  check(vamd_row_softmax_stats_as(r.data(), r.type, r.n(), r.vocab(), r.ld,
+                                  entropy ? nullptr : labels.const_data_ptr<int64_t>(), entropy ? nullptr : out,
+                                  entropy ? out : nullptr, row_type(type), f32_out(lse), f32_out(mean_z), stream_of(dev)));
+  return {value, lse, mean_z};
+}
+
+// The gradient of the logits in `shape`, or an undefined tensor where it went into the other node's.
+Tensor row_gradient(const Rows& r, const Tensor& labels, const Tensor& lse, const Tensor& mean_z, const Tensor& upstream,
+                    at::IntArrayRef shape, bool in_place, bool may_join) {
+  const at::Device dev = r.t.device();
+  const c10::DeviceGuard guard(dev);
+  const at::ScalarType type = upstream.scalar_type() == r.t.scalar_type() ? upstream.scalar_type() : at::kFloat;
+  const Tensor g = upstream.detach().reshape({-1}).to(dev, type).contiguous();
+  const bool entropy = mean_z.defined();
+  const Tensor sum = may_join && !in_place ? gradient_to_join(shape, r.t.scalar_type(), dev) : Tensor();
+  const Tensor out = in_place ? r.t : sum.defined() ? sum : at::empty(shape, r.t.options());
+  check((sum.defined() ? vamd_row_softmax_backward_add : vamd_row_softmax_backward_as)(
+      r.data(), r.type, r.n(), r.vocab(), r.ld, entropy ? nullptr : labels.const_data_ptr<int64_t>(), f32(lse), f32(mean_z),
+      entropy ? nullptr : g.const_data_ptr(), entropy ? g.const_data_ptr() : nullptr, row_type(type), out.mutable_data_ptr(),
+      in_place ? r.ld : r.vocab(), stream_of(dev)));
+  if (sum.defined()) return Tensor();
+  if (in_place) return out.view(shape);
+  if (may_join) gradient_returned(out);
+  return out;
+}
+
+class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
+ public:
+  static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels, bool inplace_backward) {
+    const Tensor lab = label_rows(labels, logits);
+    const Rows r = logit_rows(logits);
+    const RowStats s = row_stats(logits, r, lab, logits.scalar_type(), true);
+    ctx->save_for_backward({r.t, lab, s.lse});
+    ctx->saved_data["ld"] = r.ld;
+    ctx->saved_data["shape"] = logits.sizes().vec();
+    // writing the gradient over the logits needs the rows to be the caller's storage, and never overwrites a parameter
+    ctx->saved_data["in_place"] = inplace_backward && r.data() == logits.const_data_ptr() && logits.is_contiguous() &&
+                                  !(logits.is_leaf() && logits.requires_grad());
+    return s.value;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const bool records = at::GradMode::is_enabled();
+    Tensor d;
+    {
+      at::AutoGradMode no_grad(false);
+      const auto saved = ctx->get_saved_variables();
+      const bool in_place = ctx->saved_data["in_place"].toBool();
+      if (in_place) {
+        // the logits are about to become their own gradient: a second pass over this node would read gradients where
+        // it expects logits
+        TORCH_CHECK(!ctx->saved_data.count("logits_overwritten"),
+                    "logprobs_from_logits(inplace_backward=True) wrote the gradient over the logits in its first backward "
+                    "pass and cannot run a second one; pass inplace_backward=False to keep the logits");
+        ctx->saved_data["logits_overwritten"] = true;
+      }
+      const Rows r{saved[0], ctx->saved_data["ld"].toInt(), row_type(saved[0].scalar_type())};
+      d = row_gradient(r, saved[1], saved[2], Tensor(), grads[0], ctx->saved_data["shape"].toIntVector(), in_place, !records);
+    }
+    if (records)  // the gradient is no function of its own to differentiate
+      d = torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable",
+                                        1)({d.detach().requires_grad_()})[0];
+    return {d, Tensor(), Tensor()};
+  }
+};
+
+class RowEntropy : public torch::autograd::Function<RowEntropy> {
+ public:
+  static Tensor forward(AutogradContext* ctx, const Tensor& logits, bool fp32_output) {
+    const Rows r = logit_rows(logits);
+    const RowStats s = row_stats(logits, r, Tensor(), fp32_output ? at::kFloat : logits.scalar_type(), true);
+    ctx->save_for_backward({r.t, s.lse, s.mean_z});
+    ctx->saved_data["ld"] = r.ld;
+    ctx->saved_data["shape"] = logits.sizes().vec();
+    return s.value;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const bool records = at::GradMode::is_enabled();
+    at::AutoGradMode no_grad(false);
+    const auto saved = ctx->get_saved_variables();
+    const Rows r{saved[0], ctx->saved_data["ld"].toInt(), row_type(saved[0].scalar_type())};
+    return {row_gradient(r, Tensor(), saved[1], saved[2], grads[0], ctx->saved_data["shape"].toIntVector(), false, !records),
+            Tensor()};
+  }
+};
+
+Tensor logprobs_from_logits(const Tensor& logits, const Tensor& labels, bool inplace_backward) {
+  refuse_tangents("logprobs_from_logits", {&logits});
+  if (wants_gradient(logits)) return RowLogprobs::apply(logits, labels, inplace_backward);
+  at::AutoGradMode no_grad(false);
+  const Tensor lab = label_rows(labels, logits);
+  return row_stats(logits, logit_rows(logits), lab, logits.scalar_type(), false).value;
+}
+
+Tensor entropy_from_logits(const Tensor& logits, bool fp32_output) {
+  refuse_tangents("entropy_from_logits", {&logits});
+  if (wants_gradient(logits)) return RowEntropy::apply(logits, fp32_output);
+  at::AutoGradMode no_grad(false);
+  return row_stats(logits, logit_rows(logits), Tensor(), fp32_output ? at::kFloat : logits.scalar_type(), false).value;
 }
 
 // ---- policy loss ---------------------------------------------------------------------------------------------
@@ -615,6 +847,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     if (!dev.has_index()) dev.set_index(c10::hip::current_device());
     return ticket_workspace((size_t)(bytes < 0 ? 0 : bytes), dev);
   });
+  m.def("logprobs_from_logits", &logprobs_from_logits);
+  m.def("entropy_from_logits", &entropy_from_logits);
   m.def("policy_loss", &policy_loss);
   m.def("value_loss", &value_loss);
   m.def("kl_loss", &kl_loss);

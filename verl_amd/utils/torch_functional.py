@@ -65,6 +65,14 @@ def _row_backward(rows, ld, labels, lse, mean_z, d_logprobs, d_entropy, in_place
     return out
 
 
+def _native_rows(name: str, traced, logits: torch.Tensor, *rest):
+    """The row function ``name`` of the native host side; while ``torch.jit.trace`` records, the Python function ``traced``,
+    which a trace keeps as one operation."""
+    if not logits.is_cuda or torch._C._get_tracing_state() is not None:
+        return traced.apply(logits, *rest)
+    return getattr(_cabi.ops(), name)(logits, *rest)
+
+
 class _LogProbsFromLogits(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, labels, inplace_backward: bool):
@@ -119,30 +127,30 @@ def logprobs_from_logits(logits: torch.Tensor, labels: torch.Tensor, inplace_bac
     (``cross_entropy_loss(..., inplace_backward=True)``); the reference does so only where flash-attn is
     installed, this function always.  Pass ``False`` when the logits are read again after the backward pass or
     the graph is backpropagated twice (a second pass raises instead of differentiating gradients)."""
-    return _LogProbsFromLogits.apply(logits, labels, inplace_backward)
+    return _native_rows("logprobs_from_logits", _LogProbsFromLogits, logits, labels, bool(inplace_backward))
 
 
 def logprobs_from_logits_naive(logits: torch.Tensor, labels: torch.Tensor) -> torch.Tensor:
     """``log_softmax`` + gather (reference torch_functional.py:148-163)."""
-    return _LogProbsFromLogits.apply(logits, labels, False)
+    return _native_rows("logprobs_from_logits", _LogProbsFromLogits, logits, labels, False)
 
 
 def logprobs_from_logits_v2(logits: torch.Tensor, labels: torch.Tensor) -> torch.Tensor:
     """``logits[label] - logsumexp(logits)`` row by row (reference torch_functional.py:166-200); fp32 arithmetic for
     every input dtype, one rounding to the dtype of ``logits`` at the end."""
-    return _LogProbsFromLogits.apply(logits, labels, False)
+    return _native_rows("logprobs_from_logits", _LogProbsFromLogits, logits, labels, False)
 
 
 def entropy_from_logits(logits: torch.Tensor) -> torch.Tensor:
     """``logsumexp(logits) - sum(softmax(logits) * logits)`` (reference torch_functional.py:224-238), dtype of
     ``logits``."""
-    return _EntropyFromLogits.apply(logits, False)
+    return _native_rows("entropy_from_logits", _EntropyFromLogits, logits, False)
 
 
 def entropy_from_logits_with_chunking(logits: torch.Tensor, chunk_size: int = 2048) -> torch.Tensor:
     """The same in fp32 whatever the dtype of ``logits`` (reference torch_functional.py:241-263).  ``chunk_size``
     is accepted for the signature: the kernel walks a row at a time and holds no ``[chunk, vocab]`` temporaries."""
-    return _EntropyFromLogits.apply(logits, True)
+    return _native_rows("entropy_from_logits", _EntropyFromLogits, logits, True)
 
 
 class _ClipByValue(torch.autograd.Function):

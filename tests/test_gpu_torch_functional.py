@@ -604,3 +604,26 @@ def test_row_gradient_is_not_added_to_the_logits(dev):
         _cabi.check(_cabi.lib().vamd_row_softmax_backward_add(
             z.data_ptr(), 0, 2, 64, 64, None, lse.data_ptr(), lse.data_ptr(), None, lse.data_ptr(), 0, z.data_ptr(), 64,
             _cabi.stream_ptr(z.device)))
+
+
+@pytest.mark.parametrize("dtype,n,v", [(torch.float32, 160, 524288), (torch.float32, 161, 524287), (torch.bfloat16, 322, 524289)])
+def test_logits_at_the_size_of_the_memory_side_cache(dev, dtype, n, v):
+    """320 MB of logits and just over: the last row read with plain loads and the first one read past the caches."""
+    import verl_amd.utils.torch_functional as F
+    z = torch.randn(n, v, generator=torch.Generator(device=dev).manual_seed(v), device=dev).to(dtype)
+    labels = torch.arange(n, device=dev) * 7
+    x = z.requires_grad_()
+    lp, ent = F.logprobs_from_logits(x, labels, inplace_backward=False), F.entropy_from_logits_with_chunking(x)
+    d, = torch.autograd.grad(lp.float().sum() + ent.sum(), x)
+    for r in [0, 1, *range(100, 120), *range(n - 110, n)]:
+        z64 = z[r].detach().double()
+        lse = torch.logsumexp(z64, -1)
+        p = torch.exp(z64 - lse)
+        want_ent = lse - (p * z64).sum()
+        one = torch.zeros_like(p)
+        one[labels[r]] = 1
+        for got, want, kind, what, atol in ((lp[r], z64[labels[r]] - lse, dtype, "log-prob", 1e-5),
+                                            (ent[r], want_ent, torch.float32, "entropy", 2e-5),
+                                            (d[r], one - p - p * (z64 - (p * z64).sum()), dtype, "gradient", 1e-7)):
+            bound = atol + (1e-5 + 2 * HALF_ULP[kind]) * want.abs()
+            assert ((got.detach().double() - want).abs() <= bound).all(), (r, what)

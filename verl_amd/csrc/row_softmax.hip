@@ -54,10 +54,12 @@ struct Group {
   using type = std::conditional_t<VEC, u32x4_t, std::conditional_t<sizeof(typename D::type) == 4, u32x4_at4_t, u32x4_at2_t>>;
 };
 
-// logits are read once and never again by a launch: non-temporal, which is worth 7 % of HBM bandwidth here
-template <class D, bool VEC>
+// A launch reads logits once.  STREAM: non-temporal, which is worth 7 % of HBM bandwidth over logits that no cache holds.
+template <class D, bool VEC, bool STREAM>
 __device__ __forceinline__ u32x4_t load_whole(const typename D::type* __restrict__ p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const typename Group<D, VEC>::type*>(p));
+  const auto* const q = reinterpret_cast<const typename Group<D, VEC>::type*>(p);
+  if constexpr (STREAM) return __builtin_nontemporal_load(q);
+  else return *q;
 }
 
 // The ragged group a row ends in: elements at or beyond `cols` read as `fill`.
@@ -101,6 +103,7 @@ struct StatsArgs {
   bool typed;      // they have the element type of the logits
   float* lse;
   float* mean_z;
+  int64_t cached_rows;  // cached_rows()
 };
 
 // Element r of a per-row vector whose elements are D's (typed) or fp32.  16-bit callers' results leave and their upstream
@@ -131,14 +134,11 @@ __device__ __forceinline__ float load_row_value(const void* p, unsigned r, unsig
   else return (float)__builtin_bit_cast(_Float16, bits);
 }
 
-template <class D, bool VEC, int NT>
-__global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
-  using T = typename D::type;
+// One thread's part of a row: running state in the log2 domain, m = max of z log2(e), s = sum 2^(y - m), sz = sum 2^(y - m) z
+template <class D, bool VEC, bool STREAM, int NT>
+__device__ __forceinline__ void walk_row(const typename D::type* __restrict__ row, const StatsArgs& a, float& m, float& s,
+                                         float& sz) {
   constexpr int G = D::kVec;
-  const int64_t r = blockIdx.x;
-  const T* __restrict__ row = static_cast<const T*>(a.logits) + r * a.ld;
-  // running state in the log2 domain: m = max of z log2(e), s = sum 2^(y - m), sz = sum 2^(y - m) z
-  float m = kNegBig, s = 0.f, sz = 0.f;
   const int64_t stride = (int64_t)NT * G;
   for (int64_t c0 = (int64_t)threadIdx.x * G; c0 < a.cols; c0 += stride * kInFlight) {
     // whole 16-byte groups are all requested first; a ragged last group is fetched element by element afterwards
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
       const int64_t c = c0 + u * stride;
-      if (c + G <= a.cols) raw[u] = load_whole<D, VEC>(row + c);
+      if (c + G <= a.cols) raw[u] = load_whole<D, VEC, STREAM>(row + c);
     }
     float x[kInFlight][G];
 #pragma unroll
@@ -185,6 +185,16 @@ __global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
         sz = fmaf(ex, z, sz);  // padding: 0 * -1e30; a true -inf logit gives NaN, as softmax(z) * z does
       }
   }
+}
+
+template <class D, bool VEC, int NT>
+__global__ __launch_bounds__(NT) void row_softmax_stats_kernel(StatsArgs a) {
+  using T = typename D::type;
+  const int64_t r = blockIdx.x;
+  const T* __restrict__ row = static_cast<const T*>(a.logits) + r * a.ld;
+  float m = kNegBig, s = 0.f, sz = 0.f;
+  if (r < a.cached_rows) walk_row<D, VEC, false, NT>(row, a, m, s, sz);
+  else walk_row<D, VEC, true, NT>(row, a, m, s, sz);
   // wavefront, then workgroup
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
@@ -240,7 +250,7 @@ struct BackwardArgs {
 // over two and autograd's own sum over three (log-probs, entropies and both gradients, 3001 x 152064 bf16: 1315 -> 988 us).
 // TYPED: d_logprobs and d_entropy have the element type of the logits (a kernel of its own: every one of its many small
 // workgroups would start with the choice).
-template <class D, bool VEC, bool TYPED, bool ADD>
+template <class D, bool VEC, bool TYPED, bool ADD, bool STREAM>
 __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(BackwardArgs a) {
   using T = typename D::type;
   constexpr int G = D::kVec, F = D::kBackwardLoads;
@@ -258,8 +268,8 @@ __global__ __launch_bounds__(kRowThreads) void row_softmax_backward_kernel(Backw
   for (int u = 0; u < F; ++u) {
     const int64_t c = c0 + u * stride;
     if (c + G <= a.cols) {
-      raw[u] = load_whole<D, VEC>(row + c);
-      if constexpr (ADD) before[u] = load_whole<D, VEC>(out + c);
+      raw[u] = load_whole<D, VEC, STREAM>(row + c);
+      if constexpr (ADD) before[u] = load_whole<D, VEC, true>(out + c);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -348,6 +358,19 @@ bool rows_vectorizable(const void* base, int64_t ld) {
   return reinterpret_cast<uintptr_t>(base) % 16 == 0 && (ld * (int64_t)sizeof(typename D::type)) % 16 == 0;
 }
 
+// Rows of the logits that are read with plain loads, which leave them in the 256 MB memory-side cache for the next pass over the
+// same logits (log-probs, entropies and the two gradients are four).  Logits that about fit are all read so; of larger ones the
+// forward pass reads the first 224 MB so, the rest with the non-temporal hint, which does not displace them.  The four passes, all
+// non-temporal and so, us: bf16 300 x 152064 (91 MB) 130 -> 117, 500 rows 180 -> 160, 800 rows (243 MB) 280 -> 258, 1000 rows
+// (304 MB) 334 -> 327, 1500 rows 501 -> 493, 3001 rows 985 -> 976; fp32 400 x 151936 (243 MB) 280 -> 240, 500 rows 334 -> 312,
+// 1500 rows 1030 -> 1013.  With plain loads for everything 1500 rows bf16 take 513, 3001 rows 1023; with the choice inside the
+// backward kernel, whose small workgroups it delays, 800 rows 296.
+constexpr int64_t kFittingBytes = 320ll << 20, kCachedBytes = 224ll << 20;
+int64_t cached_rows(int64_t n_rows, int64_t ld, size_t element) {
+  const int64_t pitch = ld * (int64_t)element;
+  return n_rows * pitch <= kFittingBytes ? n_rows : kCachedBytes / pitch;
+}
+
 int check_rows(const char* what, const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t ld) {
   VAMD_REQUIRE(logits != nullptr, "%s: null logits", what);
   VAMD_REQUIRE(dtype >= VAMD_DT_F32 && dtype <= VAMD_DT_F16, "%s: unknown element type code %d", what, dtype);
@@ -400,9 +423,10 @@ extern "C" int vamd_row_softmax_stats_as(const void* logits, int dtype, int64_t 
                "row_softmax_stats: outputs are fp32 or of the logits' type, not of type %d", out_dtype);
   VAMD_REQUIRE((logprobs == nullptr) || labels, "row_softmax_stats: logprobs need labels");
   VAMD_REQUIRE(logprobs || entropy || lse || mean_z, "row_softmax_stats: no output requested");
-  StatsArgs a{logits, ld, labels, vocab, logprobs, entropy, out_dtype == dtype, lse, mean_z};
+  StatsArgs a{logits, ld, labels, vocab, logprobs, entropy, out_dtype == dtype, lse, mean_z, 0};
   hipStream_t s = static_cast<hipStream_t>(stream);
   VAMD_DTYPE_DISPATCH(dtype, D, {
+    a.cached_rows = cached_rows(n_rows, ld, sizeof(typename D::type));
     if (rows_vectorizable<D>(logits, ld)) launch_stats<D, true>(a, n_rows, s);
     else launch_stats<D, false>(a, n_rows, s);
   });
@@ -437,17 +461,23 @@ static int row_backward(const char* what, bool add, const void* logits, int dtyp
     const int64_t per_wg = (int64_t)kRowThreads * D::kVec * D::kBackwardLoads;
     const int64_t chunks = (vocab + per_wg - 1) / per_wg;
     VAMD_REQUIRE(n_rows * chunks < (1ll << 31), "%s: too many workgroups", what);
-    BackwardArgs a{logits, ld, labels, lse, mean_z, d_logprobs, d_entropy, (unsigned)n_rows, d_logits, ld_out, vocab, (int)chunks};
+    BackwardArgs a{logits, ld, labels, lse, mean_z, d_logprobs, d_entropy, (unsigned)n_rows, d_logits, ld_out, vocab,
+                   (int)chunks};
     const dim3 grid((unsigned)(n_rows * chunks));
     const bool vec = rows_vectorizable<D>(logits, ld) && rows_vectorizable<D>(d_logits, ld_out);
     constexpr bool kSmall = sizeof(typename D::type) < 4;
     const bool typed = kSmall && grad_dtype == dtype;
-    void (*const kernels[2][2][2])(BackwardArgs) = {
-        {{row_softmax_backward_kernel<D, false, false, false>, row_softmax_backward_kernel<D, false, false, true>},
-         {row_softmax_backward_kernel<D, false, kSmall, false>, row_softmax_backward_kernel<D, false, kSmall, true>}},
-        {{row_softmax_backward_kernel<D, true, false, false>, row_softmax_backward_kernel<D, true, false, true>},
-         {row_softmax_backward_kernel<D, true, kSmall, false>, row_softmax_backward_kernel<D, true, kSmall, true>}}};
-    hipLaunchKernelGGL(kernels[vec][typed][add], grid, dim3(kRowThreads), 0, s, a);
+    const bool stream = cached_rows(n_rows, ld, sizeof(typename D::type)) < n_rows;
+    void (*const kernels[2][2][2][2])(BackwardArgs) = {
+        {{{row_softmax_backward_kernel<D, false, false, false, false>, row_softmax_backward_kernel<D, false, false, false, true>},
+          {row_softmax_backward_kernel<D, false, false, true, false>, row_softmax_backward_kernel<D, false, false, true, true>}},
+         {{row_softmax_backward_kernel<D, false, kSmall, false, false>, row_softmax_backward_kernel<D, false, kSmall, false, true>},
+          {row_softmax_backward_kernel<D, false, kSmall, true, false>, row_softmax_backward_kernel<D, false, kSmall, true, true>}}},
+        {{{row_softmax_backward_kernel<D, true, false, false, false>, row_softmax_backward_kernel<D, true, false, false, true>},
+          {row_softmax_backward_kernel<D, true, false, true, false>, row_softmax_backward_kernel<D, true, false, true, true>}},
+         {{row_softmax_backward_kernel<D, true, kSmall, false, false>, row_softmax_backward_kernel<D, true, kSmall, false, true>},
+          {row_softmax_backward_kernel<D, true, kSmall, true, false>, row_softmax_backward_kernel<D, true, kSmall, true, true>}}}};
+    hipLaunchKernelGGL(kernels[vec][typed][add][stream], grid, dim3(kRowThreads), 0, s, a);
   });
   VAMD_LAUNCH_CHECK();
   return VAMD_OK;

@@ -154,7 +154,7 @@ struct FwdArgs {
   float4* partials;  // [plan.slots()][256] : (max in the log2 domain, sum e, sum e x with x = hidden . weight, label logit)
   float* z_cache;    // optional [n_tokens][vocab] fp32 logits / temperature, kept for the backward
   float* pi2_partials;  // optional [plan.slots()][256] : sum of e^2 relative to the same max
-  int stream_weight;    // lce_forward_few_kernel: streams_weight()
+  int stream_from;      // lce_forward_few_kernel: stream_from()
 };
 
 // The tiles of one workgroup.  The two ways of sharing out are kernels of their own: with both in one kernel the split
@@ -572,12 +572,13 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
 // 93 x 3584 x 152064 5.4 TB/s, 93 x 4096 x 128256 5.7 TB/s.  From 129 tokens on the 256-token tile's padding is less than half.  A wavefront owns 64 tokens
 // x 64 columns (2 x 4 wavefronts) and keeps the softmax state of its tokens in registers to the end.
 constexpr int kFewTokens = 128;
-// The few-token kernels read every piece of the weight in one workgroup.  From three times the 256 MB memory-side cache on, when
-// little of the weight can still be there in the next pass, they read it with the non-temporal hint, which also leaves the caches to
-// the logits and the panel.  Forward pass over 64 tokens at 151936 columns, without and with it, us: hidden size 896 (272 MB)
-// 52.7 and 57.2, 1536 (467 MB) 96 and 90, 2560 (778 MB) 152 and 146; 4096 x 128256 (1.05 GB) 187 and 170; with the backward pass
-// 896 203 and 211, 2048 (622 MB) 392 and 405, 2560 480 and 473, 3584 x 152064 621 and 617, 128 tokens 716 and 689.
-constexpr int64_t kStreamWeightBytes = 768ll << 20;
+// The few-token kernels read every piece of the weight in one workgroup, and the backward pass reads it again.  A weight that about
+// fits the 256 MB memory-side cache is read with plain loads; of a larger one the workgroups on the first 200 MB, and the others
+// with the non-temporal hint, which leaves those there.  Everything with plain loads, everything with the hint and so, us: forward
+// pass over 64 tokens at 151936 columns, hidden size 1536 (467 MB) 98, 92 and 88, 2048 138, 130 and 111, 3584 x 152064 194, 187
+// and 183; with the backward pass 1536 313, 310 and 293, 2048 392, 407 and 363, 2560 483, 474 and 459, 3584 621, 618 and 608,
+// 128 tokens 716, 690 and 675.  896 (272 MB) 203, 211 and with 200 MB kept 208.
+constexpr int64_t kFittingWeightBytes = 320ll << 20, kCachedWeightBytes = 200ll << 20;
 constexpr int kFewStageBytes = (kFewTokens + kTile) * kBK * 2;
 constexpr int kFewStages = 3;
 constexpr int kFewLds = kFewStages * kFewStageBytes;
@@ -646,7 +647,7 @@ __global__ __launch_bounds__(kThreads) void lce_forward_few_kernel(FwdArgs a) {
     const unsigned base = lds_address(lds) + (unsigned)fill * kFewStageBytes;
 #pragma unroll
     for (int i = 0; i < kFewLoadsR; ++i) dma.issue_one(i, r, base);
-    few_fetch_weight(dma, c, base + kFewTokens * kBK * 2, a.stream_weight);
+    few_fetch_weight(dma, c, base + kFewTokens * kBK * 2, c_begin >= a.stream_from);
     fill = fill == kFewStages - 1 ? 0 : fill + 1;
     if (t2 == tiles - 1 && k2 == a.k_slabs - 1) return;
     if (++k2 == a.k_slabs) {
@@ -1335,8 +1336,8 @@ struct FewHiddenArgs {
   Operand dz;      // R: [n_tokens][panel pitch], k = panel column
   Operand weight;  // C: K-major, [vocab][hidden]
   int k_slabs, split_slabs, col_tiles;
-  int stream_weight;
-  float* acc32;  // [pieces][n_tokens][hidden]
+  int stream_from;  // stream_from()
+  float* acc32;     // [pieces][n_tokens][hidden]
   int n_tokens, hidden;
 };
 
@@ -1367,7 +1368,7 @@ __global__ __launch_bounds__(kThreads) void lce_dhidden_few_kernel(FewHiddenArgs
     const unsigned base = lds_address(lds) + (unsigned)fill * kFewStageBytes;
 #pragma unroll
     for (int i = 0; i < kFewLoadsR; ++i) dma_r.issue_one(i, r, base);
-    few_fetch_weight(dma_c, c, base + kFewTokens * kBK * 2, a.stream_weight);
+    few_fetch_weight(dma_c, c, base + kFewTokens * kBK * 2, k_begin * kBK >= a.stream_from);
     fill = fill == kFewStages - 1 ? 0 : fill + 1;
     if (k2 < slabs - 1) ++k2;
   };
@@ -1618,7 +1619,11 @@ static GradPlan plan_few_hidden(int64_t hidden_size, int64_t vocab, int cus) {
   return p;
 }
 
-static bool streams_weight(int64_t hidden_size, int64_t vocab) { return vocab * hidden_size * 2 >= kStreamWeightBytes; }
+// The first weight row that the few-token kernels read past the caches.
+static int stream_from(int64_t hidden_size, int64_t vocab) {
+  const int64_t row_bytes = hidden_size * 2;
+  return (int)(vocab * row_bytes <= kFittingWeightBytes ? vocab : kCachedWeightBytes / row_bytes);
+}
 
 }  // namespace vamd
 
@@ -1694,7 +1699,7 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
                                                   (size_t)a.plan.slots() * kTile * sizeof(float4))
                        : nullptr;
   a.z_cache = logits_cache;
-  a.stream_weight = streams_weight(hidden_size, vocab);
+  a.stream_from = stream_from(hidden_size, vocab);
   hipStream_t s = static_cast<hipStream_t>(stream);
   {
     ScopedTiming tm(kTagForward, s);
@@ -2025,7 +2030,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     gw.ld_out = hidden_size;
     if (few) {
       const FewHiddenArgs f{gh.R, gh.C, gh.k_slabs, hp.split_slabs, h_tiles,
-                            streams_weight(hidden_size, vocab), acc32, (int)n_tokens, (int)hidden_size};
+                            stream_from(hidden_size, vocab), acc32, (int)n_tokens, (int)hidden_size};
       {
         ScopedTiming tm(kTagDGrad, s);
         hipLaunchKernelGGL(lce_dhidden_few_kernel, dim3(h_tiles * pieces), dim3(kThreads), kFewLds, s, f);

@@ -947,3 +947,29 @@ def test_d_hidden_over_few_tokens(dev, n, h, v):
     _, _, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)
     _close_bf16(dh, want_dh, "d_hidden", e_dh)
     _close_bf16(dw, want_dw, "d_weight", e_dw)
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (257, 896, 20000),     # one row in the last token tile, half a column tile
+    (320, 128, 33001),     # rows for one wavefront in four exactly
+    (321, 640, 33001),     # and for one more
+    (513, 384, 40000),     # pieces of several tiles in one workgroup's share
+    (769, 1152, 6000),     # whole tiles, some workgroups with empty and full rows
+])
+@pytest.mark.parametrize("cached", [False, True])
+def test_token_and_column_tiles_that_are_nearly_empty(dev, n, h, v, cached):
+    """Wavefronts without rows and columns that are not fetched, against the fp32 ground truth with the bound for d_logits staged
+    in bf16."""
+    from verl_amd.utils.kernel import linear_cross_entropy as K
+    hidden, weight, labels = _make(n, h, v, seed=n + v, dist="normal")
+    g_lp = torch.randn(n, generator=torch.Generator().manual_seed(n))
+    hd, wd, ld, gd = (t.to(dev) for t in (hidden, weight, labels, g_lp))
+    cache = torch.full((n, v), float("nan"), device=dev) if cached and v % 8 == 0 else None
+    lp, ent, lse, mz = K.efficient_entropy_forward(hd, wd, ld, 0, 0.9, logits_cache=cache)
+    if cache is not None:
+        assert bool(torch.isfinite(cache).all())
+    dh, dw = K.efficient_entropy_backward(gd, None, hd, wd, ld, lse, mz, 0, 0.9, logits_cache=cache)
+    want_lp, want_ent, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)
+    assert (lp - want_lp).abs().max() <= ATOL and (ent - want_ent).abs().max() <= ATOL
+    _close_bf16(dh, want_dh, "d_hidden", e_dh)
+    _close_bf16(dw, want_dw, "d_weight", e_dw)

@@ -187,6 +187,7 @@ struct FwdSched<false> {
   }
   __device__ __forceinline__ int slab0(int) const { return 0; }
   __device__ __forceinline__ int slabs(int) const { return k_slabs; }
+  __device__ __forceinline__ bool rows_outside(int row, int extent) const { return tn * kTile + row >= extent; }
 };
 
 // bands: the workgroup's column of every band its XCD's share of the rounds touches
@@ -248,6 +249,7 @@ struct FwdSched<true> {
   }
   __device__ __forceinline__ int slab0(int) const { return 0; }
   __device__ __forceinline__ int slabs(int) const { return k_slabs; }
+  __device__ __forceinline__ bool rows_outside(int, int) const { return false; }
 };
 
 // The epilogues that write matrices hand the accumulators through an LDS patch private to the
@@ -1354,6 +1356,7 @@ __global__ __launch_bounds__(kThreads) void lce_dhidden_few_kernel(FewHiddenArgs
   SlabDma<true> dma_c;
   dma_r.init(a.dz);
   dma_c.init(a.weight);
+  dma_c.set_tile(a.weight, c0);
   FragAddr<false> fr;
   FragAddr<true> fc;
   fr.init(wr * kNB, kNB);
@@ -1933,6 +1936,9 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
   const uint16_t* hid = static_cast<const uint16_t*>(hidden);
   const uint16_t* wgt = static_cast<const uint16_t*>(weight);
   const int h_tiles = (int)ceil_div(hidden_size, kTile);
+  // Columns past the hidden size are not fetched (SlabDma::set_tile), except over 129 to 256 tokens, where the products wait for
+  // memory and nothing is gained (200 x 896 x 151936 318 us, without them 323).
+  const int col_extent = tok_tiles > 1 || few ? (int)hidden_size : h_tiles * kTile;
 
   for (int ci = 0; ci < n_chunks; ++ci) {
     const int64_t c0 = (int64_t)ci * cv;
@@ -1998,7 +2004,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     GemmOutArgs gh;
     // (the panel has no rows past n_tokens: they read as zero through the operand's bounds)
     gh.R = Operand{dz, pitch, (int)n_tokens, (int)cv};
-    gh.C = Operand{wgt + c0 * hidden_size, hidden_size, (int)hidden_size, (int)left};
+    gh.C = Operand{wgt + c0 * hidden_size, hidden_size, col_extent, (int)left};
     gh.k_slabs = (int)ceil_div(cols, kBK);
     gh.r_tiles = d_hidden && !few ? tok_tiles : 0;  // an input that needs no gradient leaves its GEMM an empty tile list
     gh.c_tiles = h_tiles;
@@ -2018,7 +2024,7 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
     // d_weight rows of this chunk: k runs over tokens (staged zeros beyond n_tokens)
     GemmOutArgs gw;
     gw.R = Operand{dz, pitch, (int)(ceil_div(cols, 8) * 8), (int)n_tokens};
-    gw.C = Operand{hid, hidden_size, (int)hidden_size, (int)n_tokens};
+    gw.C = Operand{hid, hidden_size, col_extent, (int)n_tokens};
     gw.k_slabs = (int)ceil_div(n_tokens, kBK);
     gw.r_tiles = want_dw ? chunk_tiles : 0;
     gw.c_tiles = h_tiles;

@@ -79,34 +79,55 @@ __global__ __launch_bounds__(kRcThreads) void rollout_stats_kernel(RcArgs a, con
     load_mask_groups<VEC>(mask, pos, m, streaming);
 #pragma unroll
     for (int k = 0; k < kGroups; ++k) {
-      float wt[4];  // the group's weights leave as soon as they exist: 16 registers fewer than holding the chunk's
+      float wt[4] = {0.f, 0.f, 0.f, 0.f};  // the group's weights leave as soon as they exist: 16 registers fewer than holding the chunk's
+      // A wavefront skips groups without a valid token; in the others masked tokens (and elements past the end, which read as
+      // masked) are selected away, four tokens' arithmetic interleaved: with a branch per token, 1024 x 3072 int64 mask 20.0 us
+      // and 18.8 so, 744 x 12000 41.2 and 38.0, 64 x 1000 one-byte mask 7.1 and 6.6 (of 14.1 us without the arithmetic).
+      const bool some = m[k][0] != 0.f || m[k][1] != 0.f || m[k][2] != 0.f || m[k][3] != 0.f;
+      if (__any(some)) {
+        float d[4], w[4], ed[4];
+        bool on[4], clamped = false;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        wt[e] = 0.f;
-        if (e >= pos.valid[k] || m[k][e] == 0.f) continue;
-        s[kRcM] += 1.f;
-        s[kRcOld] += o[k][e];
-        if (!a.roll_lp) continue;
-        const float d = o[k][e] - r[k][e];
-        const float dc = fminf(fmaxf(d, -kSafetyBound), kSafetyBound);
-        const float w = expf(dc);
-        const float ed = d == dc ? w : expf(d);  // one exponential per token unless the clamp acted
-        s[kRcRoll] += r[k][e];
-        s[kRcD] += d;
-        s[kRcK3] += ed - d - 1.f;
-        s[kRcRho2] += w * w;
-        if (a.level == VAMD_IS_TOKEN) {
-          const float c = fminf(fmaxf(w, a.lower), a.thr);
-          const float t = fminf(w, a.thr);
-          s[kRcW] += w;
-          s[kRcC] += c;
-          s[kRcC2] += c * c;
-          s[kRcTrunc] += t;
-          s[kRcHigh] += w > a.thr ? 1.f : 0.f;
-          s[kRcLow] += w < a.lower ? 1.f : 0.f;
-          wmax = fmaxf(wmax, w);
-          wmin = fminf(wmin, w);
-          wt[e] = t;
+        for (int e = 0; e < 4; ++e) {
+          on[e] = m[k][e] != 0.f;
+          s[kRcM] += on[e] ? 1.f : 0.f;
+          s[kRcOld] += on[e] ? o[k][e] : 0.f;
+        }
+        if (a.roll_lp) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            d[e] = o[k][e] - r[k][e];
+            const float dc = fminf(fmaxf(d[e], -kSafetyBound), kSafetyBound);
+            w[e] = ed[e] = expf(dc);
+            clamped = clamped || (on[e] && d[e] != dc);
+          }
+          if (__any(clamped)) {  // one exponential per token unless the clamp acted
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ed[e] = d[e] == fminf(fmaxf(d[e], -kSafetyBound), kSafetyBound) ? ed[e] : expf(d[e]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            s[kRcRoll] += on[e] ? r[k][e] : 0.f;
+            s[kRcD] += on[e] ? d[e] : 0.f;
+            s[kRcK3] += on[e] ? ed[e] - d[e] - 1.f : 0.f;
+            s[kRcRho2] += on[e] ? w[e] * w[e] : 0.f;
+          }
+          if (a.level == VAMD_IS_TOKEN) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float c = fminf(fmaxf(w[e], a.lower), a.thr);
+              const float t = fminf(w[e], a.thr);
+              s[kRcW] += on[e] ? w[e] : 0.f;
+              s[kRcC] += on[e] ? c : 0.f;
+              s[kRcC2] += on[e] ? c * c : 0.f;
+              s[kRcTrunc] += on[e] ? t : 0.f;
+              s[kRcHigh] += on[e] && w[e] > a.thr ? 1.f : 0.f;
+              s[kRcLow] += on[e] && w[e] < a.lower ? 1.f : 0.f;
+              wmax = on[e] ? fmaxf(wmax, w[e]) : wmax;
+              wmin = on[e] ? fminf(wmin, w[e]) : wmin;
+              wt[e] = on[e] ? t : 0.f;
+            }
+          }
         }
       }
       if (a.level == VAMD_IS_TOKEN && a.weights && pos.valid[k] > 0)

@@ -573,6 +573,22 @@ def test_gradients_are_summed_apart_where_somebody_sees_them(dev):
     assert torch.equal(got, want) and torch.equal(y.detach(), alone["lp"])
 
 
+def test_saved_logits_that_come_back_in_other_strides(dev):
+    """Rows 40 elements apart, handed back by hooks on saved tensors with no gaps: the same gradients."""
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(7, 300, torch.float32, seed=4)
+    lab = labels.to(dev)
+    zd = torch.zeros(7, 340, device=dev)[:, :300].copy_(z).requires_grad_()
+    want, = torch.autograd.grad(_summed(F, zd, lab, ("lp", "ent")), zd)
+    for traced in (False, True):
+        lp, ent = ((lambda x, y, _: F._LogProbsFromLogits.apply(x, y, False), lambda x: F._EntropyFromLogits.apply(x, False))
+                   if traced else (F.logprobs_from_logits, F.entropy_from_logits))
+        with torch.autograd.graph.save_on_cpu():
+            loss = lp(zd, lab, False).sum() + ent(zd).sum()
+        got, = torch.autograd.grad(loss, zd)
+        assert torch.equal(got, want)
+
+
 def test_row_functions_traced_and_transformed(dev):
     """A trace runs them on its own inputs; forward-mode differentiation and functorch's transforms are refused, a second
     derivative raises."""

@@ -300,6 +300,14 @@ Rows logit_rows(const Tensor& logits) {
   if (rows.stride(1) != 1 || (rows.size(0) > 1 && rows.stride(0) < vocab)) rows = rows.contiguous();
   return {rows, rows.size(0) > 1 ? rows.stride(0) : vocab, type};
 }
+// The logits that a node saved.  Hooks on saved tensors may hand them back in other strides (save_on_cpu keeps none), so the
+// pitch is that of what comes back.
+Rows saved_rows(const Tensor& rows, at::IntArrayRef shape) {
+  const Rows r = logit_rows(rows);
+  if (r.t.numel() != c10::multiply_integers(shape) || r.vocab() != shape.back())
+    raise_assertion("saved logits came back as " + shape_text(rows));
+  return r;
+}
 Tensor label_rows(const Tensor& labels, const Tensor& logits) {
   if (logits.dim() < 1 || labels.sizes() != logits.sizes().slice(0, logits.dim() - 1))
     raise_assertion("labels " + shape_text(labels) + " do not match logits " + shape_text(logits));
@@ -351,7 +359,6 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
     const Rows r = logit_rows(logits);
     const RowStats s = row_stats(logits, r, lab, logits.scalar_type(), true);
     ctx->save_for_backward({r.t, lab, s.lse});
-    ctx->saved_data["ld"] = r.ld;
     ctx->saved_data["shape"] = logits.sizes().vec();
     // writing the gradient over the logits needs the rows to be the caller's storage, and never overwrites a parameter
     ctx->saved_data["in_place"] = inplace_backward && r.data() == logits.const_data_ptr() && logits.is_contiguous() &&
@@ -373,8 +380,8 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
                     "pass and cannot run a second one; pass inplace_backward=False to keep the logits");
         ctx->saved_data["logits_overwritten"] = true;
       }
-      const Rows r{saved[0], ctx->saved_data["ld"].toInt(), row_type(saved[0].scalar_type())};
-      d = row_gradient(r, saved[1], saved[2], Tensor(), grads[0], ctx->saved_data["shape"].toIntVector(), in_place, !records);
+      const auto shape = ctx->saved_data["shape"].toIntVector();
+      d = row_gradient(saved_rows(saved[0], shape), saved[1], saved[2], Tensor(), grads[0], shape, in_place, !records);
     }
     if (records)  // the gradient is no function of its own to differentiate
       d = torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable",
@@ -389,7 +396,6 @@ class RowEntropy : public torch::autograd::Function<RowEntropy> {
     const Rows r = logit_rows(logits);
     const RowStats s = row_stats(logits, r, Tensor(), fp32_output ? at::kFloat : logits.scalar_type(), true);
     ctx->save_for_backward({r.t, s.lse, s.mean_z});
-    ctx->saved_data["ld"] = r.ld;
     ctx->saved_data["shape"] = logits.sizes().vec();
     return s.value;
   }
@@ -397,8 +403,8 @@ class RowEntropy : public torch::autograd::Function<RowEntropy> {
     const bool records = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const auto saved = ctx->get_saved_variables();
-    const Rows r{saved[0], ctx->saved_data["ld"].toInt(), row_type(saved[0].scalar_type())};
-    return {row_gradient(r, Tensor(), saved[1], saved[2], grads[0], ctx->saved_data["shape"].toIntVector(), false, !records),
+    const auto shape = ctx->saved_data["shape"].toIntVector();
+    return {row_gradient(saved_rows(saved[0], shape), Tensor(), saved[1], saved[2], grads[0], shape, false, !records),
             Tensor()};
   }
 };

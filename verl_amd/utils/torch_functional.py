@@ -33,6 +33,13 @@ def _logit_rows(logits: torch.Tensor):
     return rows, (rows.stride(0) if rows.shape[0] > 1 else vocab)
 
 
+def _saved_rows(rows: torch.Tensor, shape):
+    """The logits that a node saved: hooks on saved tensors may hand them back in other strides (``save_on_cpu`` keeps none), so
+    the pitch is that of what comes back."""
+    assert rows.numel() == shape.numel() and rows.shape[-1] == shape[-1], f"saved logits came back as {tuple(rows.shape)}"
+    return _logit_rows(rows)
+
+
 def _row_stats(rows, ld, labels, want_logprobs: bool, want_entropy: bool, want_mean_z: bool,
                dtype=torch.float32):
     """Log-probs and entropies come in ``dtype`` (fp32 or that of the logits), the backward pass's values in fp32."""
@@ -81,7 +88,7 @@ class _LogProbsFromLogits(torch.autograd.Function):
         lab = labels.reshape(-1).to(device=rows.device, dtype=torch.int64).contiguous()
         logprobs, _, lse, _ = _row_stats(rows, ld, lab, True, False, False, logits.dtype)
         ctx.save_for_backward(rows, lab, lse)
-        ctx.ld, ctx.shape = ld, logits.shape
+        ctx.shape = logits.shape
         # writing the gradient over the logits needs the rows to BE the caller's storage
         ctx.in_place = (bool(inplace_backward) and rows.data_ptr() == logits.data_ptr() and logits.is_contiguous()
                         and not (logits.is_leaf and logits.requires_grad))   # never overwrite a parameter
@@ -99,7 +106,8 @@ class _LogProbsFromLogits(torch.autograd.Function):
                                    "its first backward pass and cannot run a second one; pass inplace_backward=False "
                                    "to keep the logits")
             ctx.logits_overwritten = True
-        d = _row_backward(rows, ctx.ld, lab, lse, None, g, None, ctx.in_place)
+        rows, ld = _saved_rows(rows, ctx.shape)
+        d = _row_backward(rows, ld, lab, lse, None, g, None, ctx.in_place)
         return d.view(ctx.shape), None, None
 
 
@@ -110,13 +118,14 @@ class _EntropyFromLogits(torch.autograd.Function):
         _, entropy, lse, mean_z = _row_stats(rows, ld, None, False, True, True,
                                              torch.float32 if fp32_output else logits.dtype)
         ctx.save_for_backward(rows, lse, mean_z)
-        ctx.ld, ctx.shape = ld, logits.shape
+        ctx.shape = logits.shape
         return entropy.view(logits.shape[:-1])
 
     @staticmethod
     def backward(ctx, g):
         rows, lse, mean_z = ctx.saved_tensors
-        d = _row_backward(rows, ctx.ld, None, lse, mean_z, None, g, False)
+        rows, ld = _saved_rows(rows, ctx.shape)
+        d = _row_backward(rows, ld, None, lse, mean_z, None, g, False)
         return d.view(ctx.shape), None
 
 

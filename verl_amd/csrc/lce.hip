@@ -157,15 +157,18 @@ struct FwdArgs {
   int stream_from;      // lce_forward_few_kernel: stream_from()
 };
 
-// The tiles of one workgroup.  The two ways of sharing out are kernels of their own: with both in one kernel the split
+// The tiles of one workgroup.  The ways of sharing out are kernels of their own: with both in one kernel the split
 // walk, whose token tile never changes, carried the bands' lookups and the state's write-out through its tile loop, with 41
 // scalar registers spilled (16384 x 3584 x 152064 12.50 ms, apart 12.47; 3300 x 896 x 151936, in bands, 706 and 699 us).
-template <bool BANDS>
-struct FwdSched;
+// Splits whose last token tile leaves wavefronts without rows, which skip the products, are a third: with that in the kernel,
+// launches
+// without such wavefronts took 0.4 to 0.6 % longer (us: 2048 x 896 x 151936 439.6, apart 437.5; 21503 x 4096 x 128256 15738,
+// apart 15601).
+enum Walk { kSplits, kSplitsIdle, kBands, kWalks };
 
 // splits: one range of the vocabulary for one token tile
-template <>
-struct FwdSched<false> {
+template <Walk WALK>
+struct FwdSched {
   int k_slabs, tn, vt_begin, ntiles;
   int64_t slot;  // where the state goes
 
@@ -187,12 +190,14 @@ struct FwdSched<false> {
   }
   __device__ __forceinline__ int slab0(int) const { return 0; }
   __device__ __forceinline__ int slabs(int) const { return k_slabs; }
-  __device__ __forceinline__ bool rows_outside(int row, int extent) const { return tn * kTile + row >= extent; }
+  __device__ __forceinline__ bool rows_outside(int row, int extent) const {
+    return WALK == kSplitsIdle && tn * kTile + row >= extent;
+  }
 };
 
 // bands: the workgroup's column of every band its XCD's share of the rounds touches
 template <>
-struct FwdSched<true> {
+struct FwdSched<kBands> {
   const FwdPlan* plan;
   int k_slabs, ntiles;
   int xcd, member, wave_count;  // this XCD, workgroup within it, its tiles of a wave
@@ -329,7 +334,7 @@ __device__ __forceinline__ void merge_state(float& m, float& s, float& sy, float
 // backward pass can form d_logits without repeating the GEMM.
 // With PI2 a fifth running sum, sum_j e_j^2, is carried, from which sum_j softmax(z)_j^2 follows
 // (calculate_sum_pi_squared_from_logits, verl/utils/torch_functional.py:680-694).
-template <bool CACHE, bool PI2, bool BANDS>
+template <bool CACHE, bool PI2, Walk WALK>
 struct FwdEpi {
   LanePos p;
   float scale2;
@@ -344,7 +349,7 @@ struct FwdEpi {
                                       // [kThreads][kNB]; states [256] float4, then squared sums [256]
   char* patches;  // CACHE: the wavefronts' exchange patches
   const FwdArgs* args;
-  FwdSched<BANDS> sched;
+  FwdSched<WALK> sched;
   int64_t slot;  // where the state of the token tile at hand goes
   float rcp_t;
 
@@ -352,7 +357,7 @@ struct FwdEpi {
   // a token past the end reads as label 0, whose sums nobody looks at.  They go into the set that is not in use: other
   // wavefronts may still be in the epilogue that reads this one.
   __device__ __forceinline__ void prefetch(int tile, int r0, int) {
-    if constexpr (BANDS) {
+    if constexpr (WALK == kBands) {
       const auto here = sched.at(tile);
       if (here.slot == slot) return;
       if (tile > 0) write_state();  // (here no accumulators are alive)
@@ -537,20 +542,20 @@ struct FwdEpi {
   }
 };
 
-template <bool CACHE, bool PI2, bool BANDS>
+template <bool CACHE, bool PI2, Walk WALK>
 __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  FwdSched<BANDS> sched;
+  FwdSched<WALK> sched;
   sched.init(a.plan, a.k_slabs, xcd_regroup(blockIdx.x, gridDim.x));
 
-  FwdEpi<CACHE, PI2, BANDS> epi;
+  FwdEpi<CACHE, PI2, WALK> epi;
   epi.p = lane_pos();
   epi.scale2 = a.scale2;
   epi.vocab = a.vocab;
   epi.rcp_t = a.rcp_t;
   epi.args = &a;
   epi.sched = sched;
-  if constexpr (BANDS) epi.slot = -1;
+  if constexpr (WALK == kBands) epi.slot = -1;
   else epi.slot = sched.slot;
   epi.reset();
   typedef float __attribute__((address_space(3))) * lds_f32_t;
@@ -1442,6 +1447,18 @@ static int allow_big_lds(K kernel, int bytes = kLdsBytes) {
   return VAMD_OK;
 }
 
+typedef void (*ForwardKernel)(FwdArgs);
+// [walk, or few tokens][logits kept][squared sums]
+static const ForwardKernel kForwardKernels[kWalks + 1][2][2] = {
+    {{lce_forward_kernel<false, false, kSplits>, lce_forward_kernel<false, true, kSplits>},
+     {lce_forward_kernel<true, false, kSplits>, lce_forward_kernel<true, true, kSplits>}},
+    {{lce_forward_kernel<false, false, kSplitsIdle>, lce_forward_kernel<false, true, kSplitsIdle>},
+     {lce_forward_kernel<true, false, kSplitsIdle>, lce_forward_kernel<true, true, kSplitsIdle>}},
+    {{lce_forward_kernel<false, false, kBands>, lce_forward_kernel<false, true, kBands>},
+     {lce_forward_kernel<true, false, kBands>, lce_forward_kernel<true, true, kBands>}},
+    {{lce_forward_few_kernel<false, false>, lce_forward_few_kernel<false, true>},
+     {lce_forward_few_kernel<true, false>, lce_forward_few_kernel<true, true>}}};
+
 // The kernels use more LDS than the default launch limit; the limit is a per-device function
 // attribute, so it is raised once on every device the library is used on.
 static int ensure_lds_attributes() {
@@ -1453,14 +1470,11 @@ static int ensure_lds_attributes() {
   std::lock_guard<std::mutex> lock(mu);
   if (done[dev]) return VAMD_OK;
   int s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, false, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, true, false>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, false, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<false, true, true>, kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, false, false>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, true, false>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, false, true>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_forward_kernel<true, true, true>, kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+  for (int w = 0; w < kWalks; ++w)
+    for (int pi2 = 0; pi2 < 2; ++pi2) {
+      if ((s = allow_big_lds(kForwardKernels[w][0][pi2], kLdsBytes + kFwdTokenLds)) != VAMD_OK) return s;
+      if ((s = allow_big_lds(kForwardKernels[w][1][pi2], kLdsBytes + kFwdCacheLds)) != VAMD_OK) return s;
+    }
   if ((s = allow_big_lds(lce_forward_few_kernel<false, false>, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_few_kernel<false, true>, kFewLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_forward_few_kernel<true, false>, kFewCacheLds)) != VAMD_OK) return s;
@@ -1667,18 +1681,6 @@ extern "C" size_t vamd_lce_forward_workspace_bytes(int64_t n_tokens, int64_t hid
   return (size_t)plan_forward(n_tokens, vocab).slots() * kTile * (sizeof(float4) + sizeof(float));  // state + squared sums
 }
 
-typedef void (*ForwardKernel)(FwdArgs);
-static ForwardKernel forward_kernel(bool cache, bool pi2, const FwdPlan& plan) {
-  static const ForwardKernel kernels[3][2][2] = {
-      {{lce_forward_few_kernel<false, false>, lce_forward_few_kernel<false, true>},
-       {lce_forward_few_kernel<true, false>, lce_forward_few_kernel<true, true>}},
-      {{lce_forward_kernel<false, false, false>, lce_forward_kernel<false, true, false>},
-       {lce_forward_kernel<true, false, false>, lce_forward_kernel<true, true, false>}},
-      {{lce_forward_kernel<false, false, true>, lce_forward_kernel<false, true, true>},
-       {lce_forward_kernel<true, false, true>, lce_forward_kernel<true, true, true>}}};
-  return kernels[plan.few_cols ? 0 : plan.splits ? 1 : 2][cache][pi2];
-}
-
 // Forward launches shared by the two entry points; `workspace` holds at least
 // vamd_lce_forward_workspace_bytes() bytes and the arguments have been checked.
 static int lce_forward_launch(const void* hidden, const void* weight, const int64_t* labels, int64_t n_tokens,
@@ -1709,7 +1711,9 @@ static int lce_forward_launch(const void* hidden, const void* weight, const int6
     const dim3 grid(a.plan.splits ? a.plan.tok_tiles * a.plan.splits : a.plan.group * kXcds), block(kThreads);
     const bool pi2 = sum_pi_squared != nullptr, cache = logits_cache != nullptr;
     const int lds_bytes = a.plan.few_cols ? (cache ? kFewCacheLds : kFewLds) : kLdsBytes + (cache ? kFwdCacheLds : kFwdTokenLds);
-    hipLaunchKernelGGL(forward_kernel(cache, pi2, a.plan), grid, block, lds_bytes, s, a);
+    const bool idle = ceil_div(n_tokens, kNB * kBlk) % (kTile / (kNB * kBlk)) != 0;  // a wavefront owns kNB blocks of tokens
+    const int walk = a.plan.few_cols ? kWalks : !a.plan.splits ? kBands : idle ? kSplitsIdle : kSplits;
+    hipLaunchKernelGGL(kForwardKernels[walk][cache][pi2], grid, block, lds_bytes, s, a);
   }
   VAMD_LAUNCH_CHECK();
 

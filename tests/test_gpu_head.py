@@ -955,6 +955,8 @@ def test_d_hidden_over_few_tokens(dev, n, h, v):
     (321, 640, 33001),     # and for one more
     (513, 384, 40000),     # pieces of several tiles in one workgroup's share
     (769, 1152, 6000),     # whole tiles, some workgroups with empty and full rows
+    (448, 128, 33001),     # the last tile has rows for three wavefronts in four
+    (449, 128, 33001),     # and for all: the forward pass takes the kernel without idle wavefronts
 ])
 @pytest.mark.parametrize("cached", [False, True])
 def test_token_and_column_tiles_that_are_nearly_empty(dev, n, h, v, cached):

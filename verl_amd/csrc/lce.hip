@@ -161,9 +161,8 @@ struct FwdArgs {
 // walk, whose token tile never changes, carried the bands' lookups and the state's write-out through its tile loop, with 41
 // scalar registers spilled (16384 x 3584 x 152064 12.50 ms, apart 12.47; 3300 x 896 x 151936, in bands, 706 and 699 us).
 // Splits whose last token tile leaves wavefronts without rows, which skip the products, are a third: with that in the kernel,
-// launches
-// without such wavefronts took 0.4 to 0.6 % longer (us: 2048 x 896 x 151936 439.6, apart 437.5; 21503 x 4096 x 128256 15738,
-// apart 15601).
+// launches without such wavefronts took 0.4 to 0.6 % longer (us: 2048 x 896 x 151936 439.6, apart 437.5; 21503 x 4096 x
+// 128256 15738, apart 15601).
 enum Walk { kSplits, kSplitsIdle, kBands, kWalks };
 
 // splits: one range of the vocabulary for one token tile

@@ -529,6 +529,125 @@ def test_summed_gradients_need_no_second_buffer(dev):
     assert got.nbytes <= torch.cuda.max_memory_allocated(dev) - before < 1.5 * got.nbytes
 
 
+class _Step(torch.autograd.Function):
+    """The identity, which runs ``step`` in the backward pass."""
+
+    @staticmethod
+    def forward(ctx, x, step):
+        ctx.step = step
+        return x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, g):
+        ctx.step()
+        return g, None
+
+
+def _pairs(dev):
+    """Two functions of the same tensor whose gradients are summed, and a tensor of 16 MiB for them."""
+    import types
+    import verl_amd.utils.torch_functional as F
+    from verl_amd.trainer.ppo import core_algos as CA
+    g = torch.Generator().manual_seed(7)
+    labels = torch.randint(0, 65536, (64,), generator=g).to(dev)
+    old, adv, ref, log_prob = (torch.randn(1024, 4096, generator=g).to(dev) for _ in range(4))
+    mask = torch.ones(1024, 4096, device=dev)
+    cfg = types.SimpleNamespace(clip_ratio=0.2, clip_ratio_low=None, clip_ratio_high=None, clip_ratio_c=3.0, global_batch_info={},
+                                get=lambda k, d=None: d)
+    return {"rows": (torch.randn(64, 65536, generator=g).to(dev), F.entropy_from_logits,
+                     lambda z: F.logprobs_from_logits(z, labels, inplace_backward=False)),
+            "losses": (log_prob, lambda x: CA.compute_kl_loss(x, ref, mask),
+                       lambda x: CA.compute_policy_loss_vanilla(old, x, adv, mask, "token-mean", cfg)[0])}
+
+
+@pytest.mark.parametrize("kind", ["rows", "losses"])
+def test_summed_gradients_beside_one_from_another_thread(dev, kind):
+    """A copy to the host is differentiated on the thread that called backward(), which adds to autograd's buffer for the tensor
+    whenever it gets there.  The two functions' sum is formed outside that buffer: here the copy's gradient arrives between
+    them, and theirs still take one allocation."""
+    import threading
+    x, first, second = _pairs(dev)[kind]
+    x.requires_grad_()
+    alone = [torch.autograd.grad(f(x).sum(), x)[0] for f in (second, first)]
+    one_ran, arrived = threading.Event(), threading.Event()
+
+    def between():               # device thread, after the node that runs first and before the other one
+        one_ran.set()
+        assert arrived.wait(60)
+
+    # of the nodes that are ready a thread runs the one made last
+    leaf = torch.ones((), requires_grad=True)
+    last = _Step.apply(leaf, arrived.set)
+    on_host = _Step.apply(x.cpu(), lambda: one_ran.wait(60)).sum()
+    late = _Step.apply(first(x), between).sum()
+    total = (last + on_host) + (late + second(x).sum()).cpu()
+    torch.cuda.synchronize()
+    count = lambda: torch.cuda.memory_stats(dev)["allocation.large_pool.allocated"]
+    before = count()
+    got, _ = torch.autograd.grad(total, (x, leaf))
+    assert one_ran.is_set() and arrived.is_set()
+    assert count() - before == 2, "the copy's gradient and the sum of the two"
+    want = 1.0 + (alone[0] + alone[1])
+    assert (got - want).abs().max() <= 4 * 2.0 ** -24 * (1 + alone[0].abs().max() + alone[1].abs().max())
+
+
+@pytest.mark.parametrize("kind", ["rows", "losses"])
+def test_a_sum_takes_one_allocation_and_a_hook_two(dev, kind):
+    x, first, second = _pairs(dev)[kind]
+    x.requires_grad_()
+    count = lambda: torch.cuda.memory_stats(dev)["allocation.large_pool.allocated"]
+    for kept, hooked in ((False, None), (True, None), (False, 0), (False, 1)):
+        a, b = first(x), second(x)
+        if hooked is not None:
+            (a, b)[hooked].grad_fn.register_hook(lambda ins, outs: None)
+        total = a.sum() + b.sum()
+        for retain in (kept, False) if kept else (False,):
+            before = count()
+            torch.autograd.grad(total, x, retain_graph=retain)
+            assert count() - before == (1 if hooked is None else 2)
+
+
+class _Nothing(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("kind", ["rows", "losses"])
+def test_a_gradient_left_with_a_node_is_not_lost(dev, kind):
+    """The other node has no gradient of its own; the pass fails between the two and is run again; it needs only one of them."""
+    x, first, second = _pairs(dev)[kind]
+    x.requires_grad_()
+    alone = [torch.autograd.grad(f(x).sum(), x)[0] for f in (second, first)]
+    got, = torch.autograd.grad(_Nothing.apply(first(x)).sum() + second(x).sum(), x)
+    assert torch.equal(got, alone[0])
+    fails = [True]
+
+    def between():
+        if fails[0]:
+            raise RuntimeError("between the two")
+
+    a, b = first(x), second(x)
+    total = _Step.apply(a, between).sum() + b.sum()
+    with pytest.raises(RuntimeError, match="between the two"):
+        torch.autograd.grad(total, x, retain_graph=True)
+    fails[0] = False
+    for _ in range(2):
+        assert torch.equal(torch.autograd.grad(total, x, retain_graph=True)[0], alone[0] + alone[1])
+    assert torch.equal(torch.autograd.grad(total, b, retain_graph=True)[0], torch.ones_like(b))
+    y = x * 1.0
+    a, b, c = first(y), second(y), first(y)
+    total = a.sum() + b.sum() + c.sum()
+    for of, want in (((b,), None), ((y,), alone[1] + alone[0] + alone[1]), ((y, a), alone[1] + alone[0] + alone[1])):
+        got = torch.autograd.grad(total, of, retain_graph=True)[0]
+        if want is not None:
+            assert torch.equal(got, want)
+
+
 def test_gradients_are_summed_apart_where_somebody_sees_them(dev):
     """A third gradient, hooks, a graph of the gradients, a receiver on another stream, a caller that keeps the first gradient."""
     import verl_amd.utils.torch_functional as F

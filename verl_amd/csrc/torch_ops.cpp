@@ -164,10 +164,10 @@ void save_form(AutogradContext* ctx, const Tensor& input, const at::Device& dev)
   ctx->saved_data["device"] = input.device();
   ctx->saved_data["dtype"] = (int64_t)input.scalar_type();
 }
+bool in_kernel_form(AutogradContext* ctx) { return ctx->saved_data.find("shape") == ctx->saved_data.end(); }
 Tensor in_saved_form(AutogradContext* ctx, Tensor g) {
-  auto it = ctx->saved_data.find("shape");
-  if (it == ctx->saved_data.end()) return g;
-  return g.view(it->second.toIntVector())
+  if (in_kernel_form(ctx)) return g;
+  return g.view(ctx->saved_data["shape"].toIntVector())
       .to(ctx->saved_data["device"].toDevice(), (at::ScalarType)ctx->saved_data["dtype"].toInt());
 }
 
@@ -175,110 +175,177 @@ Tensor upstream(const Tensor& d_loss, const at::Device& dev) { return as_f32(d_l
 
 // ---- sums of gradients ---------------------------------------------------------------------------------------
 // Two nodes that differentiate the same tensor (entropy and log-probs of the logits, KL loss and policy loss of the
-// log-probs) each hand autograd a gradient, which it adds up in a pass of its own: two tensors read and one written.  The
-// node that runs second may add its gradient to the first one's instead, in the kernel that forms it, and hand back none.
-// Both gradients go to the same input of the same node of one running backward pass, which cannot read the sum before both
-// have arrived, so the only thing to make sure of is that the first gradient is as its node left it and is held by autograd
-// alone: a weak reference to it is kept, per thread, and it is joined only if
-//   - the same backward pass (its id is never used again) still runs, on this thread, and records no graph of its own;
-//   - one reference to the tensor and one to its storage are left, and its version is that of then: nobody else (a hook, a
-//     third gradient that was added to it or that it was added to) has it or has had it;
-//   - neither node has hooks, which would see the gradients apart, and anomaly detection, which looks at each, is off;
-//   - both kernels run on the stream on which the node that receives the sum runs.
-// Otherwise the second node hands back a gradient of its own, as ever.  (Figures: scale_rows_add_kernel and
-// row_softmax_backward_kernel.)
+// log-probs) each hand autograd a gradient, which it adds up in a pass of its own: two tensors read and one written.
+// Instead the node that runs first may leave its gradient with the other one and hand back none; the other one adds its own
+// to it in the kernel that forms that, and hands back the sum.  What autograd has been given is not touched: its buffers
+// belong to all its threads, and a node of another one (a copy of the same tensor to the host or to another GPU) may add to
+// them at any time.  A gradient is left with a node only if
+//   - it differentiates the same input of the same receiver, and the backward pass at hand includes it and needs it;
+//   - it has not run in this pass.  Ids of passes grow, so a node whose newest run was in an older pass has not;
+//   - it runs on the same device, so on this thread or one that takes over from it, and on the same stream;
+//   - nothing was left with it by another pass that still runs or has failed;
+//   - neither node has hooks, which would see the gradients apart, the pass records no graph of its own, and anomaly
+//     detection, which looks at each gradient, is off.
+// Otherwise each node hands back its own gradient, as ever.  What was left lies in the other node's saved data: if the pass
+// fails in between it goes with the graph.  (Figures: scale_rows_add_kernel and row_softmax_backward_kernel.)
 using torch::autograd::Edge;
-struct Summand {
-  int pass = -1;  // id of the backward pass
-  torch::autograd::Node* receiver = nullptr;
-  uint32_t input = 0, version = 0;
-  std::optional<c10::weak_intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>> grad;
+using torch::autograd::Node;
+
+// The newest nodes that can add to a gradient left with them, of all threads: where a running node looks for another one.
+// All that counts is asked of the node itself; a node that is no longer among them is not found.
+constexpr int kJoinable = 32;
+struct Joinable {
+  Node* key = nullptr;  // compared, never followed
+  std::weak_ptr<Node> node;
+  AutogradContext* ctx = nullptr;  // lives in the node
 };
-constexpr int kSummands = 4;  // the newest gradients of a thread
-struct Summands {
-  std::array<Summand, kSummands> list;
+struct Joinables {
+  std::mutex mu;  // also guards kRan, kLeft and kLeftPass of every node's saved data
+  std::array<Joinable, kJoinable> newest;
   int next = 0;
 };
-Summands& summands() {
-  static thread_local Summands s;
-  return s;
+Joinables& joinables() {
+  static auto* j = new Joinables;  // never destroyed: at exit threads of autograd may still run
+  return *j;
+}
+constexpr const char *kRan = "ran", *kLeft = "left", *kLeftPass = "left_pass";
+
+// The node of F that made `output` can add to a gradient left with it, unless its own takes another form or another's place.
+template <class F>
+void joinable(const Tensor& output) {
+  const auto& node = output.grad_fn();
+  auto* const made = dynamic_cast<torch::autograd::CppNode<F>*>(node.get());
+  if (!made || !in_kernel_form(&made->ctx_)) return;
+  const auto in_place = made->ctx_.saved_data.find("in_place");
+  if (in_place != made->ctx_.saved_data.end() && in_place->second.toBool()) return;
+  Joinables& all = joinables();
+  std::lock_guard<std::mutex> lock(all.mu);
+  all.newest[all.next] = {node.get(), node, &made->ctx_};
+  all.next = (all.next + 1) % kJoinable;
 }
 
-// Where the running node's gradient of its input 0 goes, if that may be summed here.
-std::optional<Edge> sum_edge(const at::Device& dev) {
-  if (torch::autograd::get_current_graph_task_id() < 0 || at::GradMode::is_enabled() ||
-      torch::autograd::AnomalyMode::is_enabled())
-    return std::nullopt;
-  const auto node = torch::autograd::get_current_node();
-  if (!node || node->num_outputs() == 0 || !node->post_hooks().empty()) return std::nullopt;
-  const Edge edge = node->next_edge(0);
-  if (!edge.is_valid()) return std::nullopt;
-  const auto stream = edge.function->stream();
-  const auto mine = c10::hip::getCurrentHIPStream(dev.index());
-  if (!stream || stream->device_index() != mine.device_index() || stream->id() != mine.id()) return std::nullopt;
-  return edge;
-}
+// The other node with which the running one may sum up, if there is one, and what was left with that already.
+struct Partner {
+  std::shared_ptr<Node> node;
+  AutogradContext* ctx = nullptr;
+  Tensor left;
+};
 
-// The gradient that the running node may add its own to (and then return none), or an undefined tensor.
-Tensor gradient_to_join(at::IntArrayRef shape, at::ScalarType dtype, const at::Device& dev) {
-  const auto edge = sum_edge(dev);
-  if (!edge) return Tensor();
-  const int pass = torch::autograd::get_current_graph_task_id();
-  for (Summand& s : summands().list) {
-    if (s.pass != pass || s.receiver != edge->function.get() || s.input != edge->input_nr || !s.grad) continue;
-    auto held = s.grad->lock();
-    if (!held || held.use_count() != 2) continue;  // autograd's reference and this one
-    const Tensor sum(std::move(held));
-    if (sum._version() == s.version && sum.storage().use_count() == 1 && sum.sizes() == shape &&
-        sum.scalar_type() == dtype && sum.device() == dev)
-      return sum;
+// One node's part in the sum, from the start of its backward function.
+class Summing {
+ public:
+  explicit Summing(AutogradContext* ctx)
+      : pass_(torch::autograd::get_current_graph_task_id()),
+        seen_apart_(at::GradMode::is_enabled() || torch::autograd::AnomalyMode::is_enabled()) {
+    if (pass_ < 0) return;
+    std::lock_guard<std::mutex> lock(joinables().mu);
+    auto& data = ctx->saved_data;
+    const auto ran = data.find(kRan);
+    if (ran == data.end() || ran->second.toInt() < pass_) data[kRan] = (int64_t)pass_;
+    const auto left = data.find(kLeft);
+    if (left == data.end() || data[kLeftPass].toInt() != pass_) return;
+    left_ = left->second.toTensor();
+    data.erase(left);
   }
-  return Tensor();
-}
 
-// The running node is about to return `grad`, which it made itself, as its gradient of input 0.
-void gradient_returned(const Tensor& grad) {
-  if (!grad.defined() || !grad.is_cuda() || !grad.is_contiguous()) return;
-  const auto edge = sum_edge(grad.device());
-  if (!edge) return;
-  Summands& all = summands();
-  Summand& s = all.list[all.next];
-  all.next = (all.next + 1) % kSummands;
-  s.pass = torch::autograd::get_current_graph_task_id();
-  s.receiver = edge->function.get();  // compared, never followed
-  s.input = edge->input_nr;
-  s.version = grad._version();
-  s.grad.emplace(grad.getIntrusivePtr());
-}
+  // Looks for a partner.  Where the node's gradient of the form given goes: a tensor to which it adds its own, or an
+  // undefined tensor, and then it makes one.
+  Tensor target(at::IntArrayRef shape, at::ScalarType type, const at::Device& dev) {
+    find_partner(dev);
+    Tensor& sum = left_.defined() ? left_ : partner_.left;
+    if (sum.defined() && sum.sizes() == shape && sum.scalar_type() == type && sum.device() == dev) return sum;
+    return Tensor();
+  }
+
+  // What the node hands back for `grad`, which holds its gradient and that of target(), if one was defined.
+  Tensor result(const Tensor& grad) {
+    Tensor sum = grad;
+    if (left_.defined() && !(sum.defined() && sum.is_same(left_))) sum = sum.defined() ? sum.add(left_) : left_;
+    if (!partner_.node || !sum.defined()) return sum;
+    if (partner_.left.defined()) return sum.is_same(partner_.left) ? Tensor() : sum;
+    if (!sum.is_cuda() || !sum.is_contiguous()) return sum;
+    std::lock_guard<std::mutex> lock(joinables().mu);
+    if (!may_take(partner_.ctx) || partner_.ctx->saved_data.count(kLeft)) return sum;
+    partner_.ctx->saved_data[kLeftPass] = (int64_t)pass_;
+    partner_.ctx->saved_data[kLeft] = sum;
+    return Tensor();
+  }
+
+ private:
+  bool may_take(AutogradContext* ctx) const {
+    const auto& data = ctx->saved_data;
+    const auto ran = data.find(kRan);
+    return ran == data.end() || ran->second.toInt() < pass_;
+  }
+
+  void find_partner(const at::Device& dev) {
+    const auto* const nodes = torch::autograd::get_current_graph_task_nodes_in_graph();
+    if (pass_ < 0 || !nodes || seen_apart_) return;
+    const auto me = torch::autograd::get_current_node();
+    if (!me || me->num_outputs() == 0 || !me->post_hooks().empty()) return;
+    const Edge edge = me->next_edge(0);
+    if (!edge.is_valid()) return;
+    const auto* const needed = torch::autograd::get_current_graph_task_exec_info();
+    const auto mine = c10::hip::getCurrentHIPStream(dev.index());
+    std::array<std::shared_ptr<Node>, kJoinable> seen;  // (a node whose last owner this is goes after the lock)
+    Joinables& all = joinables();
+    std::lock_guard<std::mutex> lock(all.mu);
+    for (int i = 0; i < kJoinable; ++i) {
+      const Joinable& j = all.newest[i];
+      if (!j.key || j.key == me.get() || !nodes->count(j.key)) continue;
+      const auto& node = seen[i] = j.node.lock();
+      if (!node || node->num_outputs() == 0 || node->next_edge(0) != edge || node->device() != me->device() ||
+          !node->post_hooks().empty() || !may_take(j.ctx))
+        continue;
+      const auto stream = node->stream();
+      if (!stream || stream->device_index() != mine.device_index() || stream->id() != mine.id()) continue;
+      if (needed && !needed->empty()) {
+        const auto info = needed->find(node.get());
+        if (info == needed->end() || !info->second.needed_) continue;
+      }
+      const auto left = j.ctx->saved_data.find(kLeft);
+      if (left != j.ctx->saved_data.end()) {
+        if (j.ctx->saved_data.at(kLeftPass).toInt() != pass_) continue;
+        partner_.left = left->second.toTensor();
+      }
+      partner_.node = node;
+      partner_.ctx = j.ctx;
+      return;
+    }
+  }
+
+  int pass_;
+  bool seen_apart_;  // the pass records a graph of its gradients, or looks at each
+  Tensor left_;      // what was left with this node
+  Partner partner_;
+};
 
 // The gradient of a loss whose forward pass left it per unit upstream gradient.
 variable_list scaled_gradient(AutogradContext* ctx, const variable_list& grads, float extra_scale, size_t inputs) {
-  const bool records = at::GradMode::is_enabled();
+  Summing summing(ctx);
   at::AutoGradMode no_grad(false);
   variable_list result(inputs);
   const auto saved = ctx->get_saved_variables();
   TORCH_CHECK(saved.size() == 2, "the forward pass was not asked for a gradient of this input");
-  if (!grads[0].defined()) return result;
+  if (!grads[0].defined()) {
+    result[0] = summing.result(Tensor());
+    return result;
+  }
   const Tensor &g = saved[0], &coef = saved[1];
   const at::Device dev = g.device();
   const c10::DeviceGuard guard(dev);
   const Tensor d = upstream(grads[0], dev);
-  const bool may_join = !records && ctx->saved_data.find("shape") == ctx->saved_data.end();
-  const Tensor sum = may_join ? gradient_to_join(g.sizes(), at::kFloat, dev) : Tensor();
-  if (sum.defined()) {
-    check(vamd_scale_rows_add(f32(g), f32(coef), f32(d), extra_scale, g.size(0), g.size(1), f32_out(sum), stream_of(dev)));
-    return result;
-  }
-  const Tensor out = at::empty_like(g);
-  check(vamd_scale_rows(f32(g), f32(coef), f32(d), extra_scale, g.size(0), g.size(1), f32_out(out), stream_of(dev)));
-  result[0] = in_saved_form(ctx, out);
-  if (may_join) gradient_returned(out);
+  const Tensor sum = in_kernel_form(ctx) ? summing.target(g.sizes(), at::kFloat, dev) : Tensor();
+  const Tensor out = sum.defined() ? sum : at::empty_like(g);
+  check((sum.defined() ? vamd_scale_rows_add : vamd_scale_rows)(f32(g), f32(coef), f32(d), extra_scale, g.size(0),
+                                                                g.size(1), f32_out(out), stream_of(dev)));
+  result[0] = summing.result(in_saved_form(ctx, out));
   return result;
 }
 
 // ---- log-probs and entropies of materialised logits ----------------------------------------------------------
-// Nodes in C++ because two of them on the same logits sum their gradients (a gradient that Python has seen is never autograd's
-// alone), and because up to a few hundred rows the host is what a call waits for.
+// Nodes in C++ because two of them on the same logits sum their gradients, and because up to a few hundred rows the host is what
+// a call waits for.
 struct Rows {
   Tensor t;     // [rows, vocab], unit stride along the vocabulary
   int64_t ld;   // row pitch
@@ -332,24 +399,21 @@ RowStats row_stats(const Tensor& logits, const Rows& r, const Tensor& labels, at
   return {value, lse, mean_z};
 }
 
-// The gradient of the logits in `shape`, or an undefined tensor where it went into the other node's.
+// What a node hands back for the logits, in `shape`.
 Tensor row_gradient(const Rows& r, const Tensor& labels, const Tensor& lse, const Tensor& mean_z, const Tensor& upstream,
-                    at::IntArrayRef shape, bool in_place, bool may_join) {
+                    at::IntArrayRef shape, bool in_place, Summing& summing) {
   const at::Device dev = r.t.device();
   const c10::DeviceGuard guard(dev);
   const at::ScalarType type = upstream.scalar_type() == r.t.scalar_type() ? upstream.scalar_type() : at::kFloat;
   const Tensor g = upstream.detach().reshape({-1}).to(dev, type).contiguous();
   const bool entropy = mean_z.defined();
-  const Tensor sum = may_join && !in_place ? gradient_to_join(shape, r.t.scalar_type(), dev) : Tensor();
+  const Tensor sum = in_place ? Tensor() : summing.target(shape, r.t.scalar_type(), dev);
   const Tensor out = in_place ? r.t : sum.defined() ? sum : at::empty(shape, r.t.options());
   check((sum.defined() ? vamd_row_softmax_backward_add : vamd_row_softmax_backward_as)(
       r.data(), r.type, r.n(), r.vocab(), r.ld, entropy ? nullptr : labels.const_data_ptr<int64_t>(), f32(lse), f32(mean_z),
       entropy ? nullptr : g.const_data_ptr(), entropy ? g.const_data_ptr() : nullptr, row_type(type), out.mutable_data_ptr(),
       in_place ? r.ld : r.vocab(), stream_of(dev)));
-  if (sum.defined()) return Tensor();
-  if (in_place) return out.view(shape);
-  if (may_join) gradient_returned(out);
-  return out;
+  return summing.result(in_place ? out.view(shape) : out);
 }
 
 class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
@@ -359,7 +423,7 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
     const Rows r = logit_rows(logits);
     const RowStats s = row_stats(logits, r, lab, logits.scalar_type(), true);
     ctx->save_for_backward({r.t, lab, s.lse});
-    ctx->saved_data["shape"] = logits.sizes().vec();
+    ctx->saved_data["logits_shape"] = logits.sizes().vec();
     // writing the gradient over the logits needs the rows to be the caller's storage, and never overwrites a parameter
     ctx->saved_data["in_place"] = inplace_backward && r.data() == logits.const_data_ptr() && logits.is_contiguous() &&
                                   !(logits.is_leaf() && logits.requires_grad());
@@ -367,6 +431,7 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const bool records = at::GradMode::is_enabled();
+    Summing summing(ctx);
     Tensor d;
     {
       at::AutoGradMode no_grad(false);
@@ -380,8 +445,8 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
                     "pass and cannot run a second one; pass inplace_backward=False to keep the logits");
         ctx->saved_data["logits_overwritten"] = true;
       }
-      const auto shape = ctx->saved_data["shape"].toIntVector();
-      d = row_gradient(saved_rows(saved[0], shape), saved[1], saved[2], Tensor(), grads[0], shape, in_place, !records);
+      const auto shape = ctx->saved_data["logits_shape"].toIntVector();
+      d = row_gradient(saved_rows(saved[0], shape), saved[1], saved[2], Tensor(), grads[0], shape, in_place, summing);
     }
     if (records)  // the gradient is no function of its own to differentiate
       d = torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable",
@@ -396,22 +461,26 @@ class RowEntropy : public torch::autograd::Function<RowEntropy> {
     const Rows r = logit_rows(logits);
     const RowStats s = row_stats(logits, r, Tensor(), fp32_output ? at::kFloat : logits.scalar_type(), true);
     ctx->save_for_backward({r.t, s.lse, s.mean_z});
-    ctx->saved_data["shape"] = logits.sizes().vec();
+    ctx->saved_data["logits_shape"] = logits.sizes().vec();
     return s.value;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    const bool records = at::GradMode::is_enabled();
+    Summing summing(ctx);
     at::AutoGradMode no_grad(false);
     const auto saved = ctx->get_saved_variables();
-    const auto shape = ctx->saved_data["shape"].toIntVector();
-    return {row_gradient(saved_rows(saved[0], shape), Tensor(), saved[1], saved[2], grads[0], shape, false, !records),
+    const auto shape = ctx->saved_data["logits_shape"].toIntVector();
+    return {row_gradient(saved_rows(saved[0], shape), Tensor(), saved[1], saved[2], grads[0], shape, false, summing),
             Tensor()};
   }
 };
 
 Tensor logprobs_from_logits(const Tensor& logits, const Tensor& labels, bool inplace_backward) {
   refuse_tangents("logprobs_from_logits", {&logits});
-  if (wants_gradient(logits)) return RowLogprobs::apply(logits, labels, inplace_backward);
+  if (wants_gradient(logits)) {
+    const Tensor logprobs = RowLogprobs::apply(logits, labels, inplace_backward);
+    joinable<RowLogprobs>(logprobs);
+    return logprobs;
+  }
   at::AutoGradMode no_grad(false);
   const Tensor lab = label_rows(labels, logits);
   return row_stats(logits, logit_rows(logits), lab, logits.scalar_type(), false).value;
@@ -419,7 +488,11 @@ Tensor logprobs_from_logits(const Tensor& logits, const Tensor& labels, bool inp
 
 Tensor entropy_from_logits(const Tensor& logits, bool fp32_output) {
   refuse_tangents("entropy_from_logits", {&logits});
-  if (wants_gradient(logits)) return RowEntropy::apply(logits, fp32_output);
+  if (wants_gradient(logits)) {
+    const Tensor entropy = RowEntropy::apply(logits, fp32_output);
+    joinable<RowEntropy>(entropy);
+    return entropy;
+  }
   at::AutoGradMode no_grad(false);
   return row_stats(logits, logit_rows(logits), Tensor(), fp32_output ? at::kFloat : logits.scalar_type(), false).value;
 }
@@ -487,6 +560,7 @@ std::pair<Tensor, Tensor> policy_loss(const Tensor& log_prob, const Tensor& old_
   refuse_tangents("the policy loss", {&log_prob, &old_log_prob, &advantages, &mask, &weights});
   if (wants_gradient(log_prob)) {
     const auto r = PolicyLoss::apply(log_prob, old_log_prob, advantages, mask, is_weights, a);
+    joinable<PolicyLoss>(r[0]);
     return {r[0], r[1]};
   }
   const LossResult r = policy_forward(log_prob, old_log_prob, advantages, mask, is_weights, a, false);
@@ -535,6 +609,7 @@ std::pair<Tensor, Tensor> value_loss(const Tensor& vpreds, const Tensor& returns
   refuse_tangents("the value loss", {&vpreds, &returns, &values, &mask});
   if (wants_gradient(vpreds)) {
     const auto r = ValueLoss::apply(vpreds, returns, values, mask, clip, mode);
+    joinable<ValueLoss>(r[0]);
     return {r[0], r[1].select(0, 1)};
   }
   const LossResult r = value_forward(vpreds, returns, values, mask, clip, mode, false);
@@ -585,7 +660,11 @@ Tensor kl_loss(const Tensor& logprob, const Tensor& ref_logprob, const Tensor& m
                int mode, double dp_size, double bnt, double gbs, double lsf) {
   const KlArgs a{kind, straight_through, {mode, dp_size, bnt, gbs, lsf}};
   refuse_tangents("the KL loss", {&logprob, &ref_logprob, &mask});
-  if (wants_gradient(logprob) || wants_gradient(ref_logprob)) return KlLoss::apply(logprob, ref_logprob, mask, a);
+  if (wants_gradient(logprob) || wants_gradient(ref_logprob)) {
+    const Tensor loss = KlLoss::apply(logprob, ref_logprob, mask, a);
+    joinable<KlLoss>(loss);
+    return loss;
+  }
   return kl_forward(logprob, ref_logprob, mask, a, false).loss;
 }
 

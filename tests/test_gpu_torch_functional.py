@@ -726,9 +726,25 @@ def test_row_functions_traced_and_transformed(dev):
         with pytest.raises(RuntimeError):
             torch.vmap(fn)(zd[None])
     x = zd.clone().requires_grad_()
-    d, = torch.autograd.grad(F.logprobs_from_logits(x, lab, inplace_backward=False).sum(), x, create_graph=True)
+    # (squared: where the upstream gradient is a constant the gradient is one too, which the next test is about)
+    d, = torch.autograd.grad((F.logprobs_from_logits(x, lab, inplace_backward=False) ** 2).sum(), x, create_graph=True)
     with pytest.raises(RuntimeError, match="once_differentiable"):
         d.sum().backward()
+
+
+def test_gradients_of_a_recorded_pass_without_a_second_derivative(dev):
+    """A recorded pass whose upstream gradient is a constant leaves a gradient to which others may be added and differentiated."""
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(5, 300, torch.float32, seed=8)
+    lab = labels.to(dev)
+    x = z.to(dev).requires_grad_()
+    want, = torch.autograd.grad(F.logprobs_from_logits(x, lab, inplace_backward=False).sum(), x)
+    d, = torch.autograd.grad(F.logprobs_from_logits(x, lab, inplace_backward=False).sum(), x, create_graph=True)
+    assert torch.equal(d, want) and not d.requires_grad
+    twice, = torch.autograd.grad((d + x * x).sum(), x)
+    assert torch.equal(twice, 2 * x.detach())
+    F.logprobs_from_logits(x, lab, inplace_backward=False).sum().backward(create_graph=True)
+    assert not x.grad.requires_grad
 
 
 def test_row_gradient_is_not_added_to_the_logits(dev):

@@ -448,7 +448,7 @@ class RowLogprobs : public torch::autograd::Function<RowLogprobs> {
       const auto shape = ctx->saved_data["logits_shape"].toIntVector();
       d = row_gradient(saved_rows(saved[0], shape), saved[1], saved[2], Tensor(), grads[0], shape, in_place, summing);
     }
-    if (records)  // the gradient is no function of its own to differentiate
+    if (records && grads[0].requires_grad())  // the gradient is no function of its own to differentiate
       d = torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable",
                                         1)({d.detach().requires_grad_()})[0];
     return {d, Tensor(), Tensor()};

@@ -747,6 +747,17 @@ def test_gradients_of_a_recorded_pass_without_a_second_derivative(dev):
     assert not x.grad.requires_grad
 
 
+def test_labels_that_alone_require_a_gradient(dev):
+    """The log-probs belong to a graph, which can be differentiated and has no gradient for the labels."""
+    import verl_amd.utils.torch_functional as F
+    z, labels = _logits(5, 300, torch.float32, seed=9)
+    lab = labels.to(dev).float().requires_grad_()
+    lp = F.logprobs_from_logits(z.to(dev), lab, inplace_backward=False)
+    assert lp.requires_grad
+    lp.sum().backward()
+    assert lab.grad is None
+
+
 def test_row_gradient_is_not_added_to_the_logits(dev):
     from verl_amd import _cabi
     z = torch.randn(2, 64, device=dev)

@@ -476,7 +476,8 @@ class RowEntropy : public torch::autograd::Function<RowEntropy> {
 
 Tensor logprobs_from_logits(const Tensor& logits, const Tensor& labels, bool inplace_backward) {
   refuse_tangents("logprobs_from_logits", {&logits});
-  if (wants_gradient(logits)) {
+  // (labels of a floating type may require a gradient, and get none)
+  if (wants_gradient(logits) || wants_gradient(labels)) {
     const Tensor logprobs = RowLogprobs::apply(logits, labels, inplace_backward);
     joinable<RowLogprobs>(logprobs);
     return logprobs;

@@ -7,6 +7,7 @@ on the same values in fp64).  bf16 / fp16 logits -> the kernels compute in fp32 
 so the result must lie within half a unit in the last place of that dtype (2**-8 resp. 2**-11 relative) of the
 fp64 value, plus the fp32 slack.
 """
+import gc
 import math
 
 import pytest
@@ -523,6 +524,7 @@ def test_summed_gradients_need_no_second_buffer(dev):
     z, labels = _logits(64, 65536, torch.float32, seed=1)
     zd, lab = z.to(dev).requires_grad_(), labels.to(dev)
     loss = _summed(F, zd, lab, ("lp", "ent"))
+    gc.collect()                # what earlier tests left in cycles is not freed in between
     torch.cuda.reset_peak_memory_stats(dev)
     before = torch.cuda.memory_allocated(dev)
     got, = torch.autograd.grad(loss, zd)

@@ -893,7 +893,8 @@ def test_logits_are_kept_where_they_are_a_small_part_of_the_free_memory(dev, mon
         assert (held()[1] >= 4 * n * v) is kept
 
 
-@pytest.mark.parametrize("n,h,v", [(1, 128, 8), (65, 384, 257), (64, 128, 250), (200, 640, 300), (300, 256, 1031), (130, 896, 512)])
+@pytest.mark.parametrize("n,h,v", [(1, 128, 8), (65, 384, 257), (64, 128, 250), (200, 640, 300), (300, 256, 1031), (130, 896, 512),
+                                   (65, 1024, 102400), (130, 1024, 102401)])   # 200 MB, and the first row past the caches
 @pytest.mark.parametrize("offset", [0, 4])          # elements: d_weight on an 8-byte boundary only
 def test_weight_gradient_stored_in_whole_lines(dev, n, h, v, offset):
     """Stored in bf16 it is the same bits as added to zeros, at ragged vocabularies and hidden sizes that end in half a

@@ -1242,6 +1242,17 @@ struct LineExchange {
   }
 };
 
+// STREAM: a d_weight stored in bf16 goes past the caches.  One that does not fit the memory-side cache is written back while
+// whatever comes next reads; of one that fits, the next reader (accumulation, norm, optimizer) finds it there.  The line lies at
+// the 200 MB that the cache holds beside other data (kCachedWeightBytes).  Forward and backward and then a norm of d_weight, after a
+// pass that fills the cache with other data, plain and STREAM, us: 300 x 1024 x 32000 (66 MB) 155 and 177, 300 x 1024 x 64000
+// (131 MB) 282 and 297, 300 x 1024 x 96000 (197 MB) 407 and 411, 64 tokens 277 and 297; 300 x 1024 x 128000 (262 MB) 543 and 524,
+// 64 x 2048 x 64000 398 and 372, 300 x 896 x 151936 (272 MB) 566 and 554, 128 tokens 472 and 439, 2048 tokens 2018 and 2012,
+// 128 x 3584 x 152064 (1.09 GB) 1335 and 1236; with an addition to another gradient in the norm's place 156 and 175, 274 and 287,
+// 399 and 400, 292 and 285; 534 and 512, 386 and 367, 556 and 544, 460 and 430, 2014 and 2004, 1379 and 1277.  Without a reader
+// 300 x 1024 x 32000 to 96000 within 2 %, the larger ones 324 and 308 (128 x 896), 807 and 732 (128 x 3584), 1346 and 1331 (300);
+// only 64 x 3584 x 152064 loses (682 and 695, and gains with either reader).
+template <bool STREAM>
 struct DWeightEpi {
   LanePos p;
   const GemmOutArgs* a;
@@ -1259,14 +1270,13 @@ struct DWeightEpi {
           line.run(acc, mb, nb, v);
           const int col = c0 + p.wc * 128 + mb * 64 + 8 * line.rd_chunk;  // c_valid % 128 == 0: 8 columns are all in or all out
           const int row0 = r0 + p.wr * (kNB * kBlk) + nb * 32 + line.rd_row;
-          // Non-temporal: a large d_weight left behind in the memory-side cache is written back while the next pass reads the
-          // weight (128 x 3584 x 152064 forward and backward 858 -> 817 us, 300 x 896 x 151936 424 -> 407; the forward pass
-          // behind a d_weight of 1.09 GB 260 -> 205; sizes from 777 tokens on and small heads the same within 1 %).
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (col < A.c_valid && row0 + 8 * i < A.r_valid)
-              __builtin_nontemporal_store(
-                  v[i], reinterpret_cast<u32x4_at8*>(A.out + (int64_t)(row0 + 8 * i) * A.ld_out + col));
+            if (col < A.c_valid && row0 + 8 * i < A.r_valid) {
+              auto* const dst = reinterpret_cast<u32x4_at8*>(A.out + (int64_t)(row0 + 8 * i) * A.ld_out + col);
+              if constexpr (STREAM) __builtin_nontemporal_store(v[i], dst);
+              else *dst = v[i];
+            }
         }
       return;
     }
@@ -1306,6 +1316,7 @@ struct DWeightEpi {
 
 // Both gradient GEMMs of one vocabulary chunk in a single launch: a workgroup first walks its share of the d_hidden
 // units, then its share of the d_weight tiles, shared out by plan_gradients() so that all workgroups finish together.
+template <bool STREAM>
 __global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, GemmOutArgs gw, GradPlan plan) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int nwg = gridDim.x;
@@ -1323,7 +1334,7 @@ __global__ __launch_bounds__(kThreads) void lce_dgrad_kernel(GemmOutArgs gh, Gem
   __syncthreads();
   {
     LateStartSched sched{TileGrid{gw.r_tiles, gw.c_tiles}, gw.k_slabs, nwg, wg, plan.extra, plan.late};
-    DWeightEpi epi;
+    DWeightEpi<STREAM> epi;
     epi.p = pos;
     epi.a = &gw;
     epi.ex.init(lds + kLdsBytes, pos);
@@ -1480,7 +1491,8 @@ static int ensure_lds_attributes() {
   if ((s = allow_big_lds(lce_forward_few_kernel<true, true>, kFewCacheLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_recompute_kernel, kLdsBytes + kRecomputeExtraLds)) != VAMD_OK) return s;
   if ((s = allow_big_lds(lce_dhidden_few_kernel, kFewLds)) != VAMD_OK) return s;
-  if ((s = allow_big_lds(lce_dgrad_kernel, kLdsBytes + kGradStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_dgrad_kernel<false>, kLdsBytes + kGradStageBytes)) != VAMD_OK) return s;
+  if ((s = allow_big_lds(lce_dgrad_kernel<true>, kLdsBytes + kGradStageBytes)) != VAMD_OK) return s;
   done[dev] = true;
   return VAMD_OK;
 }
@@ -2050,7 +2062,9 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
       const GradPlan plan = plan_gradients(n_tokens, hidden_size, cols, gh.r_tiles > 0, want_dw, workgroups, few ? 1 : pieces);
       {
         ScopedTiming tm(kTagDGrad, s);
-        hipLaunchKernelGGL(lce_dgrad_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes + kGradStageBytes, s, gh, gw, plan);
+        const bool stream_dw = vocab * hidden_size * 2 > kCachedWeightBytes;
+        hipLaunchKernelGGL(stream_dw ? lce_dgrad_kernel<true> : lce_dgrad_kernel<false>, dim3(workgroups), dim3(kThreads),
+                           kLdsBytes + kGradStageBytes, s, gh, gw, plan);
       }
       VAMD_LAUNCH_CHECK();
     }

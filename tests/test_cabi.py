@@ -3,6 +3,7 @@ include/verl_amd.h declares, answers its size queries, and the host wrappers ref
 without a GPU instead of falling back."""
 import ctypes
 import os
+import pathlib
 import re
 
 import numpy as np
@@ -37,6 +38,17 @@ def test_every_declared_symbol_is_exported_and_bound(lib):
     assert lib.vamd_abi_version() == _cabi.ABI_VERSION
     header = open(os.path.join(os.path.dirname(__file__), "..", "include", "verl_amd.h")).read()
     assert f"#define VAMD_ABI_VERSION {_cabi.ABI_VERSION}\n" in header
+
+
+def test_documents_state_the_version_of_the_header():
+    """A binding is written from them: the version, and that each names the two calls that add to a gradient."""
+    root = pathlib.Path(ROOT)
+    stated = [(p.name, int(n)) for p in root.glob("*.md")
+              for n in re.findall(r"`VAMD_ABI_VERSION` (?:=|is) (\d+)", p.read_text())]
+    assert stated and all(n == _cabi.ABI_VERSION for _, n in stated), stated
+    for name in {doc for doc, _ in stated}:
+        text = (root / name).read_text()
+        assert "vamd_row_softmax_backward_add" in text and "vamd_scale_rows_add" in text, name
 
 
 def test_stale_binaries_are_told_to_be_rebuilt(monkeypatch):

@@ -964,12 +964,14 @@ def test_token_and_column_tiles_that_are_nearly_empty(dev, n, h, v, cached):
     """Wavefronts without rows and columns that are not fetched, against the fp32 ground truth with the bound for d_logits staged
     in bf16."""
     from verl_amd.utils.kernel import linear_cross_entropy as K
+    if cached:
+        v -= v % 8          # kept logits need it: 33000 is still ragged in tiles of 256
     hidden, weight, labels = _make(n, h, v, seed=n + v, dist="normal")
     g_lp = torch.randn(n, generator=torch.Generator().manual_seed(n))
     hd, wd, ld, gd = (t.to(dev) for t in (hidden, weight, labels, g_lp))
-    cache = torch.full((n, v), float("nan"), device=dev) if cached and v % 8 == 0 else None
+    cache = torch.full((n, v), float("nan"), device=dev) if cached else None
     lp, ent, lse, mz = K.efficient_entropy_forward(hd, wd, ld, 0, 0.9, logits_cache=cache)
-    if cache is not None:
+    if cached:
         assert bool(torch.isfinite(cache).all())
     dh, dw = K.efficient_entropy_backward(gd, None, hd, wd, ld, lse, mz, 0, 0.9, logits_cache=cache)
     want_lp, want_ent, want_dh, want_dw, e_dh, e_dw = _oracle_with_scale(hidden, weight, labels, 0.9, g_lp, torch.zeros(n), dev)

@@ -607,6 +607,12 @@ def test_a_sum_takes_one_allocation_and_a_hook_two(dev, kind):
             before = count()
             torch.autograd.grad(total, x, retain_graph=retain)
             assert count() - before == (1 if hooked is None else 2)
+    # nodes that are no longer among the newest are not looked for
+    total, want = first(x).sum() + second(x).sum(), torch.autograd.grad(first(x).sum() + second(x).sum(), x)[0]
+    newer = [first(x) for _ in range(20)]
+    before = count()
+    got, = torch.autograd.grad(total, x)
+    assert count() - before == 2 and len(newer) == 20 and torch.equal(got, want)
 
 
 class _Nothing(torch.autograd.Function):

@@ -192,44 +192,42 @@ using torch::autograd::Edge;
 using torch::autograd::Node;
 
 // The newest nodes that can add to a gradient left with them, of all threads: where a running node looks for another one.
-// All that counts is asked of the node itself; a node that is no longer among them is not found.
-constexpr int kJoinable = 32;
-struct Joinable {
-  Node* key = nullptr;  // compared, never followed
-  std::weak_ptr<Node> node;
-  AutogradContext* ctx = nullptr;  // lives in the node
-};
+// All that counts is asked of the node itself; a node that is no longer among them is not found.  In vectors, because a
+// backward pass finds them in another core's cache: where there is nothing to sum it reads four lines of them (asking 32 nodes
+// one by one whether they belong to the pass cost 3 us of the 165 us of a call with two losses).
+constexpr int kJoinable = 16;
 struct Joinables {
-  std::mutex mu;  // also guards kRan, kLeft and kLeftPass of every node's saved data
-  std::array<Joinable, kJoinable> newest;
+  std::mutex mu;  // also guards kLeft and kLeftPass of every node's saved data
   int next = 0;
+  std::array<Node*, kJoinable> key{}, receiver{};  // compared, never followed
+  std::array<int, kJoinable> ran{};                // the newest pass in which the node has run
+  std::array<std::weak_ptr<Node>, kJoinable> node;
+  std::array<AutogradContext*, kJoinable> ctx{};  // lives in the node
 };
 Joinables& joinables() {
   static auto* j = new Joinables;  // never destroyed: at exit threads of autograd may still run
   return *j;
 }
-constexpr const char *kRan = "ran", *kLeft = "left", *kLeftPass = "left_pass";
+constexpr const char *kLeft = "left", *kLeftPass = "left_pass";
 
 // The node of F that made `output` can add to a gradient left with it, unless its own takes another form or another's place.
 template <class F>
 void joinable(const Tensor& output) {
   const auto& node = output.grad_fn();
   auto* const made = dynamic_cast<torch::autograd::CppNode<F>*>(node.get());
-  if (!made || !in_kernel_form(&made->ctx_)) return;
+  if (!made || made->num_outputs() == 0 || !made->next_edge(0).is_valid() || !in_kernel_form(&made->ctx_)) return;
   const auto in_place = made->ctx_.saved_data.find("in_place");
   if (in_place != made->ctx_.saved_data.end() && in_place->second.toBool()) return;
   Joinables& all = joinables();
   std::lock_guard<std::mutex> lock(all.mu);
-  all.newest[all.next] = {node.get(), node, &made->ctx_};
-  all.next = (all.next + 1) % kJoinable;
+  const int i = all.next;
+  all.next = (i + 1) % kJoinable;
+  all.key[i] = made;
+  all.receiver[i] = made->next_edge(0).function.get();
+  all.ran[i] = -1;
+  all.node[i] = node;
+  all.ctx[i] = &made->ctx_;
 }
-
-// The other node with which the running one may sum up, if there is one, and what was left with that already.
-struct Partner {
-  std::shared_ptr<Node> node;
-  AutogradContext* ctx = nullptr;
-  Tensor left;
-};
 
 // One node's part in the sum, from the start of its backward function.
 class Summing {
@@ -238,86 +236,87 @@ class Summing {
       : pass_(torch::autograd::get_current_graph_task_id()),
         seen_apart_(at::GradMode::is_enabled() || torch::autograd::AnomalyMode::is_enabled()) {
     if (pass_ < 0) return;
-    std::lock_guard<std::mutex> lock(joinables().mu);
+    me_ = torch::autograd::get_current_node();
+    Joinables& all = joinables();
+    std::lock_guard<std::mutex> lock(all.mu);
+    for (int i = 0; i < kJoinable; ++i)
+      if (all.key[i] == me_.get() && all.ran[i] < pass_) all.ran[i] = pass_;
     auto& data = ctx->saved_data;
-    const auto ran = data.find(kRan);
-    if (ran == data.end() || ran->second.toInt() < pass_) data[kRan] = (int64_t)pass_;
     const auto left = data.find(kLeft);
     if (left == data.end() || data[kLeftPass].toInt() != pass_) return;
     left_ = left->second.toTensor();
     data.erase(left);
   }
 
-  // Looks for a partner.  Where the node's gradient of the form given goes: a tensor to which it adds its own, or an
+  // Looks for the other node.  Where this node's gradient of the form given goes: a tensor to which it adds its own, or an
   // undefined tensor, and then it makes one.
   Tensor target(at::IntArrayRef shape, at::ScalarType type, const at::Device& dev) {
-    find_partner(dev);
-    Tensor& sum = left_.defined() ? left_ : partner_.left;
+    find_other(dev);
+    const Tensor& sum = left_.defined() ? left_ : left_there_;
     if (sum.defined() && sum.sizes() == shape && sum.scalar_type() == type && sum.device() == dev) return sum;
     return Tensor();
   }
 
-  // What the node hands back for `grad`, which holds its gradient and that of target(), if one was defined.
+  // What the node hands back for `grad`, which holds its gradient and what was in target().
   Tensor result(const Tensor& grad) {
     Tensor sum = grad;
     if (left_.defined() && !(sum.defined() && sum.is_same(left_))) sum = sum.defined() ? sum.add(left_) : left_;
-    if (!partner_.node || !sum.defined()) return sum;
-    if (partner_.left.defined()) return sum.is_same(partner_.left) ? Tensor() : sum;
+    if (!other_ || !sum.defined()) return sum;
+    if (left_there_.defined()) return sum.is_same(left_there_) ? Tensor() : sum;
     if (!sum.is_cuda() || !sum.is_contiguous()) return sum;
-    std::lock_guard<std::mutex> lock(joinables().mu);
-    if (!may_take(partner_.ctx) || partner_.ctx->saved_data.count(kLeft)) return sum;
-    partner_.ctx->saved_data[kLeftPass] = (int64_t)pass_;
-    partner_.ctx->saved_data[kLeft] = sum;
+    Joinables& all = joinables();
+    std::lock_guard<std::mutex> lock(all.mu);
+    auto& data = all.ctx[slot_]->saved_data;
+    if (all.key[slot_] != other_.get() || all.ran[slot_] >= pass_ || data.count(kLeft)) return sum;
+    data[kLeftPass] = (int64_t)pass_;
+    data[kLeft] = sum;
     return Tensor();
   }
 
  private:
-  bool may_take(AutogradContext* ctx) const {
-    const auto& data = ctx->saved_data;
-    const auto ran = data.find(kRan);
-    return ran == data.end() || ran->second.toInt() < pass_;
-  }
-
-  void find_partner(const at::Device& dev) {
-    const auto* const nodes = torch::autograd::get_current_graph_task_nodes_in_graph();
-    if (pass_ < 0 || !nodes || seen_apart_) return;
-    const auto me = torch::autograd::get_current_node();
-    if (!me || me->num_outputs() == 0 || !me->post_hooks().empty()) return;
-    const Edge edge = me->next_edge(0);
+  void find_other(const at::Device& dev) {
+    if (pass_ < 0 || seen_apart_ || !me_ || me_->num_outputs() == 0 || !me_->post_hooks().empty()) return;
+    const Edge& edge = me_->next_edge(0);
     if (!edge.is_valid()) return;
-    const auto* const needed = torch::autograd::get_current_graph_task_exec_info();
-    const auto mine = c10::hip::getCurrentHIPStream(dev.index());
     std::array<std::shared_ptr<Node>, kJoinable> seen;  // (a node whose last owner this is goes after the lock)
     Joinables& all = joinables();
     std::lock_guard<std::mutex> lock(all.mu);
     for (int i = 0; i < kJoinable; ++i) {
-      const Joinable& j = all.newest[i];
-      if (!j.key || j.key == me.get() || !nodes->count(j.key)) continue;
-      const auto& node = seen[i] = j.node.lock();
-      if (!node || node->num_outputs() == 0 || node->next_edge(0) != edge || node->device() != me->device() ||
-          !node->post_hooks().empty() || !may_take(j.ctx))
-        continue;
-      const auto stream = node->stream();
-      if (!stream || stream->device_index() != mine.device_index() || stream->id() != mine.id()) continue;
-      if (needed && !needed->empty()) {
-        const auto info = needed->find(node.get());
-        if (info == needed->end() || !info->second.needed_) continue;
+      if (all.receiver[i] != edge.function.get() || all.key[i] == me_.get() || all.ran[i] >= pass_) continue;
+      const auto& node = seen[i] = all.node[i].lock();
+      if (!node || !runs_later(*node, edge, dev)) continue;
+      const auto& data = all.ctx[i]->saved_data;
+      const auto left = data.find(kLeft);
+      if (left != data.end()) {
+        if (data.at(kLeftPass).toInt() != pass_) continue;
+        left_there_ = left->second.toTensor();
       }
-      const auto left = j.ctx->saved_data.find(kLeft);
-      if (left != j.ctx->saved_data.end()) {
-        if (j.ctx->saved_data.at(kLeftPass).toInt() != pass_) continue;
-        partner_.left = left->second.toTensor();
-      }
-      partner_.node = node;
-      partner_.ctx = j.ctx;
+      other_ = node;
+      slot_ = i;
       return;
     }
   }
 
+  // Whether the pass at hand runs `node`, which has not run in it, after this one, as the comment above asks.
+  bool runs_later(Node& node, const Edge& edge, const at::Device& dev) const {
+    const auto* const nodes = torch::autograd::get_current_graph_task_nodes_in_graph();
+    if (!nodes || !nodes->count(&node) || node.num_outputs() == 0 || node.next_edge(0) != edge ||
+        node.device() != me_->device() || !node.post_hooks().empty())
+      return false;
+    const auto stream = node.stream();
+    const auto mine = c10::hip::getCurrentHIPStream(dev.index());
+    if (!stream || stream->device_index() != mine.device_index() || stream->id() != mine.id()) return false;
+    const auto* const needed = torch::autograd::get_current_graph_task_exec_info();
+    if (!needed || needed->empty()) return true;
+    const auto info = needed->find(&node);
+    return info != needed->end() && info->second.needed_;
+  }
+
   int pass_;
   bool seen_apart_;  // the pass records a graph of its gradients, or looks at each
-  Tensor left_;      // what was left with this node
-  Partner partner_;
+  std::shared_ptr<Node> me_, other_;
+  int slot_ = 0;     // the other node's place among the joinable ones
+  Tensor left_, left_there_;  // what was left with this node, and with the other one
 };
 
 // The gradient of a loss whose forward pass left it per unit upstream gradient.

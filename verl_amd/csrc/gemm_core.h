@@ -203,10 +203,11 @@ struct SlabDma {
   unsigned step;      // scalar byte offset between consecutive loads
   unsigned lds_wave;  // byte offset of this wavefront's first block inside the slab
   unsigned col;       // kmajor: the column of the tile that the lane fetches
-  unsigned voff_tile;  // kmajor: voff, or past every buffer's end
+  unsigned voff_tile;  // kmajor: voff, or past the buffer's end
 
   // A kmajor tile's columns past the operand's would be the next row's first ones: they are not fetched and read as zero, which
-  // the matrix cores multiply for a good deal less energy.  On a board at its power limit that is time: hidden size 896 (the last
+  // the matrix cores multiply for a good deal less energy.  (Not in operands of more than 3.75 GB, whose bounds the offset does not
+  // pass: there other values of the operand are read.  Nothing depends on the zeros, products of these columns are never stored.)  On a board at its power limit that is time: hidden size 896 (the last
   // of four column tiles is half empty), forward and backward over 777 tokens x 151936 852 -> 829 us, 2048 tokens 1939 -> 1911.
   __device__ __forceinline__ void set_tile(const Operand& op, int x0) {
     if constexpr (KMAJOR) voff_tile = (int)col + x0 < op.x_extent ? voff : 0xf0000000u;

@@ -580,10 +580,18 @@ __global__ __launch_bounds__(kThreads) void lce_forward_kernel(FwdArgs a) {
 constexpr int kFewTokens = 128;
 // The few-token kernels read every piece of the weight in one workgroup, and the backward pass reads it again.  A weight that about
 // fits the 256 MB memory-side cache is read with plain loads; of a larger one the workgroups on the first 200 MB, and the others
-// with the non-temporal hint, which leaves those there.  Everything with plain loads, everything with the hint and so, us: forward
-// pass over 64 tokens at 151936 columns, hidden size 1536 (467 MB) 98, 92 and 88, 2048 138, 130 and 111, 3584 x 152064 194, 187
-// and 183; with the backward pass 1536 313, 310 and 293, 2048 392, 407 and 363, 2560 483, 474 and 459, 3584 621, 618 and 608,
-// 128 tokens 716, 690 and 675.  896 (272 MB) 203, 211 and with 200 MB kept 208.
+// with the non-temporal hint, which leaves those there for the backward pass.  Everything with plain loads, everything with the hint
+// and so, us, 64 tokens:
+//                        the cache full of other data, read       the same, written            pass after pass
+//                        forward          and backward            forward        and backward  forward        and backward
+//   1536 x 151936        98   94   95     318  311  304           156   94  144  375  315  355   96   90   84  309  305  290
+//   2048 x 151936       140  134  134     402  408  392           197  135  191  461  413  447  138  130  103  388  402  355
+//   3584 x 152064       191  178  178     619  609  605           251  179  260  681  629  696  191  179  177  617  607  593
+//   4096 x 128256       191  166  167     586  557  550           243  167  249  644  560  632  187  162  157  570  551  538
+//   896 (272 MB, plain)  61   59   61     210  208  208           113   60  113  264  213  261   53   53   53  201  201  200
+// (runs differ by 1 to 2 %).  The last two columns find the weight of the pass before in the cache, which no update does.  Where
+// the cache is full of what was just written, as behind a trunk's forward pass, plain loads wait for that to be written back,
+// and everything with the hint is quicker at every size: what the rule gains is the backward pass on a cache without such data.
 constexpr int64_t kFittingWeightBytes = 320ll << 20, kCachedWeightBytes = 200ll << 20;
 constexpr int kFewStageBytes = (kFewTokens + kTile) * kBK * 2;
 constexpr int kFewStages = 3;
@@ -595,7 +603,7 @@ constexpr int kFewLoadsR = kFewTokens * 8 / kThreads;  // transfers per lane of 
 static_assert(kFewLoadsR + kLoads == 6, "the s_waitcnt vmcnt(6) of lce_forward_few_kernel counts the transfers of one slab");
 static_assert(kFewTokens == kFewWavesR * kNB * kBlk, "a wavefront owns kNB blocks of tokens");
 
-// the weight's slab of a stage; `stream` is the same for the whole launch
+// the weight's slab of a stage; `stream` is the same for the whole workgroup
 template <bool KMAJOR>
 __device__ __forceinline__ void few_fetch_weight(const SlabDma<KMAJOR>& dma, const SlabSrc& src, unsigned slab_lds, int stream) {
   if (stream) {
@@ -1581,12 +1589,13 @@ static int64_t default_vocab_chunk(int64_t n_tokens, int64_t hidden_size, int64_
 // each summed in fp32 into an accumulator of its own, and the d_weight tiles are shared out so that the workgroups
 // with a piece more get correspondingly fewer tiles.  The number of pieces is the one whose slowest workgroup is
 // quickest, counting in slabs (1.4 us each): an epilogue about 2, and a d_weight tile of up to 3 slabs 7 in all: with every CU
-// storing, its 128 KB take 6 us, and a slab or three more hardly show.  Gradient products over few tokens with 2 for every
-// epilogue, and as it is: 64 x 3584 x 152064 623 -> 490 us, 93 tokens 645 -> 487, 150 tokens 681 -> 588; 128 x 4096 x 128256
-// 600 -> 523.  The 7 and where it ends are a fit, not a law: four slabs stay at 4 + 2 = 6, below three, because 7 is slower
-// there (256 tokens, with 6 and 7, us: 896 192 and 201, 3584 646 and 675, 4096 585 and 613), while 6 for all four is quicker at
-// some sizes and slower at others (192 x 896 177 and 184, 128 x 3584 567 and 593; 64 x 3584 524 and 477, 128 x 4096 555 and
-// 522).  Results in fp32 or added to what is there, which move two to four times the bytes, are counted alike: not measured.
+// storing, its 128 KB take 6 us, and a slab or three more hardly show.  It decides over 129 to 192 tokens (three slabs; up to 128
+// tokens d_hidden has a kernel of its own, but for vocabularies below kFewMinVocab, where it makes no difference, 64 x 1024 x 512
+// 20.1 us and 64 x 2048 x 768 24.4, and for several chunks, which are not measured).  Backward pass with 2 for every epilogue, and as it is, us: 130 x 896 x 151936 193 and 190, 130 x 3584 x 152064 692
+// and 615, 130 x 4096 x 128256 630 and 545; 160 tokens 200 and 198, 712 and 616; 192 tokens 207 and 209, 726 and 637, 643 and
+// 582; 160 x 1024 x 8192 52 both.  The 7 and where it ends are a fit, not a law: four slabs stay at 4 + 2 = 6, below three,
+// because 7 is slower there (256 tokens, with 6 and 7, us: 896 192 and 201, 3584 646 and 675, 4096 585 and 613).  Results in fp32
+// or added to what is there, which move two to four times the bytes, are counted alike: not measured.
 constexpr int kEpilogueSlabs = 2, kFewTileSlabs = 3, kFewTileCost = 7, kMaxSplits = 64, kMinPieceSlabs = 32;
 constexpr int64_t kMaxPieceBytes = 256ll << 20;  // bound on the pieces' accumulators
 static GradPlan plan_gradients(int64_t n_tokens, int64_t hidden_size, int64_t cols, bool want_dh, bool want_dw,
@@ -1952,7 +1961,10 @@ extern "C" int vamd_lce_backward_subset_rows(const void* hidden, const void* wei
   const uint16_t* wgt = static_cast<const uint16_t*>(weight);
   const int h_tiles = (int)ceil_div(hidden_size, kTile);
   // Columns past the hidden size are not fetched (SlabDma::set_tile), except over 129 to 256 tokens, where the products wait for
-  // memory and nothing is gained (200 x 896 x 151936 318 us, without them 323).
+  // memory and tiles that fetch less are no quicker but come out of step with the others.  Backward pass with them and without, us
+  // (runs differ by 0.5 to 1 %): 130 x 896 x 151936 184.5 and 184.6, 160 tokens 195 and 197, 200 tokens 206 and 214, 256 tokens
+  // 226 and 234; 200 x 1664 x 151936 333 and 352, 256 tokens 352 and 368; 256 x 384 x 151936 141 and 146; 200 x 1152 x 65536 121.5
+  // and 122.5; 200 x 640 x 32000 63.9 and 62.9.
   const int col_extent = tok_tiles > 1 || few ? (int)hidden_size : h_tiles * kTile;
 
   for (int ci = 0; ci < n_chunks; ++ci) {

@@ -308,8 +308,9 @@ __global__ __launch_bounds__(kRcThreads) void scale_rows_kernel(const float* __r
 }
 
 // sum[i][t] += g[i][t] * coef[i] * *d_loss * extra, product and sum rounded one after the other as two launches would: 12 bytes a
-// token where scale_rows_kernel and autograd's sum move 20.  The calls of an actor update with GRPO, 1000 x 11999 tokens 300 ->
-// 274 us, 512 x 4096 208 -> 187, 8 x 513 198 -> 176 (a launch, an allocation and an operation of torch's less on the host).
+// token where scale_rows_kernel and autograd's sum move 20.  The calls of an actor update with GRPO, 1000 x 11999 tokens 298 ->
+// 279 us, 512 x 4096 205 -> 195, 8 x 513 193 -> 184 (medians of twelve runs in turn; a launch, an allocation and an operation of
+// torch's less on the host).
 template <bool VEC>
 __global__ __launch_bounds__(kRcThreads) void scale_rows_add_kernel(const float* __restrict__ g,
                                                                     const float* __restrict__ coef,

@@ -83,8 +83,8 @@ __global__ __launch_bounds__(kRcThreads) void rollout_stats_kernel(RcArgs a, con
       // A wavefront skips groups without a valid token; in the others masked tokens (and elements past the end, which read as
       // masked) are selected away, four tokens' arithmetic interleaved.  With a branch per token, and so, the kernel call after call,
       // us: 1024 x 3072 int64 mask 20.0 and 18.7, 744 x 12000 40.2 and 37.4, 64 x 1000 one-byte mask 6.6 and 6.1, 512 x 4096 fp32
-      // mask 12.5 and 11.5; 2048 x 16384 100 both, and 1024 x 3072 behind the other statistics of a step, where its inputs
-      // are in no cache, 20.0 and 19.8: there it waits for memory.
+      // mask 12.5 and 11.5; 2048 x 16384 100 both; 1024 x 3072 among the other statistics of a step 20.0 and 19.1 to 19.8,
+      // which does not show in the step's time.
       const bool some = m[k][0] != 0.f || m[k][1] != 0.f || m[k][2] != 0.f || m[k][3] != 0.f;
       if (__any(some)) {
         float d[4], w[4], ed[4];
